@@ -357,10 +357,9 @@ int scxr_apgm_itstat(const double* obj, int32_t nobj, double obj_scale, const do
 /* ------------------------------------------------ CircularConvolve / FFT --
  * Replaces scico.linop.CircularConvolve (scico/linop/_circconv.py:79-209)
  * for real float32 input of shape (batch..., F0[, F1[, F2]]).  FFT lengths:
- * powers of two up to 4096 (radix-2 in LDS) or any length up to 512
- * (direct DFT).  The plan owns the spectrum (complex64, F-shaped) and a
- * complex workspace of batch * prod(F).  Two power-of-two axes convolve on
- * half spectra (F0 x (F1/2 + 1)) with the Hermitian part of the spectrum,
+ * powers of two up to 4096 or any length up to 512 (mixed radix).  The
+ * plan owns the spectrum (complex64, F-shaped) and a complex workspace of
+ * batch * prod(F).  Two axes of 3 or more convolve on half spectra (F0 x (F1/2 + 1)) with the Hermitian part of the spectrum,
  * which equals real(ifftn(H * fftn(x))) for any H.
  */
 typedef struct scxr_cconv_plan scxr_cconv_plan;

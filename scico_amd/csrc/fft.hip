@@ -4,10 +4,11 @@
 // Layout: data (B, F0, ..., F{d-1}) row-major, B = product of the leading
 // non-transformed axes, d <= 3 transformed axes.  One kernel performs one
 // pass of 1D transforms along one axis; each workgroup loads LPB lines
-// into LDS, transforms them and writes them back:
-//   * power-of-two lengths <= 4096: iterative radix-2 decimation in time
-//     (bit-reversed load, log2(n) butterfly stages);
-//   * other lengths <= 512: direct DFT (out-of-place in LDS).
+// into LDS, transforms them by Stockham stages and writes them back:
+//   * power-of-two lengths <= 4096: radix 16 after one stage of radix 2, 4
+//     or 8;
+//   * other lengths <= 512: mixed radix (Stages): powers of two up to 8, 3,
+//     5 and 7 in registers, a larger prime factor p as p-term sums.
 // Twiddles are float32 roundings of float64 exp(-2 pi i k / n).
 // Inverse passes scale by 1/n, like numpy / jax ifft.
 //
@@ -17,8 +18,8 @@
 // the last one writes the real part.  With d == 1 the single fused pass
 // does both.
 //
-// Real convolution over two power-of-two axes (the deconvolution workload)
-// runs on half spectra instead: rows transformed two real rows per complex
+// Real convolution over two axes (the deconvolution workload) runs on half
+// spectra instead: rows transformed two real rows per complex
 // FFT into (F1/2 + 1)-wide half spectra, one fused pass on those columns
 // with the Hermitian part of H, rows inverted back to real.  At 1024 x 1024
 // each line is one 256-thread workgroup's registers (four values per
@@ -38,10 +39,22 @@ namespace fft {
 
 constexpr int MAX_POW2 = 4096;
 constexpr int MAX_DFT = 512;
-constexpr int LDS_ELEMS = 4096;  // float2 of LDS per workgroup (32 KiB)
+
+// Stockham stages of a length that is no power of two, in order: stage s
+// has radix R[s], with Ns = R[0] ... R[s - 1] before it.  mns / mnb are
+// ceil(2^32 / Ns) and ceil(2^32 / (n / R)): the quotients of the stage's
+// indices (below 2^13, by divisors below 2^10) are exact high words.
+constexpr int MAX_STAGES = 8;
+struct Stages {
+  int count = 0;
+  int twlds = 0;  // 1: a stage takes p-term sums, whose twiddles go to LDS
+  int R[MAX_STAGES] = {};
+  uint32_t mns[MAX_STAGES] = {};
+  uint32_t mnb[MAX_STAGES] = {};
+};
 
 struct Pass {
-  int n, log2n;          // line length, log2 (pow2) or -1 (direct DFT)
+  int n, log2n;          // line length, log2 (pow2) or -1 (mixed radix)
   long long stride;      // element stride along the line
   long long inner;       // lines per outer index (= stride)
   long long lines;       // total lines
@@ -51,7 +64,7 @@ struct Pass {
   int inverse;           // direction of the (non-fused) transform
   int fused;             // forward, multiply by h (conj if conj_h), inverse
   int conj_h;
-  const float2* tw;      // pow2: n/2 twiddles; DFT: n twiddles
+  const float2* tw;      // n twiddles exp(-2 pi i k / n)
   const float2* h;       // fused: spectrum, indexed by k * stride + inner
 };
 
@@ -61,145 +74,6 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
 }
 
 __device__ __forceinline__ float2 conjf2(float2 a) { return make_float2(a.x, -a.y); }
-
-// In-place radix-2 DIT stages on lpb lines of length n stored at buf[l*n + k]
-// (input in bit-reversed order, output in natural order).
-__device__ void dit_stages(float2* buf, int n, int log2n, int lpb, const float2* __restrict__ tw,
-                           bool inv) {
-  const int half_total = lpb * (n >> 1);
-  for (int s = 1; s <= log2n; ++s) {
-    const int half = 1 << (s - 1);
-    const int tstep = n >> s;  // twiddle index step
-    __syncthreads();
-    for (int b = threadIdx.x; b < half_total; b += blockDim.x) {
-      const int l = b >> (log2n - 1);
-      const int j = b & ((n >> 1) - 1);
-      const int pos = j & (half - 1);
-      const int i0 = ((j >> (s - 1)) << s) + pos;
-      float2* line = buf + l * n;
-      float2 w = tw[pos * tstep];
-      if (inv) w = conjf2(w);
-      const float2 a = line[i0];
-      const float2 t = cmul(w, line[i0 + half]);
-      line[i0] = make_float2(__fadd_rn(a.x, t.x), __fadd_rn(a.y, t.y));
-      line[i0 + half] = make_float2(__fsub_rn(a.x, t.x), __fsub_rn(a.y, t.y));
-    }
-  }
-  __syncthreads();
-}
-
-// Direct DFT of lpb lines from src to dst (both [l*n + k]).
-__device__ void direct_dft(const float2* src, float2* dst, int n, int lpb,
-                           const float2* __restrict__ tw, bool inv) {
-  __syncthreads();
-  for (int e = threadIdx.x; e < lpb * n; e += blockDim.x) {
-    const int l = e / n, k = e - l * n;
-    const float2* x = src + l * n;
-    float re = 0.0f, im = 0.0f;
-    int idx = 0;
-    for (int m = 0; m < n; ++m) {
-      float2 w = tw[idx];
-      if (inv) w = conjf2(w);
-      const float2 p = cmul(x[m], w);
-      re = __fadd_rn(re, p.x);
-      im = __fadd_rn(im, p.y);
-      idx += k;
-      if (idx >= n) idx -= n;
-    }
-    dst[e] = make_float2(re, im);
-  }
-  __syncthreads();
-}
-
-__device__ __forceinline__ int bitrev(int k, int log2n) {
-  return static_cast<int>(__builtin_bitreverse32(static_cast<unsigned>(k)) >> (32 - log2n));
-}
-
-__global__ __launch_bounds__(256) void pass_kernel(const void* __restrict__ in,
-                                                   void* __restrict__ out, Pass P, float scale,
-                                                   const int32_t* pred) {
-  if (pred_off(pred)) return;
-  extern __shared__ float2 lds[];  // two buffers of lpb * n
-  __shared__ long long base[64];
-  const int n = P.n, lpb = P.lpb, tot = lpb * n;
-  float2* A = lds;
-  float2* B = lds + tot;
-  const long long line0 = static_cast<long long>(blockIdx.x) * lpb;
-  const int nl = static_cast<int>(min(static_cast<long long>(lpb), P.lines - line0));
-  if (threadIdx.x < lpb) {
-    const long long L = line0 + threadIdx.x;
-    const long long outer = L / P.inner, inr = L - outer * P.inner;
-    base[threadIdx.x] = outer * n * P.stride + inr;
-  }
-  __syncthreads();
-  const bool pow2 = P.log2n >= 0;
-  const bool contiguous = P.stride == 1;
-  auto split = [&](int e, int& l, int& k) {
-    if (contiguous) {
-      l = e / n;
-      k = e - l * n;
-    } else {
-      k = e / lpb;
-      l = e - k * lpb;
-    }
-  };
-  // load (bit-reversed for the radix-2 path)
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int l, k;
-    split(e, l, k);
-    float2 v = make_float2(0.0f, 0.0f);
-    if (l < nl) {
-      const long long g = base[l] + static_cast<long long>(k) * P.stride;
-      v = P.in_real ? make_float2(static_cast<const float*>(in)[g], 0.0f)
-                    : static_cast<const float2*>(in)[g];
-    }
-    A[l * n + (pow2 ? bitrev(k, P.log2n) : k)] = v;
-  }
-  // forward (or the only) transform: result in natural order in R
-  const bool inv0 = P.fused ? false : (P.inverse != 0);
-  float2* R;
-  if (pow2) {
-    dit_stages(A, n, P.log2n, lpb, P.tw, inv0);
-    R = A;
-  } else {
-    direct_dft(A, B, n, lpb, P.tw, inv0);
-    R = B;
-  }
-  if (P.fused) {
-    // multiply by the spectrum into the other buffer, then inverse transform
-    float2* Q = (R == A) ? B : A;
-    for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-      const int l = e / n, k = e - l * n;
-      float2 pr = make_float2(0.0f, 0.0f);
-      if (l < nl) {
-        const long long inr = (line0 + l) % P.inner;
-        float2 hv = P.h[static_cast<long long>(k) * P.stride + inr];
-        if (P.conj_h) hv = conjf2(hv);
-        pr = cmul(hv, R[e]);
-      }
-      Q[l * n + (pow2 ? bitrev(k, P.log2n) : k)] = pr;
-    }
-    if (pow2) {
-      dit_stages(Q, n, P.log2n, lpb, P.tw, true);
-      R = Q;
-    } else {
-      direct_dft(Q, R, n, lpb, P.tw, true);  // R is free again
-    }
-  }
-  // store
-  for (int e = threadIdx.x; e < tot; e += blockDim.x) {
-    int l, k;
-    split(e, l, k);
-    if (l < nl) {
-      const long long g = base[l] + static_cast<long long>(k) * P.stride;
-      const float2 v = R[l * n + k];
-      if (P.out_real)
-        static_cast<float*>(out)[g] = __fmul_rn(v.x, scale);
-      else
-        static_cast<float2*>(out)[g] = make_float2(__fmul_rn(v.x, scale), __fmul_rn(v.y, scale));
-    }
-  }
-}
 
 // Power-of-two lengths: Stockham auto-sort passes of radix 16 (after one
 // pass of radix 2, 4 or 8 for log2 n mod 4) on lpb lines held in one LDS
@@ -247,6 +121,28 @@ __device__ __forceinline__ float2 w16(int m, bool inv) {
   return inv ? make_float2(w.x, -w.y) : w;
 }
 
+// cos and sin of 2 pi k / R for k <= R / 2: the odd butterflies' constants
+// (indices are compile-time constants, so the tables fold).
+template <int R>
+struct OddTrig;
+template <>
+struct OddTrig<3> {
+  static constexpr float cs[2] = {1.0f, -0.5f};
+  static constexpr float sn[2] = {0.0f, 0.86602540378443865f};
+};
+template <>
+struct OddTrig<5> {
+  static constexpr float cs[3] = {1.0f, 0.30901699437494742f, -0.80901699437494742f};
+  static constexpr float sn[3] = {0.0f, 0.95105651629515357f, 0.58778525229247313f};
+};
+template <>
+struct OddTrig<7> {
+  static constexpr float cs[4] = {1.0f, 0.62348980185873353f, -0.22252093395631440f,
+                                  -0.90096886790241913f};
+  static constexpr float sn[4] = {0.0f, 0.78183148246802981f, 0.97492791218182361f,
+                                  0.43388373911755812f};
+};
+
 template <int R>
 __device__ __forceinline__ void dft_small(float2 (&v)[R], bool inv) {
   if constexpr (R == 16 || R == 8) {
@@ -275,6 +171,39 @@ __device__ __forceinline__ void dft_small(float2 (&v)[R], bool inv) {
         o[k2] = cadd(a, b);
         o[k2 + 4] = csub(a, b);
       }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) v[r] = o[r];
+  } else if constexpr (R == 3 || R == 5 || R == 7) {
+    // odd R: with s_k = x_k + x_{R-k}, d_k = x_k - x_{R-k},
+    // X_m, X_{R-m} = x_0 + sum_k cos(2 pi k m / R) s_k
+    //                -+ i sum_k sin(2 pi k m / R) d_k
+    constexpr int H = R / 2;
+    float2 sm[H], df[H];
+    float2 x0 = v[0];
+#pragma unroll
+    for (int k = 1; k <= H; ++k) {
+      sm[k - 1] = cadd(v[k], v[R - k]);
+      df[k - 1] = csub(v[k], v[R - k]);
+      x0 = cadd(x0, sm[k - 1]);
+    }
+    float2 o[R];
+    o[0] = x0;
+#pragma unroll
+    for (int m = 1; m <= H; ++m) {
+      float2 c = v[0], d = make_float2(0.0f, 0.0f);
+#pragma unroll
+      for (int k = 1; k <= H; ++k) {
+        const int t = (k * m) % R;  // a compile-time constant once unrolled
+        const float co = OddTrig<R>::cs[t <= H ? t : R - t];
+        const float si = t <= H ? OddTrig<R>::sn[t] : -OddTrig<R>::sn[R - t];
+        c = make_float2(fmaf(co, sm[k - 1].x, c.x), fmaf(co, sm[k - 1].y, c.y));
+        d = make_float2(fmaf(si, df[k - 1].x, d.x), fmaf(si, df[k - 1].y, d.y));
+      }
+      // -i d (forward) or +i d (inverse)
+      const float2 t = inv ? make_float2(-d.y, d.x) : make_float2(d.y, -d.x);
+      o[m] = cadd(c, t);
+      o[R - m] = csub(c, t);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = o[r];
@@ -347,19 +276,163 @@ __device__ __forceinline__ void stockham(float2* X, int n, int log2n, int lpb,
   for (; Ns < n; Ns *= 16) stockham_stage<16>(X, n, lpb, Ns, tw, inv);
 }
 
+// Mixed radix for lengths that are no power of two.  Bound by the latency
+// of the stages' LDS round trips and barriers (n log n work is small): 540
+// row pairs of 480 points 12 us, 723 half-spectrum columns of 360 (forward,
+// spectrum, inverse) 20 us.  Sums over all n inputs, which these lengths
+// took before, cost 454 us a pass on the full spectrum: 3 x 360 x 480
+// convolution 1380 -> 40 us, and its error against float64 1.7e-6 -> 1.7e-7.
+//
+// One stage: as stockham_stage, with the quotients by Ns and n / R taken as high words of the stage's magic
+// factors (k r tstep < n, so the twiddle index needs no reduction).
+template <int R>
+__device__ __forceinline__ void mixed_stage(float2* X, int n, int lpb, int Ns, uint32_t mns,
+                                            uint32_t mnb, const float2* tw, bool inv) {
+  constexpr int NQ = (SH_MAXV + R - 1) / R;
+  const int nb = n / R, tot = lpb * nb;  // butterflies
+  const int tstep = n / (R * Ns);
+  float2 v[NQ][R];
+  int dst[NQ];
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const int b = threadIdx.x + q * SH_THREADS;
+    dst[q] = -1;
+    if (b < tot) {
+      const int l = nb > 1 ? static_cast<int>(__umulhi(b, mnb)) : b, j = b - l * nb;
+      const int g = Ns > 1 ? static_cast<int>(__umulhi(j, mns)) : j, k = j - g * Ns;
+      const float2* x = X + l * n + j;
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[q][r] = x[r * nb];
+      if (Ns > 1) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) {
+          float2 w = tw[k * r * tstep];
+          if (inv) w = conjf2(w);
+          v[q][r] = cmul(v[q][r], w);
+        }
+      }
+      dft_small<R>(v[q], inv);
+      dst[q] = l * n + g * R * Ns + k;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    if (dst[q] >= 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) X[dst[q] + r * Ns] = v[q][r];
+    }
+  }
+  __syncthreads();
+}
+
+// A stage of any radix R (a prime above 7): output s of butterfly j is the
+// R-term sum of x[j + r n / R] w^(r (k tstep + s n / R)), w = exp(-2 pi i /
+// n), from the n twiddles in LDS.
+__device__ __forceinline__ void prime_stage(float2* X, int n, int lpb, int R, int Ns,
+                                            uint32_t mns, uint32_t mnb, const float2* tw,
+                                            bool inv) {
+  const int nb = n / R, tot = lpb * n;
+  const int tstep = n / (R * Ns);
+  float2 o[SH_MAXV];
+  // element e = (line l, output s, butterfly j), j fastest
+  auto where = [&](int e, int& l, int& s, int& g, int& k) {
+    const int ls = nb > 1 ? static_cast<int>(__umulhi(e, mnb)) : e, j = e - ls * nb;
+    l = ls / R;
+    s = ls - l * R;
+    g = Ns > 1 ? static_cast<int>(__umulhi(j, mns)) : j;
+    k = j - g * Ns;
+  };
+#pragma unroll
+  for (int q = 0; q < SH_MAXV; ++q) {
+    const int e = threadIdx.x + q * SH_THREADS;
+    if (e < tot) {
+      int l, s, g, k;
+      where(e, l, s, g, k);
+      const float2* x = X + l * n + g * Ns + k;
+      int step = k * tstep + s * nb, idx = 0;
+      if (step >= n) step -= n;
+      float re = 0.0f, im = 0.0f;
+      for (int r = 0; r < R; ++r) {
+        float2 w = tw[idx];
+        if (inv) w = conjf2(w);
+        const float2 p = cmul(x[r * nb], w);
+        re = __fadd_rn(re, p.x);
+        im = __fadd_rn(im, p.y);
+        idx += step;
+        if (idx >= n) idx -= n;
+      }
+      o[q] = make_float2(re, im);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < SH_MAXV; ++q) {
+    const int e = threadIdx.x + q * SH_THREADS;
+    if (e < tot) {
+      int l, s, g, k;
+      where(e, l, s, g, k);
+      X[l * n + g * R * Ns + k + s * Ns] = o[q];
+    }
+  }
+  __syncthreads();
+}
+
+// Mixed-radix transform of lpb lines in X; tw in LDS if S.twlds.
+__device__ __forceinline__ void mixed(float2* X, int n, const Stages& S, int lpb,
+                                      const float2* tw, bool inv) {
+  int Ns = 1;
+  for (int s = 0; s < S.count; ++s) {
+    const int R = S.R[s];
+    const uint32_t mns = S.mns[s], mnb = S.mnb[s];
+    switch (R) {
+      case 2: mixed_stage<2>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 3: mixed_stage<3>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 4: mixed_stage<4>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 5: mixed_stage<5>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 7: mixed_stage<7>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 8: mixed_stage<8>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      default: prime_stage(X, n, lpb, R, Ns, mns, mnb, tw, inv);
+    }
+    Ns *= R;
+  }
+}
+
+// The transform of a pass's lines, by length.
+template <bool MIXED>
+__device__ __forceinline__ void transform(float2* X, int n, int log2n, const Stages& S, int lpb,
+                                          const float2* tw, bool inv) {
+  if constexpr (MIXED)
+    mixed(X, n, S, lpb, tw, inv);
+  else
+    stockham(X, n, log2n, lpb, tw, inv);
+}
+
+// Twiddles of a mixed pass: copied behind the tot LDS values when a stage
+// reads one per term, else read from the table (it stays in the vector
+// cache).
+template <bool MIXED>
+__device__ __forceinline__ const float2* pass_twiddles(float2* X, int tot, int n,
+                                                       const Stages& S, const float2* tw) {
+  if (!MIXED || !S.twlds) return tw;
+  for (int k = threadIdx.x; k < n; k += SH_THREADS) X[tot + k] = tw[k];
+  return X + tot;
+}
+
+template <bool MIXED>
 __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __restrict__ in,
                                                               void* __restrict__ out, Pass P,
-                                                              float scale,
+                                                              Stages S, float scale,
                                                               const int32_t* pred) {
   if (pred_off(pred)) return;
-  extern __shared__ float2 lds[];  // lpb * n values
+  extern __shared__ float2 lds[];  // lpb * n values (and n twiddles, S.twlds)
   __shared__ long long base[64];
   __shared__ long long hoff[64];  // spectrum offset of each line (fused pass)
   const int n = P.n, lpb = P.lpb, tot = lpb * n;
   float2* X = lds;
   // twiddles are read from the n-entry table in global memory (it stays in
   // the vector cache; staging it in LDS per workgroup cost more)
-  const float2* twl = P.tw;
+  const float2* twl = pass_twiddles<MIXED>(X, tot, n, S, P.tw);
   const bool contiguous = P.stride == 1;
   // Strided passes: workgroups dispatched to one XCD (consecutive ids go to
   // the 8 XCDs in turn) take consecutive line groups, so the cache lines
@@ -418,7 +491,7 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
     }
   }
   __syncthreads();
-  stockham(X, n, P.log2n, lpb, twl, P.fused ? false : (P.inverse != 0));
+  transform<MIXED>(X, n, P.log2n, S, lpb, twl, P.fused ? false : (P.inverse != 0));
   if (P.fused) {
     for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
       const int l = e / n, k = e - l * n;
@@ -429,7 +502,7 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
       }
     }
     __syncthreads();
-    stockham(X, n, P.log2n, lpb, twl, true);
+    transform<MIXED>(X, n, P.log2n, S, lpb, twl, true);
   }
   for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
     int l, k;
@@ -447,8 +520,8 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
 
 // ------------------------------------------- real 2D convolution path --
 //
-// For two power-of-two FFT axes (F0, F1) the convolution of real data runs
-// on half spectra.  Rows are transformed two at a time: z = x_a + i x_b
+// For two FFT axes (F0, F1) the convolution of real data runs on half
+// spectra.  Rows are transformed two at a time: z = x_a + i x_b
 // has the DFT Z = X_a + i X_b with X_a, X_b Hermitian, so
 //   X_a[k] = (Z[k] + conj(Z[-k])) / 2,   X_b[k] = (Z[k] - conj(Z[-k])) / (2 i),
 // and only k = 0 .. F1/2 of each row is kept (H1 = F1/2 + 1 columns).  The
@@ -457,19 +530,22 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
 // part Hs[k] = (H[k] + conj(H[-k])) / 2 of H (equal to H for a real
 // kernel), so the plan keeps Hs on the half grid.  The inverse rows rebuild
 // Z = X_a + i X_b on the full row from the Hermitian extensions (the
-// imaginary parts of the k = 0 and k = F1/2 bins dropped, as irfft does)
-// and write x_a = Re z, x_b = Im z.
+// imaginary parts of the k = 0 and, for even F1, k = F1/2 bins dropped, as
+// irfft does) and write x_a = Re z, x_b = Im z.
 
 // Forward rows: real x (R rows of n) -> half spectra (R rows of n/2 + 1).
+template <bool MIXED>
 __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __restrict__ x,
                                                               float2* __restrict__ half, int n,
-                                                              int log2n, long long R, int lpb,
+                                                              int log2n, Stages S, long long R,
+                                                              int lpb,
                                                               const float2* __restrict__ tw,
                                                               const int32_t* pred) {
   if (pred_off(pred)) return;
   extern __shared__ float2 lds[];  // lpb * n values
   float2* X = lds;
   const int tot = lpb * n, H1 = n / 2 + 1;
+  const float2* twl = pass_twiddles<MIXED>(X, tot, n, S, tw);
   const long long row0 = 2ll * blockIdx.x * lpb;  // first real row of the workgroup
   {
     float2 vv[SH_MAXV];
@@ -491,11 +567,11 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
     }
   }
   __syncthreads();
-  stockham(X, n, log2n, lpb, tw, false);
+  transform<MIXED>(X, n, log2n, S, lpb, twl, false);
   for (int e = threadIdx.x; e < lpb * H1; e += SH_THREADS) {
     const int l = e / H1, k = e - l * H1;
     const long long ra = row0 + 2 * l, rb = ra + 1;
-    const float2 zk = X[l * n + k], zm = X[l * n + ((n - k) & (n - 1))];
+    const float2 zk = X[l * n + k], zm = X[l * n + (k ? n - k : 0)];
     if (ra < R)
       half[ra * H1 + k] = make_float2(__fmul_rn(0.5f, __fadd_rn(zk.x, zm.x)),
                                       __fmul_rn(0.5f, __fsub_rn(zk.y, zm.y)));
@@ -507,28 +583,31 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
 
 // Inverse rows: half spectra (R rows of n/2 + 1) -> real y (R rows of n),
 // times scale.
+template <bool MIXED>
 __global__ __launch_bounds__(SH_THREADS) void c2r_rows_kernel(const float2* __restrict__ half,
                                                               float* __restrict__ y, int n,
-                                                              int log2n, long long R, int lpb,
+                                                              int log2n, Stages S, long long R,
+                                                              int lpb,
                                                               const float2* __restrict__ tw,
                                                               float scale, const int32_t* pred) {
   if (pred_off(pred)) return;
   extern __shared__ float2 lds[];
   float2* X = lds;
-  const int H1 = n / 2 + 1, nh = n / 2;
+  const int H1 = n / 2 + 1;
+  const float2* twl = pass_twiddles<MIXED>(X, lpb * n, n, S, tw);
   const long long row0 = 2ll * blockIdx.x * lpb;
   for (int e = threadIdx.x; e < lpb * H1; e += SH_THREADS) {
     const int l = e / H1, k = e - l * H1;
     const long long ra = row0 + 2 * l, rb = ra + 1;
     float2 a = ra < R ? half[ra * H1 + k] : make_float2(0.0f, 0.0f);
     float2 b = rb < R ? half[rb * H1 + k] : make_float2(0.0f, 0.0f);
-    if (k == 0 || k == nh) a.y = b.y = 0.0f;
+    if (k == 0 || 2 * k == n) a.y = b.y = 0.0f;
     // Z[k] = A[k] + i B[k];  Z[n - k] = conj(A[k]) + i conj(B[k])
     X[l * n + k] = make_float2(__fsub_rn(a.x, b.y), __fadd_rn(a.y, b.x));
-    if (k > 0 && k < nh) X[l * n + n - k] = make_float2(__fadd_rn(a.x, b.y), __fsub_rn(b.x, a.y));
+    if (k > 0 && 2 * k < n) X[l * n + n - k] = make_float2(__fadd_rn(a.x, b.y), __fsub_rn(b.x, a.y));
   }
   __syncthreads();
-  stockham(X, n, log2n, lpb, tw, true);
+  transform<MIXED>(X, n, log2n, S, lpb, twl, true);
   for (int e = threadIdx.x; e < lpb * n; e += SH_THREADS) {
     const int l = e / n, k = e - l * n;
     const long long ra = row0 + 2 * l, rb = ra + 1;
@@ -875,6 +954,7 @@ __global__ __launch_bounds__(256) void cmul_kernel(long long n, const float2* __
 
 struct AxisTables {
   int n = 0, log2n = -1;
+  Stages st;  // log2n < 0
   float2* tw = nullptr;
 };
 
@@ -886,8 +966,7 @@ struct Plan {
   AxisTables ax[3];
   float2* h = nullptr;     // spectrum (fsize)
   float2* work = nullptr;  // complex workspace (batch * fsize)
-  // real 2D path (two power-of-two axes, F1 >= 4): Hermitian part of the
-  // spectrum on the half grid (F0, F1/2 + 1) and lines per workgroup of the
+  // real 2D path (two axes of 3 or more): Hermitian part of the spectrum on the half grid (F0, F1/2 + 1) and lines per workgroup of the
   // row and column passes
   bool r2c = false;
   float2* hs = nullptr;
@@ -904,12 +983,52 @@ int log2_exact(int n) {
   return l;
 }
 
+// Stages of a length that is no power of two: primes above 7 first (their
+// sums need no twiddle of an earlier stage), then 7, 5 and 3, then the power
+// of two in radices 8 and a last 4 or 2.
+Stages make_stages(int n) {
+  Stages S;
+  auto add = [&](int R) { S.R[S.count++] = R; };
+  int m = n;
+  for (int p = 11; p <= m; p += 2)
+    while (m % p == 0 && [&] {
+             for (int d = 3; d * d <= p; d += 2)
+               if (p % d == 0) return false;
+             return true;
+           }()) {
+      add(p);
+      S.twlds = 1;
+      m /= p;
+    }
+  for (int p : {7, 5, 3, 8, 4, 2})
+    while (m % p == 0) {
+      add(p);
+      m /= p;
+    }
+  auto magic = [](int d) {
+    return static_cast<uint32_t>(((1ull << 32) + d - 1) / static_cast<unsigned long long>(d));
+  };
+  for (int s = 0, Ns = 1; s < S.count; ++s) {
+    S.mns[s] = magic(Ns);  // Ns = 1 wraps to 0: the kernels skip it
+    S.mnb[s] = magic(n / S.R[s]);
+    Ns *= S.R[s];
+  }
+  return S;
+}
+
+// Dynamic LDS of a pass: lpb lines of n values and, for p-term sums, the n
+// twiddles.
+size_t pass_lds(const AxisTables& t, int lpb) {
+  return sizeof(float2) * (static_cast<size_t>(lpb) * t.n + (t.st.twlds ? t.n : 0));
+}
+
 int make_tables(AxisTables& t, int n) {
   t.n = n;
   t.log2n = log2_exact(n);
   SCXR_REQUIRE(t.log2n >= 0 ? n <= MAX_POW2 : n <= MAX_DFT, SCXR_ERR_UNSUPPORTED,
                "FFT length %d unsupported (powers of two up to %d, other lengths up to %d)", n,
                MAX_POW2, MAX_DFT);
+  if (t.log2n < 0) t.st = make_stages(n);
   const int cnt = n;  // exp(-2 pi i k / n), k < n
   std::vector<float2> tw(cnt);
   for (int k = 0; k < cnt; ++k) {
@@ -942,43 +1061,13 @@ int run_pass(const Plan& p, int a, const void* in, void* out, bool in_real, bool
   P.stride = stride;
   P.inner = stride;
   P.lines = p.batch * (p.fsize / t.n);
-  if (t.log2n >= 2) {
-    // Stockham: one LDS buffer of lpb lines (at most 8192 values); lines per
-    // workgroup chosen so that a pass has at least ~1024 workgroups.
-    const long long lines = p.batch * (p.fsize / t.n);
-    int lpb = std::max(1, 8192 / t.n);
-    { int q = 1; while (q * 2 <= lpb) q *= 2; lpb = q; }
-    while (lpb > 1 && (lines + lpb - 1) / lpb < 1024) lpb /= 2;
-    lpb = std::min(lpb, 64);
-    P.lpb = lpb;
-    P.in_real = in_real;
-    P.out_real = out_real;
-    P.inverse = inverse;
-    P.fused = fused;
-    P.conj_h = conj_h;
-    P.tw = t.tw;
-    P.h = p.h;
-    const float scale = (inverse || fused) ? 1.0f / static_cast<float>(t.n) : 1.0f;
-    const size_t lds = sizeof(float2) * lpb * t.n;
-    const unsigned grid = static_cast<unsigned>((P.lines + lpb - 1) / lpb);
-    hipLaunchKernelGGL(stockham_kernel, dim3(grid), dim3(SH_THREADS), lds, s, in, out, P, scale,
-                       pred);
-    SCXR_LAUNCHED("fft stockham pass");
-    return SCXR_OK;
-  }
-  // Two LDS buffers for the fused and direct-DFT passes, one otherwise;
-  // at most 64 KiB of LDS per workgroup in total.
-  const bool two = fused || t.log2n < 0;
-  const int cap = two ? LDS_ELEMS / 2 : LDS_ELEMS;
-  SCXR_REQUIRE(t.n <= cap, SCXR_ERR_UNSUPPORTED,
-               "FFT length %d too long for a %s pass (max %d)", t.n,
-               fused ? "fused convolution" : "direct DFT", cap);
-  int lpb = std::max(1, std::min(64, cap / t.n));
-  if (t.log2n >= 0) {  // keep lpb a power of two
-    int q = 1;
-    while (q * 2 <= lpb) q *= 2;
-    lpb = q;
-  }
+  // one LDS buffer of lpb lines (at most 7168 values, with the twiddles of
+  // p-term sums 64 KiB at most); lines per workgroup chosen so that a pass
+  // has at least ~1024 workgroups
+  int lpb = std::max(1, (t.log2n >= 0 ? 8192 : 7168) / t.n);
+  { int q = 1; while (q * 2 <= lpb) q *= 2; lpb = q; }
+  while (lpb > 1 && (P.lines + lpb - 1) / lpb < 1024) lpb /= 2;
+  lpb = std::min(lpb, 64);
   P.lpb = lpb;
   P.in_real = in_real;
   P.out_real = out_real;
@@ -988,9 +1077,13 @@ int run_pass(const Plan& p, int a, const void* in, void* out, bool in_real, bool
   P.tw = t.tw;
   P.h = p.h;
   const float scale = (inverse || fused) ? 1.0f / static_cast<float>(t.n) : 1.0f;
-  const size_t lds = sizeof(float2) * (two ? 2 : 1) * lpb * t.n;
   const unsigned grid = static_cast<unsigned>((P.lines + lpb - 1) / lpb);
-  hipLaunchKernelGGL(pass_kernel, dim3(grid), dim3(256), lds, s, in, out, P, scale, pred);
+  if (t.log2n < 0)
+    hipLaunchKernelGGL(stockham_kernel<true>, dim3(grid), dim3(SH_THREADS), pass_lds(t, lpb), s,
+                       in, out, P, t.st, scale, pred);
+  else
+    hipLaunchKernelGGL(stockham_kernel<false>, dim3(grid), dim3(SH_THREADS), pass_lds(t, lpb), s,
+                       in, out, P, t.st, scale, pred);
   SCXR_LAUNCHED("fft pass");
   return SCXR_OK;
 }
@@ -1017,9 +1110,10 @@ int convolve_r2c(const Plan& p, const float* x, float* y, bool adj, const int32_
   }
   int lr = p.lpb_rows;
   const unsigned gr = static_cast<unsigned>((cl + lr - 1) / lr);
-  const size_t lds_r = sizeof(float2) * lr * n;
-  hipLaunchKernelGGL(r2c_rows_kernel, dim3(gr), dim3(SH_THREADS), lds_r, s, x, half, n, t1.log2n,
-                     R, lr, t1.tw, pred);
+  const size_t lds_r = pass_lds(t1, lr);
+  const bool mix1 = t1.log2n < 0;
+  hipLaunchKernelGGL(mix1 ? r2c_rows_kernel<true> : r2c_rows_kernel<false>, dim3(gr),
+                     dim3(SH_THREADS), lds_r, s, x, half, n, t1.log2n, t1.st, R, lr, t1.tw, pred);
   SCXR_LAUNCHED("fft r2c rows");
   // columns of the half spectrum: n0-point transforms at stride H1
   const AxisTables& t0 = p.ax[0];
@@ -1035,11 +1129,13 @@ int convolve_r2c(const Plan& p, const float* x, float* y, bool adj, const int32_
   P.tw = t0.tw;
   P.h = p.hs;
   const unsigned gc = static_cast<unsigned>((P.lines + P.lpb - 1) / P.lpb);
-  hipLaunchKernelGGL(stockham_kernel, dim3(gc), dim3(SH_THREADS), sizeof(float2) * P.lpb * P.n, s,
-                     half, half, P, 1.0f / static_cast<float>(t0.n), pred);
+  hipLaunchKernelGGL(t0.log2n < 0 ? stockham_kernel<true> : stockham_kernel<false>, dim3(gc),
+                     dim3(SH_THREADS), pass_lds(t0, P.lpb), s, static_cast<const void*>(half),
+                     static_cast<void*>(half), P, t0.st, 1.0f / static_cast<float>(t0.n), pred);
   SCXR_LAUNCHED("fft half-spectrum columns");
-  hipLaunchKernelGGL(c2r_rows_kernel, dim3(gr), dim3(SH_THREADS), lds_r, s, half, y, n, t1.log2n,
-                     R, lr, t1.tw, 1.0f / static_cast<float>(n), pred);
+  hipLaunchKernelGGL(mix1 ? c2r_rows_kernel<true> : c2r_rows_kernel<false>, dim3(gr),
+                     dim3(SH_THREADS), lds_r, s, half, y, n, t1.log2n, t1.st, R, lr, t1.tw,
+                     1.0f / static_cast<float>(n), pred);
   SCXR_LAUNCHED("fft c2r rows");
   return SCXR_OK;
 }
@@ -1111,24 +1207,25 @@ int scxr_cconv_plan_create(int32_t ndim, const int32_t* fshape, int64_t batch,
     rc = fail(SCXR_ERR_NOMEM, "hipMalloc of the spectrum failed");
   if (rc == SCXR_OK && hipMalloc(&p.work, sizeof(float2) * p.fsize * p.batch) != hipSuccess)
     rc = fail(SCXR_ERR_NOMEM, "hipMalloc of the FFT workspace failed");
-  if (rc == SCXR_OK && ndim == 2 && p.ax[0].log2n >= 2 && p.ax[1].log2n >= 2) {
+  if (rc == SCXR_OK && ndim == 2 && p.F[0] > 2 && p.F[1] > 2) {
     p.r2c = true;
     const long long H1 = p.F[1] / 2 + 1;
     if (hipMalloc(&p.hs, sizeof(float2) * p.F[0] * H1) != hipSuccess)
       rc = fail(SCXR_ERR_NOMEM, "hipMalloc of the half spectrum failed");
-    // lines per workgroup: as many as fit 8192 LDS values while the pass
-    // keeps at least 512 workgroups (SCXR_FFT_LPB="rows,cols" overrides)
-    auto pick = [](long long lines, int n) {
-      int l = std::max(1, 8192 / n);
+    // lines per workgroup: as many as fit 8192 LDS values (7168 beside the
+    // twiddles of p-term sums; at most the 64 lines that a column pass
+    // tabulates) while the pass keeps at least 512 workgroups (SCXR_FFT_LPB="rows,cols" overrides)
+    auto pick = [](long long lines, const AxisTables& t) {
+      int l = std::max(1, std::min(64, (t.log2n >= 0 ? 8192 : 7168) / t.n));
       while (l > 1 && (lines + l - 1) / l < 512) l /= 2;
       return l;
     };
-    p.lpb_rows = pick((p.batch * p.F[0] + 1) / 2, p.F[1]);
-    p.lpb_cols = pick(p.batch * H1, p.F[0]);
+    p.lpb_rows = pick((p.batch * p.F[0] + 1) / 2, p.ax[1]);
+    p.lpb_cols = pick(p.batch * H1, p.ax[0]);
     if (const char* env = std::getenv("SCXR_FFT_LPB")) {
       int a = 0, b = 0;
-      if (std::sscanf(env, "%d,%d", &a, &b) == 2 && a >= 1 && b >= 1 &&
-          a * p.F[1] <= 8192 && b * p.F[0] <= 8192) {
+      if (std::sscanf(env, "%d,%d", &a, &b) == 2 && a >= 1 && b >= 1 && a <= 64 && b <= 64 &&
+          pass_lds(p.ax[1], a) <= 65536 && pass_lds(p.ax[0], b) <= 65536) {
         p.lpb_rows = a;
         p.lpb_cols = b;
       }

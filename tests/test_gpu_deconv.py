@@ -142,6 +142,33 @@ def test_circconv_1024_psf(gpu):
     np.testing.assert_allclose(A.h_dft.cpu().numpy(), hd, rtol=0, atol=2e-6)
 
 
+@pytest.mark.parametrize("x_shape,ndims", [((3, 5), 2), ((7, 9), 2), ((2, 11, 13), 2),
+                                           ((9, 509), 2), ((512, 507), 2), ((486, 490), 2),
+                                           ((3, 360, 480), 2), ((1, 6), 2), ((2, 45), 2),
+                                           ((5, 343), 1), ((70, 17), 1), ((5, 22, 21), 3)])
+def test_mixed_radix_lengths(gpu, x_shape, ndims):
+    """Lengths that are no power of two: products of 2, 3, 5 and 7, primes
+    above 7 (alone and as factors), odd rows (a half spectrum without a
+    Nyquist column), axes of one and two points, against float64.  Each
+    transform's float32 error is at most about eps sqrt(p) for its largest
+    prime factor p (2.7e-6 at 509); a convolution takes four."""
+    rng = np.random.default_rng(17)
+    F, axes = x_shape[-ndims:], tuple(range(len(x_shape) - ndims, len(x_shape)))
+    x = rng.standard_normal(x_shape).astype(np.float32)
+    h = (rng.standard_normal(F) + 1j * rng.standard_normal(F)).astype(np.complex64)
+    A = CircularConvolve(h, x_shape, ndims=ndims, h_is_dft=True)
+    X = np.fft.fftn(x.astype(np.float64), axes=axes)
+    h64 = h.astype(np.complex128)
+    fwd = np.fft.ifftn(h64 * X, axes=axes).real
+    adj = np.fft.ifftn(h64.conj() * X, axes=axes).real
+    e = rel_l2(A(dev(x)).cpu().numpy(), fwd), rel_l2(A.adj(dev(x)).cpu().numpy(), adj)
+    got = A.fftn(dev(x)).cpu().numpy()
+    ef = float(np.linalg.norm(got - X) / np.linalg.norm(X))
+    print(f"  mixed radix {x_shape} over {ndims}: fwd {e[0]:.2e} adj {e[1]:.2e} fftn {ef:.2e}",
+          flush=True)
+    assert max(e) <= 1e-5 and ef <= 1e-5
+
+
 @pytest.mark.parametrize("shape", [(33, 31), (8, 9, 10), (40,)])
 @pytest.mark.parametrize("iso", [True, False])
 @pytest.mark.parametrize("circular", [False, True])
