@@ -499,12 +499,13 @@ int scxr_batch_admm_itstat(const scxr_xr2d_batch* plan, const double* res, const
  * Geometries where one detector axis follows one volume axis exactly
  * (single rotation axis, e.g. matrices_from_euler_angles with seq "Y")
  * run in slice mode: slice-parallel kernels, deterministic, no atomics.
- * Others run in general mode (gathers in a fixed order, also
- * deterministic).  allow_slice is a set of flags: bit 0 clear forces
- * general mode; bit 1 set keeps the slice adjoint that reads the detector
- * rows from global memory instead of staging them in LDS (the two give
- * bitwise-equal results; the staged one is faster).  Pass 1 for the
- * default.
+ * Others run in general mode (sums in a fixed order, also deterministic).
+ * allow_slice is a set of flags: bit 0 clear forces general mode; bit 1 set
+ * keeps the slice adjoint that reads the detector rows from global memory
+ * instead of staging them in LDS (the two give bitwise-equal results; the
+ * staged one is faster); bit 2 set keeps the general-mode gathers from
+ * global memory instead of the kernels with windows in LDS (equal up to
+ * float32 rounding; the latter are faster).  Pass 1 for the default.
  */
 typedef struct scxr_xr3d_plan scxr_xr3d_plan;
 
@@ -520,6 +521,14 @@ int scxr_xr3d_info(const scxr_xr3d_plan* plan, int32_t* out);
 /* proj = H vol  (_xray3d.py:110-159). */
 int scxr_xr3d_forward(const scxr_xr3d_plan* plan, const float* vol, float* proj,
                       const int32_t* pred, void* stream);
+/* Forward with a workspace of scxr_xr3d_forward_ws(plan) floats (device; 0:
+ * none is needed, ws may be null): general-mode plans then splat into LDS
+ * windows.  The workspace belongs to the call until it has run, so calls on
+ * several streams bring one each; scxr_xr3d_forward, which has none, takes
+ * the slower gather for such plans. */
+int64_t scxr_xr3d_forward_ws(const scxr_xr3d_plan* plan);
+int scxr_xr3d_forward_with(const scxr_xr3d_plan* plan, const float* vol, float* proj, float* ws,
+                           const int32_t* pred, void* stream);
 /* vol = H^T proj  (_xray3d.py:161-204). */
 int scxr_xr3d_adjoint(const scxr_xr3d_plan* plan, const float* proj, float* vol,
                       const int32_t* pred, void* stream);

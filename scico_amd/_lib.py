@@ -100,6 +100,9 @@ SIGNATURES = [
     ("scxr_xr3d_plan_destroy", c_int32, [c_void_p]),
     ("scxr_xr3d_info", c_int32, [c_void_p, c_int32_p]),
     ("scxr_xr3d_forward", c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    ("scxr_xr3d_forward_ws", c_int64, [c_void_p]),
+    ("scxr_xr3d_forward_with", c_int32,
+     [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     ("scxr_xr3d_adjoint", c_int32, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     ("scxr_xr3d_weights", c_int32, [c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
     # finite differences, proxes

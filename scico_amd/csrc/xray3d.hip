@@ -23,8 +23,11 @@
 // volume axes, u the in-plane detector axis); a tiled transpose converts
 // to and from the caller's layout when it differs.
 //
-// General mode (any other geometry): the adjoint gathers per voxel in the
-// reference's per-view order; the forward scatters with float atomics.
+// General mode (any other geometry): the forward splats blocks of voxels
+// into detector windows held in LDS and adds the windows up in a fixed
+// order; the adjoint gathers per voxel from windows staged in LDS.  Both are
+// deterministic.  Geometries whose windows do not fit take gathers from
+// global memory.
 
 #include <hip/hip_runtime.h>
 
@@ -52,11 +55,39 @@ struct Plan {
   int spg = 2;                             // forward slots per bin group
   bool vol_direct = false, proj_direct = false;
   bool adj_staged = false;                 // adjoint rows staged in LDS (adj_slice_staged_kernel)
+  void* tables = nullptr;  // general mode: one block of the tables below (mats included)
   float* mats = nullptr;   // (V, 2, 4) float32
   float4* geom = nullptr;  // slice mode: (a, b, t, 0) in-plane row per view
   float* volc = nullptr;   // canonical volume workspace (P Q rows of 4 SQ floats)
   float* proja = nullptr;  // canonical projection workspace (V U 4 SQ)
   struct GenView* gview = nullptr;  // general mode: per-view gather set-up
+  // general mode, windows in LDS (gen_splat_kernel, gen_adj_tile_kernel)
+  bool splat = false, adj_tiled = false;
+  struct SplatView* sview = nullptr;
+  struct SplatItem* sitem = nullptr;
+  float* zterm = nullptr;             // adjoint: m[r][2] (k + 1/2), 8 voxels at a time
+  int slot = 0;                       // window floats of a splat item
+  bool need_t = false;                // some view marches along z: volume copy [z][x][y]
+  std::vector<int> ifirst;            // first item of every view (V + 1 entries)
+  std::vector<int> chunk;             // first view of every pass over the items (and V)
+  long long ws_floats = 0;            // forward workspace
+};
+
+// General-mode splat set-up of one view.  The view marches along volume axis
+// a (the one whose complementary 2 x 2 minor is largest); b < c are the other
+// two.  At plane t the whole lattice of voxel blocks is shifted by
+// (rint(bb (t - tc)), rint(bc (t - tc))) voxels along (b, c), which keeps a
+// block's projection in place, so one window of detector pixels holds all of
+// the block's planes.
+struct SplatView {
+  int a, sb, sc, pitch, rows, first, last, pad;  // items [first, last)
+  float bb, bc, tc, pad2;
+  float m[8];
+};
+// One block of 8 sb x 8 sc voxels per plane (b from p8 + shift, c from q8 +
+// shift) over planes [t0, t1), with the window at detector pixel (lo0, lo1).
+struct SplatItem {
+  int view, p8, q8, lo0, lo1, t0, t1, pad;
 };
 
 // General-mode forward set-up of one view.  The detector pixel (d0, d1)
@@ -548,6 +579,423 @@ __global__ __launch_bounds__(256) void shift_rows_kernel(const float* __restrict
 
 // ------------------------------------------------- general-mode kernels --
 
+// One detector axis of a voxel: its lower pixel and the share min(ceil(left)
+// - left, 1/2) that falls there (the reference's operations; P carries its
+// rounding order).
+__device__ __forceinline__ float axis_share(float P, int& ul) {
+  const float left = __fsub_rn(P, 0.25f);
+  ul = cvt_flr_i32(left);
+  return fminf(__fsub_rn(ceilf(left), left), 0.5f);
+}
+
+typedef __attribute__((address_space(3))) float LdsFloat;
+__device__ __forceinline__ int lds_address(const float* p) {
+  return static_cast<int>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const float*)p));
+}
+
+__device__ __forceinline__ LdsFloat* lds_at(int address) {
+  return reinterpret_cast<LdsFloat*>(static_cast<uintptr_t>(static_cast<unsigned>(address)));
+}
+
+// LDS address row * u0 + 4 * u1 + base of a window pixel in two instructions
+// (row bytes in a vector register, the window's base in a scalar one); left
+// to itself the compiler takes a 32-bit multiply at quarter rate.
+__device__ __forceinline__ int win_offset(int u0, int row, int u1, int base) {
+  int r;
+  asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(u0), "v"(row), "s"(base));
+  return r + (u1 << 2);
+}
+
+// Forward, general mode.  Each wave takes one item: a block of voxels that
+// it splats, plane by plane, into its own window of detector pixels in LDS.
+// No atomics: in one instruction the 64 lanes take an 8 x 8 lattice of
+// voxels sb and sc apart, whose 2 x 2 footprints are disjoint (the host
+// picks the strides so that any two of them are 2.0625 pixels apart along a
+// detector axis), so a plain LDS read-modify-write is race free, and LDS
+// executes a wave's accesses in order.  Every voxel's weights are evaluated
+// once (a gather per detector pixel evaluates each about four times, and
+// tests as many candidates again).
+//
+// Bound by the LDS (a read and a write of four words per voxel and view, with
+// the bank conflicts of a rotated lattice: the host takes the window pitch
+// that a bank model rates cheapest for the view) and by VALU issue together:
+// 129 x 130 x 131 with 60 views 1872 -> 212 us (window sums 22 us of it), the
+// LDS busy 90 % of the kernel, VALU issue 93 %.
+template <int A, int SB_, int SC_>
+__device__ __forceinline__ void splat_item(__amdgpu_buffer_rsrc_t vr, const SplatView& g,
+                                           const SplatItem& it, int wbase, int nb, int nc,
+                                           int sta, int stb) {
+  constexpr int B = A == 0 ? 1 : 0, C = A == 2 ? 1 : 2;
+  constexpr bool FIX = SB_ > 0;
+  const int SB = FIX ? SB_ : g.sb, SC = FIX ? SC_ : g.sc;
+  const int lane = threadIdx.x & 63;
+  const int ob = SB * (lane >> 3), oc = SC * (lane & 7);
+  const float ma0 = g.m[A], ma1 = g.m[4 + A], mb0 = g.m[B], mb1 = g.m[4 + B], mc0 = g.m[C],
+              mc1 = g.m[4 + C], mt0 = g.m[3], mt1 = g.m[7];
+  int row = 4 * g.pitch;  // bytes of a window row
+  const int base = wbase - (it.lo0 * row + 4 * it.lo1);
+  asm("" : "+v"(row));
+  auto shift = [&](float beta, int t) {
+    return __builtin_amdgcn_readfirstlane(
+        static_cast<int>(rintf(__fmul_rn(beta, __fsub_rn(static_cast<float>(t), g.tc)))));
+  };
+  // byte offset of voxel (t, b, c): an index off the volume moves it past
+  // the buffer's end (at most 2^30 bytes), where loads return zero
+  auto row_off = [&](int t, int b) {
+    return static_cast<unsigned>(b) < static_cast<unsigned>(nb)
+               ? static_cast<unsigned>(t * sta + b * stb) * 4u
+               : 0x80000000u;
+  };
+  auto col_off = [&](int c) {
+    return static_cast<unsigned>(c) < static_cast<unsigned>(nc) ? static_cast<unsigned>(c) * 4u
+                                                                : 0x40000000u;
+  };
+  // P_r = ((m_r0 x0 + m_r1 x1) + m_r2 x2) + m_r3 in the reference's order:
+  // pab holds the terms of the march axis and b where both come before c
+  // (A < 2), else b's term alone, and pa is added last
+  auto voxel = [&](float x, float pab0, float pab1, float pc0, float pc1, float pa0, float pa1) {
+    float P0 = __fadd_rn(pab0, pc0), P1 = __fadd_rn(pab1, pc1);
+    if (A == 2) {
+      P0 = __fadd_rn(P0, pa0);
+      P1 = __fadd_rn(P1, pa1);
+    }
+    int u0, u1;
+    const float w0 = axis_share(__fadd_rn(P0, mt0), u0), w1 = axis_share(__fadd_rn(P1, mt1), u1);
+    // the factor 4 of the weights (an exact scaling) is applied to the sums
+    const float v0 = __fsub_rn(0.5f, w0);
+    const float xl = __fmul_rn(w1, x), xr = __fmul_rn(__fsub_rn(0.5f, w1), x);
+    const int at = win_offset(u0, row, u1, base);
+    LdsFloat* q = lds_at(at);
+    LdsFloat* r = lds_at(at + row);
+    const float a00 = q[0], a01 = q[1], a10 = r[0], a11 = r[1];
+    q[0] = fmaf(w0, xl, a00);
+    q[1] = fmaf(w0, xr, a01);
+    r[0] = fmaf(v0, xl, a10);
+    r[1] = fmaf(v0, xr, a11);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_wave_barrier();
+  };
+  if constexpr (FIX) {
+    float nxt[SB_][SC_];
+    const unsigned lane_off = static_cast<unsigned>(ob * stb + oc) * 4u;
+    auto load = [&](int t, int sb, int sc) {
+      const int bu = it.p8 + sb, cu = it.q8 + sc;
+      if (bu >= 0 && bu + 8 * SB_ <= nb && cu >= 0 && cu + 8 * SC_ <= nc) {
+        // inside the volume: a scalar offset per row, the lane's own offset
+#pragma unroll
+        for (int rb = 0; rb < SB_; ++rb)
+#pragma unroll
+          for (int rc = 0; rc < SC_; ++rc)
+            nxt[rb][rc] =
+                bload1(vr, lane_off + 4u * rc, (t * sta + (bu + rb) * stb + cu) * 4);
+        return;
+      }
+      const int b0 = bu + ob, c0 = cu + oc;
+      unsigned co[SC_];
+#pragma unroll
+      for (int rc = 0; rc < SC_; ++rc) co[rc] = col_off(c0 + rc);
+#pragma unroll
+      for (int rb = 0; rb < SB_; ++rb) {
+        const unsigned ro = row_off(t, b0 + rb);
+#pragma unroll
+        for (int rc = 0; rc < SC_; ++rc) nxt[rb][rc] = bload1(vr, ro + co[rc], 0);
+      }
+    };
+    int sb = shift(g.bb, it.t0), sc = shift(g.bc, it.t0);
+    load(it.t0, sb, sc);
+#pragma unroll 1
+    for (int t = it.t0; t < it.t1; ++t) {
+      float cur[SB_][SC_];
+#pragma unroll
+      for (int rb = 0; rb < SB_; ++rb)
+#pragma unroll
+        for (int rc = 0; rc < SC_; ++rc) cur[rb][rc] = nxt[rb][rc];
+      const float xb0 = static_cast<float>(it.p8 + sb + ob);
+      const float xc0 = static_cast<float>(it.q8 + sc + oc);
+      if (t + 1 < it.t1) {
+        sb = shift(g.bb, t + 1);
+        sc = shift(g.bc, t + 1);
+        load(t + 1, sb, sc);
+      }
+      const float xa = __fadd_rn(static_cast<float>(t), 0.5f);
+      const float pa0 = __fmul_rn(ma0, xa), pa1 = __fmul_rn(ma1, xa);
+      float pc0[SC_], pc1[SC_];
+#pragma unroll
+      for (int rc = 0; rc < SC_; ++rc) {
+        const float xc = __fadd_rn(xc0, static_cast<float>(rc) + 0.5f);
+        pc0[rc] = __fmul_rn(mc0, xc);
+        pc1[rc] = __fmul_rn(mc1, xc);
+      }
+#pragma unroll
+      for (int rb = 0; rb < SB_; ++rb) {
+        const float xb = __fadd_rn(xb0, static_cast<float>(rb) + 0.5f);
+        float pb0 = __fmul_rn(mb0, xb), pb1 = __fmul_rn(mb1, xb);
+        if (A < 2) {
+          pb0 = __fadd_rn(pa0, pb0);
+          pb1 = __fadd_rn(pa1, pb1);
+        }
+#pragma unroll
+        for (int rc = 0; rc < SC_; ++rc)
+          voxel(cur[rb][rc], pb0, pb1, pc0[rc], pc1[rc], pa0, pa1);
+      }
+    }
+  } else {
+    for (int t = it.t0; t < it.t1; ++t) {
+      const int b0 = it.p8 + shift(g.bb, t) + ob, c0 = it.q8 + shift(g.bc, t) + oc;
+      const float xa = __fadd_rn(static_cast<float>(t), 0.5f);
+      const float pa0 = __fmul_rn(ma0, xa), pa1 = __fmul_rn(ma1, xa);
+      for (int rb = 0; rb < SB; ++rb) {
+        const float xb = __fadd_rn(static_cast<float>(b0 + rb), 0.5f);
+        const unsigned ro = row_off(t, b0 + rb);
+        float pb0 = __fmul_rn(mb0, xb), pb1 = __fmul_rn(mb1, xb);
+        if (A < 2) {
+          pb0 = __fadd_rn(pa0, pb0);
+          pb1 = __fadd_rn(pa1, pb1);
+        }
+        for (int rc = 0; rc < SC; ++rc) {
+          const float x = bload1(vr, ro + col_off(c0 + rc), 0);
+          const float xc = __fadd_rn(static_cast<float>(c0 + rc), 0.5f);
+          voxel(x, pb0, pb1, __fmul_rn(mc0, xc), __fmul_rn(mc1, xc), pa0, pa1);
+        }
+      }
+    }
+  }
+}
+
+// Strides 3 x 3 (a minor near a rotation, the usual case) are compiled;
+// other strides take run-time loops.
+__global__ __launch_bounds__(256) void gen_splat_kernel(const float* __restrict__ vol,
+                                                        const float* __restrict__ volt,
+                                                        float* __restrict__ parts,
+                                                        const SplatView* __restrict__ views,
+                                                        const SplatItem* __restrict__ items,
+                                                        int item0, int item1, int slot, int X,
+                                                        int Y, int Z,
+                                                        const int32_t* __restrict__ pred) {
+  if (pred_off(pred)) return;
+  extern __shared__ float splat_win[];  // [4 waves][slot]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int i = item0 + blockIdx.x * 4 + wave;
+  if (i >= item1) return;  // waves are independent: no workgroup barrier below
+  const SplatItem it = items[i];
+  const SplatView g = views[it.view];
+  float* win = splat_win + wave * slot;
+  const int n = g.rows * g.pitch;
+  for (int e = lane; e < n; e += 64) win[e] = 0.0f;
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_wave_barrier();
+  const __amdgpu_buffer_rsrc_t vr = make_rsrc(g.a == 2 ? volt : vol, X * Y * Z * 4);
+  const bool fix = g.sb == 3 && g.sc == 3;
+  const int wbase = lds_address(splat_win) + wave * slot * 4;
+  if (g.a == 0) {
+    if (fix)
+      splat_item<0, 3, 3>(vr, g, it, wbase, Y, Z, Y * Z, Z);
+    else
+      splat_item<0, 0, 0>(vr, g, it, wbase, Y, Z, Y * Z, Z);
+  } else if (g.a == 1) {
+    if (fix)
+      splat_item<1, 3, 3>(vr, g, it, wbase, X, Z, Z, Y * Z);
+    else
+      splat_item<1, 0, 0>(vr, g, it, wbase, X, Z, Z, Y * Z);
+  } else {
+    if (fix)
+      splat_item<2, 3, 3>(vr, g, it, wbase, X, Y, X * Y, Y);
+    else
+      splat_item<2, 0, 0>(vr, g, it, wbase, X, Y, X * Y, Y);
+  }
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_wave_barrier();
+  float* dst = parts + static_cast<size_t>(i - item0) * slot;
+  for (int e = lane; e < n; e += 64) dst[e] = __fmul_rn(4.0f, win[e]);
+}
+
+// Detector pixel = sum of the windows that cover it, in item order.  One
+// workgroup per 16 x 16 pixels of a view; each wave finds the items that
+// reach its 16 x 4 pixels by ballots over the view's items.
+__global__ __launch_bounds__(256) void gen_splat_sum_kernel(const float* __restrict__ parts,
+                                                            float* __restrict__ proj,
+                                                            const SplatView* __restrict__ views,
+                                                            const SplatItem* __restrict__ items,
+                                                            int view0, int item0, int slot, int D0,
+                                                            int D1,
+                                                            const int32_t* __restrict__ pred) {
+  if (pred_off(pred)) return;
+  const int v = view0 + blockIdx.z;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int r0 = blockIdx.y * 16 + wave * 4, c0 = blockIdx.x * 16;
+  const int d0 = r0 + (lane >> 4), d1 = c0 + (lane & 15);
+  const int rows = views[v].rows, pitch = views[v].pitch;
+  const int first = views[v].first, last = views[v].last;
+  float sum = 0.0f;
+  for (int i0 = first; i0 < last; i0 += 64) {
+    const int i = i0 + lane;
+    int lo0 = 0, lo1 = 0;
+    bool hit = false;
+    if (i < last) {
+      lo0 = items[i].lo0;
+      lo1 = items[i].lo1;
+      hit = lo0 < r0 + 4 && lo0 + rows > r0 && lo1 < c0 + 16 && lo1 + pitch > c0;
+    }
+    unsigned long long todo = __ballot(hit);
+    while (todo) {  // four windows at a time: their loads are in flight together
+      float x[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        x[q] = 0.0f;
+        if (todo) {
+          const int k = __builtin_ctzll(todo);
+          todo &= todo - 1;
+          const int r = d0 - rl(lo0, k), c = d1 - rl(lo1, k);
+          if (static_cast<unsigned>(r) < static_cast<unsigned>(rows) &&
+              static_cast<unsigned>(c) < static_cast<unsigned>(pitch))
+            x[q] = parts[static_cast<size_t>(i0 + k - item0) * slot + r * pitch + c];
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sum = __fadd_rn(sum, x[q]);
+    }
+  }
+  if (d0 < D0 && d1 < D1) proj[(static_cast<size_t>(v) * D0 + d0) * D1 + d1] = sum;
+}
+
+// Adjoint, general mode.  Each wave takes an 8 x 8 x 8 block of voxels (lane
+// (i, j), eight k per lane) and walks its share of the views: the 16 x 16
+// detector pixels that the block can reach are copied into the wave's LDS
+// window (zero off the detector, so the taps need no range tests; the next
+// view's pixels are in flight meanwhile), and every voxel reads its four
+// taps there.  The terms m[r][2] (k + 1/2) are uniform over the wave and
+// come from a table by scalar loads; (m[r][0] x0 + m[r][1] x1) serves a
+// lane's eight voxels: about 31 vector instructions per voxel and view with
+// the staging, the bound (97 % of the issue rate), against 130 for taps
+// clamped and read from global memory per voxel: 129 x 130 x 131 with 60
+// views 457 -> 84 us.
+constexpr int GA = 8, GWIN = 16, GPITCH = 17;
+
+__global__ __launch_bounds__(256) void gen_adj_tile_kernel(
+    const float* __restrict__ proj, float* __restrict__ vol, const float* __restrict__ mats,
+    const float* __restrict__ zterm, int X, int Y, int Z, int V, int D0, int D1, int vs,
+    const int32_t* __restrict__ pred) {
+  if (pred_off(pred)) return;
+  __shared__ float wins[4][GWIN * GPITCH];
+  __shared__ float share[3][GA][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int nti = (X + GA - 1) / GA, ntj = (Y + GA - 1) / GA, ntk = (Z + GA - 1) / GA;
+  const int tile = blockIdx.x * (4 / vs) + wave / vs, vg = wave % vs;
+  const bool live = tile < nti * ntj * ntk;
+  const int tk = live ? tile % ntk : 0, tj = live ? (tile / ntk) % ntj : 0,
+            ti = live ? tile / (ntk * ntj) : 0;
+  const int i = ti * GA + (lane >> 3), j = tj * GA + (lane & 7), k0 = tk * GA;
+  const float x0 = __fadd_rn(static_cast<float>(i), 0.5f);
+  const float x1 = __fadd_rn(static_cast<float>(j), 0.5f);
+  float* win = wins[wave];
+  const int wbase = lds_address(&wins[0][0]) + wave * GWIN * GPITCH * 4;
+  int row = 4 * GPITCH;
+  asm("" : "+v"(row));
+  const int chunk = (V + vs - 1) / vs;
+  const int vb = live ? min(V, vg * chunk) : 0, ve = live ? min(V, vb + chunk) : 0;
+  float acc[GA];
+#pragma unroll
+  for (int k = 0; k < GA; ++k) acc[k] = 0.0f;
+  // window origins of views [c0, c0 + 64), one per lane: the lower bound of
+  // both detector indices over the block (its lowest corner), with a margin
+  // far above the float32 rounding of the projected centres
+  int olo0 = 0, olo1 = 0;
+  auto origins = [&](int c0) {
+    const float* m = mats + 8 * min(c0 + lane, V - 1);
+    int o[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const float* mr = m + 4 * r;
+      const float c = static_cast<float>(GA - 1);
+      const float xa = static_cast<float>(ti * GA) + (mr[0] < 0.0f ? c : 0.0f) + 0.5f;
+      const float xb = static_cast<float>(tj * GA) + (mr[1] < 0.0f ? c : 0.0f) + 0.5f;
+      const float xc = static_cast<float>(tk * GA) + (mr[2] < 0.0f ? c : 0.0f) + 0.5f;
+      const float lo = mr[0] * xa + mr[1] * xb + mr[2] * xc + mr[3] - 0.26f;
+      o[r] = static_cast<int>(floorf(lo));
+    }
+    olo0 = o[0];
+    olo1 = o[1];
+  };
+  float nxt[4];
+  auto fetch = [&](int v, int lo0, int lo1) {
+    const __amdgpu_buffer_rsrc_t yr =
+        make_rsrc(proj + static_cast<size_t>(v) * D0 * D1, D0 * D1 * 4);
+    // rows off the detector fall outside the view's buffer; columns off it
+    // are moved there (rows and columns are below 2^14)
+    const int row = lo0 + (lane >> 4), col = lo1 + (lane & 15);
+    const unsigned off = static_cast<unsigned>(col) < static_cast<unsigned>(D1)
+                             ? static_cast<unsigned>(row * D1 + col) * 4u
+                             : 0x80000000u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) nxt[q] = bload1(yr, off + static_cast<unsigned>(q * 16 * D1), 0);
+  };
+  if (vb < ve) {
+    origins(vb);
+    fetch(vb, rl(olo0, 0), rl(olo1, 0));
+  }
+#pragma unroll 1
+  for (int v = vb; v < ve; ++v) {
+    const int q6 = (v - vb) & 63;
+    const int lo0 = rl(olo0, q6), lo1 = rl(olo1, q6);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) win[((lane >> 4) + 4 * q) * GPITCH + (lane & 15)] = nxt[q];
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_wave_barrier();
+    if (v + 1 < ve) {
+      if (q6 == 63) origins(v + 1);
+      const int n6 = (v + 1 - vb) & 63;
+      fetch(v + 1, rl(olo0, n6), rl(olo1, n6));
+    }
+    const float* m = mats + 8 * v;
+    const float* zt = zterm + (static_cast<size_t>(v) * ntk + tk) * (2 * GA);
+    const float a0 = __fadd_rn(__fmul_rn(m[0], x0), __fmul_rn(m[1], x1));
+    const float a1 = __fadd_rn(__fmul_rn(m[4], x0), __fmul_rn(m[5], x1));
+    const float t0 = m[3], t1 = m[7];
+    const int base = wbase - (lo0 * GPITCH + lo1) * 4;
+#pragma unroll
+    for (int k = 0; k < GA; ++k) {
+      int u0, u1;
+      const float w0 = axis_share(__fadd_rn(__fadd_rn(a0, zt[k]), t0), u0);
+      const float w1 = axis_share(__fadd_rn(__fadd_rn(a1, zt[GA + k]), t1), u1);
+      const LdsFloat* y = lds_at(win_offset(u0, row, u1, base));
+      // the factor 4 of the weights (an exact scaling) is applied to the sums
+      const float v0 = __fsub_rn(0.5f, w0), v1 = __fsub_rn(0.5f, w1);
+      const float left = fmaf(v0, y[GPITCH], __fmul_rn(w0, y[0]));
+      const float right = fmaf(v0, y[GPITCH + 1], __fmul_rn(w0, y[1]));
+      acc[k] = fmaf(v1, right, fmaf(w1, left, acc[k]));
+    }
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (vs > 1) {  // add the other waves' shares of the views, in order
+    const int slot0 = (wave / vs) * (vs - 1);
+    if (vg > 0)
+#pragma unroll
+      for (int k = 0; k < GA; ++k) share[slot0 + vg - 1][k][lane] = acc[k];
+    __syncthreads();
+    if (vg > 0) return;
+    for (int g = 1; g < vs; ++g)
+#pragma unroll
+      for (int k = 0; k < GA; ++k) acc[k] = __fadd_rn(acc[k], share[slot0 + g - 1][k][lane]);
+  }
+  if (!live || i >= X || j >= Y) return;
+#pragma unroll
+  for (int k = 0; k < GA; ++k) acc[k] = __fmul_rn(4.0f, acc[k]);
+  float* out = vol + (static_cast<size_t>(i) * Y + j) * Z + k0;
+  if (Z % 4 == 0 && k0 + GA <= Z && (reinterpret_cast<uintptr_t>(vol) & 15) == 0) {
+    reinterpret_cast<float4*>(out)[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    reinterpret_cast<float4*>(out)[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < GA; ++k)
+      if (k0 + k < Z) out[k] = acc[k];
+  }
+}
+
+// The gathers below read global memory; they take what the windows cannot
+// hold (projected voxels far apart on the detector, or nearly on one line).
+
 __global__ __launch_bounds__(256) void gen_adj_kernel(const float* __restrict__ proj,
                                                       float* __restrict__ vol,
                                                       const float* __restrict__ mats, int X,
@@ -814,12 +1262,16 @@ static bool try_slice(Plan& p, const std::vector<float>& m, int sax, int dax) {
 }
 
 void destroy(Plan& p) {
-  if (p.mats) (void)hipFree(p.mats);
+  if (p.mats && !p.tables) (void)hipFree(p.mats);
+  if (p.tables) (void)hipFree(p.tables);
+  p.tables = nullptr;
   if (p.geom) (void)hipFree(p.geom);
   if (p.volc) (void)hipFree(p.volc);
   if (p.proja) (void)hipFree(p.proja);
-  if (p.gview) (void)hipFree(p.gview);
   p.gview = nullptr;
+  p.sview = nullptr;
+  p.sitem = nullptr;
+  p.zterm = nullptr;
   p.mats = nullptr;
   p.geom = nullptr;
   p.volc = p.proja = nullptr;
@@ -831,6 +1283,265 @@ static int dev_alloc(void** ptr, size_t bytes) {
     *ptr = nullptr;
     return fail(SCXR_ERR_NOMEM, "hipMalloc of %zu bytes failed", bytes);
   }
+  return SCXR_OK;
+}
+
+// Detector coordinates of every voxel centre stay below this (float32
+// rounding of P far below the window margins, window offsets within int32).
+constexpr double GEN_PMAX = 8192.0;
+constexpr double GEN_MARGIN = 0.01;
+
+static bool gen_in_range(const Plan& p, const std::vector<float>& m) {
+  if (p.D0 > 16384 || p.D1 > 16384 || static_cast<double>(p.D0) * p.D1 > 2.6e8) return false;
+  for (int v = 0; v < p.V; ++v)
+    for (int r = 0; r < 2; ++r)
+      if (std::fabs(mat(m, v, r, 0)) * p.X + std::fabs(mat(m, v, r, 1)) * p.Y +
+              std::fabs(mat(m, v, r, 2)) * p.Z + std::fabs(mat(m, v, r, 3)) >
+          GEN_PMAX)
+        return false;
+  return true;
+}
+
+// Tables of the tiled adjoint; false if some view's 8 x 8 x 8 blocks reach
+// over more than GWIN detector pixels.
+static bool build_adj_tiles(const Plan& p, const std::vector<float>& m, std::vector<float>& zt) {
+  for (int v = 0; v < p.V; ++v)
+    for (int r = 0; r < 2; ++r) {
+      const double ext = (GA - 1.0) * (std::fabs(mat(m, v, r, 0)) + std::fabs(mat(m, v, r, 1)) +
+                                       std::fabs(mat(m, v, r, 2)));
+      if (std::floor(ext + 2 * GEN_MARGIN) + 3 > GWIN) return false;
+    }
+  const int ntk = (p.Z + GA - 1) / GA;
+  zt.resize(static_cast<size_t>(p.V) * ntk * 2 * GA);
+  for (int v = 0; v < p.V; ++v)
+    for (int t = 0; t < ntk; ++t)
+      for (int r = 0; r < 2; ++r)
+        for (int k = 0; k < GA; ++k)
+          zt[((static_cast<size_t>(v) * ntk + t) * 2 + r) * GA + k] =
+              mat(m, v, r, 2) * (static_cast<float>(t * GA + k) + 0.5f);
+  return true;
+}
+
+// Lane strides (sb, sc) of the splat: the smallest product for which any two
+// voxels of the 8 x 8 lane lattice project at least 2.0625 pixels apart along
+// one detector axis (their 2 x 2 footprints are then disjoint, with a margin
+// far above the rounding of the projected centres).
+static bool splat_strides(const double mb[2], const double mc[2], int& sb, int& sc) {
+  auto disjoint = [&](int SB, int SC) {
+    for (int a = 0; a < 8; ++a)
+      for (int b = -7; b < 8; ++b) {
+        if (a == 0 && b <= 0) continue;
+        const double d0 = std::fabs(a * SB * mb[0] + b * SC * mc[0]);
+        const double d1 = std::fabs(a * SB * mb[1] + b * SC * mc[1]);
+        if (std::max(d0, d1) < 2.0625) return false;
+      }
+    return true;
+  };
+  int best = 65;
+  for (int SB = 1; SB <= 8; ++SB)
+    for (int SC = 1; SC <= 8; ++SC)
+      if (SB * SC < best && disjoint(SB, SC)) {
+        best = SB * SC;
+        sb = SB;
+        sc = SC;
+      }
+  return best < 65;
+}
+
+// Window pitch for lane strides (sb, sc): of the width and the 16 values above
+// it, the one for which the bank model rates the lattice cheapest (the LDS
+// serves 32 lanes at a time over 32 banks, so a half-wave costs the largest
+// number of its lanes on one bank).  Over the angles of a 74 degree tilt the
+// model averages 2.1 cycles per access against 2.9 for a fixed odd pitch (and
+// the counters of that one showed 2.9).
+static int splat_pitch(const double mb[2], const double mc[2], int sb, int sc, int width) {
+  int d0[64], at[64];
+  for (int l = 0; l < 64; ++l) {
+    const double b = sb * (l >> 3), c = sc * (l & 7);
+    d0[l] = static_cast<int>(std::floor(512.31 + b * mb[0] + c * mc[0]));
+    at[l] = d0[l] * width + static_cast<int>(std::floor(512.83 + b * mb[1] + c * mc[1]));
+  }
+  int best = width, low = INT_MAX;
+  for (int pitch = width; pitch <= width + 16; ++pitch) {
+    int cost = 0;
+    for (int h = 0; h < 2; ++h) {
+      unsigned char cnt[32] = {0};
+      unsigned char mx = 0;
+      for (int l = 32 * h; l < 32 * h + 32; ++l) {
+        const unsigned char n = ++cnt[at[l] & 31];
+        mx = n > mx ? n : mx;
+        at[l] += d0[l];
+      }
+      cost += mx;
+    }
+    if (cost < low) {
+      low = cost;
+      best = pitch;
+    }
+  }
+  return best;
+}
+
+// Splat tables: march axes, lane strides, blocks and their windows.  False
+// where a view has no strides up to 8 x 8 or its windows do not fit
+// 4 x 16 KiB of LDS.
+static bool build_splat(Plan& p, const std::vector<float>& m, const std::vector<GenView>& gv,
+                        std::vector<SplatView>& views, std::vector<SplatItem>& items) {
+  const long long vox = static_cast<long long>(p.X) * p.Y * p.Z;
+  if (vox * 4 > (1LL << 30)) return false;
+  const int dims[3] = {p.X, p.Y, p.Z};
+  struct Block {
+    int p, q, lo0, lo1, t0, t1;
+  };
+  views.resize(p.V);
+  std::vector<Block> blocks;  // of all views in turn; view v's end at bend[v]
+  std::vector<size_t> bend(p.V);
+  long long planes = 0;
+  int slot = 0;
+  bool need_t = false;
+  for (int v = 0; v < p.V; ++v) {
+    SplatView g{};
+    g.a = gv[v].a;
+    const int b = g.a == 0 ? 1 : 0, c = g.a == 2 ? 1 : 2;
+    const int na = dims[g.a], nb = dims[b], nc = dims[c];
+    const double ma[2] = {mat(m, v, 0, g.a), mat(m, v, 1, g.a)};
+    const double mb[2] = {mat(m, v, 0, b), mat(m, v, 1, b)};
+    const double mc[2] = {mat(m, v, 0, c), mat(m, v, 1, c)};
+    if (!splat_strides(mb, mc, g.sb, g.sc)) return false;
+    const double det = mb[0] * mc[1] - mc[0] * mb[1];
+    const double bb = -(mc[1] * ma[0] - mc[0] * ma[1]) / det;
+    const double bc = -(-mb[1] * ma[0] + mb[0] * ma[1]) / det;
+    const double tc = na / 2;
+    g.bb = static_cast<float>(bb);
+    g.bc = static_cast<float>(bc);
+    g.tc = static_cast<float>(tc);
+    for (int k = 0; k < 8; ++k) g.m[k] = m[8 * v + k];
+    const int wb = 8 * g.sb, wc = 8 * g.sc;
+    int size[2];
+    double low[2];  // lowest corner of a block relative to its origin voxel
+    for (int r = 0; r < 2; ++r) {
+      // the shift is within half a voxel (and its rounding) of the exact one
+      low[r] = std::min(mb[r] * -0.501, mb[r] * (wb - 0.499)) +
+               std::min(mc[r] * -0.501, mc[r] * (wc - 0.499));
+      const double ext = std::fabs(mb[r]) * (wb + 0.002) + std::fabs(mc[r]) * (wc + 0.002);
+      size[r] = static_cast<int>(std::floor(ext + 2 * GEN_MARGIN)) + 3;
+    }
+    g.rows = size[0];
+    g.pitch = size[1];
+    if (g.rows * (g.pitch + 16) > 4096) return false;
+    g.pitch = splat_pitch(mb, mc, g.sb, g.sc, size[1]);
+    slot = std::max(slot, g.rows * g.pitch);
+    need_t = need_t || g.a == 2;
+    const double smb = std::fabs(bb) * (na / 2 + 1) + 1, smc = std::fabs(bc) * (na / 2 + 1) + 1;
+    const int p0 = static_cast<int>(std::floor(-smb / wb)),
+              p1 = static_cast<int>(std::floor((nb + smb) / wb));
+    const int q0 = static_cast<int>(std::floor(-smc / wc)),
+              q1 = static_cast<int>(std::floor((nc + smc) / wc));
+    for (int bp = p0; bp <= p1; ++bp)
+      for (int bq = q0; bq <= q1; ++bq) {
+        // planes where the block meets the volume: 0 <= origin + width and
+        // origin < n along both axes, half a voxel to spare for the rounding
+        double lo = 0.0, hi = na - 1.0;
+        auto meet = [&](double o, double beta, int w, int n) {
+          // -w < o + beta (t - tc) + [-0.51, 0.51] < n
+          const double l = -w - 0.51 - o, h = n + 0.51 - o;
+          if (std::fabs(beta) < 1e-12) {
+            if (!(l < 0.0 && 0.0 < h)) hi = -1.0;
+            return;
+          }
+          const double ta = tc + l / beta, tb = tc + h / beta;
+          lo = std::max(lo, std::floor(std::min(ta, tb)));
+          hi = std::min(hi, std::ceil(std::max(ta, tb)));
+        };
+        meet(static_cast<double>(bp) * wb, bb, wb, nb);
+        meet(static_cast<double>(bq) * wc, bc, wc, nc);
+        if (hi < lo) continue;
+        Block k;
+        k.p = bp * wb;
+        k.q = bq * wc;
+        k.t0 = static_cast<int>(lo);
+        k.t1 = static_cast<int>(hi) + 1;
+        int origin[2];
+        for (int r = 0; r < 2; ++r)
+          origin[r] = static_cast<int>(std::floor(ma[r] * (tc + 0.5) + mb[r] * (k.p + 0.5) +
+                                                  mc[r] * (k.q + 0.5) + mat(m, v, r, 3) + low[r] -
+                                                  0.25 - GEN_MARGIN));
+        k.lo0 = origin[0];
+        k.lo1 = origin[1];
+        // off the detector: its window would add nothing
+        if (k.lo0 >= p.D0 || k.lo0 + g.rows <= 0 || k.lo1 >= p.D1 || k.lo1 + g.pitch <= 0) continue;
+        planes += k.t1 - k.t0;
+        blocks.push_back(k);
+      }
+    views[v] = g;
+    bend[v] = blocks.size();
+  }
+  // Planes per item: about 16384 items (16 waves a SIMD) of at least 16
+  // planes, a shorter item being mostly the clearing and writing of its
+  // window; 8 planes where 16 would leave most of the chip idle.  Measured
+  // with a 74 degree tilt, items of 8192, 16384 at least 16, 16384 at least 8
+  // planes: 144^3 with 90 views 407, 380, 383 us, with 20 views 107, 108, 115
+  // us; 64^3 with 3 views (about 500 items of 16) 26.5, 26.5, 20.4 us.
+  const int most = std::max(p.X, std::max(p.Y, p.Z));
+  const long long least = planes / 16 < 1024 ? 8 : 16;
+  const int len = static_cast<int>(
+      std::min<long long>(most, std::max<long long>(least, (planes + 16383) / 16384)));
+  p.ifirst.assign(p.V + 1, 0);
+  for (int v = 0; v < p.V; ++v) {
+    views[v].first = static_cast<int>(items.size());
+    for (size_t e = v ? bend[v - 1] : 0; e < bend[v]; ++e) {
+      const Block& k = blocks[e];
+      const int n = k.t1 - k.t0, parts = (n + len - 1) / len;
+      for (int s = 0; s < parts; ++s)
+        items.push_back(SplatItem{v, k.p, k.q, k.lo0, k.lo1, k.t0 + n * s / parts,
+                                  k.t0 + n * (s + 1) / parts, 0});
+    }
+    views[v].last = static_cast<int>(items.size());
+    p.ifirst[v + 1] = views[v].last;
+  }
+  // Passes of whole views whose windows fit 128 MiB (the last-level cache
+  // holds 256 MiB), at most 65535 views (the grid's z extent).
+  const long long room = (32LL << 20) / std::max(slot, 1);
+  long long most_items = 1;
+  p.chunk.assign(1, 0);
+  for (int v = 0; v < p.V; ++v) {
+    const int c0 = p.chunk.back();
+    if (v > c0 && (p.ifirst[v + 1] - p.ifirst[c0] > room || v - c0 >= 65535)) p.chunk.push_back(v);
+    most_items = std::max<long long>(most_items, p.ifirst[v + 1] - p.ifirst[p.chunk.back()]);
+  }
+  p.chunk.push_back(p.V);
+  p.slot = slot;
+  p.need_t = need_t;
+  p.ws_floats = most_items * slot + (need_t ? vox : 0);
+  return true;
+}
+
+// General mode: one device block for every table (one allocation and one
+// copy, which set the time of making a plan).
+static int upload_tables(Plan& p, const std::vector<float>& m, const std::vector<GenView>& gv,
+                         const std::vector<SplatView>& views, const std::vector<SplatItem>& items,
+                         const std::vector<float>& zt) {
+  std::vector<char> host;
+  auto add = [&](const void* src, size_t bytes) {
+    const size_t at = (host.size() + 255) & ~static_cast<size_t>(255);
+    host.resize(at + bytes);
+    if (bytes) std::memcpy(host.data() + at, src, bytes);
+    return at;
+  };
+  const size_t am = add(m.data(), m.size() * sizeof(float));
+  const size_t ag = add(gv.data(), gv.size() * sizeof(GenView));
+  const size_t av = add(views.data(), views.size() * sizeof(SplatView));
+  const size_t ai = add(items.data(), items.size() * sizeof(SplatItem));
+  const size_t az = add(zt.data(), zt.size() * sizeof(float));
+  const int rc = dev_alloc(&p.tables, host.size());
+  if (rc) return rc;
+  SCXR_HIP(hipMemcpy(p.tables, host.data(), host.size(), hipMemcpyHostToDevice));
+  char* base = static_cast<char*>(p.tables);
+  p.mats = reinterpret_cast<float*>(base + am);
+  p.gview = reinterpret_cast<GenView*>(base + ag);
+  p.sview = reinterpret_cast<SplatView*>(base + av);
+  p.sitem = reinterpret_cast<SplatItem*>(base + ai);
+  p.zterm = reinterpret_cast<float*>(base + az);
   return SCXR_OK;
 }
 
@@ -849,9 +1560,7 @@ int create(Plan& p, int X, int Y, int Z, int V, const float* mats, int D0, int D
     for (int dax = 1; dax >= 0 && p.mode != MODE_SLICE; --dax)
       for (int sax = 0; sax < 3 && p.mode != MODE_SLICE; ++sax) try_slice(p, m, sax, dax);
   }
-  int rc = dev_alloc(reinterpret_cast<void**>(&p.mats), m.size() * sizeof(float));
-  if (rc) return rc;
-  SCXR_HIP(hipMemcpy(p.mats, m.data(), m.size() * sizeof(float), hipMemcpyHostToDevice));
+  int rc;
   if (p.mode == MODE_GENERAL) {
     std::vector<GenView> gv(V);
     for (int v = 0; v < V; ++v) {
@@ -886,10 +1595,18 @@ int create(Plan& p, int X, int Y, int Z, int V, const float* mats, int D0, int D
       g.nc = static_cast<int>(std::floor(2.0 * hc)) + 2;
       gv[v] = g;
     }
-    rc = dev_alloc(reinterpret_cast<void**>(&p.gview), V * sizeof(GenView));
-    if (rc) return rc;
-    SCXR_HIP(hipMemcpy(p.gview, gv.data(), V * sizeof(GenView), hipMemcpyHostToDevice));
+    std::vector<SplatView> views;
+    std::vector<SplatItem> items;
+    std::vector<float> zt;
+    if (!(allow_slice & 4) && gen_in_range(p, m)) {
+      p.splat = build_splat(p, m, gv, views, items);
+      p.adj_tiled = build_adj_tiles(p, m, zt);
+    }
+    return upload_tables(p, m, gv, views, items, zt);
   }
+  rc = dev_alloc(reinterpret_cast<void**>(&p.mats), m.size() * sizeof(float));
+  if (rc) return rc;
+  SCXR_HIP(hipMemcpy(p.mats, m.data(), m.size() * sizeof(float), hipMemcpyHostToDevice));
   if (p.mode == MODE_SLICE) {
     const int e = 1 - p.dax;
     std::vector<float4> g(V);
@@ -1008,8 +1725,40 @@ static int canon_to_proj(const Plan& p, const float* yc, float* y, const int32_t
                    static_cast<long long>(p.D0) * p.D1, p.D1, pred, s);
 }
 
-int forward(const Plan& p, const float* vol, float* proj, const int32_t* pred, hipStream_t s) {
+// Splat forward: ws holds the transposed volume (if a view marches along z),
+// then the windows of one pass over the items.
+static int forward_splat(const Plan& p, const float* vol, float* proj, float* ws,
+                         const int32_t* pred, hipStream_t s) {
+  const float* volt = vol;
+  float* parts = ws;
+  if (p.need_t) {
+    const int XY = p.X * p.Y;  // vol[xy][z] -> volt[z][xy]
+    const int rc = transpose(vol, ws, 1, XY, p.Z, XY, p.Z, 0, 0, 0, p.Z, 0, XY, pred, s);
+    if (rc) return rc;
+    volt = ws;
+    parts = ws + static_cast<size_t>(XY) * p.Z;
+  }
+  for (size_t c = 0; c + 1 < p.chunk.size(); ++c) {
+    const int v0 = p.chunk[c], v1 = p.chunk[c + 1];
+    const int i0 = p.ifirst[v0], i1 = p.ifirst[v1];
+    if (i1 > i0) {
+      hipLaunchKernelGGL(gen_splat_kernel, dim3(ceil_div(i1 - i0, 4)), dim3(256),
+                         4 * p.slot * sizeof(float), s, vol, volt, parts, p.sview, p.sitem, i0, i1,
+                         p.slot, p.X, p.Y, p.Z, pred);
+      SCXR_LAUNCHED("xr3d general forward");
+    }
+    hipLaunchKernelGGL(gen_splat_sum_kernel, dim3(ceil_div(p.D1, 16), ceil_div(p.D0, 16), v1 - v0),
+                       dim3(256), 0, s, parts, proj, p.sview, p.sitem, v0, i0, p.slot, p.D0, p.D1,
+                       pred);
+    SCXR_LAUNCHED("xr3d general forward window sums");
+  }
+  return SCXR_OK;
+}
+
+int forward(const Plan& p, const float* vol, float* proj, float* ws, const int32_t* pred,
+            hipStream_t s) {
   if (p.mode == MODE_GENERAL) {
+    if (p.splat && ws) return forward_splat(p, vol, proj, ws, pred, s);
     const long long npix = static_cast<long long>(p.D0) * p.D1;
     hipLaunchKernelGGL(gen_fwd_kernel, dim3(ceil_div(npix, 64), p.V), dim3(64 * GEN_W), 0, s, vol,
                        proj, p.mats, p.gview, p.X, p.Y, p.Z, p.D0, p.D1, pred);
@@ -1053,6 +1802,20 @@ int forward(const Plan& p, const float* vol, float* proj, const int32_t* pred, h
 int adjoint(const Plan& p, const float* proj, float* vol, const int32_t* pred, hipStream_t s) {
   if (p.mode == MODE_GENERAL) {
     const long long n = static_cast<long long>(p.X) * p.Y * p.Z;
+    if (p.adj_tiled) {
+      // The four waves of a workgroup take four shares of one block's views,
+      // or two of two blocks' where a share would be under 8 views: more and
+      // shorter waves, also where there are blocks enough to fill the chip.
+      // 1, 2, 4 shares: 48^3 with 90 views 81, 42, 23.5 us, 130^3 with 90
+      // views 144, 128, 123 us; 64^3 with 20 views 20.7, 12.0, 15.1 us, 144^3
+      // with 3 views 13.0, 13.0, 15.8 us.
+      const int tiles = ceil_div(p.X, GA) * ceil_div(p.Y, GA) * ceil_div(p.Z, GA);
+      const int vs = p.V >= 32 ? 4 : 2;
+      hipLaunchKernelGGL(gen_adj_tile_kernel, dim3(ceil_div(tiles, 4 / vs)), dim3(256), 0, s, proj,
+                         vol, p.mats, p.zterm, p.X, p.Y, p.Z, p.V, p.D0, p.D1, vs, pred);
+      SCXR_LAUNCHED("xr3d general adjoint (tiled)");
+      return SCXR_OK;
+    }
     hipLaunchKernelGGL(gen_adj_kernel, dim3(ceil_div(n, 256)), dim3(256), 0, s, proj, vol, p.mats,
                        p.X, p.Y, p.Z, p.V, p.D0, p.D1, pred);
     SCXR_LAUNCHED("xr3d general adjoint");
@@ -1129,7 +1892,18 @@ int scxr_xr3d_info(const scxr_xr3d_plan* plan, int32_t* out) {
 int scxr_xr3d_forward(const scxr_xr3d_plan* plan, const float* vol, float* proj,
                       const int32_t* pred, void* stream) {
   SCXR_REQUIRE(plan && vol && proj, SCXR_ERR_ARG, "null argument to xr3d_forward");
-  return xr3d::forward(plan->p, vol, proj, pred, as_stream(stream));
+  return xr3d::forward(plan->p, vol, proj, nullptr, pred, as_stream(stream));
+}
+
+int64_t scxr_xr3d_forward_ws(const scxr_xr3d_plan* plan) {
+  return plan && plan->p.splat ? static_cast<int64_t>(plan->p.ws_floats) : 0;
+}
+
+int scxr_xr3d_forward_with(const scxr_xr3d_plan* plan, const float* vol, float* proj, float* ws,
+                           const int32_t* pred, void* stream) {
+  SCXR_REQUIRE(plan && vol && proj, SCXR_ERR_ARG, "null argument to xr3d_forward_with");
+  SCXR_REQUIRE(ws || !plan->p.splat, SCXR_ERR_ARG, "xr3d_forward_with needs its workspace");
+  return xr3d::forward(plan->p, vol, proj, ws, pred, as_stream(stream));
 }
 
 int scxr_xr3d_adjoint(const scxr_xr3d_plan* plan, const float* proj, float* vol,

@@ -56,6 +56,8 @@ class XRayTransform3D(LinearOperator):
         self._plan = None
         self._allow_slice = True
         self._stage_adjoint = True
+        self._windows = True
+        self._ws_floats = 0
         super().__init__(
             input_shape=self.input_shape,
             output_shape=self.output_shape,
@@ -76,9 +78,11 @@ class XRayTransform3D(LinearOperator):
                 "scxr_xr3d_plan_create", X, Y, Z, self.output_shape[0],
                 self.matrices.ctypes.data_as(ctypes.POINTER(ctypes.c_float)),
                 self.det_shape[0], self.det_shape[1],
-                int(self._allow_slice) | (0 if self._stage_adjoint else 2), ctypes.byref(h),
+                int(self._allow_slice) | (0 if self._stage_adjoint else 2) |
+                (0 if self._windows else 4), ctypes.byref(h),
             )
             self._plan = h
+            self._ws_floats = int(lib.scxr_xr3d_forward_ws(h))
             self._finalizer = weakref.finalize(self, lib.scxr_xr3d_plan_destroy, h)
         return self._plan
 
@@ -95,7 +99,11 @@ class XRayTransform3D(LinearOperator):
         """X-ray projection (``_xray3d.py:95-100``)."""
         im = dev.input_array(im, self.input_shape, "im")
         out = dev.output_buffer(out, self.output_shape)
-        call("scxr_xr3d_forward", self.plan, im.data_ptr(), out.data_ptr(),
+        plan = self.plan
+        # general mode: detector windows, from the caching allocator so that
+        # calls on several streams (and captured ones) have their own
+        ws = dev.empty((self._ws_floats,)) if self._ws_floats else None
+        call("scxr_xr3d_forward_with", plan, im.data_ptr(), out.data_ptr(), dev.ptr(ws),
              dev.ptr(_pred.resolve(pred)), dev.stream())
         return out
 

@@ -181,3 +181,69 @@ def test_staged_adjoint_bitwise(gpu, case):
     if case in ("full", "slab"):
         assert staged
     assert torch.equal(H.T(y), Hg.T(y))
+
+
+def _tilted(shape, det, seq, n, **kw):
+    ang = np.stack(np.broadcast_arrays(74.0, np.linspace(0, 180, n, endpoint=False)), axis=-1)
+    return _mats(shape, det, seq, ang, degrees=True, **kw)
+
+
+# (shape, det, matrices): blocks of the splat are 24 voxels, of the adjoint 8;
+# march axes x, y and z; detectors smaller and larger than the object; few
+# and many views; other voxel spacings (other lane strides); spacings whose
+# windows do not fit (the gathers)
+WINDOW_CASES = {
+    "tilt": ((33, 30, 31), (40, 42), lambda s, d: _tilted(s, d, "XY", 5)),
+    "one_voxel": ((1, 1, 1), (3, 3), lambda s, d: _tilted(s, d, "XY", 3)),
+    "edges": ((24, 8, 25), (16, 17), lambda s, d: _tilted(s, d, "XY", 4)),
+    "march_z": ((17, 49, 40), (60, 31), lambda s, d: _mats(
+        s, d, "XY", np.random.default_rng(1).uniform(-0.3, 0.3, (4, 2)))),
+    "march_x": ((47, 26, 23), (33, 50), lambda s, d: _mats(
+        s, d, "YX", np.pi / 2 + np.random.default_rng(2).uniform(-0.3, 0.3, (4, 2)))),
+    "any": ((40, 28, 36), (48, 48), lambda s, d: _mats(
+        s, d, "XYZ", np.random.default_rng(3).uniform(0, np.pi, (70, 3)))),
+    "fine": ((40, 40, 40), (24, 24), lambda s, d: _tilted(s, d, "XY", 4,
+                                                          voxel_spacing=[0.6, 0.6, 0.6])),
+    "stretched": ((20, 24, 18), (40, 40), lambda s, d: _tilted(s, d, "XY", 4,
+                                                               voxel_spacing=[1.0, 1.3, 0.8])),
+    "too_wide": ((12, 12, 12), (64, 64), lambda s, d: _tilted(s, d, "XY", 3,
+                                                              voxel_spacing=[4.0, 4.0, 4.0])),
+}
+
+
+@pytest.mark.parametrize("case", list(WINDOW_CASES))
+def test_general_windows(gpu, case):
+    """General-mode projections through detector windows in LDS against the
+    oracle and the gathers from global memory (sums of the same terms in
+    another order: a few float32 roundings of relative size 6e-8 each, as
+    the bars of the other parity tests); twice the same bits; into an output
+    that is not 16-byte aligned; and on a side stream while the default
+    stream projects another volume with the same operator."""
+    shape, det, mk = WINDOW_CASES[case]
+    M = mk(shape, det)
+    H = XRayTransform3D(shape, M, det)
+    G = XRayTransform3D(shape, M, det)
+    G._windows = False
+    assert H.info()["mode"] == "general"
+    rng = np.random.default_rng(11)
+    x = torch.as_tensor(rng.random(shape).astype(np.float32), device="cuda")
+    y = torch.as_tensor(rng.standard_normal(H.output_shape).astype(np.float32), device="cuda")
+    p, b = H(x), H.adj(y)
+    e = (rel_l2(p.cpu(), X.project_3d(x.cpu().numpy(), H.matrices, det)),
+         rel_l2(b.cpu(), X.back_project_3d(y.cpu().numpy(), H.matrices, shape)),
+         rel_l2(p.cpu(), G(x).cpu()), rel_l2(b.cpu(), G.adj(y).cpu()))
+    print(f"  {case}: oracle fwd {e[0]:.2e} adj {e[1]:.2e}, gathers fwd {e[2]:.2e} adj {e[3]:.2e}",
+          flush=True)
+    assert max(e) <= 1e-5
+    assert torch.equal(p, H(x)) and torch.equal(b, H.adj(y))
+    off = torch.empty(b.numel() + 1, device="cuda")[1:]
+    assert torch.equal(H.back_project(y, out=off).reshape(shape), b)
+    off = torch.empty(p.numel() + 1, device="cuda")[1:]
+    assert torch.equal(H.project(x, out=off).reshape(p.shape), p)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ps = [H(x) for _ in range(4)]
+    pd = [H(2.0 * x) for _ in range(4)]
+    torch.cuda.synchronize()
+    assert all(torch.equal(q, p) for q in ps) and all(torch.equal(q, 2.0 * p) for q in pd)
