@@ -187,6 +187,7 @@ int create(Batch& b, int ns, const int32_t* dims, const float* angles, const dou
     to += tx * ty;
     wo += Gs;
   }
+  rw.resize(rw.size() + xr2d::RW_PAD, 1.0);  // read past the last slice's end
   b.n_img = io;
   b.n_sino = so;
   b.n_tiles = to;

@@ -77,6 +77,17 @@ __device__ __forceinline__ int cvt_flr_i32(float x) {
   return r;
 }
 
+// LDS addresses as integers, for kernels that form them with their own
+// arithmetic (a generic pointer costs an extra add per access).
+typedef __attribute__((address_space(3))) float LdsFloat;
+__device__ __forceinline__ int lds_address(const float* p) {
+  return static_cast<int>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const float*)p));
+}
+__device__ __forceinline__ LdsFloat* lds_at(int address) {
+  return reinterpret_cast<LdsFloat*>(static_cast<uintptr_t>(static_cast<unsigned>(address)));
+}
+
 // Sum of one double per thread over a 256-thread workgroup (fixed order:
 // wave shuffles, then the 4 wave sums left to right).  Thread 0 gets the
 // result.  `sh` holds 4 doubles of LDS.

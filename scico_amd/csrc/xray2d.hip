@@ -310,12 +310,14 @@ int create(Plan& p, int M, int N, int A, int D, const double* x0, const double* 
   p.n_groups = static_cast<int>(h.groups.size());
   p.adj_w = h.adj_w;
   const std::vector<float4>& geom = h.geom;
-  const std::vector<double>& rw = h.rw;
+  std::vector<double>& rw = h.rw;
   const std::vector<int4>& groups = h.groups;
   const std::vector<int>& order = h.order;
   const std::vector<float>& clo = h.clo;
 
-  size_t bytes_geom = sizeof(float4) * A, bytes_rw = sizeof(double) * A;
+  // (the adjoint reads up to RW_PAD entries past the last view's)
+  rw.resize(A + RW_PAD, 1.0);
+  size_t bytes_geom = sizeof(float4) * A, bytes_rw = sizeof(double) * rw.size();
   size_t bytes_groups = sizeof(int4) * groups.size(), bytes_order = sizeof(int) * A;
   size_t bytes_clo = sizeof(float) * A;
   // block index -> forward group, balanced over the CUs
@@ -911,16 +913,22 @@ static hipError_t fwd_allow_lds(int bytes) {
 }
 
 // Adjoint (back projection).  One workgroup per pixel tile of ADJ_TI rows
-// and ADJ_TJ * PPT columns (each thread owns PPT pixels of one row, ADJ_TJ
-// apart); views are processed in chunks of ADJ_VC.  For each view the
+// and ADJ_TJ * PPT columns (each thread owns PPT pixels of one column,
+// ADJ_TI / PPT rows apart); views are processed in chunks of ADJ_VC.  For each view the
 // detector window reachable from the tile (W <= 64 bins, zero outside
 // [0, D)) and the view's geometry are staged in LDS, then every thread
 // gathers its pixels' two bins.  The windows of the next chunk are
 // prefetched into registers while the current chunk is computed, so the
 // global-load latency is hidden behind the gather arithmetic.  The two sums
 // of _xray2d.py:299-304 are kept separately and added at the end.
-// Px = (Pxmin + P0 i) + P1 j keeps the reference order; the row term
-// Pxmin + P0 i is shared by a thread's pixels.
+// Px = (Pxmin + P0 i) + P1 j keeps the reference order; the row terms
+// Pxmin + P0 i are evaluated once per view and row pair while the view is
+// staged, and one 16-byte record gives a thread both of its rows' terms, P1
+// and the window address; 1 / width comes by scalar loads.  VALU issue bounds
+// this kernel (all of the nominal rate): 13.2 -> 11.7 instructions per pixel
+// and view took 512^2 with 720 views from 61.9 to 56.7 us, bitwise unchanged.
+// (Row terms as separate 8-byte reads cost the LDS more than the VALU gained:
+// 66 us.)
 //
 // Window origin of view a for the tile at (i0, j0):
 //   lo = floor(P0 * i0 + P1 * j0 + clo[a]),
@@ -928,14 +936,13 @@ static hipError_t fwd_allow_lds(int bytes) {
 // a lower bound of floor(Px) over the tile with a one-bin margin for the
 // float32 rounding of Px; W covers the tile's projected extent plus the
 // margins, so every pixel's bins ind and ind + 1 lie inside the window.
-struct __align__(16) ViewLds {
-  float Pxmin, P0, P1;
-  // byte offset in win_all of detector bin 0 for this view: an integer
+struct __align__(16) ViewLds {  // of one view and two rows of a tile
+  float row[2];  // row terms of tile rows r and r + 8
+  float P1;
+  // LDS address of detector bin 0 in this view's window: an integer
   // (float32 bits when the weights use floor, so that 4 fl + base4 is one
   // exact float multiply-add; int32 when they use the fraction instruction)
   uint32_t base4;
-  double rw;
-  double pad;
 };
 
 // One adjoint tile (tile row by, column bx; dot partial written at index
@@ -952,51 +959,59 @@ __device__ __forceinline__ void adj_tile(const float* __restrict__ sino, float* 
                                          int dot_i) {
   constexpr int VPW = ADJ_VC / 4;  // views staged per wave
   __shared__ float win_all[VS][ADJ_VC * ADJ_WFAST];
-  __shared__ ViewLds gv_all[VS][ADJ_VC];
+  // view records of the current and the next chunk
+  __shared__ ViewLds gv_all[2][VS][ADJ_VC][8];
   __shared__ double red[4 * VS];
+  constexpr int TR = ADJ_TI / PPT;  // rows between a thread's pixels
   const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), t = threadIdx.x & 255;
   float* win = win_all[grp];
-  ViewLds* gv = gv_all[grp];
-  const int tx = t % ADJ_TJ, ty = t / ADJ_TJ;
+  const int tx = t % (ADJ_TJ * PPT), ty = t / (ADJ_TJ * PPT);
   const int i0 = by * ADJ_TI, j0 = bx * (ADJ_TJ * PPT);
-  const int i = i0 + ty;
-  int j[PPT];
+  const int j = j0 + tx;
+  int i[PPT];
   bool inside[PPT];
-  float fj[PPT];
   bool any = false;
 #pragma unroll
   for (int q = 0; q < PPT; ++q) {
-    j[q] = j0 + tx + ADJ_TJ * q;
-    inside[q] = (i < M) && (j[q] < N);
-    fj[q] = static_cast<float>(j[q]);
+    i[q] = i0 + ty + TR * q;
+    inside[q] = (i[q] < M) && (j < N);
     any = any || inside[q];
   }
-  const float fi = static_cast<float>(i);
+  const float fj = static_cast<float>(j);
   const float fi0 = static_cast<float>(i0), fj0 = static_cast<float>(j0);
   const int wave = t >> 6, lane = t & 63;
-  const char* winb = reinterpret_cast<const char*>(&win_all[0][0]);
-  const int gbase4 = grp * (ADJ_VC * ADJ_WFAST * 4);
+  const int gbase4 = lds_address(win);
   // this group's views [vb, ve); every group runs the same number of chunks
   const int share = (A + VS - 1) / VS;
   const int vb = min(A, grp * share), ve = min(A, vb + share);
   const int nchunk = (share + ADJ_VC - 1) / ADJ_VC;
 
   // Staging is spread over the lanes: lane 8 sq + sw of a wave handles
-  // view slot sv = wave + 4 sq of a chunk; it computes that view's window
-  // origin and writes word sw of its LDS record.  The windows themselves
+  // view slot sv = wave + 4 sq of a chunk: it computes that view's window
+  // origin and writes its record for tile rows sw and sw + 8.  The windows themselves
   // are read by the whole wave, one view at a time, through a buffer
   // resource bounded to the view's sinogram row, so bins outside [0, D)
   // read zero.
   const int wv = __builtin_amdgcn_readfirstlane(wave);
   const int sq = lane >> 3, sw = lane & 7, sv = wv + 4 * sq;
   float pf[VPW];
-  int lo_nx = 0;  // window origin of this lane's view slot in the prefetched chunk
-  auto prefetch = [&](int a0) {
+  auto prefetch = [&](int a0, int buf) {
     const int a = a0 + sv;
     const int as = a < ve ? a : 0;
     const float4 g = geom[as];
     const int lo = static_cast<int>(floorf(fmaf(g.y, fi0, fmaf(g.z, fj0, clo[as]))));
-    lo_nx = a < ve ? lo : 0;
+    // padded views get zero geometry
+    const bool real = a < ve;
+    const int b4 = gbase4 + 4 * (sv * W - (real ? lo : 0));
+    ViewLds rec;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float ti = __fadd_rn(g.x, __fmul_rn(g.y, static_cast<float>(i0 + sw + 8 * h)));
+      rec.row[h] = real ? ti : 0.0f;
+    }
+    rec.P1 = real ? g.z : 0.0f;
+    rec.base4 = FR ? static_cast<uint32_t>(b4) : __float_as_uint(static_cast<float>(b4));
+    gv_all[buf][grp][sv][sw] = rec;
 #pragma unroll
     for (int q = 0; q < VPW; ++q) {
       const int aq = a0 + wv + 4 * q;
@@ -1013,7 +1028,7 @@ __device__ __forceinline__ void adj_tile(const float* __restrict__ sino, float* 
   float acc0[PPT], acc1[PPT];
 #pragma unroll
   for (int q = 0; q < PPT; ++q) acc0[q] = acc1[q] = 0.0f;
-  prefetch(vb);
+  prefetch(vb, 0);
   for (int c = 0; c < nchunk; ++c) {
     const int a0 = vb + c * ADJ_VC;
     const int nv = max(0, min(ADJ_VC, ve - a0));
@@ -1024,43 +1039,38 @@ __device__ __forceinline__ void adj_tile(const float* __restrict__ sino, float* 
       const int v = wv + 4 * q;
       if (v < nv4 && lane < W) win[v * W + lane] = v < nv ? pf[q] : 0.0f;
     }
-    if (sv < nv4) {
-      // record words: Pxmin, P0, P1, base4, rw (2 words), pad (2 words);
-      // padded views get zero geometry and rw = 1
-      const bool real = sv < nv;
-      const int a = real ? a0 + sv : 0;
-      uint32_t word = 0;
-      if (sw < 3) {
-        word = real ? reinterpret_cast<const uint32_t*>(geom)[4 * a + sw] : 0u;
-      } else if (sw == 3) {
-        const int b4 = gbase4 + 4 * (sv * W - (real ? lo_nx : 0));
-        word = FR ? static_cast<uint32_t>(b4) : __float_as_uint(static_cast<float>(b4));
-      } else if (sw < 6) {
-        word = real ? reinterpret_cast<const uint32_t*>(rwt)[2 * a + (sw - 4)]
-                    : (sw == 5 ? 0x3ff00000u : 0u);
-      }
-      reinterpret_cast<uint32_t*>(gv)[8 * sv + sw] = word;
-    }
     __syncthreads();
-    if (a0 + ADJ_VC < ve) prefetch(a0 + ADJ_VC);
+    // (the other buffer's last readers passed the barrier above)
+    if (a0 + ADJ_VC < ve) prefetch(a0 + ADJ_VC, (c + 1) & 1);
+    const ViewLds(*gv)[8] = gv_all[c & 1][grp];
     if (any) {
       for (int v = 0; v < nv4; v += 4) {
         float w[4][PPT];
         int k[4][PPT];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          const ViewLds tv = gv[v + u];
-          const float ti = __fadd_rn(tv.Pxmin, __fmul_rn(tv.P0, fi));
+          const ViewLds tv = gv[v + u][ty & 7];
+          // 1 / width of the view: scalar loads (the table is padded: a
+          // padded view's window is zero, so any finite value serves it)
+          const double rw = rwt[a0 + v + u];
+          float ti[PPT];
+          if constexpr (PPT == 2) {
+            ti[0] = tv.row[0];
+            ti[1] = tv.row[1];
+          } else {
+            ti[0] = ty < 8 ? tv.row[0] : tv.row[1];
+          }
+          const float tj = __fmul_rn(tv.P1, fj);
 #pragma unroll
           for (int q = 0; q < PPT; ++q) {
-            const float Px = __fadd_rn(ti, __fmul_rn(tv.P1, fj[q]));
+            const float Px = __fadd_rn(ti[q], tj);
             if (FR) {
-              w[u][q] = weight_frac(Px, tv.rw);
+              w[u][q] = weight_frac(Px, rw);
               k[u][q] = (cvt_flr_i32(Px) << 2) + static_cast<int>(tv.base4);
             } else {
               const float fl = floorf(Px);
               const float dd = __fsub_rn(1.0f, __fsub_rn(Px, fl));
-              w[u][q] = div_rn_sat(dd, tv.rw);
+              w[u][q] = div_rn_sat(dd, rw);
               k[u][q] = static_cast<int>(
                   static_cast<unsigned>(__fmaf_rn(fl, 4.0f, __uint_as_float(tv.base4))));
             }
@@ -1071,8 +1081,9 @@ __device__ __forceinline__ void adj_tile(const float* __restrict__ sino, float* 
         for (int u = 0; u < 4; ++u)
 #pragma unroll
           for (int q = 0; q < PPT; ++q) {
-            y0[u][q] = *reinterpret_cast<const float*>(winb + k[u][q]);
-            y1[u][q] = *reinterpret_cast<const float*>(winb + k[u][q] + 4);
+            const LdsFloat* y = lds_at(k[u][q]);
+            y0[u][q] = y[0];
+            y1[u][q] = y[1];
           }
 #pragma unroll
         for (int u = 0; u < 4; ++u)
@@ -1115,12 +1126,12 @@ __device__ __forceinline__ void adj_tile(const float* __restrict__ sino, float* 
       if (!inside[q]) continue;
       float v = __fadd_rn(acc0[q], acc1[q]);
       if (epi.kind == EPI_GRAM) {  // (rho * C^T C)(p) + A^T A p   (_admmaux.py:222-229)
-        v = __fadd_rn(__fmul_rn(epi.rho, fd::gram2d(epi.p, M, N, i, j[q], circ)), v);
+        v = __fadd_rn(__fmul_rn(epi.rho, fd::gram2d(epi.p, M, N, i[q], j, circ)), v);
       } else if (epi.kind == EPI_RHS) {  // A^T y + rho * C^T (z - u)   (_admmaux.py:245-256)
-        v = __fadd_rn(v, __fmul_rn(epi.rho, fd::adj2d_diff(epi.z, epi.u, M, N, i, j[q], circ)));
+        v = __fadd_rn(v, __fmul_rn(epi.rho, fd::adj2d_diff(epi.z, epi.u, M, N, i[q], j, circ)));
       }
-      out[static_cast<size_t>(i) * N + j[q]] = v;
-      if (epi.dot_ws) dot += static_cast<double>(epi.p[static_cast<size_t>(i) * N + j[q]]) * v;
+      out[static_cast<size_t>(i[q]) * N + j] = v;
+      if (epi.dot_ws) dot += static_cast<double>(epi.p[static_cast<size_t>(i[q]) * N + j]) * v;
     }
   }
   if (epi.dot_ws) {  // per-tile partial of sum p * out (CG curvature p^T A p)
@@ -1318,8 +1329,11 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void fwd_batch_kernel(BatchTabs t, 
   }
 }
 
+// At least six waves per SIMD: 73 registers instead of 89, so that two
+// workgroups of 12 waves share a CU (32 ragged slices, both directions:
+// 1261 -> 1148 us).
 template <int PPT, bool FR, int VS>
-__global__ __launch_bounds__(256 * VS) __attribute__((amdgpu_waves_per_eu(4))) void adj_batch_kernel(BatchTabs t, const float* __restrict__ sino,
+__global__ __launch_bounds__(256 * VS) __attribute__((amdgpu_waves_per_eu(6))) void adj_batch_kernel(BatchTabs t, const float* __restrict__ sino,
                                                         float* __restrict__ out, BatchEpi be,
                                                         const int32_t* pred, int pstride) {
   for (int it = blockIdx.x; it < t.na; it += gridDim.x) {

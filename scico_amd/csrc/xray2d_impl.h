@@ -17,6 +17,7 @@ constexpr int ADJ_TJ = 16;
 constexpr int ADJ_VC = 32;
 constexpr int ADJ_VS = 3;  // groups of 256 threads splitting the views of a tile
 constexpr int ADJ_WFAST = 64;  // window slots (one per lane)
+constexpr int RW_PAD = 3;      // entries that end a table of 1 / width per view
 
 // Forward: FWD_WAVES waves x ch chains (2, or 1 for wide detectors)
 // private LDS copies of (D + 4) bins per owned view.
@@ -58,7 +59,7 @@ struct Plan {
   bool fwd_generic = false, adj_generic = false;
   void* dev_block = nullptr;  // device tables (one allocation)
   float4* geom = nullptr;     // (Pxmin, P0, P1, width) per view
-  double* rw = nullptr;       // RN64(1 / width) per view
+  double* rw = nullptr;       // RN64(1 / width) per view, RW_PAD more entries
   int4* groups = nullptr;     // forward groups: (first, count, class, 0)
   int* order = nullptr;       // views grouped by class
   int* gblock = nullptr;      // forward group of each forward block index

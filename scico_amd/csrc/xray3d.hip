@@ -588,16 +588,6 @@ __device__ __forceinline__ float axis_share(float P, int& ul) {
   return fminf(__fsub_rn(ceilf(left), left), 0.5f);
 }
 
-typedef __attribute__((address_space(3))) float LdsFloat;
-__device__ __forceinline__ int lds_address(const float* p) {
-  return static_cast<int>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const float*)p));
-}
-
-__device__ __forceinline__ LdsFloat* lds_at(int address) {
-  return reinterpret_cast<LdsFloat*>(static_cast<uintptr_t>(static_cast<unsigned>(address)));
-}
-
 // LDS address row * u0 + 4 * u1 + base of a window pixel in two instructions
 // (row bytes in a vector register, the window's base in a scalar one); left
 // to itself the compiler takes a 32-bit multiply at quarter rate.
