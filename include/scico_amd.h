@@ -325,10 +325,10 @@ int scxr_tv_norm(int32_t ndim, const int32_t* shape, const float* x, int32_t iso
                  int32_t circular, double* out, double* ws, const int32_t* pred, void* stream);
 
 /* ------------------------------- fused AcceleratedPGM deconvolution --
- * One AcceleratedPGM-TV iteration (scico/optimize/_pgm.py:183-252) on a
- * 1024 x 1024 image with f = 0.5 ||A x - y||^2, A a real CircularConvolve,
- * g = lam TV (2D), constant step 1/L, in four launches that also record
- * its statistics row:
+ * One AcceleratedPGM-TV iteration (scico/optimize/_pgm.py:183-252) on one
+ * image (both sides of 3 or more pixels) with f = 0.5 ||A x - y||^2, A a real
+ * CircularConvolve, g = lam TV (2D), constant step 1/L, in four launches that
+ * also record its statistics row:
  *   scxr_tv_prox_apgm:  x <- prox_{tau TV}(u) (tau = lam / L), the
  *     partials of ||x - v||^2 and of TV(x), v <- x + c (x - x_prev)
  *     (c = (t_k - 1) / t_{k+1});
@@ -346,6 +346,12 @@ int32_t scxr_tv_prox_apgm_parts(int32_t M, int32_t N);
 int scxr_tv_prox_apgm(int32_t M, int32_t N, const float* u, float* x, float* v, float tau,
                       int32_t isotropic, int32_t circular, float c, double* res_ws,
                       double* tv_ws, const int32_t* pred, void* stream);
+/* The same from x and v into x_new and v_new (x_new = x and v_new = v:
+ * in place; otherwise x and v are only read). */
+int scxr_tv_prox_apgm_to(int32_t M, int32_t N, const float* u, const float* x, const float* v,
+                         float* x_new, float* v_new, float tau, int32_t isotropic,
+                         int32_t circular, float c, double* res_ws, double* tv_ws,
+                         const int32_t* pred, void* stream);
 /* hist[2 row] = obj_scale * sum(obj) + lam * sum(tv), hist[2 row + 1] =
  * sqrt(sum(res)), row = *counter (skipped at or beyond hist_cap), then
  * *counter += 1. */
@@ -377,18 +383,27 @@ int scxr_cconv_spectrum(const scxr_cconv_plan* plan, float* out, void* stream);
  * (_circconv.py:188-209). */
 int scxr_cconv_apply(const scxr_cconv_plan* plan, const float* x, float* y, int32_t adjoint,
                      const int32_t* pred, void* stream);
-/* Gradient step of the fused AcceleratedPGM iteration, for a plan of one
- * 1024 x 1024 real convolution (SCXR_ERR_UNSUPPORTED otherwise); G = A^T A
- * is the convolution by gs = |Hs|^2 (Hs the Hermitian part of the spectrum
- * on the half grid k0 < 1024, k1 < 513; gs float32 and Yh complex64 are
- * stored transposed, gs[k1 1024 + k0]):
+/* Fused AcceleratedPGM deconvolution, for a plan of one real two-axis
+ * convolution F0 x F1 (both 3 or more; SCXR_ERR_UNSUPPORTED otherwise).
+ * Half grid: k0 < F0, k1 < H1 = F1/2 + 1; its arrays are stored [k0 H1 + k1],
+ * at 1024 x 1024 transposed, [k1 1024 + k0].
+ * scxr_cconv_apgm_parts: objective partials of a gradient step (workgroups
+ * of its column pass); 0 if the plan is not supported.
+ * scxr_cconv_apgm_setup: gs (F0 H1 floats) = |Hs|^2, Hs the Hermitian part of
+ * the spectrum, and Yh (F0 H1 complex64) = fft2(y), both evaluated in float64
+ * and rounded once; ws: scxr_cconv_apgm_setup_ws(plan) doubles. */
+int32_t scxr_cconv_apgm_parts(const scxr_cconv_plan* plan);
+int64_t scxr_cconv_apgm_setup_ws(const scxr_cconv_plan* plan);
+int scxr_cconv_apgm_setup(const scxr_cconv_plan* plan, const float* y, float* gs, float* Yh,
+                          double* ws, void* stream);
+/* Gradient step of the fused iteration; G = A^T A is the convolution by gs:
  *   gx <- G x;  u <- v + b ((1 + c) gx - c gx_prev - aty)
  * with gx_prev the gx on entry (G v for v = x + c (x - x_prev), by
  * linearity; c = 0 at the first step, with gx zero), aty = A^T y and
- * b = -1/L.  If obj is non-NULL, obj[k] (513 doubles) = w_k sum over the
- * column k of |Hs X - Yh|^2 (X = fft2(x), Yh = fft2(y) on the half grid;
- * w_k = 1 for k = 0 and 512, else 2), so that sum(obj) / 1024^2
- * = ||A x - y||^2 (Parseval).  No reference counterpart as one call: it
+ * b = -1/L.  If obj is non-NULL, obj[g] (scxr_cconv_apgm_parts doubles) =
+ * sum over the columns k1 of workgroup g of w |Hs X - Yh|^2 (X = fft2(x) on
+ * the half grid; w = 1 for k1 = 0 and 2 k1 = F1, else 2), so that
+ * sum(obj) / (F0 F1) = ||A x - y||^2 (Parseval).  No reference counterpart as one call: it
  * is the gradient of SquaredL2Loss (scico/loss.py:208-209) and the
  * objective evaluation of _pgm.py:151-156, one convolution instead of
  * three. */
@@ -397,11 +412,11 @@ int scxr_cconv_apgm_grad(const scxr_cconv_plan* plan, const float* x, const floa
                          const float* aty, float c, float b, float* u, const int32_t* pred,
                          void* stream);
 /* scxr_cconv_apgm_grad with obj and Yh required, followed in its last
- * launch by the statistics row of scxr_apgm_itstat(obj, 513, obj_scale,
+ * launch by the statistics row of scxr_apgm_itstat(obj, parts, obj_scale,
  * tv, ntv, lam, res, nres, hist, counter, hist_cap): the row sums the
  * objective partials of this call and the prox partials (tv, res) that
  * earlier work on the stream wrote.  The sums' double roundings may differ
- * from scxr_apgm_itstat's (512 threads instead of 1024).  A call whose
+ * from scxr_apgm_itstat's (fewer threads than its 1024).  A call whose
  * predicate is 0 records no row.  No reference counterpart as one call
  * (see scxr_cconv_apgm_grad; the row is _pgm.py:242-248's itstat). */
 int scxr_cconv_apgm_grad_itstat(const scxr_cconv_plan* plan, const float* x, const float* gs,

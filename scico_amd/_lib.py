@@ -163,6 +163,13 @@ SIGNATURES = [
     ("scxr_tv_prox_apgm", c_int32,
      [c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_float, c_int32, c_int32, c_float,
       c_void_p, c_void_p, c_void_p, c_void_p]),
+    ("scxr_tv_prox_apgm_to", c_int32,
+     [c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_int32,
+      c_int32, c_float, c_void_p, c_void_p, c_void_p, c_void_p]),
+    ("scxr_cconv_apgm_parts", c_int32, [c_void_p]),
+    ("scxr_cconv_apgm_setup_ws", c_int64, [c_void_p]),
+    ("scxr_cconv_apgm_setup", c_int32,
+     [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     ("scxr_apgm_itstat", c_int32,
      [c_void_p, c_int32, c_double, c_void_p, c_int32, c_double, c_void_p, c_int32, c_void_p,
       c_void_p, c_int32, c_void_p]),

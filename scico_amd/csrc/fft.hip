@@ -75,6 +75,23 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
 
 __device__ __forceinline__ float2 conjf2(float2 a) { return make_float2(a.x, -a.y); }
 
+// The same in float64, for the spectra that a solver prepares once.
+__device__ __forceinline__ double2 cmul(double2 a, double2 b) {
+  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+}
+__device__ __forceinline__ double2 conjf2(double2 a) { return make_double2(a.x, -a.y); }
+template <class V>
+using Real = decltype(V::x);
+template <class V>
+__device__ __forceinline__ V cmake(Real<V> x, Real<V> y) {
+  V v;
+  v.x = x;
+  v.y = y;
+  return v;
+}
+__device__ __forceinline__ float fma_(float a, float b, float c) { return fmaf(a, b, c); }
+__device__ __forceinline__ double fma_(double a, double b, double c) { return fma(a, b, c); }
+
 // Power-of-two lengths: Stockham auto-sort passes of radix 16 (after one
 // pass of radix 2, 4 or 8 for log2 n mod 4) on lpb lines held in one LDS
 // buffer.  Each
@@ -94,13 +111,20 @@ __device__ __forceinline__ float2 csub(float2 a, float2 b) {
   return make_float2(__fsub_rn(a.x, b.x), __fsub_rn(a.y, b.y));
 }
 
+__device__ __forceinline__ double2 cadd(double2 a, double2 b) {
+  return make_double2(a.x + b.x, a.y + b.y);
+}
+__device__ __forceinline__ double2 csub(double2 a, double2 b) {
+  return make_double2(a.x - b.x, a.y - b.y);
+}
+
 // 4-point DFT of a[0], a[s], a[2 s], a[3 s] in place (natural order).
-template <int S, int N>
-__device__ __forceinline__ void dft4_strided(float2 (&v)[N], int o, bool inv) {
-  const float2 s02 = cadd(v[o], v[o + 2 * S]), d02 = csub(v[o], v[o + 2 * S]);
-  const float2 s13 = cadd(v[o + S], v[o + 3 * S]), d13 = csub(v[o + S], v[o + 3 * S]);
+template <int S, int N, class V>
+__device__ __forceinline__ void dft4_strided(V (&v)[N], int o, bool inv) {
+  const V s02 = cadd(v[o], v[o + 2 * S]), d02 = csub(v[o], v[o + 2 * S]);
+  const V s13 = cadd(v[o + S], v[o + 3 * S]), d13 = csub(v[o + S], v[o + 3 * S]);
   // -i d13 (forward) or +i d13 (inverse)
-  const float2 t = inv ? make_float2(-d13.y, d13.x) : make_float2(d13.y, -d13.x);
+  const V t = inv ? cmake<V>(-d13.y, d13.x) : cmake<V>(d13.y, -d13.x);
   v[o] = cadd(s02, s13);
   v[o + 2 * S] = csub(s02, s13);
   v[o + S] = cadd(d02, t);
@@ -110,15 +134,14 @@ __device__ __forceinline__ void dft4_strided(float2 (&v)[N], int o, bool inv) {
 // exp(-2 pi i m / 16) = (cos(pi m / 8), -sin(pi m / 8)) for m = 0 .. 15,
 // conjugated for the inverse: the internal twiddles of the 8- and 16-point
 // butterflies (m is a compile-time constant there, so the tables fold).
-__device__ __forceinline__ float2 w16(int m, bool inv) {
-  constexpr float c1 = 0.92387953251128674f, s1 = 0.38268343236508978f;
-  constexpr float h = 0.70710678118654752f;
-  constexpr float cs[16] = {1.0f, c1, h, s1, 0.0f, -s1, -h, -c1,
-                            -1.0f, -c1, -h, -s1, 0.0f, s1, h, c1};
-  constexpr float sn[16] = {0.0f, s1, h, c1, 1.0f, c1, h, s1,
-                            0.0f, -s1, -h, -c1, -1.0f, -c1, -h, -s1};
-  const float2 w = make_float2(cs[m & 15], -sn[m & 15]);
-  return inv ? make_float2(w.x, -w.y) : w;
+template <class V>
+__device__ __forceinline__ V w16(int m, bool inv) {
+  using T = Real<V>;
+  constexpr T c1 = static_cast<T>(0.92387953251128674), s1 = static_cast<T>(0.38268343236508978);
+  constexpr T h = static_cast<T>(0.70710678118654752), o = 1, z = 0;
+  constexpr T cs[16] = {o, c1, h, s1, z, -s1, -h, -c1, -o, -c1, -h, -s1, z, s1, h, c1};
+  constexpr T sn[16] = {z, s1, h, c1, o, c1, h, s1, z, -s1, -h, -c1, -o, -c1, -h, -s1};
+  return cmake<V>(cs[m & 15], inv ? sn[m & 15] : -sn[m & 15]);
 }
 
 // cos and sin of 2 pi k / R for k <= R / 2: the odd butterflies' constants
@@ -127,24 +150,24 @@ template <int R>
 struct OddTrig;
 template <>
 struct OddTrig<3> {
-  static constexpr float cs[2] = {1.0f, -0.5f};
-  static constexpr float sn[2] = {0.0f, 0.86602540378443865f};
+  static constexpr double cs[2] = {1.0, -0.5};
+  static constexpr double sn[2] = {0.0, 0.86602540378443865};
 };
 template <>
 struct OddTrig<5> {
-  static constexpr float cs[3] = {1.0f, 0.30901699437494742f, -0.80901699437494742f};
-  static constexpr float sn[3] = {0.0f, 0.95105651629515357f, 0.58778525229247313f};
+  static constexpr double cs[3] = {1.0, 0.30901699437494742, -0.80901699437494742};
+  static constexpr double sn[3] = {0.0, 0.95105651629515357, 0.58778525229247313};
 };
 template <>
 struct OddTrig<7> {
-  static constexpr float cs[4] = {1.0f, 0.62348980185873353f, -0.22252093395631440f,
-                                  -0.90096886790241913f};
-  static constexpr float sn[4] = {0.0f, 0.78183148246802981f, 0.97492791218182361f,
-                                  0.43388373911755812f};
+  static constexpr double cs[4] = {1.0, 0.62348980185873353, -0.22252093395631440,
+                                   -0.90096886790241913};
+  static constexpr double sn[4] = {0.0, 0.78183148246802981, 0.97492791218182361,
+                                   0.43388373911755812};
 };
 
-template <int R>
-__device__ __forceinline__ void dft_small(float2 (&v)[R], bool inv) {
+template <int R, class V>
+__device__ __forceinline__ void dft_small(V (&v)[R], bool inv) {
   if constexpr (R == 16 || R == 8) {
     // R = 4 Q: inputs n1 + 4 n2 ... as R = Q x 4 with Q = R / 4:
     // DFT over the Q-strided groups, twiddle, then 4- (or 2-) point DFTs.
@@ -156,18 +179,18 @@ __device__ __forceinline__ void dft_small(float2 (&v)[R], bool inv) {
 #pragma unroll
     for (int n1 = 1; n1 < Q; ++n1)
 #pragma unroll
-      for (int k2 = 1; k2 < 4; ++k2) v[n1 + Q * k2] = cmul(v[n1 + Q * k2], w16(n1 * k2 * (16 / R), inv));
+      for (int k2 = 1; k2 < 4; ++k2) v[n1 + Q * k2] = cmul(v[n1 + Q * k2], w16<V>(n1 * k2 * (16 / R), inv));
     // step 3: for each k2, Q-point DFT over n1; output k = k2 + 4 k1
-    float2 o[R];
+    V o[R];
 #pragma unroll
     for (int k2 = 0; k2 < 4; ++k2) {
       if constexpr (Q == 4) {
-        float2 g[4] = {v[Q * k2], v[1 + Q * k2], v[2 + Q * k2], v[3 + Q * k2]};
+        V g[4] = {v[Q * k2], v[1 + Q * k2], v[2 + Q * k2], v[3 + Q * k2]};
         dft4_strided<1, 4>(g, 0, inv);
 #pragma unroll
         for (int k1 = 0; k1 < 4; ++k1) o[k2 + 4 * k1] = g[k1];
       } else {
-        const float2 a = v[Q * k2], b = v[1 + Q * k2];
+        const V a = v[Q * k2], b = v[1 + Q * k2];
         o[k2] = cadd(a, b);
         o[k2 + 4] = csub(a, b);
       }
@@ -179,49 +202,41 @@ __device__ __forceinline__ void dft_small(float2 (&v)[R], bool inv) {
     // X_m, X_{R-m} = x_0 + sum_k cos(2 pi k m / R) s_k
     //                -+ i sum_k sin(2 pi k m / R) d_k
     constexpr int H = R / 2;
-    float2 sm[H], df[H];
-    float2 x0 = v[0];
+    V sm[H], df[H];
+    V x0 = v[0];
 #pragma unroll
     for (int k = 1; k <= H; ++k) {
       sm[k - 1] = cadd(v[k], v[R - k]);
       df[k - 1] = csub(v[k], v[R - k]);
       x0 = cadd(x0, sm[k - 1]);
     }
-    float2 o[R];
+    V o[R];
     o[0] = x0;
 #pragma unroll
     for (int m = 1; m <= H; ++m) {
-      float2 c = v[0], d = make_float2(0.0f, 0.0f);
+      V c = v[0], d = cmake<V>(0, 0);
 #pragma unroll
       for (int k = 1; k <= H; ++k) {
         const int t = (k * m) % R;  // a compile-time constant once unrolled
-        const float co = OddTrig<R>::cs[t <= H ? t : R - t];
-        const float si = t <= H ? OddTrig<R>::sn[t] : -OddTrig<R>::sn[R - t];
-        c = make_float2(fmaf(co, sm[k - 1].x, c.x), fmaf(co, sm[k - 1].y, c.y));
-        d = make_float2(fmaf(si, df[k - 1].x, d.x), fmaf(si, df[k - 1].y, d.y));
+        using T = Real<V>;
+        const T co = static_cast<T>(OddTrig<R>::cs[t <= H ? t : R - t]);
+        const T si = static_cast<T>(t <= H ? OddTrig<R>::sn[t] : -OddTrig<R>::sn[R - t]);
+        c = cmake<V>(fma_(co, sm[k - 1].x, c.x), fma_(co, sm[k - 1].y, c.y));
+        d = cmake<V>(fma_(si, df[k - 1].x, d.x), fma_(si, df[k - 1].y, d.y));
       }
       // -i d (forward) or +i d (inverse)
-      const float2 t = inv ? make_float2(-d.y, d.x) : make_float2(d.y, -d.x);
+      const V t = inv ? cmake<V>(-d.y, d.x) : cmake<V>(d.y, -d.x);
       o[m] = cadd(c, t);
       o[R - m] = csub(c, t);
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) v[r] = o[r];
   } else if constexpr (R == 2) {
-    const float2 a = v[0], b = v[1];
-    v[0] = make_float2(__fadd_rn(a.x, b.x), __fadd_rn(a.y, b.y));
-    v[1] = make_float2(__fsub_rn(a.x, b.x), __fsub_rn(a.y, b.y));
+    const V a = v[0], b = v[1];
+    v[0] = cadd(a, b);
+    v[1] = csub(a, b);
   } else {
-    const float2 s02 = make_float2(__fadd_rn(v[0].x, v[2].x), __fadd_rn(v[0].y, v[2].y));
-    const float2 d02 = make_float2(__fsub_rn(v[0].x, v[2].x), __fsub_rn(v[0].y, v[2].y));
-    const float2 s13 = make_float2(__fadd_rn(v[1].x, v[3].x), __fadd_rn(v[1].y, v[3].y));
-    const float2 d13 = make_float2(__fsub_rn(v[1].x, v[3].x), __fsub_rn(v[1].y, v[3].y));
-    // -i d13 (forward) or +i d13 (inverse)
-    const float2 t = inv ? make_float2(-d13.y, d13.x) : make_float2(d13.y, -d13.x);
-    v[0] = make_float2(__fadd_rn(s02.x, s13.x), __fadd_rn(s02.y, s13.y));
-    v[2] = make_float2(__fsub_rn(s02.x, s13.x), __fsub_rn(s02.y, s13.y));
-    v[1] = make_float2(__fadd_rn(d02.x, t.x), __fadd_rn(d02.y, t.y));
-    v[3] = make_float2(__fsub_rn(d02.x, t.x), __fsub_rn(d02.y, t.y));
+    dft4_strided<1, 4>(v, 0, inv);
   }
 }
 
@@ -285,13 +300,13 @@ __device__ __forceinline__ void stockham(float2* X, int n, int log2n, int lpb,
 //
 // One stage: as stockham_stage, with the quotients by Ns and n / R taken as high words of the stage's magic
 // factors (k r tstep < n, so the twiddle index needs no reduction).
-template <int R>
-__device__ __forceinline__ void mixed_stage(float2* X, int n, int lpb, int Ns, uint32_t mns,
-                                            uint32_t mnb, const float2* tw, bool inv) {
-  constexpr int NQ = (SH_MAXV + R - 1) / R;
+template <int R, int MAXV, class V>
+__device__ __forceinline__ void mixed_stage(V* X, int n, int lpb, int Ns, uint32_t mns,
+                                            uint32_t mnb, const V* tw, bool inv) {
+  constexpr int NQ = (MAXV + R - 1) / R;
   const int nb = n / R, tot = lpb * nb;  // butterflies
   const int tstep = n / (R * Ns);
-  float2 v[NQ][R];
+  V v[NQ][R];
   int dst[NQ];
 #pragma unroll
   for (int q = 0; q < NQ; ++q) {
@@ -300,13 +315,13 @@ __device__ __forceinline__ void mixed_stage(float2* X, int n, int lpb, int Ns, u
     if (b < tot) {
       const int l = nb > 1 ? static_cast<int>(__umulhi(b, mnb)) : b, j = b - l * nb;
       const int g = Ns > 1 ? static_cast<int>(__umulhi(j, mns)) : j, k = j - g * Ns;
-      const float2* x = X + l * n + j;
+      const V* x = X + l * n + j;
 #pragma unroll
       for (int r = 0; r < R; ++r) v[q][r] = x[r * nb];
       if (Ns > 1) {
 #pragma unroll
         for (int r = 1; r < R; ++r) {
-          float2 w = tw[k * r * tstep];
+          V w = tw[k * r * tstep];
           if (inv) w = conjf2(w);
           v[q][r] = cmul(v[q][r], w);
         }
@@ -329,12 +344,12 @@ __device__ __forceinline__ void mixed_stage(float2* X, int n, int lpb, int Ns, u
 // A stage of any radix R (a prime above 7): output s of butterfly j is the
 // R-term sum of x[j + r n / R] w^(r (k tstep + s n / R)), w = exp(-2 pi i /
 // n), from the n twiddles in LDS.
-__device__ __forceinline__ void prime_stage(float2* X, int n, int lpb, int R, int Ns,
-                                            uint32_t mns, uint32_t mnb, const float2* tw,
-                                            bool inv) {
+template <int MAXV, class V>
+__device__ __forceinline__ void prime_stage(V* X, int n, int lpb, int R, int Ns, uint32_t mns,
+                                            uint32_t mnb, const V* tw, bool inv) {
   const int nb = n / R, tot = lpb * n;
   const int tstep = n / (R * Ns);
-  float2 o[SH_MAXV];
+  V o[MAXV];
   // element e = (line l, output s, butterfly j), j fastest
   auto where = [&](int e, int& l, int& s, int& g, int& k) {
     const int ls = nb > 1 ? static_cast<int>(__umulhi(e, mnb)) : e, j = e - ls * nb;
@@ -344,30 +359,30 @@ __device__ __forceinline__ void prime_stage(float2* X, int n, int lpb, int R, in
     k = j - g * Ns;
   };
 #pragma unroll
-  for (int q = 0; q < SH_MAXV; ++q) {
+  for (int q = 0; q < MAXV; ++q) {
     const int e = threadIdx.x + q * SH_THREADS;
     if (e < tot) {
       int l, s, g, k;
       where(e, l, s, g, k);
-      const float2* x = X + l * n + g * Ns + k;
+      const V* x = X + l * n + g * Ns + k;
       int step = k * tstep + s * nb, idx = 0;
       if (step >= n) step -= n;
-      float re = 0.0f, im = 0.0f;
+      Real<V> re = 0, im = 0;
       for (int r = 0; r < R; ++r) {
-        float2 w = tw[idx];
+        V w = tw[idx];
         if (inv) w = conjf2(w);
-        const float2 p = cmul(x[r * nb], w);
-        re = __fadd_rn(re, p.x);
-        im = __fadd_rn(im, p.y);
+        const V p = cmul(x[r * nb], w);
+        re = re + p.x;
+        im = im + p.y;
         idx += step;
         if (idx >= n) idx -= n;
       }
-      o[q] = make_float2(re, im);
+      o[q] = cmake<V>(re, im);
     }
   }
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < SH_MAXV; ++q) {
+  for (int q = 0; q < MAXV; ++q) {
     const int e = threadIdx.x + q * SH_THREADS;
     if (e < tot) {
       int l, s, g, k;
@@ -379,20 +394,21 @@ __device__ __forceinline__ void prime_stage(float2* X, int n, int lpb, int R, in
 }
 
 // Mixed-radix transform of lpb lines in X; tw in LDS if S.twlds.
-__device__ __forceinline__ void mixed(float2* X, int n, const Stages& S, int lpb,
-                                      const float2* tw, bool inv) {
+template <int MAXV = SH_MAXV, class V>
+__device__ __forceinline__ void mixed(V* X, int n, const Stages& S, int lpb, const V* tw,
+                                      bool inv) {
   int Ns = 1;
   for (int s = 0; s < S.count; ++s) {
     const int R = S.R[s];
     const uint32_t mns = S.mns[s], mnb = S.mnb[s];
     switch (R) {
-      case 2: mixed_stage<2>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
-      case 3: mixed_stage<3>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
-      case 4: mixed_stage<4>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
-      case 5: mixed_stage<5>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
-      case 7: mixed_stage<7>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
-      case 8: mixed_stage<8>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
-      default: prime_stage(X, n, lpb, R, Ns, mns, mnb, tw, inv);
+      case 2: mixed_stage<2, MAXV>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 3: mixed_stage<3, MAXV>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 4: mixed_stage<4, MAXV>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 5: mixed_stage<5, MAXV>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 7: mixed_stage<7, MAXV>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      case 8: mixed_stage<8, MAXV>(X, n, lpb, Ns, mns, mnb, tw, inv); break;
+      default: prime_stage<MAXV>(X, n, lpb, R, Ns, mns, mnb, tw, inv);
     }
     Ns *= R;
   }
@@ -581,21 +597,14 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
   }
 }
 
-// Inverse rows: half spectra (R rows of n/2 + 1) -> real y (R rows of n),
-// times scale.
+// Inverse rows: half spectra (R rows of n/2 + 1) of row pairs row0 + 2 l ->
+// transformed lines X (real rows row0 + 2 l and row0 + 2 l + 1, unscaled).
 template <bool MIXED>
-__global__ __launch_bounds__(SH_THREADS) void c2r_rows_kernel(const float2* __restrict__ half,
-                                                              float* __restrict__ y, int n,
-                                                              int log2n, Stages S, long long R,
-                                                              int lpb,
-                                                              const float2* __restrict__ tw,
-                                                              float scale, const int32_t* pred) {
-  if (pred_off(pred)) return;
-  extern __shared__ float2 lds[];
-  float2* X = lds;
+__device__ __forceinline__ void c2r_lines(const float2* __restrict__ half, float2* X, int n,
+                                          int log2n, const Stages& S, long long R, int lpb,
+                                          long long row0, const float2* __restrict__ tw) {
   const int H1 = n / 2 + 1;
   const float2* twl = pass_twiddles<MIXED>(X, lpb * n, n, S, tw);
-  const long long row0 = 2ll * blockIdx.x * lpb;
   for (int e = threadIdx.x; e < lpb * H1; e += SH_THREADS) {
     const int l = e / H1, k = e - l * H1;
     const long long ra = row0 + 2 * l, rb = ra + 1;
@@ -608,6 +617,21 @@ __global__ __launch_bounds__(SH_THREADS) void c2r_rows_kernel(const float2* __re
   }
   __syncthreads();
   transform<MIXED>(X, n, log2n, S, lpb, twl, true);
+}
+
+// Inverse rows to real y (R rows of n), times scale.
+template <bool MIXED>
+__global__ __launch_bounds__(SH_THREADS) void c2r_rows_kernel(const float2* __restrict__ half,
+                                                              float* __restrict__ y, int n,
+                                                              int log2n, Stages S, long long R,
+                                                              int lpb,
+                                                              const float2* __restrict__ tw,
+                                                              float scale, const int32_t* pred) {
+  if (pred_off(pred)) return;
+  extern __shared__ float2 lds[];
+  float2* X = lds;
+  const long long row0 = 2ll * blockIdx.x * lpb;
+  c2r_lines<MIXED>(half, X, n, log2n, S, R, lpb, row0, tw);
   for (int e = threadIdx.x; e < lpb * n; e += SH_THREADS) {
     const int l = e / n, k = e - l * n;
     const long long ra = row0 + 2 * l, rb = ra + 1;
@@ -809,16 +833,141 @@ __global__ __launch_bounds__(2 * QT) void q1k_c2r_kernel(const float2* __restric
 
 // ---------------------------------- fused AcceleratedPGM gradient step --
 //
-// For f(x) = 0.5 ||A x - y||^2 with A the 1024 x 1024 real circular
-// convolution, one convolution per iteration serves both the gradient and
+// For f(x) = 0.5 ||A x - y||^2 with A a real circular convolution over two
+// axes (F0, F1), one convolution per iteration serves both the gradient and
 // the objective:
 //   * G x (G = A^T A: the convolution by |Hs|^2, real on the half grid),
 //     and G v = (1 + c) G x - c G x_prev for the extrapolated point
 //     v = x + c (x - x_prev) (linearity), so u = v - (1/L) (G v - A^T y);
 //   * ||A x - y||^2 = sum_k w_k |Hs[k] X[k] - Y[k]|^2 / (F0 F1) over the
-//     half spectrum (Parseval; w_k = 1 on the first and the Nyquist column,
-//     2 elsewhere), X and Y the spectra of x and y.
-// All half-grid arrays are transposed (column k1 contiguous).
+//     half spectrum (Parseval; w_k = 1 on the first and, for even F1, the
+//     Nyquist column, 2 elsewhere), X and Y the spectra of x and y.
+// Half-grid arrays are F0 x (F1/2 + 1); at 1024 x 1024 they are transposed
+// (column k1 contiguous).
+
+// Set-up: gs = |Hs|^2 on the half grid, evaluated in float64 from the
+// plan's spectrum and rounded once.
+__global__ __launch_bounds__(256) void gram_spectrum_kernel(const float2* __restrict__ h,
+                                                            float* __restrict__ gs, int F0, int F1,
+                                                            int trans) {
+  const int H1 = F1 / 2 + 1;
+  const long long tot = static_cast<long long>(F0) * H1;
+  for (long long e = blockIdx.x * 256ll + threadIdx.x; e < tot; e += 256ll * gridDim.x) {
+    const int k0 = static_cast<int>(e / H1), k1 = static_cast<int>(e - static_cast<long long>(k0) * H1);
+    const float2 a = h[static_cast<long long>(k0) * F1 + k1];
+    const float2 b = h[static_cast<long long>((F0 - k0) % F0) * F1 + (F1 - k1) % F1];
+    const double re = 0.5 * (static_cast<double>(a.x) + static_cast<double>(b.x));
+    const double im = 0.5 * (static_cast<double>(a.y) - static_cast<double>(b.y));
+    gs[trans ? static_cast<long long>(k1) * F0 + k0 : e] = static_cast<float>(re * re + im * im);
+  }
+}
+
+// Set-up: Yh = rfft2(y) in float64, rounded once to complex64.  Runs once per
+// solve (rows 18 us, columns 11 us at 1024 x 1024), one line per workgroup in
+// LDS: once, so a simple kernel serves.
+__global__ __launch_bounds__(256) void twiddle64_kernel(double2* __restrict__ tw, int n) {
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  if (k >= n) return;
+  double sn, cs;
+  sincospi(-2.0 * k / n, &sn, &cs);
+  tw[k] = make_double2(cs, sn);
+}
+
+constexpr int MAXV64 = MAX_POW2 / SH_THREADS;  // values per thread of a line
+
+__global__ __launch_bounds__(SH_THREADS) void rows64_kernel(const float* __restrict__ y,
+                                                            double2* __restrict__ half, int n,
+                                                            Stages S,
+                                                            const double2* __restrict__ tw) {
+  extern __shared__ double2 lds64[];
+  const int H1 = n / 2 + 1;
+  const long long row = blockIdx.x;
+  for (int k = threadIdx.x; k < n; k += SH_THREADS)
+    lds64[k] = make_double2(static_cast<double>(y[row * n + k]), 0.0);
+  __syncthreads();
+  mixed<MAXV64>(lds64, n, S, 1, tw, false);
+  for (int k = threadIdx.x; k < H1; k += SH_THREADS) half[row * H1 + k] = lds64[k];
+}
+
+__global__ __launch_bounds__(SH_THREADS) void cols64_kernel(const double2* __restrict__ half,
+                                                            float2* __restrict__ out, int n,
+                                                            int H1, Stages S,
+                                                            const double2* __restrict__ tw,
+                                                            int trans) {
+  extern __shared__ double2 lds64[];
+  // consecutive columns on one XCD: they share the cache lines of their rows
+  int c = blockIdx.x;
+  {
+    const int G8 = (gridDim.x / 8) * 8;
+    if (c < G8) c = (c % 8) * (G8 / 8) + c / 8;
+  }
+  for (int k = threadIdx.x; k < n; k += SH_THREADS)
+    lds64[k] = half[static_cast<long long>(k) * H1 + c];
+  __syncthreads();
+  mixed<MAXV64>(lds64, n, S, 1, tw, false);
+  for (int k = threadIdx.x; k < n; k += SH_THREADS)
+    out[trans ? static_cast<long long>(c) * n + k : static_cast<long long>(k) * H1 + c] =
+        make_float2(static_cast<float>(lds64[k].x), static_cast<float>(lds64[k].y));
+}
+
+// Columns of any length (the 1024-point ones below keep their line in
+// registers): forward, objective partial of the workgroup's columns (if
+// obj), times gs, inverse, times 1/F0.
+template <bool MIXED>
+__global__ __launch_bounds__(SH_THREADS) void cols_gram_kernel(
+    float2* __restrict__ half, const float2* __restrict__ hs, const float* __restrict__ gs,
+    const float2* __restrict__ Yh, double* __restrict__ obj, int n, int log2n, Stages S, int H1,
+    int F1, int lpb, const float2* __restrict__ tw, float scale, const int32_t* pred) {
+  if (pred_off(pred)) return;
+  extern __shared__ float2 lds[];
+  __shared__ double sh[4];
+  float2* X = lds;
+  const int tot = lpb * n;
+  const float2* twl = pass_twiddles<MIXED>(X, tot, n, S, tw);
+  int blk = blockIdx.x;  // neighbouring columns on one XCD, as in stockham_kernel
+  {
+    const int G8 = (gridDim.x / 8) * 8;
+    if (blk < G8) blk = (blk % 8) * (G8 / 8) + blk / 8;
+  }
+  const int c0 = blk * lpb, nl = min(lpb, H1 - c0);
+  for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
+    const int k = e / lpb, l = e - k * lpb;
+    X[l * n + k] = l < nl ? half[static_cast<long long>(k) * H1 + c0 + l] : make_float2(0.f, 0.f);
+  }
+  __syncthreads();
+  transform<MIXED>(X, n, log2n, S, lpb, twl, false);
+  double acc = 0.0;
+  for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
+    const int k = e / lpb, l = e - k * lpb;
+    if (l < nl) {
+      const long long o = static_cast<long long>(k) * H1 + c0 + l;
+      const float2 a = X[l * n + k];
+      if (obj) {
+        const float2 p = cmul(hs[o], a), yk = Yh[o];
+        const double dx = static_cast<double>(p.x) - static_cast<double>(yk.x);
+        const double dy = static_cast<double>(p.y) - static_cast<double>(yk.y);
+        const double d = dx * dx + dy * dy;
+        acc += (c0 + l == 0 || 2 * (c0 + l) == F1) ? d : 2.0 * d;
+      }
+      const float g = gs[o];
+      X[l * n + k] = make_float2(__fmul_rn(g, a.x), __fmul_rn(g, a.y));
+    }
+  }
+  if (obj) {
+    acc = block_sum_f64(acc, sh);
+    if (threadIdx.x == 0) obj[blockIdx.x] = acc;
+  }
+  __syncthreads();
+  transform<MIXED>(X, n, log2n, S, lpb, twl, true);
+  for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
+    const int k = e / lpb, l = e - k * lpb;
+    if (l < nl) {
+      const float2 a = X[l * n + k];
+      half[static_cast<long long>(k) * H1 + c0 + l] =
+          make_float2(__fmul_rn(a.x, scale), __fmul_rn(a.y, scale));
+    }
+  }
+}
 
 // Columns: forward, objective partial of the column (if obj), times gsT,
 // inverse, times 1/1024.
@@ -922,6 +1071,36 @@ __global__ __launch_bounds__(2 * QT) void q1k_c2r_step_kernel(
       u[e] = __fadd_rn(v[e], __fmul_rn(b, __fsub_rn(gv, aty[e])));
       gx[e] = gn;
     }
+  }
+}
+
+// The same for rows of any length: workgroup 0 reduces the statistics row if
+// STATS, the others take lpb row pairs each.
+template <bool MIXED, bool STATS>
+__global__ __launch_bounds__(SH_THREADS) void c2r_step_kernel(
+    const float2* __restrict__ half, float* __restrict__ gx, const float* __restrict__ v,
+    const float* __restrict__ aty, float c1, float c, float b, float* __restrict__ u, int n,
+    int log2n, Stages S, long long R, int lpb, const float2* __restrict__ tw, float scale,
+    ApgmStats st, const int32_t* pred) {
+  if (pred_off(pred)) return;
+  if (STATS && blockIdx.x == 0) {
+    apgm_stats_block<SH_THREADS>(st.obj, st.nobj, st.obj_scale, st.tv, st.ntv, st.lam, st.res,
+                                 st.nres, st.hist, st.counter, st.hist_cap);
+    return;
+  }
+  extern __shared__ float2 lds[];
+  float2* X = lds;
+  const long long row0 = 2ll * (blockIdx.x - (STATS ? 1 : 0)) * lpb;
+  c2r_lines<MIXED>(half, X, n, log2n, S, R, lpb, row0, tw);
+  for (int q = threadIdx.x; q < 2 * lpb * n; q += SH_THREADS) {
+    const int r = q / n, k = q - r * n;  // real row row0 + r
+    if (row0 + r >= R) break;
+    const float2 z = X[(r >> 1) * n + k];
+    const long long e = (row0 + r) * n + k;
+    const float gn = __fmul_rn(r & 1 ? z.y : z.x, scale);
+    const float gv = __fsub_rn(__fmul_rn(c1, gn), __fmul_rn(c, gx[e]));
+    u[e] = __fadd_rn(v[e], __fmul_rn(b, __fsub_rn(gv, aty[e])));
+    gx[e] = gn;
   }
 }
 
@@ -1289,6 +1468,14 @@ int scxr_cconv_apply(const scxr_cconv_plan* plan, const float* x, float* y, int3
 
 }  // extern "C"
 
+// Workgroups of the fused gradient step's column pass, one objective partial
+// each (0: the plan is not one real two-axis convolution).
+static int apgm_parts(const Plan& p) {
+  if (!p.r2c || p.batch != 1) return 0;
+  const int H1 = p.F[1] / 2 + 1;
+  return q1k_path(p) ? H1 : static_cast<int>(ceil_div(H1, p.lpb_cols));
+}
+
 // The three kernels of one fused gradient step; st (nullable) adds the
 // statistics row to the last of them.
 static int apgm_grad(const scxr_cconv_plan* plan, const float* x, const float* gs,
@@ -1298,10 +1485,38 @@ static int apgm_grad(const scxr_cconv_plan* plan, const float* x, const float* g
   SCXR_REQUIRE(plan && x && gs && gx && v && aty && u && (!obj || Yh), SCXR_ERR_ARG,
                "null argument to cconv_apgm_grad");
   const Plan& p = plan->p;
-  SCXR_REQUIRE(q1k_path(p) && p.batch == 1, SCXR_ERR_UNSUPPORTED,
-               "fused APGM gradient needs a single 1024 x 1024 real convolution plan");
-  constexpr int H1 = Q1K / 2 + 1;
+  SCXR_REQUIRE(apgm_parts(p) > 0, SCXR_ERR_UNSUPPORTED,
+               "fused APGM gradient needs a plan of one real two-axis convolution");
   float2* half = p.work;
+  if (!q1k_path(p)) {
+    const AxisTables &t0 = p.ax[0], &t1 = p.ax[1];
+    const int n0 = t0.n, n1 = t1.n, H1 = n1 / 2 + 1, lr = p.lpb_rows;
+    const bool mix0 = t0.log2n < 0, mix1 = t1.log2n < 0;
+    const unsigned gr = ceil_div((n0 + 1) / 2, lr);
+    hipLaunchKernelGGL(mix1 ? r2c_rows_kernel<true> : r2c_rows_kernel<false>, dim3(gr),
+                       dim3(SH_THREADS), pass_lds(t1, lr), s, x, half, n1, t1.log2n, t1.st,
+                       static_cast<long long>(n0), lr, t1.tw, pred);
+    SCXR_LAUNCHED("fft r2c rows");
+    hipLaunchKernelGGL(mix0 ? cols_gram_kernel<true> : cols_gram_kernel<false>,
+                       dim3(apgm_parts(p)), dim3(SH_THREADS), pass_lds(t0, p.lpb_cols), s, half,
+                       p.hs, gs, reinterpret_cast<const float2*>(Yh), obj, n0, t0.log2n, t0.st, H1,
+                       n1, p.lpb_cols, t0.tw, 1.0f / static_cast<float>(n0), pred);
+    SCXR_LAUNCHED("fft gram columns");
+    const float sc = 1.0f / static_cast<float>(n1);
+    if (st)
+      hipLaunchKernelGGL((mix1 ? c2r_step_kernel<true, true> : c2r_step_kernel<false, true>),
+                         dim3(gr + 1), dim3(SH_THREADS), pass_lds(t1, lr), s, half, gx, v, aty,
+                         1.0f + c, c, b, u, n1, t1.log2n, t1.st, static_cast<long long>(n0), lr,
+                         t1.tw, sc, *st, pred);
+    else
+      hipLaunchKernelGGL((mix1 ? c2r_step_kernel<true, false> : c2r_step_kernel<false, false>),
+                         dim3(gr), dim3(SH_THREADS), pass_lds(t1, lr), s, half, gx, v, aty,
+                         1.0f + c, c, b, u, n1, t1.log2n, t1.st, static_cast<long long>(n0), lr,
+                         t1.tw, sc, ApgmStats{}, pred);
+    SCXR_LAUNCHED("fft c2r gradient step");
+    return SCXR_OK;
+  }
+  constexpr int H1 = Q1K / 2 + 1;
   hipLaunchKernelGGL(q1k_r2c_kernel, dim3(Q1K / QR), dim3(2 * QT), 0, s, x, half, p.ax[1].tw,
                      pred);
   SCXR_LAUNCHED("fft r2c rows (1024)");
@@ -1322,6 +1537,42 @@ static int apgm_grad(const scxr_cconv_plan* plan, const float* x, const float* g
 
 extern "C" {
 
+int32_t scxr_cconv_apgm_parts(const scxr_cconv_plan* plan) {
+  return plan ? apgm_parts(plan->p) : 0;
+}
+
+int64_t scxr_cconv_apgm_setup_ws(const scxr_cconv_plan* plan) {
+  if (!plan || apgm_parts(plan->p) <= 0) return 0;
+  const Plan& p = plan->p;
+  return 2 * (static_cast<int64_t>(p.F[0]) * (p.F[1] / 2 + 1) + p.F[0] + p.F[1]);
+}
+
+int scxr_cconv_apgm_setup(const scxr_cconv_plan* plan, const float* y, float* gs, float* Yh,
+                          double* ws, void* stream) {
+  SCXR_REQUIRE(plan && y && gs && Yh && ws, SCXR_ERR_ARG, "null argument to cconv_apgm_setup");
+  const Plan& p = plan->p;
+  SCXR_REQUIRE(apgm_parts(p) > 0, SCXR_ERR_UNSUPPORTED,
+               "fused APGM set-up needs a plan of one real two-axis convolution");
+  const hipStream_t s = as_stream(stream);
+  const int n0 = p.F[0], n1 = p.F[1], H1 = n1 / 2 + 1, trans = q1k_path(p);
+  double2* half = reinterpret_cast<double2*>(ws);
+  double2* tw0 = half + static_cast<long long>(n0) * H1;
+  double2* tw1 = tw0 + n0;
+  hipLaunchKernelGGL(gram_spectrum_kernel, dim3(1024), dim3(256), 0, s, p.h, gs, n0, n1, trans);
+  SCXR_LAUNCHED("cconv gram spectrum");
+  hipLaunchKernelGGL(twiddle64_kernel, dim3(ceil_div(n0, 256)), dim3(256), 0, s, tw0, n0);
+  SCXR_LAUNCHED("cconv twiddles");
+  hipLaunchKernelGGL(twiddle64_kernel, dim3(ceil_div(n1, 256)), dim3(256), 0, s, tw1, n1);
+  SCXR_LAUNCHED("cconv twiddles");
+  hipLaunchKernelGGL(rows64_kernel, dim3(n0), dim3(SH_THREADS), sizeof(double2) * n1, s, y, half,
+                     n1, make_stages(n1), tw1);
+  SCXR_LAUNCHED("cconv float64 rows");
+  hipLaunchKernelGGL(cols64_kernel, dim3(H1), dim3(SH_THREADS), sizeof(double2) * n0, s, half,
+                     reinterpret_cast<float2*>(Yh), n0, H1, make_stages(n0), tw0, trans);
+  SCXR_LAUNCHED("cconv float64 columns");
+  return SCXR_OK;
+}
+
 int scxr_cconv_apgm_grad(const scxr_cconv_plan* plan, const float* x, const float* gs,
                          const float* Yh, double* obj, float* gx, const float* v,
                          const float* aty, float c, float b, float* u, const int32_t* pred,
@@ -1337,7 +1588,8 @@ int scxr_cconv_apgm_grad_itstat(const scxr_cconv_plan* plan, const float* x, con
                                 const int32_t* pred, void* stream) {
   SCXR_REQUIRE(obj && Yh && tv && res && hist && counter && ntv > 0 && nres > 0 && hist_cap > 0,
                SCXR_ERR_ARG, "bad cconv_apgm_grad_itstat arguments");
-  const ApgmStats st{obj, Q1K / 2 + 1, obj_scale, tv, ntv, lam, res, nres, hist, counter,
+  SCXR_REQUIRE(plan, SCXR_ERR_ARG, "null argument to cconv_apgm_grad");
+  const ApgmStats st{obj, apgm_parts(plan->p), obj_scale, tv, ntv, lam, res, nres, hist, counter,
                      hist_cap};
   return apgm_grad(plan, x, gs, Yh, obj, gx, v, aty, c, b, u, &st, pred, as_stream(stream));
 }

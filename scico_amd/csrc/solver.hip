@@ -848,11 +848,12 @@ __global__ __launch_bounds__(256) void tv_prox_kernel(const float* __restrict__ 
 constexpr int TVT = 16;
 template <int EXT>
 __global__ __launch_bounds__(256) void tv_prox2d_kernel(const float* __restrict__ v,
-                                                        float* __restrict__ out, TvDims t,
+                                                        float* out, TvDims t,
                                                         float tau, float invK, int iso,
                                                         const float* __restrict__ w,
                                                         const int32_t* pred,
-                                                        float* __restrict__ vm, float c,
+                                                        const float* xold, const float* vold,
+                                                        float* vm, float c,
                                                         double* __restrict__ res_ws,
                                                         double* __restrict__ tv_ws) {
   if (pred_off(pred)) return;
@@ -935,7 +936,7 @@ __global__ __launch_bounds__(256) void tv_prox2d_kernel(const float* __restrict_
     if (pi < M && pj < N) {
       const float xn = xs[ty][tx];
       const int64_t e = static_cast<int64_t>(pi) * N + pj;
-      const float xo = out[e], vo = vm[e];
+      const float xo = xold[e], vo = vold[e];
       const double d = static_cast<double>(xn) - static_cast<double>(vo);
       res = d * d;
       vm[e] = __fadd_rn(xn, __fmul_rn(c, __fsub_rn(xn, xo)));
@@ -1524,8 +1525,8 @@ int scxr_tv_prox(int32_t ndim, const int32_t* shape, const float* v, float* out,
   if (ndim == 2) {
     const dim3 g(ceil_div(t.d[2], solver::TVT), ceil_div(t.d[1], solver::TVT));
     hipLaunchKernelGGL(solver::tv_prox2d_kernel<0>, g, dim3(256), 0, as_stream(stream), v,
-                       out, t, tau, 0.25f, isotropic, nullptr, pred, nullptr, 0.0f, nullptr,
-                       nullptr);
+                       out, t, tau, 0.25f, isotropic, nullptr, pred, nullptr, nullptr, nullptr,
+                       0.0f, nullptr, nullptr);
   } else {
     hipLaunchKernelGGL(solver::tv_prox_kernel, dim3(solver::elem_grid(n)), dim3(256), 0,
                        as_stream(stream), v, out, t, tau, 1.0f / static_cast<float>(2 * ndim),
@@ -1543,15 +1544,24 @@ int32_t scxr_tv_prox_apgm_parts(int32_t M, int32_t N) {
 int scxr_tv_prox_apgm(int32_t M, int32_t N, const float* u, float* x, float* v, float tau,
                       int32_t isotropic, int32_t circular, float c, double* res_ws,
                       double* tv_ws, const int32_t* pred, void* stream) {
-  SCXR_REQUIRE(u && x && v && res_ws && tv_ws && u != x && u != v && x != v, SCXR_ERR_ARG,
-               "bad tv_prox_apgm arguments (u, x and v must be distinct)");
+  return scxr_tv_prox_apgm_to(M, N, u, x, v, x, v, tau, isotropic, circular, c, res_ws, tv_ws,
+                              pred, stream);
+}
+
+int scxr_tv_prox_apgm_to(int32_t M, int32_t N, const float* u, const float* x, const float* v,
+                         float* x_new, float* v_new, float tau, int32_t isotropic,
+                         int32_t circular, float c, double* res_ws, double* tv_ws,
+                         const int32_t* pred, void* stream) {
+  SCXR_REQUIRE(u && x && v && x_new && v_new && res_ws && tv_ws && u != x_new && u != v_new &&
+                   x_new != v_new && x_new != v && v_new != x,
+               SCXR_ERR_ARG, "bad tv_prox_apgm arguments (u, x and v must be distinct)");
   const int32_t shape[2] = {M, N};
   solver::TvDims t;
   const int rc = tv_dims(2, shape, circular, t);
   if (rc) return rc;
   const dim3 g(ceil_div(N, solver::TVT), ceil_div(M, solver::TVT));
-  hipLaunchKernelGGL(solver::tv_prox2d_kernel<1>, g, dim3(256), 0, as_stream(stream), u, x, t,
-                     tau, 0.25f, isotropic, nullptr, pred, v, c, res_ws, tv_ws);
+  hipLaunchKernelGGL(solver::tv_prox2d_kernel<1>, g, dim3(256), 0, as_stream(stream), u, x_new, t,
+                     tau, 0.25f, isotropic, nullptr, pred, x, v, v_new, c, res_ws, tv_ws);
   SCXR_LAUNCHED("tv prox apgm");
   return SCXR_OK;
 }
@@ -1568,7 +1578,8 @@ int scxr_tv_prox_w(int32_t ndim, const int32_t* shape, const float* v, const flo
   if (ndim == 2) {
     const dim3 g(ceil_div(t.d[2], solver::TVT), ceil_div(t.d[1], solver::TVT));
     hipLaunchKernelGGL(solver::tv_prox2d_kernel<0>, g, dim3(256), 0, as_stream(stream), v,
-                       out, t, tau, 0.25f, isotropic, w, pred, nullptr, 0.0f, nullptr, nullptr);
+                       out, t, tau, 0.25f, isotropic, w, pred, nullptr, nullptr, nullptr, 0.0f,
+                       nullptr, nullptr);
   } else {
     hipLaunchKernelGGL(solver::tv_prox_kernel, dim3(solver::elem_grid(n)), dim3(256), 0,
                        as_stream(stream), v, out, t, tau, 1.0f / static_cast<float>(2 * ndim),

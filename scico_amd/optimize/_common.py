@@ -20,10 +20,11 @@ from ..util import DeviceElapsed, Timer
 def itstat_func_and_object(itstat_fields: dict, itstat_attrib: list,
                            itstat_options: Optional[dict] = None):
     """``_common.py:28-74``: build the insertion function and the stats object."""
-    attribs = list(itstat_attrib)
+    # compiled once: parsing the expressions took 20 us of every iteration
+    attribs = [compile("obj." + a, "<itstat>", "eval") for a in itstat_attrib]
 
     def itstat_func(obj):
-        return tuple(eval("obj." + a, {"obj": obj}) for a in attribs)
+        return tuple(eval(a, {"obj": obj}) for a in attribs)
 
     opts = {"fields": itstat_fields, "itstat_func": itstat_func, "display": False}
     if itstat_options:

@@ -5,8 +5,8 @@
 ``f`` with a gradient and ``g`` with a prox.  For the deconvolution
 structure
 
-    f = SquaredL2Loss(y, CircularConvolve (one real 1024 x 1024 image),
-                      scale=0.5),
+    f = SquaredL2Loss(y, CircularConvolve (one real image, both axes of 3 or
+                      more pixels), scale=0.5),
     g = lam * IsotropicTVNorm() or lam * AnisotropicTVNorm()  (2D),
     constant step size,
 
@@ -28,7 +28,7 @@ import torch
 
 from .. import _device as dev
 from .. import _vec as vec
-from .._lib import call, load
+from .._lib import ScxrError, call, load
 from ._common import Optimizer
 
 
@@ -130,6 +130,8 @@ class AcceleratedPGM(PGM):
 
     def step(self):
         if self._fused is not None:
+            self._fused = self._fused.current()
+        if self._fused is not None:
             self._fused.step(self._momentum())
             return
         x_old = self.x
@@ -171,14 +173,43 @@ class _FusedDeconv:
         if not (type(f) is SquaredL2Loss and f.scale == 0.5 and type(f.A) is CircularConvolve):
             return None
         A = f.A
-        if not (A.ndims == 2 and A.batch == 1 and A.input_shape == (1024, 1024)):
+        if not (A.ndims == 2 and A.input_shape == A.fft_shape and
+                tuple(f.y.shape) == A.input_shape):
             return None
         scale, base = (g.scale, g.functional) if isinstance(g, ScaledFunctional) else (1.0, g)
         if not isinstance(base, TVNorm) or base.axes is not None:
             return None
         if tuple(pgm.x.shape) != A.input_shape or pgm.x.dtype != torch.float32:
             return None
+        try:
+            if int(load().scxr_cconv_apgm_parts(A.plan)) <= 0:
+                return None
+        except ScxrError:  # no plan for this size: the generic path reports it when used
+            return None
         return _FusedDeconv(pgm, float(scale), base)
+
+    @staticmethod
+    def _inputs(pgm):
+        """What the set-up was made from (objects, and versions that torch
+        counts up when a tensor is modified in place)."""
+        f, g = pgm.f, pgm.g
+        base = getattr(g, "functional", g)
+        return (f, f.A, f.scale, f.y, f.y._version, g, getattr(g, "scale", 1.0), base,
+                getattr(base, "isotropic", None), getattr(base, "circular", None))
+
+    def current(self):
+        """This object if the solver's problem and state are the ones that it
+        left, itself brought up to date if only the state was replaced or
+        modified (or L), else what the new problem calls for (host checks)."""
+        now = self._inputs(self.pgm)
+        if any(a is not b and (i not in (2, 4, 6, 8, 9) or a != b)
+               for i, (a, b) in enumerate(zip(now, self._made_from))):
+            return _FusedDeconv.build(self.pgm)
+        p = self.pgm
+        if p.x is not self.x or p.v is not self.v or float(p.L) != self._L or \
+                (self.x._version, self.v._version) != self._versions:
+            self.adopt_state()
+        return self
 
     def __init__(self, pgm: AcceleratedPGM, lam: float, tv):
         self.pgm = pgm
@@ -192,21 +223,21 @@ class _FusedDeconv:
         f32 = dict(dtype=torch.float32, device=dev.DEVICE)
         f64 = dict(dtype=torch.float64, device=dev.DEVICE)
         y = dev.as_device(pgm.f.y)
-        # G = A^T A on the half grid: |Hs|^2 with Hs the Hermitian part of
-        # the spectrum (float64, rounded once), as SquaredL2Loss's gram
-        hd = dev.to_numpy(self.A.h_dft).astype(np.complex128)
-        hneg = np.roll(np.flip(hd, (0, 1)), 1, (0, 1))
-        hs = 0.5 * (hd + np.conj(hneg))
+        self._made_from = self._inputs(pgm)
+        # the half-grid spectra of G = A^T A and of y, formed in float64 on the
+        # device and rounded once (host FFTs took 15 ms of a new 1024 x 1024
+        # problem)
         H1 = self.N // 2 + 1
-        # half-grid arrays transposed (column k1 contiguous), as the kernels
-        # keep the half spectrum
-        self.gs = dev.as_device(np.ascontiguousarray((hs.real**2 + hs.imag**2)[:, :H1].T,
-                                                     dtype=np.float32))
-        yh = np.fft.rfft2(dev.to_numpy(y).astype(np.float64))
-        self.Yh = torch.as_tensor(np.ascontiguousarray(yh.T.astype(np.complex64)),
-                                  device=dev.DEVICE)
+        self.gs = torch.empty(self.M * H1, **f32)
+        self.Yh = torch.empty(2 * self.M * H1, **f32)
+        ws = torch.empty(int(lib.scxr_cconv_apgm_setup_ws(self.A.plan)), **f64)
+        call("scxr_cconv_apgm_setup", self.A.plan, y.data_ptr(), self.gs.data_ptr(),
+             self.Yh.data_ptr(), ws.data_ptr(), dev.stream())
+        # at 1024 x 1024 the iterates are updated in place (a captured step
+        # may be replayed on its own results); other sizes get new ones
+        self.in_place = (self.M, self.N) == (1024, 1024)
         self.aty = self.A.adj(y)
-        self.n_obj = H1
+        self.n_obj = int(lib.scxr_cconv_apgm_parts(self.A.plan))
         self.n_res = int(lib.scxr_tv_prox_apgm_parts(self.M, self.N))
         self.n_tv = self.n_res  # the prox kernel's TV partials, one per workgroup
         self.ws_obj = torch.empty(self.n_obj, **f64)
@@ -220,7 +251,7 @@ class _FusedDeconv:
         self.counter = torch.zeros(1, dtype=torch.int32, device=dev.DEVICE)
         self.n_steps = 0
         self._reserve(max(64, pgm.maxiter))
-        self.adopt_state()
+        self.adopt_state(same=getattr(pgm, "itnum", 0) == 0 and pgm.t == 1.0)
 
     def _reserve(self, rows: int):
         if rows <= self.hist_cap:
@@ -241,20 +272,23 @@ class _FusedDeconv:
                     np.float32(lam_eff))
         return b, tau
 
-    def adopt_state(self):
-        """Own contiguous x and v, and the first gradient step from them."""
+    def adopt_state(self, same: bool = False):
+        """Own contiguous x and v, and the first gradient step from them
+        (``same``: v is known to equal x, as in a new solver)."""
         p = self.pgm
         self.x = p.x.contiguous().clone()
         self.v = p.v.contiguous().clone() if hasattr(p, "v") else self.x.clone()
         self._publish()
-        self._prime()
+        self._L = float(p.L)
+        self._prime(same)
 
     def _publish(self):
         self.pgm.x = self.x
         if hasattr(self.pgm, "v"):
             self.pgm.v = self.v
+        self._versions = (self.x._version, self.v._version)
 
-    def _prime(self):
+    def _prime(self, same: bool):
         """The state a step starts from: u = v - (1/L) grad f(v) and gx = G x
         (the step forms G v_next = (1 + c) G x_next - c gx)."""
         b, _ = self._consts()
@@ -263,7 +297,7 @@ class _FusedDeconv:
         vec.fill(self.gx, 0.0)
         call("scxr_cconv_apgm_grad", self.A.plan, P(self.v), P(self.gs), None, None, P(self.gx),
              P(self.v), P(self.aty), 0.0, b, P(self.u), None, s)
-        if not torch.equal(self.v, self.x):  # a restored mid-run state: gx = G x as well
+        if not same and not torch.equal(self.v, self.x):  # a mid-run state: gx = G x as well
             scratch = torch.empty_like(self.u)
             call("scxr_cconv_apgm_grad", self.A.plan, P(self.x), P(self.gs), None, None,
                  P(self.gx), P(self.x), P(self.aty), 0.0, b, P(scratch), None, s)
@@ -275,14 +309,18 @@ class _FusedDeconv:
         self.enqueue(c)
         self.n_steps += 1
         self._publish()
+        self.pgm.fixed_point_residual = self.stat(1)
 
     def enqueue(self, c: float):
         """One iteration (no host synchronisation; capturable)."""
         b, tau = self._consts()
         P = lambda t: t.data_ptr()
         s = dev.stream()
-        call("scxr_tv_prox_apgm", self.M, self.N, P(self.u), P(self.x), P(self.v), tau, self.iso,
-             self.circ, c, P(self.ws_res), P(self.ws_tv), None, s)
+        x, v = self.x, self.v
+        if not self.in_place:
+            self.x, self.v = torch.empty_like(x), torch.empty_like(v)
+        call("scxr_tv_prox_apgm_to", self.M, self.N, P(self.u), P(x), P(v), P(self.x), P(self.v),
+             tau, self.iso, self.circ, c, P(self.ws_res), P(self.ws_tv), None, s)
         call("scxr_cconv_apgm_grad_itstat", self.A.plan, P(self.x), P(self.gs), P(self.Yh),
              P(self.ws_obj), P(self.gx), P(self.v), P(self.aty), c, b, P(self.u), self.obj_scale,
              P(self.ws_tv), self.n_tv, self.lam, P(self.ws_res), self.n_res, P(self.hist),

@@ -455,3 +455,74 @@ def test_fused_apgm_tv_variants(gpu, iso, circular):
     print(f"  fused APGM iso={iso} circ={circular}: 10 steps rel-L2 {e:.2e}, objective "
           f"{d_obj:.2e}, residual {d_res:.2e}", flush=True)
     assert e <= 1e-6 and d_obj <= 1e-6 and d_res <= 1e-6
+
+
+@pytest.mark.parametrize("shape", [(3, 3), (64, 48), (45, 50), (256, 512), (33, 501), (2048, 20)])
+def test_fused_apgm_any_size(gpu, shape):
+    """The fused deconvolution iteration at sizes other than 1024 x 1024
+    (mixed-radix and power-of-two lines, odd rows, several columns and one
+    per workgroup): iterates, which are new tensors, within 1e-6 of the
+    generic iteration's over 10 steps and after a step constant, the state
+    and the data were changed between steps; the statistics those of its own
+    iterates.  Bars of the statistics: the residual is a float64 sum of exact
+    differences; the objective takes A x, whose relative error is at most
+    1e-6 of ||y||, so f differs by at most ||A x - y|| times that and half
+    its square, and the TV norm by 1e-6 of itself."""
+    from scico_amd.optimize import _pgm
+
+    M, N = shape
+    rng = np.random.default_rng(23)
+    xg = rng.random(shape).astype(np.float32)
+    psf = gaussian_psf(min(15, M, N) | 1, 1.5)[:M, :N]
+    A = CircularConvolve(psf, shape)
+    y = A(dev(xg)) + 0.01 * dev(rng.standard_normal(shape).astype(np.float32))
+    H = A.h_dft.cpu().numpy().astype(np.complex128)
+    L0 = float(np.max(np.abs(H) ** 2))
+    x1 = dev(rng.random(shape).astype(np.float32))
+    lam = 2e-2
+
+    def run(fused):
+        _pgm._FusedDeconv.enabled = fused
+        try:
+            s = AcceleratedPGM(f=loss.SquaredL2Loss(y=y.clone(), A=A),
+                               g=lam * functional.IsotropicTVNorm(), L0=L0,
+                               x0=torch.zeros(shape, device="cuda"), maxiter=10)
+        finally:
+            _pgm._FusedDeconv.enabled = True
+        assert (s._fused is not None) == fused
+        kept = []
+        for k in range(10):
+            v = s.v.clone()
+            s.step()
+            kept.append((s.x, v, float(s.objective()), float(s.norm_residual()),
+                         float(s.fixed_point_residual)))
+        ten = [t[0].clone() for t in kept]
+        s.L = 1.5 * L0
+        s.step()
+        a = s.x.clone()
+        s.x = x1.clone()
+        s.v = 0.5 * x1
+        s.step()
+        b = s.x.clone()
+        s.f.y.mul_(0.5)
+        s.step()
+        return ten, kept, (a, b, s.x.clone())
+
+    tf, kept, cf = run(True)
+    tg, _, cg = run(False)
+    e = max(rel_l2(p.cpu(), q.cpu()) for p, q in zip(tf, tg))
+    ec = max(rel_l2(p.cpu(), q.cpu()) for p, q in zip(cf, cg))
+    y64 = y.cpu().numpy().astype(np.float64)
+    ny = np.linalg.norm(y64)
+    worst = 0.0
+    for x, v, obj, res, fpr in kept:
+        x64 = x.cpu().numpy().astype(np.float64)
+        r = np.linalg.norm(np.fft.ifft2(H * np.fft.fft2(x64)).real - y64)
+        tv = S.tv_norm(x64)
+        bar = 1e-6 * (ny * r + 0.5e-6 * ny**2 + lam * tv)
+        worst = max(worst, abs(obj - (0.5 * r**2 + lam * tv)) / bar)
+        ref = np.linalg.norm(x64 - v.cpu().numpy().astype(np.float64))
+        assert abs(res - ref) <= 1e-9 * ref and fpr == res
+    print(f"  fused APGM {shape}: 10 steps rel-L2 {e:.2e}, after changes {ec:.2e}, objective "
+          f"{worst:.2e} of its bar", flush=True)
+    assert e <= 1e-6 and ec <= 1e-6 and worst <= 1.0
