@@ -834,30 +834,14 @@ __global__ __launch_bounds__(256) void tv_prox_kernel(const float* __restrict__ 
 // of once per neighbouring output, and every output combines the
 // coefficients at p, p - e0 and p - e1 with the same operations, in the
 // same order, as tv_prox_kernel (so the results are bitwise equal).
-//
-// APGM (EXT = 1): the AcceleratedPGM step that follows the prox
-// (scico/optimize/_pgm.py:221-240) and the TV value of its result, fused.
-// The tile computes one extra row and column of outputs (the first of the
-// next tiles, bitwise as they compute them) so that every pixel's forward
-// differences are at hand.  With out holding x_prev and vm the previous
-// extrapolated point v, each stored output x gives the partial sums of
-// (x - v)^2 (the fixed-point residual) and of the TV norm of x (as
-// tv_norm_kernel: sqrt of the squared differences or their absolute
-// values, float64), one each per workgroup, and v <- x + c (x - x_prev),
-// with the operations of the unfused path.
 constexpr int TVT = 16;
-template <int EXT>
 __global__ __launch_bounds__(256) void tv_prox2d_kernel(const float* __restrict__ v,
-                                                        float* out, TvDims t,
+                                                        float* __restrict__ out, TvDims t,
                                                         float tau, float invK, int iso,
                                                         const float* __restrict__ w,
-                                                        const int32_t* pred,
-                                                        const float* xold, const float* vold,
-                                                        float* vm, float c,
-                                                        double* __restrict__ res_ws,
-                                                        double* __restrict__ tv_ws) {
+                                                        const int32_t* pred) {
   if (pred_off(pred)) return;
-  constexpr int NO = TVT + EXT;  // outputs per tile side
+  constexpr int NO = TVT;  // outputs per tile side
   __shared__ float vs[NO + 2][NO + 3];
   __shared__ float cH[2][NO + 1][NO + 2], cL[2][NO + 1][NO + 2];
   const float s = 0.70710677f;
@@ -923,40 +907,139 @@ __global__ __launch_bounds__(256) void tv_prox2d_kernel(const float* __restrict_
   };
   const int ty = tid / TVT, tx = tid - ty * TVT;
   const int pi = i0 + ty, pj = j0 + tx;
-  if constexpr (EXT == 0) {
-    if (pi < M && pj < N) out[static_cast<int64_t>(pi) * N + pj] = output(ty, tx);
-  } else {
-    __shared__ float xs[NO][NO + 1];
-    for (int e = tid; e < NO * NO; e += 256) {
-      const int r = e / NO, cc = e - r * NO;
-      xs[r][cc] = output(r, cc);
+  if (pi < M && pj < N) out[static_cast<int64_t>(pi) * N + pj] = output(ty, tx);
+}
+
+// The AcceleratedPGM step that follows the prox (scico/optimize/_pgm.py:
+// 221-240) and the TV value of its result, fused with the prox of an (M, N)
+// image.  x and v hold the previous iterate and extrapolated point; each
+// output x_new gives the partial sums of (x_new - v)^2 (the fixed-point
+// residual) and of the TV norm of x_new (as tv_norm_kernel: sqrt of the
+// squared differences or their absolute values, float64), one each per
+// workgroup, and v_new = x_new + c (x_new - x), with the operations of the
+// unfused path; x_new and v_new may be x and v.
+//
+// Each wave marches down TVR rows of a strip of TVC columns, one column per
+// lane: the rows it needs are loaded at once, a row's coefficients stay in
+// registers for the next row, and the next column's values come from the
+// neighbouring lane by wave shifts.  Bound by VALU issue (the shrink's
+// square root and quotients, the float64 TV norm) and memory together;
+// 1024 x 1024: 16.1 us on 16 x 16 tiles in LDS (326 instructions per pixel,
+// each stage of a tile leaving most of its last pass idle) -> 11.7 us.
+constexpr int TVR = 4;   // rows per wave (8: 12.8 us, 2: 12.0 us at 1024 x 1024)
+constexpr int TVC = 61;  // columns per wave: lanes 1 .. 61 (lane 62 ends the differences)
+
+// The value of the next / previous lane (0 past the ends).
+__device__ __forceinline__ float lane_next(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x130, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float lane_prev(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
+}
+
+__global__ __launch_bounds__(256) void tv_prox_apgm_kernel(
+    const float* __restrict__ u, TvDims t, float tau, int iso, const float* x, const float* v,
+    float* x_new, float* v_new, float c, int strips, int chunks, double* __restrict__ res_ws,
+    double* __restrict__ tv_ws, const int32_t* pred) {
+  if (pred_off(pred)) return;
+  const float s = 0.70710677f, invK = 0.25f;
+  const int M = t.d[1], N = t.d[2], P0 = t.P[1], P1 = t.P[2];
+  const bool circ = t.circ != 0;
+  const int lane = threadIdx.x & 63;
+  // consecutive workgroups of an XCD (they go to the 8 XCDs in turn) take
+  // neighbouring strips and chunks, which share rows and cache lines
+  int blk = blockIdx.x;
+  {
+    const int G8 = (gridDim.x / 8) * 8;
+    if (blk < G8) blk = (blk % 8) * (G8 / 8) + blk / 8;
+  }
+  const int item = blk * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool live = item < strips * chunks;
+  double res = 0.0, tv = 0.0;
+  if (live) {
+    const int chunk = item / strips, strip = item - chunk * strips;
+    const int i0 = chunk * TVR, j = strip * TVC - 1 + lane;  // this lane's column
+    // padded location q in [-1, ...) modulo P
+    auto wrap = [](int q, int P) {
+      if (q < 0) return q + P;
+      if (q >= P) {
+        q -= P;
+        if (q >= P) q %= P;
+      }
+      return q;
+    };
+    const int jw = wrap(j, P1), js = min(jw, N - 1);
+    const bool jin = circ || jw < N;  // coefficients of this column are shrunk
+    const bool col = lane >= 1 && lane <= TVC && j < N;  // an output column
+    float uu[TVR + 3], xo[TVR], vo[TVR];
+#pragma unroll
+    for (int r = 0; r < TVR + 3; ++r)
+      uu[r] = u[static_cast<int64_t>(min(wrap(i0 - 1 + r, P0), M - 1)) * N + js];
+#pragma unroll
+    for (int r = 0; r < TVR; ++r) {
+      xo[r] = vo[r] = 0.0f;
+      if (col && i0 + r < M) {
+        const int64_t e = static_cast<int64_t>(i0 + r) * N + j;
+        xo[r] = x[e];
+        vo[r] = v[e];
+      }
     }
-    __syncthreads();
-    double res = 0.0, tv = 0.0;
-    if (pi < M && pj < N) {
-      const float xn = xs[ty][tx];
-      const int64_t e = static_cast<int64_t>(pi) * N + pj;
-      const float xo = xold[e], vo = vold[e];
-      const double d = static_cast<double>(xn) - static_cast<double>(vo);
-      res = d * d;
-      vm[e] = __fadd_rn(xn, __fmul_rn(c, __fsub_rn(xn, xo)));
-      out[e] = xn;
-      const bool circ = t.circ != 0;
-      const float g0 = fd::diff_fwd(xn, xs[ty + 1][tx], pi, M, circ);
-      const float g1 = fd::diff_fwd(xn, xs[ty][tx + 1], pj, N, circ);
-      if (iso)
-        tv = sqrt(static_cast<double>(g0) * g0 + static_cast<double>(g1) * g1);
-      else
-        tv = fabs(static_cast<double>(g0)) + fabs(static_cast<double>(g1));
+    float h0p = 0.0f, l0p = 0.0f, xp = 0.0f, xpn = 0.0f;  // of the row above
+#pragma unroll
+    for (int r = 0; r < TVR + 2; ++r) {
+      // coefficients at padded row i0 - 1 + r
+      const float vq = uu[r], vn0 = uu[r + 1], vn1 = lane_next(vq);
+      float H[2] = {__fmul_rn(s, __fsub_rn(vn0, vq)), __fmul_rn(s, __fsub_rn(vn1, vq))};
+      const float L0 = __fmul_rn(s, __fadd_rn(vq, vn0)), L1 = __fmul_rn(s, __fadd_rn(vq, vn1));
+      if (jin && (circ || wrap(i0 - 1 + r, P0) < M)) {
+        if (iso) {
+          l21_shrink(H, 2, tau);
+        } else {
+          H[0] = l1_shrink(H[0], tau);
+          H[1] = l1_shrink(H[1], tau);
+        }
+      }
+      if (r > 0) {  // output row i0 + r - 1: p, p - e0 (row above), p - e1 (lane below)
+        const float lo0 = __fmul_rn(s, __fadd_rn(L0, l0p));
+        const float hi0 = __fmul_rn(s, __fsub_rn(h0p, H[0]));
+        const float lo1 = __fmul_rn(s, __fadd_rn(L1, lane_prev(L1)));
+        const float hi1 = __fmul_rn(s, __fsub_rn(lane_prev(H[1]), H[1]));
+        const float xn = __fmul_rn(invK, __fadd_rn(__fadd_rn(lo0, hi0), __fadd_rn(lo1, hi1)));
+        if (r > 1) {  // TV of row i0 + r - 2, whose next row is at hand now
+          const int pi = i0 + r - 2;
+          if (col && pi < M) {
+            const float g0 = fd::diff_fwd(xp, xn, pi, M, circ);
+            const float g1 = fd::diff_fwd(xp, xpn, j, N, circ);
+            if (iso)
+              tv += sqrt(static_cast<double>(g0) * g0 + static_cast<double>(g1) * g1);
+            else
+              tv += fabs(static_cast<double>(g0)) + fabs(static_cast<double>(g1));
+          }
+        }
+        if (r <= TVR) {
+          const int pi = i0 + r - 1;
+          if (col && pi < M) {
+            const double d = static_cast<double>(xn) - static_cast<double>(vo[r - 1]);
+            res += d * d;
+            const int64_t e = static_cast<int64_t>(pi) * N + j;
+            v_new[e] = __fadd_rn(xn, __fmul_rn(c, __fsub_rn(xn, xo[r - 1])));
+            x_new[e] = xn;
+          }
+        }
+        xp = xn;
+        xpn = lane_next(xn);
+      }
+      h0p = H[0];
+      l0p = L0;
     }
-    __shared__ double sh[4];
-    res = block_sum_f64(res, sh);
-    __syncthreads();
-    tv = block_sum_f64(tv, sh);
-    if (tid == 0) {
-      res_ws[by * gridDim.x + bx] = res;
-      tv_ws[by * gridDim.x + bx] = tv;
-    }
+  }
+  __shared__ double sh[4];
+  res = block_sum_f64(res, sh);
+  __syncthreads();
+  tv = block_sum_f64(tv, sh);
+  if (threadIdx.x == 0) {
+    res_ws[blockIdx.x] = res;
+    tv_ws[blockIdx.x] = tv;
   }
 }
 
@@ -1524,9 +1607,8 @@ int scxr_tv_prox(int32_t ndim, const int32_t* shape, const float* v, float* out,
   const int64_t n = static_cast<int64_t>(t.d[0]) * t.d[1] * t.d[2];
   if (ndim == 2) {
     const dim3 g(ceil_div(t.d[2], solver::TVT), ceil_div(t.d[1], solver::TVT));
-    hipLaunchKernelGGL(solver::tv_prox2d_kernel<0>, g, dim3(256), 0, as_stream(stream), v,
-                       out, t, tau, 0.25f, isotropic, nullptr, pred, nullptr, nullptr, nullptr,
-                       0.0f, nullptr, nullptr);
+    hipLaunchKernelGGL(solver::tv_prox2d_kernel, g, dim3(256), 0, as_stream(stream), v, out, t,
+                       tau, 0.25f, isotropic, nullptr, pred);
   } else {
     hipLaunchKernelGGL(solver::tv_prox_kernel, dim3(solver::elem_grid(n)), dim3(256), 0,
                        as_stream(stream), v, out, t, tau, 1.0f / static_cast<float>(2 * ndim),
@@ -1538,7 +1620,8 @@ int scxr_tv_prox(int32_t ndim, const int32_t* shape, const float* v, float* out,
 
 int32_t scxr_tv_prox_apgm_parts(int32_t M, int32_t N) {
   if (M <= 0 || N <= 0) return -1;
-  return static_cast<int32_t>(ceil_div(M, solver::TVT) * ceil_div(N, solver::TVT));
+  return static_cast<int32_t>(ceil_div(
+      static_cast<long long>(ceil_div(N, solver::TVC)) * ceil_div(M, solver::TVR), 4));
 }
 
 int scxr_tv_prox_apgm(int32_t M, int32_t N, const float* u, float* x, float* v, float tau,
@@ -1559,9 +1642,11 @@ int scxr_tv_prox_apgm_to(int32_t M, int32_t N, const float* u, const float* x, c
   solver::TvDims t;
   const int rc = tv_dims(2, shape, circular, t);
   if (rc) return rc;
-  const dim3 g(ceil_div(N, solver::TVT), ceil_div(M, solver::TVT));
-  hipLaunchKernelGGL(solver::tv_prox2d_kernel<1>, g, dim3(256), 0, as_stream(stream), u, x_new, t,
-                     tau, 0.25f, isotropic, nullptr, pred, x, v, v_new, c, res_ws, tv_ws);
+  const int strips = static_cast<int>(ceil_div(N, solver::TVC));
+  const int chunks = static_cast<int>(ceil_div(M, solver::TVR));
+  hipLaunchKernelGGL(solver::tv_prox_apgm_kernel, dim3(scxr_tv_prox_apgm_parts(M, N)), dim3(256),
+                     0, as_stream(stream), u, t, tau, isotropic, x, v, x_new, v_new, c, strips,
+                     chunks, res_ws, tv_ws, pred);
   SCXR_LAUNCHED("tv prox apgm");
   return SCXR_OK;
 }
@@ -1577,9 +1662,8 @@ int scxr_tv_prox_w(int32_t ndim, const int32_t* shape, const float* v, const flo
   const int64_t n = static_cast<int64_t>(t.d[0]) * t.d[1] * t.d[2];
   if (ndim == 2) {
     const dim3 g(ceil_div(t.d[2], solver::TVT), ceil_div(t.d[1], solver::TVT));
-    hipLaunchKernelGGL(solver::tv_prox2d_kernel<0>, g, dim3(256), 0, as_stream(stream), v,
-                       out, t, tau, 0.25f, isotropic, w, pred, nullptr, nullptr, nullptr, 0.0f,
-                       nullptr, nullptr);
+    hipLaunchKernelGGL(solver::tv_prox2d_kernel, g, dim3(256), 0, as_stream(stream), v, out, t,
+                       tau, 0.25f, isotropic, w, pred);
   } else {
     hipLaunchKernelGGL(solver::tv_prox_kernel, dim3(solver::elem_grid(n)), dim3(256), 0,
                        as_stream(stream), v, out, t, tau, 1.0f / static_cast<float>(2 * ndim),
