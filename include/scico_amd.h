@@ -186,6 +186,9 @@ int scxr_vec_copy(int64_t n, const float* x, float* z, const int32_t* pred, void
 /* z = x * y elementwise. */
 int scxr_vec_mul(int64_t n, const float* x, const float* y, float* z, const int32_t* pred,
                  void* stream);
+/* z = (a x) y elementwise (scxr_vec_scale, then scxr_vec_mul, in one pass). */
+int scxr_vec_scale_mul(int64_t n, float a, const float* x, const float* y, float* z,
+                       const int32_t* pred, void* stream);
 /* z = (x >= thr) ? v : 0. */
 int scxr_vec_ge(int64_t n, const float* x, float thr, float v, float* z, const int32_t* pred,
                 void* stream);

@@ -83,6 +83,14 @@ def mul(x, y, out=None, pred=None):
     return out
 
 
+def scale_mul(a, x, y, out=None, pred=None):
+    """``(a x) y`` in one pass (``mul(scale(a, x), y)``)."""
+    out = torch.empty_like(x) if out is None else out
+    call("scxr_vec_scale_mul", _n(x), float(a), x.data_ptr(), y.data_ptr(), out.data_ptr(),
+         dev.ptr(_pred.resolve(pred)), dev.stream())
+    return out
+
+
 def ge(x, thr, v=1.0, out=None, pred=None):
     """``(x >= thr) * v``."""
     out = torch.empty_like(x) if out is None else out

@@ -59,6 +59,16 @@ __global__ __launch_bounds__(256) void mul_kernel(int64_t n, const float* __rest
     z[e] = __fmul_rn(x[e], y[e]);
 }
 
+// z = (a x) y, both products rounded
+__global__ __launch_bounds__(256) void scale_mul_kernel(int64_t n, float a,
+                                                        const float* __restrict__ x,
+                                                        const float* y, float* z,
+                                                        const int32_t* pred) {
+  if (pred_off(pred)) return;
+  for (int64_t e = blockIdx.x * 256ll + threadIdx.x; e < n; e += 256ll * gridDim.x)
+    z[e] = __fmul_rn(__fmul_rn(a, x[e]), y[e]);
+}
+
 // z = (x >= thr) ? v : 0
 __global__ __launch_bounds__(256) void ge_kernel(int64_t n, const float* __restrict__ x, float thr,
                                                  float v, float* __restrict__ z,
@@ -261,6 +271,16 @@ int scxr_vec_mul(int64_t n, const float* x, const float* y, float* z, const int3
   hipLaunchKernelGGL(vec::mul_kernel, dim3(vec::grid_for(n)), dim3(256), 0, as_stream(stream), n,
                      x, y, z, pred);
   SCXR_LAUNCHED("mul");
+  return SCXR_OK;
+}
+
+int scxr_vec_scale_mul(int64_t n, float a, const float* x, const float* y, float* z,
+                       const int32_t* pred, void* stream) {
+  SCXR_REQUIRE(n >= 0 && (n == 0 || (x && y && z)), SCXR_ERR_ARG, "bad scale_mul arguments");
+  if (n == 0) return SCXR_OK;
+  hipLaunchKernelGGL(vec::scale_mul_kernel, dim3(vec::grid_for(n)), dim3(256), 0,
+                     as_stream(stream), n, a, x, y, z, pred);
+  SCXR_LAUNCHED("scale_mul");
   return SCXR_OK;
 }
 

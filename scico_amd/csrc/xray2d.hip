@@ -1159,26 +1159,81 @@ __global__ __launch_bounds__(256 * ADJ_VS) __attribute__((amdgpu_waves_per_eu(4)
 // FBP row filter (_xray2d.py:187-194): the reference convolves each row
 // with the ramp taps h[0..D) by zero-padded FFT of length 2D - 1 and keeps
 // [s, 2D - 1 - s), s = (D - 1) / 2; here the same linear convolution is
-// summed directly: out[a, t] = sum_m h[m] y[a, t + s - m], 0 <= t + s - m < D.
+// summed directly: out[a, t] = sum_k y[a, k] h[t + s - k], a product of the
+// rows with the Toeplitz matrix of the taps, on the float32 matrix cores.
+// A workgroup takes 16 rows x 64 outputs (16 x 16 per wave) and walks the
+// inputs that reach them in chunks of 256 through LDS, four per MFMA; two
+// accumulators take alternate steps.  Bound by the latency of one or two
+// waves per SIMD (a sinogram has few rows); 301 rows of 595: 54 -> 9.9 us
+// against one row per workgroup with two LDS reads per multiply-add.
+// The matrix products include the zeros beyond the taps, so a tile with an
+// input that is not finite takes the plain sums, which leave them out.
+constexpr int RAMP_K = 256, RAMP_T = 64, RAMP_A = 16;
+
 __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
                                                    float* __restrict__ out,
-                                                   const float* __restrict__ taps, int D, int Dout,
-                                                   int s, const int32_t* pred) {
+                                                   const float* __restrict__ taps, int A, int D,
+                                                   int Dout, int s, const int32_t* pred) {
   if (pred_off(pred)) return;
-  __shared__ float row[4096];
-  __shared__ float h[4096];
-  const int a = blockIdx.x;
-  for (int k = threadIdx.x; k < D; k += 256) {
-    row[k] = y[static_cast<size_t>(a) * D + k];
-    h[k] = taps[k];
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  __shared__ float rows[RAMP_A][RAMP_K + 4];
+  __shared__ float h[RAMP_K + RAMP_T];
+  __shared__ int bad;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int a0 = blockIdx.y * RAMP_A, t0 = blockIdx.x * RAMP_T;
+  if (threadIdx.x == 0) bad = 0;
+  // inputs k with 0 <= t + s - k < D for some output t of the tile
+  const int kb = max(0, t0 + s - (D - 1)), ke = min(D, t0 + RAMP_T + s);
+  f4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  const int i = lane & 15, kk = lane >> 4;
+  bool fin = true;
+  for (int k0 = kb; k0 < ke; k0 += RAMP_K) {
+    __syncthreads();
+    float v[RAMP_A];  // all loads in flight at once
+#pragma unroll
+    for (int r = 0; r < RAMP_A; ++r) {
+      const int a = a0 + r, k = k0 + threadIdx.x;
+      v[r] = (a < A && k < ke) ? y[static_cast<size_t>(a) * D + k] : 0.0f;
+    }
+#pragma unroll
+    for (int r = 0; r < RAMP_A; ++r) {
+      fin = fin && fabsf(v[r]) <= 3.402823466e38f;
+      rows[r][threadIdx.x] = v[r];
+    }
+    // h[e] = tap of distance t - k = e - (RAMP_K - 1) from the chunk's origin
+    for (int e = threadIdx.x; e < RAMP_K + RAMP_T; e += 256) {
+      const int m = t0 - k0 + s + e - (RAMP_K - 1);
+      const float g = m >= 0 && m < D ? taps[m] : 0.0f;
+      fin = fin && fabsf(g) <= 3.402823466e38f;
+      h[e] = g;
+    }
+    __syncthreads();
+    const float* hp = h + 16 * wave + i + (RAMP_K - 1) - kk;
+    const float* rp = &rows[i][kk];
+    const int steps = (min(RAMP_K, ke - k0) + 3) / 4;  // rounded up to 8 below: rows are 0 there
+    for (int q0 = 0; q0 < steps; q0 += 8) {
+#pragma unroll
+      for (int q = q0; q < q0 + 8; ++q)
+        acc[q & 1] =
+            __builtin_amdgcn_mfma_f32_16x16x4f32(rp[4 * q], hp[-4 * q], acc[q & 1], 0, 0, 0);
+    }
   }
+  if (!fin) bad = 1;
   __syncthreads();
-  for (int t = threadIdx.x; t < Dout; t += 256) {
-    const int c = t + s;
-    const int m0 = max(0, c - D + 1), m1 = min(D - 1, c);
-    float acc = 0.0f;
-    for (int m = m0; m <= m1; ++m) acc = fmaf(h[m], row[c - m], acc);
-    out[static_cast<size_t>(a) * Dout + t] = acc;
+  const int t = t0 + 16 * wave + i;
+  if (t >= Dout) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int a = a0 + 4 * kk + r;
+    if (a >= A) break;
+    float v = acc[0][r] + acc[1][r];
+    if (bad) {
+      const int c = t + s;
+      v = 0.0f;
+      for (int m = max(0, c - D + 1); m <= min(D - 1, c); ++m)
+        v = fmaf(taps[m], y[static_cast<size_t>(a) * D + c - m], v);
+    }
+    out[static_cast<size_t>(a) * Dout + t] = v;
   }
 }
 
@@ -1630,8 +1685,8 @@ int scxr_ramp_filter(int32_t A, int32_t D, int32_t Dout, int32_t shift, const fl
                      const float* y, float* out, const int32_t* pred, void* stream) {
   SCXR_REQUIRE(A > 0 && D > 0 && D <= 4096 && Dout > 0 && taps && y && out, SCXR_ERR_ARG,
                "bad ramp_filter arguments (D must be in [1, 4096])");
-  hipLaunchKernelGGL(ramp_kernel, dim3(A), dim3(256), 0, as_stream(stream), y, out, taps, D, Dout,
-                     shift, pred);
+  hipLaunchKernelGGL(ramp_kernel, dim3(ceil_div(Dout, RAMP_T), ceil_div(A, RAMP_A)), dim3(256), 0,
+                     as_stream(stream), y, out, taps, A, D, Dout, shift, pred);
   SCXR_LAUNCHED("ramp filter");
   return SCXR_OK;
 }

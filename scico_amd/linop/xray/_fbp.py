@@ -55,4 +55,4 @@ def fbp(H, y):
          hy.data_ptr(), None, dev.stream())
     bp = H.back_project(hy)
     c = float(np.float32(np.pi * float(np.asarray(H.dx[0])) * float(np.asarray(H.dx[1])) / A))
-    return vec.mul(vec.scale(c, H.fbp_mask), bp)
+    return vec.scale_mul(c, H.fbp_mask, bp, out=bp)

@@ -304,3 +304,39 @@ def test_general_geometry_kernels(gpu, dx, dc):
         finally:
             admm_mod._FusedTV.enabled = old
     assert rel_l2(xs[0], xs[1]) <= 1e-4
+
+
+@pytest.mark.parametrize("A,D", [(1, 2), (15, 3), (16, 64), (17, 65), (5, 300), (33, 595),
+                                 (2, 4096)])
+def test_ramp_filter_rows(gpu, A, D):
+    """FBP's row filter at the edges of its tiles (16 rows, 64 outputs, chunks
+    of 256 inputs) against the float64 convolution; the sum of D products in
+    float32 is off by at most D eps sum |h| |y|.  A value that is not finite
+    reaches the outputs within D - 1 - s taps of it and no others."""
+    from scico_amd._lib import call
+    from scico_amd.linop.xray._fbp import filter_window, ramp_filter
+
+    rng = np.random.default_rng(A * 10000 + D)
+    s, Dout = filter_window(D)
+    h = ramp_filter(np.arange(D) - s, 1.0)
+    y = rng.standard_normal((A, D)).astype(np.float32)
+    out = torch.empty((A, Dout), device="cuda")
+
+    def run(rows):
+        hd, yd = torch.as_tensor(h, device="cuda"), torch.as_tensor(rows, device="cuda")
+        call("scxr_ramp_filter", A, D, Dout, s, hd.data_ptr(), yd.data_ptr(), out.data_ptr(), None,
+             torch.cuda.current_stream().cuda_stream)
+        return out.cpu().numpy()
+
+    got = run(y)
+    h64, y64 = h.astype(np.float64), y.astype(np.float64)
+    ref = np.stack([np.convolve(r, h64)[s : s + Dout] for r in y64])
+    bar = D * 2.0**-24 * np.stack([np.convolve(np.abs(r), np.abs(h64))[s : s + Dout] for r in y64])
+    assert np.all(np.abs(got - ref) <= bar + 1e-30)
+    y[A - 1, D // 2] = np.inf
+    bad = run(y)
+    t = np.arange(Dout)
+    reach = (t + s - D // 2 >= 0) & (t + s - D // 2 < D)
+    np.testing.assert_array_equal(np.isfinite(bad[A - 1]), ~reach)
+    assert np.all(np.abs(bad[A - 1, ~reach] - ref[A - 1, ~reach]) <= bar[A - 1, ~reach] + 1e-30)
+    assert np.all(np.abs(bad[: A - 1] - ref[: A - 1]) <= bar[: A - 1] + 1e-30)
