@@ -112,8 +112,8 @@ int scxr_ramp_filter(int32_t A, int32_t D, int32_t Dout, int32_t shift, const fl
  * `parts` workgroups (1..8) whose partial sinograms are added in part
  * order, which balances the CUs when there are few views.  parts = 0
  * restores the automatic choice made at plan creation (4 for images of at
- * least 256 x 256 pixels with fewer than two forward workgroups per CU,
- * else 1).  The split changes the
+ * least 256 x 256 pixels with fewer than two forward groups per CU and for
+ * images of at least 128 x 128 pixels with at most 3/4 of one, else 1).  The split changes the
  * float32 summation order of a detector bin (results move by rounding,
  * relative L2 about 1e-7); with parts = 1 the plan's forward is bitwise
  * equal to the batched projector's for the same slice.  The effective

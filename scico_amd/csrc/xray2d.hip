@@ -10,6 +10,7 @@
 // (_xray2d.py:326-347).
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "common.h"
@@ -271,6 +272,16 @@ int build_tables(HostTables& h, int M, int N, int A, int D, const double* x0, co
 
 static hipError_t fwd_allow_lds(int bytes);
 
+// Distance of staged image columns (rows past the image are zero, at least
+// four of them): the columns start 4 banks apart (16 columns x 4 rows are
+// written at once) and 16-byte aligned.  0 for strides without a compiled
+// walk.
+static int column_pitch(const HostTables& h, int M) {
+  for (const int4& g : h.groups)
+    if ((g.z & 1) && (g.w < 3 || g.w > 5)) return 0;
+  return (M + 31) / 32 * 32 + 4;
+}
+
 int create(Plan& p, int M, int N, int A, int D, const double* x0, const double* dx,
            double y0, const float* angles) {
   p.M = M;
@@ -308,6 +319,7 @@ int create(Plan& p, int M, int N, int A, int D, const double* x0, const double* 
   p.host_geom = h.geom;
   p.any_colfast = h.any_colfast;
   p.n_groups = static_cast<int>(h.groups.size());
+  p.fwd_pitch = p.vpg == 1 && p.any_colfast && !h.fwd_generic ? column_pitch(h, M) : 0;
   p.adj_w = h.adj_w;
   const std::vector<float4>& geom = h.geom;
   std::vector<double>& rw = h.rw;
@@ -317,43 +329,41 @@ int create(Plan& p, int M, int N, int A, int D, const double* x0, const double* 
 
   // (the adjoint reads up to RW_PAD entries past the last view's)
   rw.resize(A + RW_PAD, 1.0);
-  size_t bytes_geom = sizeof(float4) * A, bytes_rw = sizeof(double) * rw.size();
-  size_t bytes_groups = sizeof(int4) * groups.size(), bytes_order = sizeof(int) * A;
-  size_t bytes_clo = sizeof(float) * A;
   // block index -> forward group, balanced over the CUs
   std::vector<int> gblock;
   if (!groups.empty()) {
     int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        cus <= 0)
-      cus = 256;
-    gblock = place_groups(h.gcost, cus);
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+        cus > 0)
+      p.cus = cus;
+    gblock = place_groups(h.gcost, p.cus);
   }
-  size_t bytes_gblock = sizeof(int) * gblock.size();
-  size_t total =
-      bytes_geom + bytes_rw + bytes_groups + bytes_order + bytes_clo + bytes_gblock + 256 * 6;
-  if (hipMalloc(&p.dev_block, total) != hipSuccess)
-    return fail(SCXR_ERR_NOMEM, "hipMalloc of %zu bytes for the plan tables failed", total);
-  char* base = static_cast<char*>(p.dev_block);
-  auto carve = [&](size_t bytes) {
-    char* r = base;
-    base += (bytes + 255) & ~static_cast<size_t>(255);
-    return r;
+  std::vector<FwdBlock> blocks;
+  for (int gi : gblock) {
+    const int a = order[groups[gi].x];
+    blocks.push_back(FwdBlock{geom[a], rw[a], a, gi, groups[gi]});
+  }
+  // one allocation and one copy: the tables, each 256-byte aligned
+  std::vector<char> host;
+  auto put = [&](const auto& v) {
+    const size_t at = host.size(), bytes = sizeof(v[0]) * v.size();
+    host.resize(at + (bytes + 255) / 256 * 256);
+    if (bytes) std::memcpy(host.data() + at, v.data(), bytes);
+    return at;
   };
-  p.geom = reinterpret_cast<float4*>(carve(bytes_geom));
-  p.rw = reinterpret_cast<double*>(carve(bytes_rw));
-  p.groups = reinterpret_cast<int4*>(carve(bytes_groups));
-  p.order = reinterpret_cast<int*>(carve(bytes_order));
-  p.clo = reinterpret_cast<float*>(carve(bytes_clo));
-  p.gblock = reinterpret_cast<int*>(carve(bytes_gblock));
-  if (bytes_gblock)
-    SCXR_HIP(hipMemcpy(p.gblock, gblock.data(), bytes_gblock, hipMemcpyHostToDevice));
-  SCXR_HIP(hipMemcpy(p.clo, clo.data(), bytes_clo, hipMemcpyHostToDevice));
-  SCXR_HIP(hipMemcpy(p.geom, geom.data(), bytes_geom, hipMemcpyHostToDevice));
-  SCXR_HIP(hipMemcpy(p.rw, rw.data(), bytes_rw, hipMemcpyHostToDevice));
-  SCXR_HIP(hipMemcpy(p.groups, groups.data(), bytes_groups, hipMemcpyHostToDevice));
-  SCXR_HIP(hipMemcpy(p.order, order.data(), bytes_order, hipMemcpyHostToDevice));
+  const size_t at_geom = put(geom), at_rw = put(rw), at_order = put(order), at_clo = put(clo),
+               at_blocks = put(blocks), at_done = put(std::vector<int>(groups.size(), 0));
+  if (hipMalloc(&p.dev_block, host.size()) != hipSuccess)
+    return fail(SCXR_ERR_NOMEM, "hipMalloc of %zu bytes for the plan tables failed", host.size());
+  SCXR_HIP(hipMemcpy(p.dev_block, host.data(), host.size(), hipMemcpyHostToDevice));
+  char* base = static_cast<char*>(p.dev_block);
+  p.geom = reinterpret_cast<float4*>(base + at_geom);
+  p.rw = reinterpret_cast<double*>(base + at_rw);
+  p.order = reinterpret_cast<int*>(base + at_order);
+  p.clo = reinterpret_cast<float*>(base + at_clo);
+  p.gblock = reinterpret_cast<FwdBlock*>(base + at_blocks);
+  p.done = reinterpret_cast<int*>(base + at_done);
   if (p.any_colfast) {
     if (hipMalloc(&p.work, sizeof(float) * static_cast<size_t>(M) * N) != hipSuccess)
       return fail(SCXR_ERR_NOMEM, "hipMalloc of the transpose workspace failed");
@@ -366,25 +376,22 @@ int create(Plan& p, int M, int N, int A, int D, const double* x0, const double* 
 // A forward group's lines can be split over several workgroups, whose
 // partial rows are added in a fixed order afterwards: with one workgroup
 // per view, a few hundred views leave the 256 CUs unevenly loaded.
-// Automatic choice, from a sweep of 1..8 parts on MI355X (90..720 views,
-// 128^2..512^2 pixels): 4 parts (within 10 % of the best count in every
-// case measured; 512^2 with 360 views 94 -> 65 us, with 90 views 51 ->
-// 35 us) for images of at least 256 x 256 pixels with fewer than two
-// forward groups per CU.  Smaller images keep one workgroup per group (the
-// extra launch costs more than the split saves: 128^2 with 60 views 12.5 ->
-// 14.8 us), and so do plans with more groups: at 512^2 with 720 views the
-// split would save 13 % of the forward, but its rounding took a 100-step
+// Automatic choice, from a sweep of 1..8 parts on MI355X (30..720 views,
+// 48^2..600^2 pixels): 4 parts (512^2 with 360 views 69 -> 59 us, with 90
+// views 50 -> 30 us) for images of at least 256 x 256 pixels with fewer than
+// two forward groups per CU, and from 128 x 128 pixels with up to 3/4 of one
+// (128^2 with 60 views 11.5 -> 7.1 us, with 180 views 11.9 -> 10.1 us, with
+// 360 views 12 -> 17 us).  Smaller images keep one workgroup per group (the
+// split gains a tenth: 64^2 with 60 views 6.0 -> 5.6 us), and so do plans
+// with more groups: at 512^2 with 720 views the
+// split would save 5 % of the forward, but its rounding took a 100-step
 // ADMM-TV run with early-stopping CG outside the drift envelope of the
 // reference-arithmetic runs at one iteration, which the unsplit projector
 // stays well inside.
 int auto_split(const Plan& p) {
-  if (p.fwd_generic || static_cast<long long>(p.M) * p.N < 65536) return 1;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus <= 0)
-    return 1;
-  return p.n_groups < 2 * cus ? 4 : 1;
+  const long long px = static_cast<long long>(p.M) * p.N;
+  if (p.fwd_generic || px < 16384) return 1;
+  return p.n_groups < 2 * p.cus && (px >= 65536 || 4 * p.n_groups <= 3 * p.cus) ? 4 : 1;
 }
 
 // Sets the forward split (1..FWD_SP_MAX parts; 1 for the general-geometry
@@ -749,35 +756,114 @@ __device__ __forceinline__ void fwd_body_s(const float* __restrict__ src, float*
   }
 }
 
-// One forward group (gi indexes groups[]); acc is the dynamic LDS array.
-template <int V, int CH, bool FR>
+// Copies the image columns of the workgroup's share into LDS (`share`,
+// `pitch` apart, zeros past the image), for the column-fast walk without a
+// transposed image: a small forward is latency and launches, and the launch
+// that transposes costs it 2 us (128^2 with 60 views in 4 parts 9.3 -> 7.1 us).
+template <int CH>
+__device__ __forceinline__ void fwd_stage(const float* __restrict__ im, float* share, int pitch,
+                                          int M, int N) {
+  constexpr int K = FWD_WAVES * CH, RP = 64 * FWD_WAVES / K;
+  const int scol = threadIdx.x % K, srow = threadIdx.x / K;
+  float* dst = share + scol * pitch;
+  for (int base = K * static_cast<int>(blockIdx.y); base < N;
+       base += K * static_cast<int>(gridDim.y), dst += K * pitch) {
+    const bool in = base + scol < N;
+    const float* src = im + base + scol;
+#pragma unroll 8
+    for (int r = srow; r < pitch; r += RP)
+      dst[r] = in && r < M ? src[static_cast<size_t>(r) * N] : 0.0f;
+  }
+}
+
+// The column-fast walk over the staged share: same pixels, lanes and order as
+// fwd_body_s, so the same result bit for bit.
+template <int CH, int S, bool FR>
+__device__ __forceinline__ void fwd_body_staged(float* acc, const float* share, int pitch, int L,
+                                                int kmul, const float* Pxmin, const float* P0,
+                                                const float* P1, const double* rw, int M, int N,
+                                                int D) {
+  constexpr int K = FWD_WAVES * CH;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const float Dmax = static_cast<float>(D);
+  constexpr int span = 64 * S;
+  const int loff = S * ((lane * kmul) & 63);
+  int row[CH][1];
+#pragma unroll
+  for (int c = 0; c < CH; ++c) row[c][0] = (wave * CH + c) * L + 2;
+  float flr[S];
+#pragma unroll
+  for (int r = 0; r < S; ++r) flr[r] = static_cast<float>(loff + r);
+  const float* col = share + wave * pitch;
+  for (int base = K * static_cast<int>(blockIdx.y); base < N;
+       base += K * static_cast<int>(gridDim.y), col += K * pitch) {
+    float t[CH][1];
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+      t[c][0] = __fmul_rn(P1[0], static_cast<float>(base + wave + FWD_WAVES * c));
+    for (int c0 = 0; c0 < M; c0 += span) {
+      const float fc0 = static_cast<float>(c0);
+      float cur[CH][S];
+#pragma unroll
+      for (int c = 0; c < CH; ++c) {
+        // lanes past the image read the zeros that end the column
+        const float* p = col + FWD_WAVES * c * pitch;
+        if constexpr (S == 4) {
+          const float4 v = *reinterpret_cast<const float4*>(p + min(c0 + loff, pitch - 4));
+          cur[c][0] = v.x, cur[c][1] = v.y, cur[c][2] = v.z, cur[c][3] = v.w;
+        } else {
+#pragma unroll
+          for (int r = 0; r < S; ++r) cur[c][r] = p[min(c0 + loff + r, pitch - 1)];
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < S; ++r) {
+        float val[CH];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) val[c] = cur[c][r];
+        fwd_phase<1, CH, true, FR>(acc, row, t, val, __fadd_rn(fc0, flr[r]), 1, Pxmin, P0, P1, rw,
+                                   Dmax);
+      }
+    }
+  }
+}
+
+// One of a group's views.
+struct FwdView {
+  float4 g;
+  double rw;
+  int view;
+};
+
+// Forward group gi (grp: its row of groups[]; view_of(v): its views); acc is
+// the dynamic LDS array.  STG: column-fast groups stage columns of im
+// `pitch` apart behind the rows in acc.  part: the rows go to another
+// workgroup, so they are stored at agent scope.
+template <int V, int CH, bool FR, bool STG, class Views>
 __device__ __forceinline__ void fwd_group(const float* __restrict__ im,
                                           const float* __restrict__ imT,
-                                          float* __restrict__ sino,
-                                          const float4* __restrict__ geom,
-                                          const double* __restrict__ rwt,
-                                          const int4* __restrict__ groups,
-                                          const int* __restrict__ order, int M, int N, int D,
+                                          float* __restrict__ sino, const Views& view_of,
+                                          const int4 grp, int M, int N, int D,
                                           const float* __restrict__ yres,
-                                          double* __restrict__ res_ws, int gi, float* acc) {
+                                          double* __restrict__ res_ws, int gi, float* acc,
+                                          int pitch, bool part) {
   __shared__ double red[FWD_WAVES];
   const int L = D + 4;
-  const int4 grp = groups[gi];
   const int cnt = grp.y;
-  float Pxmin[V], P0[V], P1[V], wd[V];
+  float Pxmin[V], P0[V], P1[V];
   double rw[V];
   int view[V];
 #pragma unroll
   for (int v = 0; v < V; ++v) {
-    const int a = order[grp.x + (v < cnt ? v : 0)];
-    view[v] = a;
-    const float4 g = geom[a];
-    Pxmin[v] = g.x;
-    P0[v] = g.y;
-    P1[v] = g.z;
-    wd[v] = g.w;
-    rw[v] = rwt[a];
+    const FwdView w = view_of(v < cnt ? v : 0);
+    view[v] = w.view;
+    Pxmin[v] = w.g.x;
+    P0[v] = w.g.y;
+    P1[v] = w.g.z;
+    rw[v] = w.rw;
   }
+  if constexpr (STG)
+    if (grp.z & 1) fwd_stage<CH>(im, acc + FWD_WAVES * CH * L, pitch, M, N);
   for (int e = threadIdx.x; e < V * FWD_WAVES * CH * L; e += 64 * FWD_WAVES) acc[e] = 0.0f;
   __syncthreads();
   // lane strides 3 to 5 cover unit-spaced detectors with pixel sizes
@@ -786,7 +872,13 @@ __device__ __forceinline__ void fwd_group(const float* __restrict__ im,
   const int kmul = grp.z >> 1;  // lane permutation multiplier (odd)
   const float* src = colf ? imT : im;
 #define SCXR_FWD_S(SS)                                                                 \
-  if (colf)                                                                            \
+  if constexpr (STG) {                                                                 \
+    if (colf)                                                                          \
+      fwd_body_staged<CH, SS, FR>(acc, acc + FWD_WAVES * CH * L, pitch, L, kmul, Pxmin, P0, P1, \
+                                  rw, M, N, D);                                        \
+    else                                                                               \
+      fwd_body_s<V, CH, false, SS, FR>(im, acc, L, cnt, kmul, Pxmin, P0, P1, rw, M, N, D); \
+  } else if (colf)                                                                     \
     fwd_body_s<V, CH, true, SS, FR>(src, acc, L, cnt, kmul, Pxmin, P0, P1, rw, M, N, D);   \
   else                                                                                 \
     fwd_body_s<V, CH, false, SS, FR>(src, acc, L, cnt, kmul, Pxmin, P0, P1, rw, M, N, D);
@@ -801,7 +893,7 @@ __device__ __forceinline__ void fwd_group(const float* __restrict__ im,
       SCXR_FWD_S(5)
       break;
     default:
-      if (colf)
+      if (!STG && colf)
         fwd_body<V, CH, true, FR>(src, acc, L, cnt, grp.w, kmul, Pxmin, P0, P1, rw, M, N, D);
       else
         fwd_body<V, CH, false, FR>(src, acc, L, cnt, grp.w, kmul, Pxmin, P0, P1, rw, M, N, D);
@@ -818,7 +910,10 @@ __device__ __forceinline__ void fwd_group(const float* __restrict__ im,
       for (int b = threadIdx.x; b < D; b += 64 * FWD_WAVES) {
         float val = r[b];
         for (int c = 1; c < FWD_WAVES * CH; ++c) val = __fadd_rn(val, r[c * L + b]);
-        dst[b] = val;
+        if (part)
+          __hip_atomic_store(dst + b, val, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+          dst[b] = val;
         if (yrow) {
           const double d = static_cast<double>(__fsub_rn(yrow[b], val));
           res += d * d;
@@ -842,53 +937,65 @@ __device__ __forceinline__ void fwd_group(const float* __restrict__ im,
 
 // Workgroup (b, part) of a grid (groups, SP) runs forward group gblock[b]
 // (the CU-balanced placement of the plan), taking every SP-th set of
-// FWD_WAVES * CH lines of it, from set `part`; with SP > 1 it writes
-// its rows to partial sinogram `part` of `parts` (A x D each), which
-// fwd_parts_kernel adds up.
-template <int V, int CH, bool FR>
+// FWD_WAVES * CH lines of it, from set `part`.  With SP > 1 it writes its
+// rows to partial sinogram `part` of `parts` (A x D each), and the
+// workgroup of a group that finishes last adds the parts up, in part order
+// whichever it is (a launch of its own for the sums: 17.8 us against 15.8 at
+// 256^2 with 180 views, 4 parts).  The parts cross between workgroups, so
+// they are stored and loaded at agent scope, past the XCD's cache, and every
+// wave's stores are complete before the workgroup is counted.  (A release
+// fence instead writes the whole L2 back in every workgroup: 130 us.)
+template <int V, int CH, bool FR, bool STG>
 __global__ __launch_bounds__(64 * FWD_WAVES) void fwd_kernel(const float* __restrict__ im,
                                                   const float* __restrict__ imT,
                                                   float* __restrict__ sino,
                                                   const float4* __restrict__ geom,
                                                   const double* __restrict__ rwt,
-                                                  const int4* __restrict__ groups,
                                                   const int* __restrict__ order, int M, int N,
                                                   int D, const float* __restrict__ yres,
                                                   double* __restrict__ res_ws,
-                                                  float* __restrict__ parts, int A,
-                                                  const int* __restrict__ gblock,
-                                                  const int32_t* pred) {
+                                                  float* parts, int A,
+                                                  const FwdBlock* __restrict__ gblock, int* done,
+                                                  int pitch, const int32_t* pred) {
   if (pred_off(pred)) return;
-  extern __shared__ float acc[];  // [V][FWD_WAVES waves][CH chains][L]
-  const int gi = gblock[blockIdx.x];
-  if (gridDim.y > 1)
-    fwd_group<V, CH, FR>(im, imT, parts + static_cast<size_t>(blockIdx.y) * A * D, geom, rwt,
-                         groups, order, M, N, D, nullptr, nullptr, gi, acc);
-  else
-    fwd_group<V, CH, FR>(im, imT, sino, geom, rwt, groups, order, M, N, D, yres, res_ws, gi,
-                         acc);
-}
-
-// sino = parts[0] + parts[1] + ... (in part order) for the views of group
-// blockIdx.x, with that group's residual partial as fwd_group writes it.
-__global__ __launch_bounds__(256) void fwd_parts_kernel(const float* __restrict__ parts, int sp,
-                                                        int A, int D, float* __restrict__ sino,
-                                                        const int4* __restrict__ groups,
-                                                        const int* __restrict__ order,
-                                                        const float* __restrict__ yres,
-                                                        double* __restrict__ res_ws,
-                                                        const int32_t* pred) {
-  if (pred_off(pred)) return;
-  __shared__ double red[4];
-  const int gi = blockIdx.x;
-  const int4 grp = groups[gi];
+  extern __shared__ __align__(16) float acc[];  // [V][FWD_WAVES waves][CH chains][L], strip
+  const FwdBlock blk = gblock[blockIdx.x];
+  const int gi = blk.gi;
+  const int4 grp = blk.grp;
+  auto view_of = [&](int v) {
+    if constexpr (V == 1) return FwdView{blk.geom, blk.rw, blk.view};
+    const int a = order[grp.x + v];
+    return FwdView{geom[a], rwt[a], a};
+  };
+  if (gridDim.y == 1) {
+    fwd_group<V, CH, FR, STG>(im, imT, sino, view_of, grp, M, N, D, yres, res_ws, gi, acc, pitch,
+                              false);
+    return;
+  }
+  __shared__ int last;
   const size_t plane = static_cast<size_t>(A) * D;
+  fwd_group<V, CH, FR, STG>(im, imT, parts + blockIdx.y * plane, view_of, grp, M, N, D, nullptr,
+                            nullptr, gi, acc, pitch, true);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = atomicInc(reinterpret_cast<unsigned*>(done + gi), gridDim.y - 1) == gridDim.y - 1;
+  __syncthreads();
+  if (!last) return;
+  __shared__ double red[FWD_WAVES];
   double res = 0.0;
   for (int v = 0; v < grp.y; ++v) {
-    const size_t row = static_cast<size_t>(order[grp.x + v]) * D;
-    for (int b = threadIdx.x; b < D; b += 256) {
-      float val = parts[row + b];
-      for (int q = 1; q < sp; ++q) val = __fadd_rn(val, parts[q * plane + row + b]);
+    const size_t row = static_cast<size_t>(V == 1 ? blk.view : order[grp.x + v]) * D;
+    for (int b = threadIdx.x; b < D; b += 64 * FWD_WAVES) {
+      float q[FWD_SP_MAX];
+#pragma unroll
+      for (int k = 0; k < FWD_SP_MAX; ++k)
+        if (k < static_cast<int>(gridDim.y)) q[k] = __hip_atomic_load(parts + k * plane + row + b, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT);
+      float val = q[0];
+#pragma unroll
+      for (int k = 1; k < FWD_SP_MAX; ++k)
+        if (k < static_cast<int>(gridDim.y)) val = __fadd_rn(val, q[k]);
       sino[row + b] = val;
       if (yres) {
         const double d = static_cast<double>(__fsub_rn(yres[row + b], val));
@@ -897,18 +1004,25 @@ __global__ __launch_bounds__(256) void fwd_parts_kernel(const float* __restrict_
     }
   }
   if (res_ws) {
-    res = block_sum_f64(res, red);
-    if (threadIdx.x == 0) res_ws[gi] = res;
+    for (int off = 32; off > 0; off >>= 1) res += __shfl_down(res, off, 64);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = res;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double t = red[0];
+      for (int w = 1; w < FWD_WAVES; ++w) t += red[w];
+      res_ws[gi] = t;
+    }
   }
 }
 
 // Dynamic LDS beyond 64 KiB for the one-view, one-chain forward (wide
 // detectors).
 static hipError_t fwd_allow_lds(int bytes) {
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<1, 1, false>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  const hipError_t e =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<1, 1, false, false>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
   if (e != hipSuccess) return e;
-  return hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<1, 1, true>),
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<1, 1, true, false>),
                              hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
@@ -1377,9 +1491,14 @@ __global__ __launch_bounds__(64 * FWD_WAVES) void fwd_batch_kernel(BatchTabs t, 
     const int4 sh = t.shape[s];
     const int64_t io = t.ioff[s], so = t.soff[s];
     const int vo = t.voff[s], go = t.goff[s];
-    fwd_group<V, CH, FR>(im + io, imT + io, sino + so, t.geom + vo, t.rw + vo, t.groups + go,
-                 t.order + vo, sh.x, sh.y, sh.w, yres ? yres + so : nullptr,
-                 res_ws ? res_ws + go : nullptr, w.y, acc);
+    const int4 grp = t.groups[go + w.y];
+    auto view_of = [&](int v) {
+      const int a = t.order[vo + grp.x + v];
+      return FwdView{t.geom[vo + a], t.rw[vo + a], a};
+    };
+    fwd_group<V, CH, FR, false>(im + io, imT + io, sino + so, view_of, grp, sh.x, sh.y, sh.w,
+                                yres ? yres + so : nullptr, res_ws ? res_ws + go : nullptr, w.y,
+                                acc, 0, false);
     __syncthreads();  // the next item re-zeroes acc
   }
 }
@@ -1491,49 +1610,66 @@ int forward(const Plan& p, const float* im, float* sino, const int32_t* pred, hi
     SCXR_LAUNCHED("xr2d general forward");
     return SCXR_OK;
   }
-  // column-fast views stream the transposed image: the caller's, or the
-  // plan's workspace filled here
+  // Column-fast views stream the transposed image (the caller's, or the
+  // plan's workspace filled here) or stage their columns of the image itself:
+  // where rows and share take at most 64 KiB (128^2 unsplit takes 78: 12.5 us
+  // staged, 11.5 transposed; 100 x 80 takes 50: 8.8 against 9.4) and every
+  // workgroup of the launch finds room on a CU at once (256^2 in 8 parts with
+  // 45 views 10.2 -> 9.7 us, but with 180 views, three turns, 16 -> 21 us).
+  const size_t rows_lds = fwd_lds_bytes(p.vpg, p.D, p.fwd_ch);
+  const size_t share = fwd_share_bytes(p.fwd_ch, p.N, p.fwd_sp, p.fwd_pitch);
+  const bool stage = !imT && p.fwd_pitch > 0 && rows_lds + share <= FWD_LDS_MAX &&
+                     static_cast<size_t>(p.n_groups) * p.fwd_sp <=
+                         p.cus * (LDS_PER_CU / (rows_lds + share));
   const float* srcT = imT ? imT : p.work;
-  if (p.any_colfast && !imT) {
+  if (p.any_colfast && !imT && !stage) {
     dim3 g(ceil_div(p.N, 32), ceil_div(p.M, 32));
     hipLaunchKernelGGL(transpose_kernel, g, dim3(256), 0, s, im, p.work, p.M, p.N, pred);
     SCXR_LAUNCHED("xr2d transpose");
   }
-  const size_t lds = fwd_lds_bytes(p.vpg, p.D, p.fwd_ch);
+  const size_t lds = rows_lds + (stage ? share : 0);
   const dim3 fgrid(p.n_groups, p.fwd_sp);
-#define SCXR_FWD(VV, CC)                                                                      \
-  do {                                                                                         \
-    if (p.adj_fract)                                                                           \
-      hipLaunchKernelGGL((fwd_kernel<VV, CC, true>), fgrid, dim3(64 * FWD_WAVES), lds, s, im,  \
-                         srcT, sino, p.geom, p.rw, p.groups, p.order, p.M, p.N, p.D, yres,    \
-                         res_ws, p.parts, p.A, p.gblock, pred);                               \
-    else                                                                                       \
-      hipLaunchKernelGGL((fwd_kernel<VV, CC, false>), fgrid, dim3(64 * FWD_WAVES), lds, s, im, \
-                         srcT, sino, p.geom, p.rw, p.groups, p.order, p.M, p.N, p.D, yres,    \
-                         res_ws, p.parts, p.A, p.gblock, pred);                               \
-  } while (0)
-  if (p.fwd_ch == 2) {
-    if (p.vpg == 1)
-      SCXR_FWD(1, 2);
-    else if (p.vpg == 2)
-      SCXR_FWD(2, 2);
-    else
-      SCXR_FWD(4, 2);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, fgrid, dim3(64 * FWD_WAVES), lds, s, im, srcT, sino, p.geom, p.rw,
+                       p.order, p.M, p.N, p.D, yres, res_ws, p.parts, p.A, p.gblock,
+                       p.done, stage ? p.fwd_pitch : 0, pred);
+  };
+#define SCXR_FWD(VV, CC)                                      \
+  if (p.adj_fract)                                            \
+    go(fwd_kernel<VV, CC, true, false>);                      \
+  else                                                        \
+    go(fwd_kernel<VV, CC, false, false>);
+  if (stage) {
+    if (p.fwd_ch == 2) {
+      if (p.adj_fract)
+        go(fwd_kernel<1, 2, true, true>);
+      else
+        go(fwd_kernel<1, 2, false, true>);
+    } else {
+      if (p.adj_fract)
+        go(fwd_kernel<1, 1, true, true>);
+      else
+        go(fwd_kernel<1, 1, false, true>);
+    }
+  } else if (p.fwd_ch == 2) {
+    if (p.vpg == 1) {
+      SCXR_FWD(1, 2)
+    } else if (p.vpg == 2) {
+      SCXR_FWD(2, 2)
+    } else {
+      SCXR_FWD(4, 2)
+    }
   } else {
-    if (p.vpg == 1)
-      SCXR_FWD(1, 1);
-    else if (p.vpg == 2)
-      SCXR_FWD(2, 1);
-    else
-      SCXR_FWD(4, 1);
+    if (p.vpg == 1) {
+      SCXR_FWD(1, 1)
+    } else if (p.vpg == 2) {
+      SCXR_FWD(2, 1)
+    } else {
+      SCXR_FWD(4, 1)
+    }
   }
 #undef SCXR_FWD
   SCXR_LAUNCHED("xr2d forward");
-  if (p.fwd_sp > 1) {
-    hipLaunchKernelGGL(fwd_parts_kernel, dim3(p.n_groups), dim3(256), 0, s, p.parts, p.fwd_sp,
-                       p.A, p.D, sino, p.groups, p.order, yres, res_ws, pred);
-    SCXR_LAUNCHED("xr2d forward part sums");
-  }
   return SCXR_OK;
 }
 

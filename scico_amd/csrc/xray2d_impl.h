@@ -24,10 +24,18 @@ constexpr int RW_PAD = 3;      // entries that end a table of 1 / width per view
 constexpr int FWD_WAVES = 8;
 constexpr int FWD_SP_MAX = 8;  // most workgroups one forward group's lines are split over
 constexpr size_t FWD_LDS_MAX = 64 * 1024;
+constexpr size_t LDS_PER_CU = 160 * 1024;
 constexpr int FWD_SMAX = 64;  // largest lane stride of the forward projector
 inline size_t fwd_lds_bytes(int vpg, int D, int ch) {
   return sizeof(float) * static_cast<size_t>(vpg) * FWD_WAVES * ch *
          (static_cast<size_t>(D) + 4);
+}
+// Image columns that a workgroup of column-fast views stages
+// (fwd_body_staged): its share of the N columns over sp workgroups, in sets
+// of FWD_WAVES * ch, `pitch` rows apart.
+inline size_t fwd_share_bytes(int ch, int N, int sp, int pitch) {
+  const int K = FWD_WAVES * ch, sets = (N + K - 1) / K;
+  return sizeof(float) * static_cast<size_t>((sets + sp - 1) / sp) * K * pitch;
 }
 // Chains per wave for vpg views of D bins: 2 when the rows fit, else 1
 // (0: too wide).
@@ -44,12 +52,23 @@ inline int fwd_chains_ext(int vpg, int D, size_t lds_cap) {
   return (vpg == 1 && fwd_lds_bytes(1, D, 1) <= lds_cap) ? 1 : 0;
 }
 
+// One forward workgroup column: its group's row of groups[] and, for groups
+// of one view, that view, so that a single load precedes the walk.
+struct __align__(16) FwdBlock {
+  float4 geom;  // as Plan::geom
+  double rw;
+  int view, gi;
+  int4 grp;  // (first in order[], views, class | lane multiplier << 1, lane stride)
+};
+
 struct Plan {
   int M = 0, N = 0, A = 0, D = 0;
   int vpg = 1;         // views per forward workgroup
   int fwd_ch = 2;      // forward chains per wave
   int n_groups = 0;    // forward workgroups
+  int cus = 256;       // compute units of the device
   int fwd_sp = 1;      // workgroups per forward group, splitting its lines
+  int fwd_pitch = 0;   // rows of a staged column; 0: the image is transposed
   int adj_w = 0;       // adjoint window width (bins)
   int adj_ppt = 1;     // adjoint pixels per thread
   bool adj_fract = false;  // Px >= 1 everywhere: fraction-instruction weights
@@ -60,12 +79,12 @@ struct Plan {
   void* dev_block = nullptr;  // device tables (one allocation)
   float4* geom = nullptr;     // (Pxmin, P0, P1, width) per view
   double* rw = nullptr;       // RN64(1 / width) per view, RW_PAD more entries
-  int4* groups = nullptr;     // forward groups: (first, count, class, 0)
   int* order = nullptr;       // views grouped by class
-  int* gblock = nullptr;      // forward group of each forward block index
+  FwdBlock* gblock = nullptr; // forward group of each forward block index
   float* clo = nullptr;       // adjoint window origin offset per view
   float* work = nullptr;      // transposed image workspace (M * N)
   float* parts = nullptr;     // fwd_sp_cap partial sinograms (A x D each)
+  int* done = nullptr;        // finished parts of each forward group, 0 between launches
   int fwd_sp_cap = 1;         // parts the workspace holds (1: none)
   std::vector<float4> host_geom;
 };

@@ -340,3 +340,38 @@ def test_ramp_filter_rows(gpu, A, D):
     np.testing.assert_array_equal(np.isfinite(bad[A - 1]), ~reach)
     assert np.all(np.abs(bad[A - 1, ~reach] - ref[A - 1, ~reach]) <= bar[A - 1, ~reach] + 1e-30)
     assert np.all(np.abs(bad[: A - 1] - ref[: A - 1]) <= bar[: A - 1] + 1e-30)
+
+
+@pytest.mark.parametrize("M,N,A,parts", [
+    (1, 1, 3, 4), (3, 5, 7, 8), (16, 16, 9, 2), (17, 15, 9, 3), (64, 33, 12, 4),
+    (192, 17, 20, 8), (193, 129, 60, 4), (256, 256, 45, 8), (320, 48, 33, 7), (400, 300, 12, 8),
+])
+def test_forward_parts_and_staged_columns(gpu, M, N, A, parts):
+    """Sums of a view's parts by the workgroup that ends last, and columns
+    staged from the image in place of a transposed copy: the staged forward
+    equals the one from a transposed image bit for bit, twice in a row on
+    other images too, and both are within the float32 bound of the float64
+    sums (a bin adds n products: n eps of the absolute sum)."""
+    from scico_amd._lib import call
+
+    H = XRayTransform2D((M, N), np.linspace(0, np.pi, A, endpoint=False).astype(np.float32))
+    assert H.set_forward_split(parts) == parts
+    ind, w = (t.cpu().numpy() for t in H.weights())
+    rng = np.random.default_rng(M * 1000 + N)
+    for _ in range(3):
+        x = rng.standard_normal((M, N)).astype(np.float32)
+        xd = torch.as_tensor(x, device="cuda")
+        got = H.project(xd).cpu().numpy()
+        xt, other = xd.t().contiguous(), torch.empty(H.output_shape, device="cuda")
+        call("scxr_xr2d_forward_t", H.plan, xd.data_ptr(), xt.data_ptr(), other.data_ptr(), None,
+             torch.cuda.current_stream().cuda_stream)
+        np.testing.assert_array_equal(got, other.cpu().numpy())
+        for a in range(A):
+            ref, mag, cnt = (np.zeros(H.ny + 2) for _ in range(3))
+            for k, f in ((ind[a], w[a]), (ind[a] + 1, 1.0 - w[a].astype(np.float64))):
+                at = np.clip(k, -1, H.ny).astype(np.int64).reshape(-1) + 1
+                np.add.at(ref, at, (x.astype(np.float64) * f).reshape(-1))
+                np.add.at(mag, at, np.abs(x.astype(np.float64) * f).reshape(-1))
+                np.add.at(cnt, at, 1)
+            bar = (cnt + 2) * 2.0**-24 * mag
+            assert np.all(np.abs(got[a] - ref[1:-1]) <= bar[1:-1])
