@@ -294,10 +294,14 @@ int create(Plan& p, int M, int N, int A, int D, const double* x0, const double* 
   size_t lds_cap = FWD_LDS_MAX;
   {
     int dev = 0, v = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess &&
-        v > 0)
-      lds_cap = std::max(lds_cap, static_cast<size_t>(v));
+    if (hipGetDevice(&dev) == hipSuccess) {
+      if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) ==
+              hipSuccess && v > 0)
+        lds_cap = std::max(lds_cap, static_cast<size_t>(v));
+      if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+          v > 0)
+        p.cus = v;
+    }
   }
   p.fwd_ch = fwd_chains_ext(p.vpg, D, lds_cap);
   if (p.fwd_ch > 0 && fwd_lds_bytes(p.vpg, D, p.fwd_ch) > FWD_LDS_MAX) {
@@ -310,7 +314,12 @@ int create(Plan& p, int M, int N, int A, int D, const double* x0, const double* 
     }
   }
   HostTables h;
-  const int rc = build_tables(h, M, N, A, D, x0, dx, y0, angles, p.vpg, 0, p.fwd_ch, true);
+  // One pixel per adjoint thread where its tiles, twice as many, still have a
+  // CU each (256^2 with 180 views 11.5 -> 9.1 us, 128^2 with 180 views 11.2 ->
+  // 8.6 us); with more tiles two pixels share a view's record (320^2 with 180
+  // views 11.7 against 13.1 us).  The same sums either way.
+  const int ppt = 2LL * ceil_div(N, 2 * ADJ_TJ) * ceil_div(M, ADJ_TI) <= p.cus ? 1 : 0;
+  const int rc = build_tables(h, M, N, A, D, x0, dx, y0, angles, p.vpg, ppt, p.fwd_ch, true);
   if (rc) return rc;
   p.fwd_generic = h.fwd_generic;
   p.adj_generic = h.adj_generic;
@@ -332,11 +341,6 @@ int create(Plan& p, int M, int N, int A, int D, const double* x0, const double* 
   // block index -> forward group, balanced over the CUs
   std::vector<int> gblock;
   if (!groups.empty()) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-        cus > 0)
-      p.cus = cus;
     gblock = place_groups(h.gcost, p.cus);
   }
   std::vector<FwdBlock> blocks;
