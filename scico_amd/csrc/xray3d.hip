@@ -34,6 +34,7 @@
 #include <climits>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -44,6 +45,7 @@ namespace xr3d {
 enum { MODE_GENERAL = 0, MODE_SLICE = 1 };
 
 constexpr int FB = 8;   // forward: detector bins per wave
+constexpr int FBL = 7;  // the same of fwd_slice16_kernel: 8 bin groups of 2 slots fill a lane row
 constexpr int AR = 8;   // adjoint: pixels per wave (2 x 4 block)
 
 struct Plan {
@@ -53,6 +55,7 @@ struct Plan {
   int P = 0, Q = 0, S = 0, SQ = 0, U = 0;  // SQ = slice quads (slices padded to 4)
   int cpr = 32;                            // forward candidates per row
   int spg = 2;                             // forward slots per bin group
+  bool slot16 = false;                     // forward by fwd_slice16_kernel
   bool vol_direct = false, proj_direct = false;
   bool adj_staged = false;                 // adjoint rows staged in LDS (adj_slice_staged_kernel)
   void* tables = nullptr;  // general mode: one block of the tables below (mats included)
@@ -173,6 +176,26 @@ __device__ __forceinline__ float rlf(float v, int lane) {
 
 // ------------------------------------------------------ slice kernels --
 
+// Bin group and view group of a workgroup of the slice forward.
+__device__ __forceinline__ void slice_block(int& bg, int& vg) {
+  // Workgroup order: consecutive workgroups go to the 8 XCDs in turn; each
+  // XCD is given a contiguous run of an order that takes the view groups
+  // in blocks of about an eighth of them, every bin group of a block with
+  // its views adjacent.  Each XCD then works on its own range of views
+  // (neighbouring views' strips share most of their pixel rows, so they
+  // share its L2) across all bin groups (whose strips differ in length,
+  // so every XCD gets a similar share of work).  A bijection of the grid.
+  const int GX = gridDim.x, GY = gridDim.y, G = GX * GY, G8 = (G / 8) * 8;
+  int L = blockIdx.y * GX + blockIdx.x;
+  if (L < G8) L = (L % 8) * (G8 / 8) + L / 8;
+  const int VB = GY >= 8 ? GY / 8 : 1;  // view groups per block
+  const int blk = L / (GX * VB);
+  const int nb = min(VB, GY - blk * VB);  // the last block may be short
+  const int within = L - blk * GX * VB;
+  bg = within / nb;
+  vg = blk * VB + (within - bg * nb);
+}
+
 // Forward: each wave owns FB consecutive bins of one view for 256 slices
 // and gathers the strip of pixels that touch them, row by row along the
 // slow in-plane axis.  Lane kk of a row pass holds candidate kk of the
@@ -193,25 +216,8 @@ __global__ __launch_bounds__(256) void fwd_slice_kernel(const float4* __restrict
   constexpr int RPP = 64 / CPR;
   constexpr int BIG = INT_MAX / 2;
   const int lane = threadIdx.x & 63;
-  // Workgroup order: consecutive workgroups go to the 8 XCDs in turn; each
-  // XCD is given a contiguous run of an order that takes the view groups
-  // in blocks of about an eighth of them, every bin group of a block with
-  // its views adjacent.  Each XCD then works on its own range of views
-  // (neighbouring views' strips share most of their pixel rows, so they
-  // share its L2) across all bin groups (whose strips differ in length,
-  // so every XCD gets a similar share of work).  A bijection of the grid.
   int bg, vg;
-  {
-    const int GX = gridDim.x, GY = gridDim.y, G = GX * GY, G8 = (G / 8) * 8;
-    int L = blockIdx.y * GX + blockIdx.x;
-    if (L < G8) L = (L % 8) * (G8 / 8) + L / 8;
-    const int VB = GY >= 8 ? GY / 8 : 1;  // view groups per block
-    const int blk = L / (GX * VB);
-    const int nb = min(VB, GY - blk * VB);  // the last block may be short
-    const int within = L - blk * GX * VB;
-    bg = within / nb;
-    vg = blk * VB + (within - bg * nb);
-  }
+  slice_block(bg, vg);
   const int v = vg * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (v >= V) return;
   const int u0 = bg * FB;
@@ -322,6 +328,126 @@ __global__ __launch_bounds__(256) void fwd_slice_kernel(const float4* __restrict
   if (!qok) return;
 #pragma unroll
   for (int j = 0; j < FB; ++j)
+    if (u0 + j < U) proj[(static_cast<size_t>(v) * U + u0 + j) * SQ + quad] = acc[j];
+}
+
+// Value of lane N of every 16-lane row, for the whole row (N a constant).
+template <int N>
+__device__ __forceinline__ int row_bcast(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, 0x150 | N, 0xf, 0xf, true);
+}
+template <int N>
+__device__ __forceinline__ float4 fma4_bcast(float w, float4 x, float4 acc) {
+  const float wn = __int_as_float(row_bcast<N>(__float_as_int(w)));
+  return fma4(wn, x, acc);
+}
+
+// Forward for in-plane spacings near 1 (at most 16 candidates in a row, two
+// per bin group): the strip gather of fwd_slice_kernel with most of its scalar
+// work per pixel taken out; the same sums in the same order.  A pass
+// evaluates the taps of four image rows (16 candidates each) and files them
+// by slot, two for each of the 8 bin groups, in an LDS table of the wave.  A
+// row's 16 entries are read back into every 16-lane row, where a slot's
+// weights are a row broadcast of a constant lane and one ballot tells which
+// slots are taken.  Bound by the vector loads (a 16-byte load of 64 lanes for
+// each pixel, view and bin group: 28 TB/s from the CUs' caches at 256^3 with
+// 360 views) and their latency.  Against fwd_slice_kernel: 256^3 with 360, 180
+// and 45 views 1372, 844, 405 -> 1256, 741, 330 us, 128^3 with 90 views 194 ->
+// 153 us.  (Eight loads at a time: 1212, 787, 376, 171 us.)
+// (Sharing the pixel rows of four views through LDS takes two thirds off the
+// loads, but with a barrier per image row too little is in flight: 1602 us.)
+__global__ __launch_bounds__(256) void fwd_slice16_kernel(
+    const float4* __restrict__ vol, float4* __restrict__ proj, const float4* __restrict__ geom,
+    int P, int Q, int SQ, int U, int V, const int32_t* __restrict__ pred) {
+  if (pred_off(pred)) return;
+  constexpr int BIG = INT_MAX / 2;
+  __shared__ int4 table[4][64];
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  int bg, vg;
+  slice_block(bg, vg);
+  const int v = vg * 4 + w;
+  if (v >= V) return;
+  const int u0 = bg * FBL;
+  const unsigned quad = blockIdx.z * 64 + lane;
+  const bool qok = quad < static_cast<unsigned>(SQ);
+  const unsigned qoff = (qok ? quad : 0u) * 16u;
+  const int rowb = SQ * 16;
+  const __amdgpu_buffer_rsrc_t vr = make_rsrc(vol, P * Q * rowb);
+  const float4 g = geom[v];
+  const float a = g.x, b = g.y, t = g.z;
+  const bool qfast = fabsf(b) >= fabsf(a);
+  const float f = qfast ? b : a, sc = qfast ? a : b, rf = 1.0f / f;
+  const int nslow = qfast ? P : Q, nfast = qfast ? Q : P;
+  const float plo = static_cast<float>(u0) - 0.75f;
+  const float phi = static_cast<float>(u0 + FBL) + 0.25f;
+  const int kk = lane & 15, lr = lane >> 4;
+  int4* ent = table[w];
+
+  float4 acc[FBL];
+#pragma unroll
+  for (int j = 0; j < FBL; ++j) acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+
+  for (int r0 = 0; r0 < nslow; r0 += 4) {
+    // taps of rows r0 .. r0 + 3, filed by slot; the interval of the strip in
+    // a row is widened by one pixel each side, the exact bin decides
+    {
+      const int row = r0 + lr;
+      const float c = sc * (static_cast<float>(row) + 0.5f) + t;
+      const float ka = (plo - c) * rf - 0.5f, kb = (phi - c) * rf - 0.5f;
+      const int klo = max(0, static_cast<int>(floorf(fminf(ka, kb))) - 1);
+      const int khi = min(nfast - 1, static_cast<int>(ceilf(fmaxf(ka, kb))) + 1);
+      int gi = BIG, off = 0;
+      float wl = 0.0f, wr = 0.0f;
+      if (row < nslow && kk <= khi - klo) {
+        const int k = f > 0.0f ? klo + kk : khi - kk;  // bins do not decrease with kk
+        const int p = qfast ? row : k, q = qfast ? k : row;
+        const Tap tp = slice_tap(a, b, t, p, q, U);
+        gi = tp.ul - u0;
+        wl = tp.wl;
+        wr = tp.wr;
+        off = (p * Q + q) * rowb;
+      }
+      // the second pixel of its bin group? (lane before, within the row)
+      const int prev = __builtin_amdgcn_update_dpp(-BIG, gi, 0x111, 0xf, 0xf, false);
+      ent[lane] = make_int4(0, 0, 0, 0);
+      if (gi >= -1 && gi < FBL)
+        ent[lr * 16 + 2 * (gi + 1) + (gi == prev)] =
+            make_int4(off, __float_as_int(wl), __float_as_int(wr), 1);
+    }
+#pragma unroll 1
+    for (int rr = 0; rr < min(4, nslow - r0); ++rr) {
+      const int4 e = ent[rr * 16 + kk];
+      const unsigned occ = static_cast<unsigned>(__builtin_amdgcn_ballot_w64(e.w != 0)) & 0xffffu;
+      if (occ == 0) continue;
+      const float wl = __int_as_float(e.y), wr = __int_as_float(e.z);
+      // taken slots only (wave-uniform), all loads before the first sum
+      float4 x[16];
+      auto load = [&](auto N) {
+        constexpr int n = decltype(N)::value;
+        if (occ & (1u << n)) x[n % 16] = bload4(vr, qoff, rl(e.x, n));
+      };
+      auto use = [&](auto N) {
+        constexpr int n = decltype(N)::value, gg = n / 2 - 1;
+        if (occ & (1u << n)) {
+          if constexpr (gg >= 0) acc[gg] = fma4_bcast<n>(wl, x[n % 16], acc[gg]);
+          if constexpr (gg + 1 < FBL) acc[gg + 1] = fma4_bcast<n>(wr, x[n % 16], acc[gg + 1]);
+        }
+      };
+#define SCXR_X3_SLOT(N) std::integral_constant<int, N>{}
+      load(SCXR_X3_SLOT(0)); load(SCXR_X3_SLOT(1)); load(SCXR_X3_SLOT(2)); load(SCXR_X3_SLOT(3));
+      load(SCXR_X3_SLOT(4)); load(SCXR_X3_SLOT(5)); load(SCXR_X3_SLOT(6)); load(SCXR_X3_SLOT(7));
+      load(SCXR_X3_SLOT(8)); load(SCXR_X3_SLOT(9)); load(SCXR_X3_SLOT(10)); load(SCXR_X3_SLOT(11));
+      load(SCXR_X3_SLOT(12)); load(SCXR_X3_SLOT(13)); load(SCXR_X3_SLOT(14)); load(SCXR_X3_SLOT(15));
+      use(SCXR_X3_SLOT(0)); use(SCXR_X3_SLOT(1)); use(SCXR_X3_SLOT(2)); use(SCXR_X3_SLOT(3));
+      use(SCXR_X3_SLOT(4)); use(SCXR_X3_SLOT(5)); use(SCXR_X3_SLOT(6)); use(SCXR_X3_SLOT(7));
+      use(SCXR_X3_SLOT(8)); use(SCXR_X3_SLOT(9)); use(SCXR_X3_SLOT(10)); use(SCXR_X3_SLOT(11));
+      use(SCXR_X3_SLOT(12)); use(SCXR_X3_SLOT(13)); use(SCXR_X3_SLOT(14)); use(SCXR_X3_SLOT(15));
+#undef SCXR_X3_SLOT
+    }
+  }
+  if (!qok) return;
+#pragma unroll
+  for (int j = 0; j < FBL; ++j)
     if (u0 + j < U) proj[(static_cast<size_t>(v) * U + u0 + j) * SQ + quad] = acc[j];
 }
 
@@ -446,8 +572,8 @@ __global__ __launch_bounds__(256) void adj_slice_staged_kernel(
     mx = max(mx, __builtin_amdgcn_mov_dpp(mx, 0xB1, 0xF, 0xF, true));
     mn = min(mn, __builtin_amdgcn_mov_dpp(mn, 0x4E, 0xF, 0xF, true));  // quad_perm 2 3 0 1
     mx = max(mx, __builtin_amdgcn_mov_dpp(mx, 0x4E, 0xF, 0xF, true));
-    lo = min(max(mn, 0), U - 1);
-    n = min(max(mx + 1, 0), U - 1) - lo + 1;
+    lo = mn;
+    n = mx - mn + 2;
   };
   int lo_c, n_c, lo_n = 0, n_n = 0;  // ranges of the current and the next 16 views
   ranges(0, lo_c, n_c);
@@ -455,7 +581,7 @@ __global__ __launch_bounds__(256) void adj_slice_staged_kernel(
   // stage view v's rows into buffer b
   auto stage_view = [&](int v, int lo, int n, int b) {
     for (int k = w; k < n; k += 4)
-      lds_row_load(yr, &stage[b][k][0], qoff, (v * U + lo + k) * rowb);
+      lds_row_load(yr, &stage[b][k][0], qoff, (v * U + min(max(lo + k, 0), U - 1)) * rowb);
   };
 
   float4 acc[AR];
@@ -465,15 +591,14 @@ __global__ __launch_bounds__(256) void adj_slice_staged_kernel(
   stage_view(0, rl(lo_c, 0), rl(n_c, 0), 0);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  int cab = 0;  // the pixel's two detector rows, clamped as adj_slice_kernel
-                // clamps them, packed as two 16-bit fields (U < 65536)
+  int ul = 0;  // the pixel's first detector row
   float wl = 0.0f, wr = 0.0f;
 #pragma unroll 1
   for (int v = 0; v < V; ++v) {
     const int j = v & 7;
     if (j == 0) {  // taps of the wave's 8 pixels for views v .. v + 7
       const int vv = v + jv;
-      int ul = 0;
+      ul = 0;
       wl = wr = 0.0f;
       if (vv < V) {
         const float4 g = geom[vv];
@@ -482,7 +607,6 @@ __global__ __launch_bounds__(256) void adj_slice_staged_kernel(
         wl = pok ? tp.wl : 0.0f;
         wr = pok ? tp.wr : 0.0f;
       }
-      cab = min(max(ul, 0), U - 1) | (min(max(ul + 1, 0), U - 1) << 16);
     }
     // this view's range, then the next view's, from the 16-view range sets
     const int lo = rl(lo_c, 4 * (v & 15));
@@ -493,26 +617,28 @@ __global__ __launch_bounds__(256) void adj_slice_staged_kernel(
       const int nn = nxt_set ? rl(n_n, kn) : rl(n_c, kn);
       stage_view(vn, lon, nn, vn & 1);
     }
-    // both rows of all eight pixels first (no reuse branches: LDS reads
+    // both rows of four pixels first (no reuse branches: LDS reads
     // are cheap), then the accumulation in adj_slice_kernel's order
     const char* sb = reinterpret_cast<const char*>(&stage[v & 1][0][0] + lane);
-    // byte offsets of both staged rows (64 float4 = 1 KiB apart): every
-    // pixel's clamped rows lie in [lo, lo + n), n <= ADJ_NW (the range is
-    // taken over the tile's corner bins), so neither 16-bit field borrows
-    // and each offset stays below 2^14
-    const unsigned rab = static_cast<unsigned>(cab - (lo | (lo << 16))) << 10;
-    float4 ya[AR], yb[AR];
+    // byte offset of the first staged row (64 float4 = 1 KiB apart): every
+    // pixel's rows lie in [lo, lo + n), n <= ADJ_NW (the range is taken over
+    // the tile's corner bins)
+    const int ra = (ul - lo) * 1024;
 #pragma unroll
-    for (int i = 0; i < AR; ++i) {
-      const unsigned x = static_cast<unsigned>(rl(static_cast<int>(rab), j * AR + i));
-      ya[i] = *reinterpret_cast<const float4*>(sb + (x & 0xffffu));
-      yb[i] = *reinterpret_cast<const float4*>(sb + (x >> 16));
-    }
+    for (int i0 = 0; i0 < AR; i0 += 4) {
+      float4 ya[4], yb[4];
 #pragma unroll
-    for (int i = 0; i < AR; ++i) {
-      const int L = j * AR + i;
-      const float cl = rlf(wl, L), cr = rlf(wr, L);
-      acc[i] = fma4(cr, yb[i], fma4(cl, ya[i], acc[i]));
+      for (int i = 0; i < 4; ++i) {
+        const float4* y = reinterpret_cast<const float4*>(sb + rl(ra, j * AR + i0 + i));
+        ya[i] = y[0];
+        yb[i] = y[64];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int L = j * AR + i0 + i;
+        const float cl = rlf(wl, L), cr = rlf(wr, L);
+        acc[i0 + i] = fma4(cr, yb[i], fma4(cl, ya[i], acc[i0 + i]));
+      }
     }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -1229,6 +1355,9 @@ static bool try_slice(Plan& p, const std::vector<float>& m, int sax, int dax) {
   const double spg = std::ceil(1.0 / static_cast<double>(fmin) + 0.01);
   if (spg > 3.0) return false;
   p.spg = spg <= 2.0 ? 2 : 3;
+  // 16 candidates hold a strip of FBL + 1 bins, rounded outwards and widened
+  // by a pixel each side
+  p.slot16 = (FBL + 1) / static_cast<double>(fmin) < 11.99;
   p.mode = MODE_SLICE;
   p.sax = sax;
   p.dax = dax;
@@ -1762,9 +1891,17 @@ int forward(const Plan& p, const float* vol, float* proj, float* ws, const int32
     vc = p.volc;
   }
   float* yc = p.proj_direct ? proj : p.proja;
-  dim3 grid(ceil_div(p.U, FB), ceil_div(p.V, 4), ceil_div(p.SQ, 64));
   const float4* v4 = reinterpret_cast<const float4*>(vc);
   float4* y4 = reinterpret_cast<float4*>(yc);
+  if (p.slot16) {
+    const dim3 g16(ceil_div(p.U, FBL), ceil_div(p.V, 4), ceil_div(p.SQ, 64));
+    hipLaunchKernelGGL(fwd_slice16_kernel, g16, dim3(256), 0, s, v4, y4, p.geom, p.P, p.Q, p.SQ,
+                       p.U, p.V, pred);
+    SCXR_LAUNCHED("xr3d slice forward (16 slots)");
+    if (!p.proj_direct) return canon_to_proj(p, yc, proj, pred, s);
+    return SCXR_OK;
+  }
+  const dim3 grid(ceil_div(p.U, FB), ceil_div(p.V, 4), ceil_div(p.SQ, 64));
 #define SCXR_FWD3(C, G)                                                                       \
   hipLaunchKernelGGL((fwd_slice_kernel<C, G>), grid, dim3(256), 0, s, v4, y4, p.geom, p.P, p.Q, \
                      p.SQ, p.U, p.V, pred)

@@ -247,3 +247,50 @@ def test_general_windows(gpu, case):
     pd = [H(2.0 * x) for _ in range(4)]
     torch.cuda.synchronize()
     assert all(torch.equal(q, p) for q in ps) and all(torch.equal(q, 2.0 * p) for q in pd)
+
+
+@pytest.mark.parametrize("shape,views,scale,shift", [
+    ((1, 4, 1), 2, 1.0, 0.0),  # one pixel
+    ((5, 4, 9), 3, 1.0, 0.0),  # rows no multiple of 4, bins no multiple of 7
+    ((33, 12, 20), 6, 1.0, -7.3),  # strip partly off the detector
+    ((16, 260, 16), 5, 1.0, 0.0),  # more than 64 slice quads
+    ((21, 8, 30), 9, 0.945, 2.5),  # spacing just above and just below the limit of
+    ((21, 8, 30), 9, 0.942, 2.5),  # 16 candidates in a row
+    ((24, 8, 24), 8, 1.3, 0.0),  # wide spacing: empty bin groups
+    ((24, 8, 24), 8, 0.72, 0.0),  # three pixels in a bin group
+])
+def test_slice_strips(gpu, shape, views, scale, shift):
+    """Slice-mode forward and adjoint against float64 sums of the operator's
+    own weights, over the forms of the forward's strips; n products added in
+    float32 are off by at most n eps times the absolute sum."""
+    th = np.linspace(0, np.pi, views, endpoint=False)
+    rows = np.zeros((views, 2, 3))
+    rows[:, 0, 0], rows[:, 0, 2] = scale * np.cos(th), scale * np.sin(th)
+    rows[:, 1, 1] = 1.0
+    det = (int(np.ceil(scale * np.hypot(shape[0], shape[2]))) + 1, shape[1])
+    t = np.asarray(det) / 2 - rows @ (np.asarray(shape) / 2)
+    t[:, 0] += shift
+    H = XRayTransform3D(shape, np.concatenate((rows, t[..., None]), axis=2), det)
+    assert H.info()["mode"] == "slice"
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal(shape).astype(np.float32)
+    y = rng.standard_normal(H.output_shape).astype(np.float32)
+    fwd = H.project(torch.as_tensor(x, device="cuda")).cpu().numpy()
+    adj = H.back_project(torch.as_tensor(y, device="cuda")).cpu().numpy()
+    ref = np.zeros((3, views, det[0] + 2, det[1]))  # sum, absolute sum, products
+    back = np.zeros((2, *shape))
+    for v in range(views):
+        ul, w = (a.cpu().numpy() for a in H.weights(v))
+        at1 = np.clip(ul[1], 0, det[1] - 1)
+        for k in (0, 1):  # detector rows ul and ul + 1 (the slice axis has one tap)
+            at0 = np.clip(ul[0] + k, -1, det[0]) + 1
+            prod = x.astype(np.float64) * w[k]
+            np.add.at(ref[0, v], (at0, at1), prod)
+            np.add.at(ref[1, v], (at0, at1), np.abs(prod))
+            np.add.at(ref[2, v], (at0, at1), 1)
+            yv = np.pad(y[v].astype(np.float64), ((1, 1), (0, 0)))[at0, at1]
+            back[0] += yv * w[k]
+            back[1] += np.abs(yv * w[k])
+    eps = 2.0**-24
+    assert np.all(np.abs(fwd - ref[0, :, 1:-1]) <= eps * (ref[2] * ref[1])[:, 1:-1] + 1e-30)
+    assert np.all(np.abs(adj - back[0]) <= eps * 2 * views * back[1] + 1e-30)
