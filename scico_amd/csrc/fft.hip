@@ -102,7 +102,12 @@ __device__ __forceinline__ double fma_(double a, double b, double c) { return fm
 // natural order, so the fused convolution pass multiplies by the spectrum
 // and runs the inverse stages on the same buffer.
 constexpr int SH_THREADS = 256;
-constexpr int SH_MAXV = 32;  // values per thread per stage (lpb n <= 8192)
+// Values per thread and stage: 4 for workgroups of at most 1024 values, else 32
+// (lpb n <= 8192).  The kernels unroll over them for every radix, and at 32
+// the mixed-radix column pass is 160 KB of code, which does not stay in the
+// instruction cache (convolution of 3 x 360 x 480: 39 -> 25 us, 512 x 512: 27 ->
+// 22 us).
+constexpr int SH_MAXV = 32, SH_FEW = 4;
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) {
   return make_float2(__fadd_rn(a.x, b.x), __fadd_rn(a.y, b.y));
@@ -240,15 +245,16 @@ __device__ __forceinline__ void dft_small(V (&v)[R], bool inv) {
   }
 }
 
-template <int R>
+template <int R, int MAXV>
 __device__ __forceinline__ void stockham_stage(float2* X, int n, int lpb, int Ns,
                                                const float2* tw, bool inv) {
   const int nb = n / R, tot = lpb * nb;  // butterflies
   const int tstep = n / (R * Ns);
-  float2 v[SH_MAXV / R][R];
-  int dst[SH_MAXV / R];
+  constexpr int NQ = (MAXV + R - 1) / R;
+  float2 v[NQ][R];
+  int dst[NQ];
 #pragma unroll
-  for (int q = 0; q < SH_MAXV / R; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     const int b = threadIdx.x + q * SH_THREADS;
     dst[q] = -1;
     if (b < tot) {
@@ -269,7 +275,7 @@ __device__ __forceinline__ void stockham_stage(float2* X, int n, int lpb, int Ns
   }
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < SH_MAXV / R; ++q) {
+  for (int q = 0; q < NQ; ++q) {
     if (dst[q] >= 0) {
 #pragma unroll
       for (int r = 0; r < R; ++r) X[dst[q] + r * Ns] = v[q][r];
@@ -278,25 +284,26 @@ __device__ __forceinline__ void stockham_stage(float2* X, int n, int lpb, int Ns
   __syncthreads();
 }
 
+template <int MAXV>
 __device__ __forceinline__ void stockham(float2* X, int n, int log2n, int lpb,
                                          const float2* tw, bool inv) {
   // one stage of radix 2, 4 or 8 for log2 n mod 4, then radix-16 stages
   int Ns = 1;
   switch (log2n & 3) {
-    case 1: stockham_stage<2>(X, n, lpb, Ns, tw, inv); Ns = 2; break;
-    case 2: stockham_stage<4>(X, n, lpb, Ns, tw, inv); Ns = 4; break;
-    case 3: stockham_stage<8>(X, n, lpb, Ns, tw, inv); Ns = 8; break;
+    case 1: stockham_stage<2, MAXV>(X, n, lpb, Ns, tw, inv); Ns = 2; break;
+    case 2: stockham_stage<4, MAXV>(X, n, lpb, Ns, tw, inv); Ns = 4; break;
+    case 3: stockham_stage<8, MAXV>(X, n, lpb, Ns, tw, inv); Ns = 8; break;
     default: break;
   }
-  for (; Ns < n; Ns *= 16) stockham_stage<16>(X, n, lpb, Ns, tw, inv);
+  for (; Ns < n; Ns *= 16) stockham_stage<16, MAXV>(X, n, lpb, Ns, tw, inv);
 }
 
 // Mixed radix for lengths that are no power of two.  Bound by the latency
 // of the stages' LDS round trips and barriers (n log n work is small): 540
-// row pairs of 480 points 12 us, 723 half-spectrum columns of 360 (forward,
-// spectrum, inverse) 20 us.  Sums over all n inputs, which these lengths
+// row pairs of 480 points 7.5 us, 723 half-spectrum columns of 360 (forward,
+// spectrum, inverse) 12.8 us.  Sums over all n inputs, which these lengths
 // took before, cost 454 us a pass on the full spectrum: 3 x 360 x 480
-// convolution 1380 -> 40 us, and its error against float64 1.7e-6 -> 1.7e-7.
+// convolution 1380 -> 25 us, and its error against float64 1.7e-6 -> 1.7e-7.
 //
 // One stage: as stockham_stage, with the quotients by Ns and n / R taken as high words of the stage's magic
 // factors (k r tstep < n, so the twiddle index needs no reduction).
@@ -394,7 +401,7 @@ __device__ __forceinline__ void prime_stage(V* X, int n, int lpb, int R, int Ns,
 }
 
 // Mixed-radix transform of lpb lines in X; tw in LDS if S.twlds.
-template <int MAXV = SH_MAXV, class V>
+template <int MAXV, class V>
 __device__ __forceinline__ void mixed(V* X, int n, const Stages& S, int lpb, const V* tw,
                                       bool inv) {
   int Ns = 1;
@@ -415,13 +422,13 @@ __device__ __forceinline__ void mixed(V* X, int n, const Stages& S, int lpb, con
 }
 
 // The transform of a pass's lines, by length.
-template <bool MIXED>
+template <bool MIXED, int MAXV>
 __device__ __forceinline__ void transform(float2* X, int n, int log2n, const Stages& S, int lpb,
                                           const float2* tw, bool inv) {
   if constexpr (MIXED)
-    mixed(X, n, S, lpb, tw, inv);
+    mixed<MAXV>(X, n, S, lpb, tw, inv);
   else
-    stockham(X, n, log2n, lpb, tw, inv);
+    stockham<MAXV>(X, n, log2n, lpb, tw, inv);
 }
 
 // Twiddles of a mixed pass: copied behind the tot LDS values when a stage
@@ -435,7 +442,7 @@ __device__ __forceinline__ const float2* pass_twiddles(float2* X, int tot, int n
   return X + tot;
 }
 
-template <bool MIXED>
+template <bool MIXED, int MAXV>
 __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __restrict__ in,
                                                               void* __restrict__ out, Pass P,
                                                               Stages S, float scale,
@@ -480,9 +487,9 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
   };
   {
     // every load of the thread is issued before the first LDS store
-    float2 vv[SH_MAXV];
+    float2 vv[MAXV];
 #pragma unroll
-    for (int q = 0; q < SH_MAXV; ++q) {
+    for (int q = 0; q < MAXV; ++q) {
       const int e = threadIdx.x + q * SH_THREADS;
       if (e < tot) {
         int l, k;
@@ -497,7 +504,7 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
       }
     }
 #pragma unroll
-    for (int q = 0; q < SH_MAXV; ++q) {
+    for (int q = 0; q < MAXV; ++q) {
       const int e = threadIdx.x + q * SH_THREADS;
       if (e < tot) {
         int l, k;
@@ -506,19 +513,36 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
       }
     }
   }
+  constexpr bool AHEAD = MAXV <= SH_FEW;  // the spectrum is loaded before the transform
+  float2 hv[AHEAD ? MAXV : 1];
+  auto spectrum = [&](int e) {
+    const int l = e / n, k = e - l * n;
+    return l < nl ? P.h[static_cast<long long>(k) * P.stride + hoff[l]] : make_float2(0.0f, 0.0f);
+  };
+  if constexpr (AHEAD) {
+    if (P.fused) {
+#pragma unroll
+      for (int q = 0; q < MAXV; ++q)
+        if (threadIdx.x + q * SH_THREADS < tot) hv[q] = spectrum(threadIdx.x + q * SH_THREADS);
+    }
+  }
   __syncthreads();
-  transform<MIXED>(X, n, P.log2n, S, lpb, twl, P.fused ? false : (P.inverse != 0));
+  transform<MIXED, MAXV>(X, n, P.log2n, S, lpb, twl, P.fused ? false : (P.inverse != 0));
   if (P.fused) {
-    for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
-      const int l = e / n, k = e - l * n;
-      if (l < nl) {
-        float2 hv = P.h[static_cast<long long>(k) * P.stride + hoff[l]];
-        if (P.conj_h) hv = conjf2(hv);
-        X[e] = cmul(hv, X[e]);
-      }
+    auto times = [&](int e, float2 h) {
+      if (P.conj_h) h = conjf2(h);
+      X[e] = cmul(h, X[e]);
+    };
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int q = 0; q < MAXV; ++q)
+        if (threadIdx.x + q * SH_THREADS < tot)
+          times(threadIdx.x + q * SH_THREADS, hv[q]);
+    } else {
+      for (int e = threadIdx.x; e < tot; e += SH_THREADS) times(e, spectrum(e));
     }
     __syncthreads();
-    transform<MIXED>(X, n, P.log2n, S, lpb, twl, true);
+    transform<MIXED, MAXV>(X, n, P.log2n, S, lpb, twl, true);
   }
   for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
     int l, k;
@@ -550,7 +574,7 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
 // irfft does) and write x_a = Re z, x_b = Im z.
 
 // Forward rows: real x (R rows of n) -> half spectra (R rows of n/2 + 1).
-template <bool MIXED>
+template <bool MIXED, int MAXV>
 __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __restrict__ x,
                                                               float2* __restrict__ half, int n,
                                                               int log2n, Stages S, long long R,
@@ -564,9 +588,9 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
   const float2* twl = pass_twiddles<MIXED>(X, tot, n, S, tw);
   const long long row0 = 2ll * blockIdx.x * lpb;  // first real row of the workgroup
   {
-    float2 vv[SH_MAXV];
+    float2 vv[MAXV];
 #pragma unroll
-    for (int q = 0; q < SH_MAXV; ++q) {
+    for (int q = 0; q < MAXV; ++q) {
       const int e = threadIdx.x + q * SH_THREADS;
       if (e < tot) {
         const int l = e / n, k = e - l * n;
@@ -577,13 +601,13 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
       }
     }
 #pragma unroll
-    for (int q = 0; q < SH_MAXV; ++q) {
+    for (int q = 0; q < MAXV; ++q) {
       const int e = threadIdx.x + q * SH_THREADS;
       if (e < tot) X[e] = vv[q];
     }
   }
   __syncthreads();
-  transform<MIXED>(X, n, log2n, S, lpb, twl, false);
+  transform<MIXED, MAXV>(X, n, log2n, S, lpb, twl, false);
   for (int e = threadIdx.x; e < lpb * H1; e += SH_THREADS) {
     const int l = e / H1, k = e - l * H1;
     const long long ra = row0 + 2 * l, rb = ra + 1;
@@ -599,7 +623,7 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
 
 // Inverse rows: half spectra (R rows of n/2 + 1) of row pairs row0 + 2 l ->
 // transformed lines X (real rows row0 + 2 l and row0 + 2 l + 1, unscaled).
-template <bool MIXED>
+template <bool MIXED, int MAXV>
 __device__ __forceinline__ void c2r_lines(const float2* __restrict__ half, float2* X, int n,
                                           int log2n, const Stages& S, long long R, int lpb,
                                           long long row0, const float2* __restrict__ tw) {
@@ -616,11 +640,11 @@ __device__ __forceinline__ void c2r_lines(const float2* __restrict__ half, float
     if (k > 0 && 2 * k < n) X[l * n + n - k] = make_float2(__fadd_rn(a.x, b.y), __fsub_rn(b.x, a.y));
   }
   __syncthreads();
-  transform<MIXED>(X, n, log2n, S, lpb, twl, true);
+  transform<MIXED, MAXV>(X, n, log2n, S, lpb, twl, true);
 }
 
 // Inverse rows to real y (R rows of n), times scale.
-template <bool MIXED>
+template <bool MIXED, int MAXV>
 __global__ __launch_bounds__(SH_THREADS) void c2r_rows_kernel(const float2* __restrict__ half,
                                                               float* __restrict__ y, int n,
                                                               int log2n, Stages S, long long R,
@@ -631,7 +655,7 @@ __global__ __launch_bounds__(SH_THREADS) void c2r_rows_kernel(const float2* __re
   extern __shared__ float2 lds[];
   float2* X = lds;
   const long long row0 = 2ll * blockIdx.x * lpb;
-  c2r_lines<MIXED>(half, X, n, log2n, S, R, lpb, row0, tw);
+  c2r_lines<MIXED, MAXV>(half, X, n, log2n, S, R, lpb, row0, tw);
   for (int e = threadIdx.x; e < lpb * n; e += SH_THREADS) {
     const int l = e / n, k = e - l * n;
     const long long ra = row0 + 2 * l, rb = ra + 1;
@@ -913,7 +937,7 @@ __global__ __launch_bounds__(SH_THREADS) void cols64_kernel(const double2* __res
 // Columns of any length (the 1024-point ones below keep their line in
 // registers): forward, objective partial of the workgroup's columns (if
 // obj), times gs, inverse, times 1/F0.
-template <bool MIXED>
+template <bool MIXED, int MAXV>
 __global__ __launch_bounds__(SH_THREADS) void cols_gram_kernel(
     float2* __restrict__ half, const float2* __restrict__ hs, const float* __restrict__ gs,
     const float2* __restrict__ Yh, double* __restrict__ obj, int n, int log2n, Stages S, int H1,
@@ -935,7 +959,7 @@ __global__ __launch_bounds__(SH_THREADS) void cols_gram_kernel(
     X[l * n + k] = l < nl ? half[static_cast<long long>(k) * H1 + c0 + l] : make_float2(0.f, 0.f);
   }
   __syncthreads();
-  transform<MIXED>(X, n, log2n, S, lpb, twl, false);
+  transform<MIXED, MAXV>(X, n, log2n, S, lpb, twl, false);
   double acc = 0.0;
   for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
     const int k = e / lpb, l = e - k * lpb;
@@ -958,7 +982,7 @@ __global__ __launch_bounds__(SH_THREADS) void cols_gram_kernel(
     if (threadIdx.x == 0) obj[blockIdx.x] = acc;
   }
   __syncthreads();
-  transform<MIXED>(X, n, log2n, S, lpb, twl, true);
+  transform<MIXED, MAXV>(X, n, log2n, S, lpb, twl, true);
   for (int e = threadIdx.x; e < tot; e += SH_THREADS) {
     const int k = e / lpb, l = e - k * lpb;
     if (l < nl) {
@@ -1076,7 +1100,7 @@ __global__ __launch_bounds__(2 * QT) void q1k_c2r_step_kernel(
 
 // The same for rows of any length: workgroup 0 reduces the statistics row if
 // STATS, the others take lpb row pairs each.
-template <bool MIXED, bool STATS>
+template <bool MIXED, int MAXV, bool STATS>
 __global__ __launch_bounds__(SH_THREADS) void c2r_step_kernel(
     const float2* __restrict__ half, float* __restrict__ gx, const float* __restrict__ v,
     const float* __restrict__ aty, float c1, float c, float b, float* __restrict__ u, int n,
@@ -1091,7 +1115,7 @@ __global__ __launch_bounds__(SH_THREADS) void c2r_step_kernel(
   extern __shared__ float2 lds[];
   float2* X = lds;
   const long long row0 = 2ll * (blockIdx.x - (STATS ? 1 : 0)) * lpb;
-  c2r_lines<MIXED>(half, X, n, log2n, S, R, lpb, row0, tw);
+  c2r_lines<MIXED, MAXV>(half, X, n, log2n, S, R, lpb, row0, tw);
   for (int q = threadIdx.x; q < 2 * lpb * n; q += SH_THREADS) {
     const int r = q / n, k = q - r * n;  // real row row0 + r
     if (row0 + r >= R) break;
@@ -1201,6 +1225,22 @@ size_t pass_lds(const AxisTables& t, int lpb) {
   return sizeof(float2) * (static_cast<size_t>(lpb) * t.n + (t.st.twlds ? t.n : 0));
 }
 
+// Lines that a workgroup may take: 1024 values, the instances of four values
+// a thread (8 x 512 x 512 convolution, 4 lines against 2: 53.7 against 48.2
+// us, 8 x 450 x 480 64.3 against 41.3 us); lines longer than that 8192 (7168
+// beside the twiddles of p-term sums).
+int line_cap(const AxisTables& t) {
+  const int values = t.n <= SH_FEW * SH_THREADS ? SH_FEW * SH_THREADS
+                                                : (t.log2n >= 0 ? 8192 : 7168);
+  return std::max(1, values / t.n);
+}
+
+// The instance of a pass's kernel for lpb lines of t (see SH_MAXV).
+#define SCXR_FFT_KERNEL(K, t, lpb, ...)                                          \
+  (static_cast<long long>(lpb) * (t).n <= SH_FEW * SH_THREADS                    \
+       ? ((t).log2n < 0 ? &K<true, SH_FEW, ##__VA_ARGS__> : &K<false, SH_FEW, ##__VA_ARGS__>) \
+       : ((t).log2n < 0 ? &K<true, SH_MAXV, ##__VA_ARGS__> : &K<false, SH_MAXV, ##__VA_ARGS__>))
+
 int make_tables(AxisTables& t, int n) {
   t.n = n;
   t.log2n = log2_exact(n);
@@ -1240,10 +1280,9 @@ int run_pass(const Plan& p, int a, const void* in, void* out, bool in_real, bool
   P.stride = stride;
   P.inner = stride;
   P.lines = p.batch * (p.fsize / t.n);
-  // one LDS buffer of lpb lines (at most 7168 values, with the twiddles of
-  // p-term sums 64 KiB at most); lines per workgroup chosen so that a pass
+  // one LDS buffer of lpb lines; lines per workgroup chosen so that a pass
   // has at least ~1024 workgroups
-  int lpb = std::max(1, (t.log2n >= 0 ? 8192 : 7168) / t.n);
+  int lpb = line_cap(t);
   { int q = 1; while (q * 2 <= lpb) q *= 2; lpb = q; }
   while (lpb > 1 && (P.lines + lpb - 1) / lpb < 1024) lpb /= 2;
   lpb = std::min(lpb, 64);
@@ -1257,12 +1296,8 @@ int run_pass(const Plan& p, int a, const void* in, void* out, bool in_real, bool
   P.h = p.h;
   const float scale = (inverse || fused) ? 1.0f / static_cast<float>(t.n) : 1.0f;
   const unsigned grid = static_cast<unsigned>((P.lines + lpb - 1) / lpb);
-  if (t.log2n < 0)
-    hipLaunchKernelGGL(stockham_kernel<true>, dim3(grid), dim3(SH_THREADS), pass_lds(t, lpb), s,
-                       in, out, P, t.st, scale, pred);
-  else
-    hipLaunchKernelGGL(stockham_kernel<false>, dim3(grid), dim3(SH_THREADS), pass_lds(t, lpb), s,
-                       in, out, P, t.st, scale, pred);
+  hipLaunchKernelGGL(SCXR_FFT_KERNEL(stockham_kernel, t, lpb), dim3(grid), dim3(SH_THREADS),
+                     pass_lds(t, lpb), s, in, out, P, t.st, scale, pred);
   SCXR_LAUNCHED("fft pass");
   return SCXR_OK;
 }
@@ -1290,9 +1325,7 @@ int convolve_r2c(const Plan& p, const float* x, float* y, bool adj, const int32_
   int lr = p.lpb_rows;
   const unsigned gr = static_cast<unsigned>((cl + lr - 1) / lr);
   const size_t lds_r = pass_lds(t1, lr);
-  const bool mix1 = t1.log2n < 0;
-  hipLaunchKernelGGL(mix1 ? r2c_rows_kernel<true> : r2c_rows_kernel<false>, dim3(gr),
-                     dim3(SH_THREADS), lds_r, s, x, half, n, t1.log2n, t1.st, R, lr, t1.tw, pred);
+  hipLaunchKernelGGL(SCXR_FFT_KERNEL(r2c_rows_kernel, t1, lr), dim3(gr), dim3(SH_THREADS), lds_r, s, x, half, n, t1.log2n, t1.st, R, lr, t1.tw, pred);
   SCXR_LAUNCHED("fft r2c rows");
   // columns of the half spectrum: n0-point transforms at stride H1
   const AxisTables& t0 = p.ax[0];
@@ -1308,12 +1341,11 @@ int convolve_r2c(const Plan& p, const float* x, float* y, bool adj, const int32_
   P.tw = t0.tw;
   P.h = p.hs;
   const unsigned gc = static_cast<unsigned>((P.lines + P.lpb - 1) / P.lpb);
-  hipLaunchKernelGGL(t0.log2n < 0 ? stockham_kernel<true> : stockham_kernel<false>, dim3(gc),
-                     dim3(SH_THREADS), pass_lds(t0, P.lpb), s, static_cast<const void*>(half),
+  hipLaunchKernelGGL(SCXR_FFT_KERNEL(stockham_kernel, t0, P.lpb), dim3(gc), dim3(SH_THREADS),
+                     pass_lds(t0, P.lpb), s, static_cast<const void*>(half),
                      static_cast<void*>(half), P, t0.st, 1.0f / static_cast<float>(t0.n), pred);
   SCXR_LAUNCHED("fft half-spectrum columns");
-  hipLaunchKernelGGL(mix1 ? c2r_rows_kernel<true> : c2r_rows_kernel<false>, dim3(gr),
-                     dim3(SH_THREADS), lds_r, s, half, y, n, t1.log2n, t1.st, R, lr, t1.tw,
+  hipLaunchKernelGGL(SCXR_FFT_KERNEL(c2r_rows_kernel, t1, lr), dim3(gr), dim3(SH_THREADS), lds_r, s, half, y, n, t1.log2n, t1.st, R, lr, t1.tw,
                      1.0f / static_cast<float>(n), pred);
   SCXR_LAUNCHED("fft c2r rows");
   return SCXR_OK;
@@ -1391,11 +1423,11 @@ int scxr_cconv_plan_create(int32_t ndim, const int32_t* fshape, int64_t batch,
     const long long H1 = p.F[1] / 2 + 1;
     if (hipMalloc(&p.hs, sizeof(float2) * p.F[0] * H1) != hipSuccess)
       rc = fail(SCXR_ERR_NOMEM, "hipMalloc of the half spectrum failed");
-    // lines per workgroup: as many as fit 8192 LDS values (7168 beside the
-    // twiddles of p-term sums; at most the 64 lines that a column pass
-    // tabulates) while the pass keeps at least 512 workgroups (SCXR_FFT_LPB="rows,cols" overrides)
+    // lines per workgroup: as many as line_cap allows (at most the 64 lines
+    // that a column pass tabulates) while the pass keeps at least 512
+    // workgroups (SCXR_FFT_LPB="rows,cols" overrides)
     auto pick = [](long long lines, const AxisTables& t) {
-      int l = std::max(1, std::min(64, (t.log2n >= 0 ? 8192 : 7168) / t.n));
+      int l = std::min(64, line_cap(t));
       while (l > 1 && (lines + l - 1) / l < 512) l /= 2;
       return l;
     };
@@ -1491,25 +1523,24 @@ static int apgm_grad(const scxr_cconv_plan* plan, const float* x, const float* g
   if (!q1k_path(p)) {
     const AxisTables &t0 = p.ax[0], &t1 = p.ax[1];
     const int n0 = t0.n, n1 = t1.n, H1 = n1 / 2 + 1, lr = p.lpb_rows;
-    const bool mix0 = t0.log2n < 0, mix1 = t1.log2n < 0;
     const unsigned gr = ceil_div((n0 + 1) / 2, lr);
-    hipLaunchKernelGGL(mix1 ? r2c_rows_kernel<true> : r2c_rows_kernel<false>, dim3(gr),
-                       dim3(SH_THREADS), pass_lds(t1, lr), s, x, half, n1, t1.log2n, t1.st,
+    hipLaunchKernelGGL(SCXR_FFT_KERNEL(r2c_rows_kernel, t1, lr), dim3(gr), dim3(SH_THREADS),
+                       pass_lds(t1, lr), s, x, half, n1, t1.log2n, t1.st,
                        static_cast<long long>(n0), lr, t1.tw, pred);
     SCXR_LAUNCHED("fft r2c rows");
-    hipLaunchKernelGGL(mix0 ? cols_gram_kernel<true> : cols_gram_kernel<false>,
+    hipLaunchKernelGGL(SCXR_FFT_KERNEL(cols_gram_kernel, t0, p.lpb_cols),
                        dim3(apgm_parts(p)), dim3(SH_THREADS), pass_lds(t0, p.lpb_cols), s, half,
                        p.hs, gs, reinterpret_cast<const float2*>(Yh), obj, n0, t0.log2n, t0.st, H1,
                        n1, p.lpb_cols, t0.tw, 1.0f / static_cast<float>(n0), pred);
     SCXR_LAUNCHED("fft gram columns");
     const float sc = 1.0f / static_cast<float>(n1);
     if (st)
-      hipLaunchKernelGGL((mix1 ? c2r_step_kernel<true, true> : c2r_step_kernel<false, true>),
+      hipLaunchKernelGGL(SCXR_FFT_KERNEL(c2r_step_kernel, t1, lr, true),
                          dim3(gr + 1), dim3(SH_THREADS), pass_lds(t1, lr), s, half, gx, v, aty,
                          1.0f + c, c, b, u, n1, t1.log2n, t1.st, static_cast<long long>(n0), lr,
                          t1.tw, sc, *st, pred);
     else
-      hipLaunchKernelGGL((mix1 ? c2r_step_kernel<true, false> : c2r_step_kernel<false, false>),
+      hipLaunchKernelGGL(SCXR_FFT_KERNEL(c2r_step_kernel, t1, lr, false),
                          dim3(gr), dim3(SH_THREADS), pass_lds(t1, lr), s, half, gx, v, aty,
                          1.0f + c, c, b, u, n1, t1.log2n, t1.st, static_cast<long long>(n0), lr,
                          t1.tw, sc, ApgmStats{}, pred);
