@@ -14,8 +14,9 @@
   (``scico/optimize/_pgm.py:183-252``) with a per-pixel TV weight map,
   differentiable with respect to the sinogram and the weight map.  The
   backward pass recomputes the forward from checkpoints every
-  ``checkpoint_every`` steps and runs the adjoint recursion with the
-  projector kernels and the TV-prox VJP kernel.
+  ``checkpoint_every`` steps (except after the last, whose prox inputs the
+  forward keeps) and runs the adjoint recursion with the projector kernels
+  and the TV-prox VJP kernel.
 """
 
 from __future__ import annotations
@@ -168,29 +169,43 @@ def _momentum(K: int) -> List[float]:
     return cs
 
 
-def _step(H, y, v, x_old, w, L, lam, c, iso):
-    """One AcceleratedPGM step; returns ``(x, v_next, u)``."""
+def _prox_input(H, y, v, L):
+    """``u = v - (1/L) H^T (H v - y)``."""
     r = vec.add(H.project(v), -1.0, y)
-    u = vec.axpby(1.0, v, -(1.0 / L), H.back_project(r))
+    return vec.axpby(1.0, v, -(1.0 / L), H.back_project(r))
+
+
+def _prox_step(u, x_old, w, L, lam, c, iso):
+    """The rest of an AcceleratedPGM step: ``(x, v_next)``."""
     x = tv_prox_weighted(u, (1.0 / L) * lam, w, isotropic=iso)
-    v_next = vec.axpby(1.0, x, c, vec.add(x, -1.0, x_old))
-    return x, v_next, u
+    return x, vec.axpby(1.0, x, c, vec.add(x, -1.0, x_old))
 
 
 class _UnrolledAPGMTV(torch.autograd.Function):
+    # The backward runs over segments of `every` steps.  The forward keeps
+    # (x, v) at the start of each, and the prox inputs of the last one, which
+    # the backward needs first (the others' it computes again: as many images,
+    # one segment at a time).
     @staticmethod
     def forward(ctx, y, w, x0, H, L, lam, K, every, iso):
         y, w = y.detach().contiguous(), w.detach().contiguous()
         cs = _momentum(K)
-        x = x0.detach().contiguous().clone()
-        v = x.clone()
-        ckpts = {}
+        x = v = x0.detach().contiguous().clone()
+        ckpts, us = {}, []
+        keep = any(ctx.needs_input_grad)
         for k in range(K):
-            if k % every == 0:
-                ckpts[k] = (x.clone(), v.clone())
-            x, v, _ = _step(H, y, v, x, w, L, lam, cs[k], iso)
+            if k % every == 0 and keep:
+                ckpts[k] = (x, v)
+                us = []
+            u = _prox_input(H, y, v, L)
+            if keep:
+                us.append(u)
+            if k + 1 < K:
+                x, v = _prox_step(u, x, w, L, lam, cs[k], iso)
+            else:
+                x = tv_prox_weighted(u, (1.0 / L) * lam, w, isotropic=iso)
         ctx.H, ctx.L, ctx.lam, ctx.K, ctx.every, ctx.iso, ctx.cs = H, L, lam, K, every, iso, cs
-        ctx.ckpts = ckpts
+        ctx.ckpts, ctx.us = ckpts, us
         ctx.save_for_backward(y, w)
         return x
 
@@ -199,19 +214,23 @@ class _UnrolledAPGMTV(torch.autograd.Function):
         y, w = ctx.saved_tensors
         H, L, lam, K, every, iso, cs = ctx.H, ctx.L, ctx.lam, ctx.K, ctx.every, ctx.iso, ctx.cs
         gam = 1.0 / L
-        xbar = gx.detach().contiguous().clone()  # cotangent of x_{k+1}
+        xbar = gx.detach().contiguous()  # cotangent of x_{k+1}
         vbar = torch.zeros_like(xbar)  # cotangent of v_{k+1}
         ybar = torch.zeros_like(y)
         wbar = torch.zeros_like(w)
         gw = torch.empty_like(w)
+        us = ctx.us
         for s in reversed(sorted(ctx.ckpts)):
-            # recompute the segment's prox inputs u_k from the checkpoint
-            x, v = (t.clone() for t in ctx.ckpts[s])
-            us = []
-            for k in range(s, min(s + every, K)):
-                x, v, u = _step(H, y, v, x, w, L, lam, cs[k], iso)
-                us.append(u)
-            for k in reversed(range(s, min(s + every, K))):
+            end = min(s + every, K)
+            if us is None:
+                # recompute the segment's prox inputs u_k from the checkpoint
+                x, v = ctx.ckpts[s]
+                us = []
+                for k in range(s, end):
+                    us.append(_prox_input(H, y, v, L))
+                    if k + 1 < end:
+                        x, v = _prox_step(us[-1], x, w, L, lam, cs[k], iso)
+            for k in reversed(range(s, end)):
                 u = us[k - s]
                 # v_{k+1} = x_{k+1} + c_k (x_{k+1} - x_k)
                 xk1 = vec.axpby(1.0, xbar, 1.0 + cs[k], vbar)
@@ -224,6 +243,7 @@ class _UnrolledAPGMTV(torch.autograd.Function):
                 vec.axpby(1.0, ybar, gam, Au, out=ybar)
                 vbar = vec.axpby(1.0, ubar, -gam, H.back_project(Au))
                 xbar = xk_part
+            us = None
         return ybar, wbar, None, None, None, None, None, None, None
 
 
