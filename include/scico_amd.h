@@ -91,6 +91,12 @@ int scxr_xr2d_forward(const scxr_xr2d_plan* plan, const float* im, float* sino,
 int scxr_xr2d_forward_t(const scxr_xr2d_plan* plan, const float* im, const float* imT,
                         float* sino, const int32_t* pred, void* stream);
 
+/* im = (c w) A^T sino elementwise, in the back projection's launch (bitwise
+ * scxr_vec_scale_mul after it; w of im's size).  SCXR_ERR_UNSUPPORTED for the
+ * general-geometry adjoint. */
+int scxr_xr2d_adjoint_mul(const scxr_xr2d_plan* plan, const float* sino, float c, const float* w,
+                          float* im, const int32_t* pred, void* stream);
+
 /* im = A^T sino  (_xray2d.py:267-306), gather form, exact adjoint of the
  * forward's weights. */
 int scxr_xr2d_adjoint(const scxr_xr2d_plan* plan, const float* sino, float* im,

@@ -190,6 +190,8 @@ SIGNATURES = [
     ("scxr_ramp_filter", c_int32,
      [c_int32, c_int32, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     ("scxr_vec_mul", c_int32, [c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    ("scxr_xr2d_adjoint_mul", c_int32,
+     [c_void_p, c_void_p, c_float, c_void_p, c_void_p, c_void_p, c_void_p]),
     ("scxr_vec_scale_mul", c_int32,
      [c_int64, c_float, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     ("scxr_vec_ge", c_int32, [c_int64, c_void_p, c_float, c_float, c_void_p, c_void_p, c_void_p]),

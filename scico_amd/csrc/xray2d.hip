@@ -1247,6 +1247,8 @@ __device__ __forceinline__ void adj_tile(const float* __restrict__ sino, float* 
         v = __fadd_rn(__fmul_rn(epi.rho, fd::gram2d(epi.p, M, N, i[q], j, circ)), v);
       } else if (epi.kind == EPI_RHS) {  // A^T y + rho * C^T (z - u)   (_admmaux.py:245-256)
         v = __fadd_rn(v, __fmul_rn(epi.rho, fd::adj2d_diff(epi.z, epi.u, M, N, i[q], j, circ)));
+      } else if (epi.kind == EPI_MUL) {
+        v = __fmul_rn(__fmul_rn(epi.rho, epi.p[static_cast<size_t>(i[q]) * N + j]), v);
       }
       out[static_cast<size_t>(i[q]) * N + j] = v;
       if (epi.dot_ws) dot += static_cast<double>(epi.p[static_cast<size_t>(i[q]) * N + j]) * v;
@@ -1772,6 +1774,16 @@ int scxr_xr2d_forward_res(const scxr_xr2d_plan* plan, const float* im, float* si
   SCXR_REQUIRE(plan && im && sino && y && res_ws, SCXR_ERR_ARG,
                "null argument to xr2d_forward_res");
   return xr2d::forward(plan->p, im, sino, pred, as_stream(stream), y, res_ws);
+}
+
+int scxr_xr2d_adjoint_mul(const scxr_xr2d_plan* plan, const float* sino, float c, const float* w,
+                          float* im, const int32_t* pred, void* stream) {
+  SCXR_REQUIRE(plan && im && sino && w, SCXR_ERR_ARG, "null argument to xr2d_adjoint_mul");
+  AdjEpi e;
+  e.kind = EPI_MUL;
+  e.rho = c;
+  e.p = w;
+  return xr2d::adjoint(plan->p, sino, im, pred, as_stream(stream), e);
 }
 
 int scxr_xr2d_adjoint(const scxr_xr2d_plan* plan, const float* sino, float* im,

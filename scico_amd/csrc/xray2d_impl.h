@@ -90,12 +90,13 @@ struct Plan {
 };
 
 // Adjoint epilogues (applied per pixel after the back projection sum).
-enum { EPI_NONE = 0, EPI_GRAM = 1, EPI_RHS = 2 };
+enum { EPI_NONE = 0, EPI_GRAM = 1, EPI_RHS = 2, EPI_MUL = 3 };
 struct AdjEpi {
   int kind = EPI_NONE;
   int circular = 0;
   float rho = 0.0f;
   const float* p = nullptr;  // EPI_GRAM: image whose FD gram is added; dot partner
+                             // EPI_MUL: image that rho times multiplies the result
   const float* z = nullptr;  // EPI_RHS: (2, M, N)
   const float* u = nullptr;  // EPI_RHS: (2, M, N), may be null
   double* dot_ws = nullptr;  // per-workgroup partials of sum p * out (nullable)

@@ -5,8 +5,10 @@ from __future__ import annotations
 import numpy as np
 
 from ... import _device as dev
+from ... import _pred
 from ... import _vec as vec
 from ..._lib import call
+from ._xray2d import XRayTransform2D
 
 
 def ramp_filter(x, tau: float) -> np.ndarray:
@@ -53,6 +55,11 @@ def fbp(H, y):
     hy = dev.empty((A, Dout))
     call("scxr_ramp_filter", A, N, Dout, s, H.fbp_filter.data_ptr(), y.data_ptr(),
          hy.data_ptr(), None, dev.stream())
-    bp = H.back_project(hy)
     c = float(np.float32(np.pi * float(np.asarray(H.dx[0])) * float(np.asarray(H.dx[1])) / A))
+    if type(H).back_project is XRayTransform2D.back_project and H.tiled:
+        out = dev.empty(H.input_shape)
+        call("scxr_xr2d_adjoint_mul", H.plan, hy.data_ptr(), c, H.fbp_mask.data_ptr(),
+             out.data_ptr(), dev.ptr(_pred.resolve(None)), dev.stream())
+        return out
+    bp = H.back_project(hy)
     return vec.scale_mul(c, H.fbp_mask, bp, out=bp)

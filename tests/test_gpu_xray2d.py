@@ -375,3 +375,24 @@ def test_forward_parts_and_staged_columns(gpu, M, N, A, parts):
                 np.add.at(cnt, at, 1)
             bar = (cnt + 2) * 2.0**-24 * mag
             assert np.all(np.abs(got[a] - ref[1:-1]) <= bar[1:-1])
+
+
+@pytest.mark.parametrize("shape,views,det", [((17, 33), 5, None), ((128, 130), 9, 91),
+                                             ((300, 500), 12, None)])
+def test_adjoint_mul_epilogue(gpu, shape, views, det):
+    """``(c w) H^T y`` in the back projection's launch is bitwise the two
+    passes (one and two pixels a thread), infinities and zeros included."""
+    from scico_amd import _vec as vec
+    from scico_amd._lib import call
+
+    H = XRayTransform2D(shape, np.linspace(0, np.pi, views, endpoint=False).astype(np.float32),
+                        det_count=det)
+    g = torch.Generator("cpu").manual_seed(2)
+    y = torch.randn(H.output_shape, generator=g).cuda()
+    w = (torch.rand(shape, generator=g) > 0.5).float().cuda()
+    y[0, H.ny // 2] = float("inf")
+    out = torch.empty(shape, device="cuda")
+    call("scxr_xr2d_adjoint_mul", H.plan, y.data_ptr(), 0.37, w.data_ptr(), out.data_ptr(), None,
+         torch.cuda.current_stream().cuda_stream)
+    ref = vec.scale_mul(0.37, w, H.back_project(y))
+    assert torch.equal(out.view(torch.int32), ref.view(torch.int32))
