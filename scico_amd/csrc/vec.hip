@@ -8,6 +8,7 @@
 #include "common.h"
 #include "vec_impl.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -152,7 +153,8 @@ __global__ __launch_bounds__(256) void reduce_pass2(int nparts, const double* __
 }
 
 unsigned grid_for(int64_t n) {
-  const int64_t b = (n + 1023) / 1024;
+  // (as solver::elem_grid)
+  const int64_t b = std::max((n + 1023) / 1024, std::min<int64_t>((n + 255) / 256, 256));
   return static_cast<unsigned>(b < 1 ? 1 : (b > 2048 ? 2048 : b));
 }
 
