@@ -185,10 +185,12 @@ __device__ __forceinline__ void slice_block(int& bg, int& vg) {
   // (neighbouring views' strips share most of their pixel rows, so they
   // share its L2) across all bin groups (whose strips differ in length,
   // so every XCD gets a similar share of work).  A bijection of the grid.
+  // (An eighth rounded up: rounded down, a run ends in the long strips of one
+  // block more; 256^3 with 360 and 180 views 1256, 741 -> 1196, 698 us.)
   const int GX = gridDim.x, GY = gridDim.y, G = GX * GY, G8 = (G / 8) * 8;
   int L = blockIdx.y * GX + blockIdx.x;
   if (L < G8) L = (L % 8) * (G8 / 8) + L / 8;
-  const int VB = GY >= 8 ? GY / 8 : 1;  // view groups per block
+  const int VB = (GY + 7) / 8;  // view groups per block
   const int blk = L / (GX * VB);
   const int nb = min(VB, GY - blk * VB);  // the last block may be short
   const int within = L - blk * GX * VB;
@@ -350,10 +352,11 @@ __device__ __forceinline__ float4 fma4_bcast(float w, float4 x, float4 acc) {
 // row's 16 entries are read back into every 16-lane row, where a slot's
 // weights are a row broadcast of a constant lane and one ballot tells which
 // slots are taken.  Bound by the vector loads (a 16-byte load of 64 lanes for
-// each pixel, view and bin group: 28 TB/s from the CUs' caches at 256^3 with
+// each pixel, view and bin group: 23 TB/s from the CUs' caches at 256^3 with
 // 360 views) and their latency.  Against fwd_slice_kernel: 256^3 with 360, 180
-// and 45 views 1372, 844, 405 -> 1256, 741, 330 us, 128^3 with 90 views 194 ->
-// 153 us.  (Eight loads at a time: 1212, 787, 376, 171 us.)
+// and 45 views 1372, 844, 405 -> 1196, 698, 323 us, 128^3 with 90 views 194 ->
+// 151 us.  (Eight loads at a time, before slice_block rounded up: 1212, 787,
+// 376, 171 against 1256, 741, 330, 153 us.)
 // (Sharing the pixel rows of four views through LDS takes two thirds off the
 // loads, but with a barrier per image row too little is in flight: 1602 us.)
 __global__ __launch_bounds__(256) void fwd_slice16_kernel(
