@@ -573,11 +573,31 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
 // imaginary parts of the k = 0 and, for even F1, k = F1/2 bins dropped, as
 // irfft does) and write x_a = Re z, x_b = Im z.
 
+// The row pairs of a pass over R rows.  A pair shares its rounding (and
+// whatever is not finite), so both rows come from one image: where the images
+// of a batch have an odd number of rows, `odd` is the number of pairs of an
+// image, the last of which is one row alone (0: rows pair throughout).
+struct RowPairs {
+  long long R;
+  unsigned odd;
+};
+// First row of a pair, and its second (R or more: there is none).
+__device__ __forceinline__ void pair_rows(const RowPairs& P, long long pair, long long& ra,
+                                          long long& rb) {
+  ra = 2 * pair;
+  rb = ra + 1;
+  if (P.odd) {
+    const unsigned q = static_cast<unsigned>(pair), im = q / P.odd;
+    ra -= im;
+    rb = q - im * P.odd == P.odd - 1 ? P.R : ra + 1;
+  }
+}
+
 // Forward rows: real x (R rows of n) -> half spectra (R rows of n/2 + 1).
 template <bool MIXED, int MAXV>
 __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __restrict__ x,
                                                               float2* __restrict__ half, int n,
-                                                              int log2n, Stages S, long long R,
+                                                              int log2n, Stages S, RowPairs P,
                                                               int lpb,
                                                               const float2* __restrict__ tw,
                                                               const int32_t* pred) {
@@ -586,7 +606,7 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
   float2* X = lds;
   const int tot = lpb * n, H1 = n / 2 + 1;
   const float2* twl = pass_twiddles<MIXED>(X, tot, n, S, tw);
-  const long long row0 = 2ll * blockIdx.x * lpb;  // first real row of the workgroup
+  const long long R = P.R, pair0 = static_cast<long long>(blockIdx.x) * lpb;
   {
     float2 vv[MAXV];
 #pragma unroll
@@ -594,7 +614,8 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
       const int e = threadIdx.x + q * SH_THREADS;
       if (e < tot) {
         const int l = e / n, k = e - l * n;
-        const long long ra = row0 + 2 * l, rb = ra + 1;
+        long long ra, rb;
+        pair_rows(P, pair0 + l, ra, rb);
         const float a = ra < R ? x[ra * n + k] : 0.0f;
         const float b = rb < R ? x[rb * n + k] : 0.0f;
         vv[q] = make_float2(a, b);
@@ -610,7 +631,8 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
   transform<MIXED, MAXV>(X, n, log2n, S, lpb, twl, false);
   for (int e = threadIdx.x; e < lpb * H1; e += SH_THREADS) {
     const int l = e / H1, k = e - l * H1;
-    const long long ra = row0 + 2 * l, rb = ra + 1;
+    long long ra, rb;
+    pair_rows(P, pair0 + l, ra, rb);
     const float2 zk = X[l * n + k], zm = X[l * n + (k ? n - k : 0)];
     if (ra < R)
       half[ra * H1 + k] = make_float2(__fmul_rn(0.5f, __fadd_rn(zk.x, zm.x)),
@@ -621,17 +643,19 @@ __global__ __launch_bounds__(SH_THREADS) void r2c_rows_kernel(const float* __res
   }
 }
 
-// Inverse rows: half spectra (R rows of n/2 + 1) of row pairs row0 + 2 l ->
-// transformed lines X (real rows row0 + 2 l and row0 + 2 l + 1, unscaled).
+// Inverse rows: half spectra (R rows of n/2 + 1) of the row pairs pair0 + l ->
+// transformed lines X (the real rows of each pair, unscaled).
 template <bool MIXED, int MAXV>
 __device__ __forceinline__ void c2r_lines(const float2* __restrict__ half, float2* X, int n,
-                                          int log2n, const Stages& S, long long R, int lpb,
-                                          long long row0, const float2* __restrict__ tw) {
+                                          int log2n, const Stages& S, const RowPairs& P, int lpb,
+                                          long long pair0, const float2* __restrict__ tw) {
   const int H1 = n / 2 + 1;
+  const long long R = P.R;
   const float2* twl = pass_twiddles<MIXED>(X, lpb * n, n, S, tw);
   for (int e = threadIdx.x; e < lpb * H1; e += SH_THREADS) {
     const int l = e / H1, k = e - l * H1;
-    const long long ra = row0 + 2 * l, rb = ra + 1;
+    long long ra, rb;
+    pair_rows(P, pair0 + l, ra, rb);
     float2 a = ra < R ? half[ra * H1 + k] : make_float2(0.0f, 0.0f);
     float2 b = rb < R ? half[rb * H1 + k] : make_float2(0.0f, 0.0f);
     if (k == 0 || 2 * k == n) a.y = b.y = 0.0f;
@@ -647,18 +671,19 @@ __device__ __forceinline__ void c2r_lines(const float2* __restrict__ half, float
 template <bool MIXED, int MAXV>
 __global__ __launch_bounds__(SH_THREADS) void c2r_rows_kernel(const float2* __restrict__ half,
                                                               float* __restrict__ y, int n,
-                                                              int log2n, Stages S, long long R,
+                                                              int log2n, Stages S, RowPairs P,
                                                               int lpb,
                                                               const float2* __restrict__ tw,
                                                               float scale, const int32_t* pred) {
   if (pred_off(pred)) return;
   extern __shared__ float2 lds[];
   float2* X = lds;
-  const long long row0 = 2ll * blockIdx.x * lpb;
-  c2r_lines<MIXED, MAXV>(half, X, n, log2n, S, R, lpb, row0, tw);
+  const long long R = P.R, pair0 = static_cast<long long>(blockIdx.x) * lpb;
+  c2r_lines<MIXED, MAXV>(half, X, n, log2n, S, P, lpb, pair0, tw);
   for (int e = threadIdx.x; e < lpb * n; e += SH_THREADS) {
     const int l = e / n, k = e - l * n;
-    const long long ra = row0 + 2 * l, rb = ra + 1;
+    long long ra, rb;
+    pair_rows(P, pair0 + l, ra, rb);
     const float2 v = X[e];
     if (ra < R) y[ra * n + k] = __fmul_rn(v.x, scale);
     if (rb < R) y[rb * n + k] = __fmul_rn(v.y, scale);
@@ -1115,7 +1140,7 @@ __global__ __launch_bounds__(SH_THREADS) void c2r_step_kernel(
   extern __shared__ float2 lds[];
   float2* X = lds;
   const long long row0 = 2ll * (blockIdx.x - (STATS ? 1 : 0)) * lpb;
-  c2r_lines<MIXED, MAXV>(half, X, n, log2n, S, R, lpb, row0, tw);
+  c2r_lines<MIXED, MAXV>(half, X, n, log2n, S, RowPairs{R, 0}, lpb, row0 / 2, tw);
   for (int q = threadIdx.x; q < 2 * lpb * n; q += SH_THREADS) {
     const int r = q / n, k = q - r * n;  // real row row0 + r
     if (row0 + r >= R) break;
@@ -1302,6 +1327,13 @@ int run_pass(const Plan& p, int a, const void* in, void* out, bool in_real, bool
   return SCXR_OK;
 }
 
+// Row pairs of a plan's images, and their number.
+RowPairs row_pairs(const Plan& p) {
+  const bool odd = p.batch > 1 && p.F[0] % 2 == 1;
+  return {p.batch * p.F[0], odd ? static_cast<unsigned>(p.F[0] + 1) / 2 : 0u};
+}
+long long pair_count(const Plan& p) { return p.batch * ((p.F[0] + 1) / 2); }
+
 // Real 2D path: rows forward (two real rows per complex FFT), fused column
 // pass on the half spectrum, rows inverse.
 int convolve_r2c(const Plan& p, const float* x, float* y, bool adj, const int32_t* pred,
@@ -1310,7 +1342,8 @@ int convolve_r2c(const Plan& p, const float* x, float* y, bool adj, const int32_
   const int n = t1.n, H1 = n / 2 + 1;
   const long long R = p.batch * p.F[0];
   float2* half = p.work;  // R rows of H1 (fits in the batch * fsize workspace)
-  const long long cl = (R + 1) / 2;  // complex row transforms
+  const RowPairs P1 = row_pairs(p);
+  const long long cl = pair_count(p);  // complex row transforms
   if (q1k_path(p)) {
     const unsigned gr = static_cast<unsigned>(R / QR);
     hipLaunchKernelGGL(q1k_r2c_kernel, dim3(gr), dim3(2 * QT), 0, s, x, half, t1.tw, pred);
@@ -1325,7 +1358,7 @@ int convolve_r2c(const Plan& p, const float* x, float* y, bool adj, const int32_
   int lr = p.lpb_rows;
   const unsigned gr = static_cast<unsigned>((cl + lr - 1) / lr);
   const size_t lds_r = pass_lds(t1, lr);
-  hipLaunchKernelGGL(SCXR_FFT_KERNEL(r2c_rows_kernel, t1, lr), dim3(gr), dim3(SH_THREADS), lds_r, s, x, half, n, t1.log2n, t1.st, R, lr, t1.tw, pred);
+  hipLaunchKernelGGL(SCXR_FFT_KERNEL(r2c_rows_kernel, t1, lr), dim3(gr), dim3(SH_THREADS), lds_r, s, x, half, n, t1.log2n, t1.st, P1, lr, t1.tw, pred);
   SCXR_LAUNCHED("fft r2c rows");
   // columns of the half spectrum: n0-point transforms at stride H1
   const AxisTables& t0 = p.ax[0];
@@ -1345,7 +1378,7 @@ int convolve_r2c(const Plan& p, const float* x, float* y, bool adj, const int32_
                      pass_lds(t0, P.lpb), s, static_cast<const void*>(half),
                      static_cast<void*>(half), P, t0.st, 1.0f / static_cast<float>(t0.n), pred);
   SCXR_LAUNCHED("fft half-spectrum columns");
-  hipLaunchKernelGGL(SCXR_FFT_KERNEL(c2r_rows_kernel, t1, lr), dim3(gr), dim3(SH_THREADS), lds_r, s, half, y, n, t1.log2n, t1.st, R, lr, t1.tw,
+  hipLaunchKernelGGL(SCXR_FFT_KERNEL(c2r_rows_kernel, t1, lr), dim3(gr), dim3(SH_THREADS), lds_r, s, half, y, n, t1.log2n, t1.st, P1, lr, t1.tw,
                      1.0f / static_cast<float>(n), pred);
   SCXR_LAUNCHED("fft c2r rows");
   return SCXR_OK;
@@ -1431,7 +1464,7 @@ int scxr_cconv_plan_create(int32_t ndim, const int32_t* fshape, int64_t batch,
       while (l > 1 && (lines + l - 1) / l < 512) l /= 2;
       return l;
     };
-    p.lpb_rows = pick((p.batch * p.F[0] + 1) / 2, p.ax[1]);
+    p.lpb_rows = pick(pair_count(p), p.ax[1]);
     p.lpb_cols = pick(p.batch * H1, p.ax[0]);
     if (const char* env = std::getenv("SCXR_FFT_LPB")) {
       int a = 0, b = 0;
@@ -1526,7 +1559,7 @@ static int apgm_grad(const scxr_cconv_plan* plan, const float* x, const float* g
     const unsigned gr = ceil_div((n0 + 1) / 2, lr);
     hipLaunchKernelGGL(SCXR_FFT_KERNEL(r2c_rows_kernel, t1, lr), dim3(gr), dim3(SH_THREADS),
                        pass_lds(t1, lr), s, x, half, n1, t1.log2n, t1.st,
-                       static_cast<long long>(n0), lr, t1.tw, pred);
+                       row_pairs(p), lr, t1.tw, pred);
     SCXR_LAUNCHED("fft r2c rows");
     hipLaunchKernelGGL(SCXR_FFT_KERNEL(cols_gram_kernel, t0, p.lpb_cols),
                        dim3(apgm_parts(p)), dim3(SH_THREADS), pass_lds(t0, p.lpb_cols), s, half,

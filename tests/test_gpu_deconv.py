@@ -526,3 +526,26 @@ def test_fused_apgm_any_size(gpu, shape):
     print(f"  fused APGM {shape}: 10 steps rel-L2 {e:.2e}, after changes {ec:.2e}, objective "
           f"{worst:.2e} of its bar", flush=True)
     assert e <= 1e-6 and ec <= 1e-6 and worst <= 1.0
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 4), (3, 45, 60), (5, 7, 9), (4, 33, 512), (70, 5, 3)])
+def test_circconv_batch_images_apart(gpu, shape):
+    """Images with an odd number of rows: each image of a batch is the one
+    convolved alone, bit for bit and so whatever its neighbours hold (values
+    1e6 times as large, infinities, NaN)."""
+    rng = np.random.default_rng(29)
+    psf = rng.standard_normal((3, 3)).astype(np.float32)
+    x = dev(rng.standard_normal(shape).astype(np.float32))
+    A = CircularConvolve(psf, shape, ndims=2)
+    A1 = CircularConvolve(psf, shape[1:], ndims=2)
+    big = x.clone()
+    big[::2] *= 1e6
+    bad = x.clone()
+    bad[0] = float("nan")
+    bad[-1, 0] = float("inf")
+    for op, one in ((A, A1), (A.adj, A1.adj)):
+        alone = torch.stack([one(xi) for xi in x])
+        ybig, ybad = op(big), op(bad)
+        assert torch.equal(op(x), alone)
+        assert torch.equal(ybig[1::2], alone[1::2])
+        assert torch.equal(ybad[1:-1], alone[1:-1]) and torch.isnan(ybad[0]).all()
