@@ -82,7 +82,7 @@ class PGM(Optimizer):
     def objective(self, x=None):
         """``f(x) + g(x)`` (``_pgm.py:151-156``), device float64."""
         fused = getattr(self, "_fused", None)
-        if x is None and fused is not None and fused.n_steps:
+        if x is None and fused is not None and fused.has_row():
             return fused.stat(0)
         x = self.x if x is None else x
         return self.f(x) + self.g(x)
@@ -197,13 +197,21 @@ class _FusedDeconv:
         return (f, f.A, f.scale, f.y, f.y._version, g, getattr(g, "scale", 1.0), base,
                 getattr(base, "isotropic", None), getattr(base, "circular", None))
 
+    def _same_problem(self):
+        return not any(a is not b and (i not in (2, 4, 6, 8, 9) or a != b)
+                       for i, (a, b) in enumerate(zip(self._inputs(self.pgm), self._made_from)))
+
+    def has_row(self):
+        """Whether the last statistics row is that of the solver's present x
+        (not replaced, modified or loaded since the step) and problem."""
+        return self._stepped and self.pgm.x is self.x and \
+            self.x._version == self._versions[0] and self._same_problem()
+
     def current(self):
         """This object if the solver's problem and state are the ones that it
         left, itself brought up to date if only the state was replaced or
         modified (or L), else what the new problem calls for (host checks)."""
-        now = self._inputs(self.pgm)
-        if any(a is not b and (i not in (2, 4, 6, 8, 9) or a != b)
-               for i, (a, b) in enumerate(zip(now, self._made_from))):
+        if not self._same_problem():
             return _FusedDeconv.build(self.pgm)
         p = self.pgm
         if p.x is not self.x or p.v is not self.v or float(p.L) != self._L or \
@@ -276,6 +284,7 @@ class _FusedDeconv:
         """Own contiguous x and v, and the first gradient step from them
         (``same``: v is known to equal x, as in a new solver)."""
         p = self.pgm
+        self._stepped = False
         self.x = p.x.contiguous().clone()
         self.v = p.v.contiguous().clone() if hasattr(p, "v") else self.x.clone()
         self._publish()
@@ -308,6 +317,7 @@ class _FusedDeconv:
             self._reserve(2 * self.hist_cap)
         self.enqueue(c)
         self.n_steps += 1
+        self._stepped = True
         self._publish()
         self.pgm.fixed_point_residual = self.stat(1)
 

@@ -549,3 +549,40 @@ def test_circconv_batch_images_apart(gpu, shape):
         assert torch.equal(op(x), alone)
         assert torch.equal(ybig[1::2], alone[1::2])
         assert torch.equal(ybad[1:-1], alone[1:-1]) and torch.isnan(ybad[0]).all()
+
+
+@pytest.mark.parametrize("shape", [(60, 64), (1024, 1024)])
+def test_fused_apgm_objective_of_present_x(gpu, shape):
+    """objective() after a step is the step's statistic, and that of the
+    solver's x once x was replaced, modified in place or loaded, or the data
+    changed, since."""
+    import tempfile
+
+    A = CircularConvolve(gaussian_psf(5, 1.0), shape)
+    y = dev(np.random.default_rng(31).random(shape).astype(np.float32))
+
+    def make():
+        return AcceleratedPGM(f=loss.SquaredL2Loss(y=y.clone(), A=A), L0=1.0,
+                              g=2e-2 * functional.IsotropicTVNorm(),
+                              x0=torch.zeros(shape, device="cuda"), maxiter=3)
+
+    s = make()
+    assert s._fused is not None
+    for change in ("replaced", "in place", "data", "loaded"):
+        s.step()
+        before = float(s.objective())
+        assert before == float(s._fused.stat(0))
+        if change == "replaced":
+            s.x = 2.0 * s.x + 1.0
+        elif change == "in place":
+            s.x.add_(0.5)
+        elif change == "data":
+            s.f.y.mul_(2.0)
+        else:
+            with tempfile.TemporaryDirectory() as d:
+                t = make()
+                t.solve()
+                t.save_state(d + "/s.npz")
+                s.load_state(d + "/s.npz")
+        now = float(s.objective())
+        assert now == float(s.f(s.x) + s.g(s.x)) and abs(now - before) > 1e-3 * before, change
