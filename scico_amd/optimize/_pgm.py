@@ -88,9 +88,6 @@ class PGM(Optimizer):
         return self.f(x) + self.g(x)
 
     def norm_residual(self):
-        fused = getattr(self, "_fused", None)
-        if fused is not None and fused.n_steps:
-            return fused.stat(1)
         return self.fixed_point_residual
 
     def _momentum(self):
@@ -190,16 +187,17 @@ class _FusedDeconv:
 
     @staticmethod
     def _inputs(pgm):
-        """What the set-up was made from (objects, and versions that torch
-        counts up when a tensor is modified in place)."""
+        """What the set-up is made from: the objects, and with their identities
+        the values that change in place (torch counts a tensor's changes)."""
         f, g = pgm.f, pgm.g
-        base = getattr(g, "functional", g)
-        return (f, f.A, f.scale, f.y, f.y._version, g, getattr(g, "scale", 1.0), base,
-                getattr(base, "isotropic", None), getattr(base, "circular", None))
+        A, y, base = f.A, f.y, getattr(g, "functional", g)
+        return (f, A, y, g, base), (id(f), id(A), id(y), id(g), id(base), f.scale, y._version,
+                                    getattr(g, "scale", 1.0), getattr(base, "isotropic", None),
+                                    getattr(base, "circular", None))
 
     def _same_problem(self):
-        return not any(a is not b and (i not in (2, 4, 6, 8, 9) or a != b)
-                       for i, (a, b) in enumerate(zip(self._inputs(self.pgm), self._made_from)))
+        # (the objects are held, so that no other can have one's identity)
+        return self._inputs(self.pgm)[1] == self._made_from[1]
 
     def has_row(self):
         """Whether the last statistics row is that of the solver's present x
@@ -241,9 +239,6 @@ class _FusedDeconv:
         ws = torch.empty(int(lib.scxr_cconv_apgm_setup_ws(self.A.plan)), **f64)
         call("scxr_cconv_apgm_setup", self.A.plan, y.data_ptr(), self.gs.data_ptr(),
              self.Yh.data_ptr(), ws.data_ptr(), dev.stream())
-        # at 1024 x 1024 the iterates are updated in place (a captured step
-        # may be replayed on its own results); other sizes get new ones
-        self.in_place = (self.M, self.N) == (1024, 1024)
         self.aty = self.A.adj(y)
         self.n_obj = int(lib.scxr_cconv_apgm_parts(self.A.plan))
         self.n_res = int(lib.scxr_tv_prox_apgm_parts(self.M, self.N))
@@ -258,6 +253,7 @@ class _FusedDeconv:
         self.hist = None
         self.counter = torch.zeros(1, dtype=torch.int32, device=dev.DEVICE)
         self.n_steps = 0
+        self._consts_of = (None, 0.0, 0.0)  # L and the b and tau of it
         self._reserve(max(64, pgm.maxiter))
         self.adopt_state(same=getattr(pgm, "itnum", 0) == 0 and pgm.t == 1.0)
 
@@ -274,11 +270,12 @@ class _FusedDeconv:
 
     def _consts(self):
         L = float(self.pgm.L)
-        b = -(1.0 / L)
-        lam_eff = (1.0 / L) * self.lam  # ScaledFunctional.prox(v, 1/L)
-        tau = float(np.float32(np.float32(np.sqrt(np.float32(2.0))) * np.float32(4)) *
-                    np.float32(lam_eff))
-        return b, tau
+        if L != self._consts_of[0]:
+            lam_eff = (1.0 / L) * self.lam  # ScaledFunctional.prox(v, 1/L)
+            tau = float(np.float32(np.float32(np.sqrt(np.float32(2.0))) * np.float32(4)) *
+                        np.float32(lam_eff))
+            self._consts_of = (L, -(1.0 / L), tau)
+        return self._consts_of[1:]
 
     def adopt_state(self, same: bool = False):
         """Own contiguous x and v, and the first gradient step from them
@@ -306,29 +303,35 @@ class _FusedDeconv:
         vec.fill(self.gx, 0.0)
         call("scxr_cconv_apgm_grad", self.A.plan, P(self.v), P(self.gs), None, None, P(self.gx),
              P(self.v), P(self.aty), 0.0, b, P(self.u), None, s)
-        if not same and not torch.equal(self.v, self.x):  # a mid-run state: gx = G x as well
+        if not same:  # a mid-run state: gx = G x as well (no look at the values: capturable)
             scratch = torch.empty_like(self.u)
             call("scxr_cconv_apgm_grad", self.A.plan, P(self.x), P(self.gs), None, None,
                  P(self.gx), P(self.x), P(self.aty), 0.0, b, P(scratch), None, s)
-            torch.cuda.current_stream().synchronize()
 
     def step(self, c: float):
         if self.n_steps >= self.hist_cap:
             self._reserve(2 * self.hist_cap)
-        self.enqueue(c)
+        # An iterate once published keeps its values: a step makes new tensors.
+        # A captured step updates the solver's own instead, so that each replay
+        # goes on from the last one's results.
+        if torch.cuda.is_current_stream_capturing():
+            self.enqueue(c)
+        else:
+            self.enqueue(c, torch.empty_like(self.x), torch.empty_like(self.v))
         self.n_steps += 1
         self._stepped = True
         self._publish()
         self.pgm.fixed_point_residual = self.stat(1)
 
-    def enqueue(self, c: float):
-        """One iteration (no host synchronisation; capturable)."""
+    def enqueue(self, c: float, x_new=None, v_new=None):
+        """One iteration (no host synchronisation; capturable), of x and v in
+        place or into new tensors."""
         b, tau = self._consts()
         P = lambda t: t.data_ptr()
         s = dev.stream()
         x, v = self.x, self.v
-        if not self.in_place:
-            self.x, self.v = torch.empty_like(x), torch.empty_like(v)
+        if x_new is not None:
+            self.x, self.v = x_new, v_new
         call("scxr_tv_prox_apgm_to", self.M, self.N, P(self.u), P(x), P(v), P(self.x), P(self.v),
              tau, self.iso, self.circ, c, P(self.ws_res), P(self.ws_tv), None, s)
         call("scxr_cconv_apgm_grad_itstat", self.A.plan, P(self.x), P(self.gs), P(self.Yh),

@@ -586,3 +586,82 @@ def test_fused_apgm_objective_of_present_x(gpu, shape):
                 s.load_state(d + "/s.npz")
         now = float(s.objective())
         assert now == float(s.f(s.x) + s.g(s.x)) and abs(now - before) > 1e-3 * before, change
+
+
+@pytest.mark.parametrize("shape", [(3, 3), (45, 50), (60, 64), (1024, 1024)])
+@pytest.mark.parametrize("what", ["step", "enqueue"])
+def test_fused_apgm_captured_steps(gpu, shape, what):
+    """A captured step, replayed, goes on from its own results at every size:
+    after each of four replays, with eager work that allocates and frees
+    images and synchronizations between them, x and v are those of as many
+    eager steps, bit for bit, and so is an eager step that follows.  Eager
+    steps leave the iterates handed out before as they were."""
+    A = CircularConvolve(gaussian_psf(3, 1.0), shape)
+    y = dev(np.random.default_rng(37).random(shape).astype(np.float32))
+    t = 3.0  # the momentum of every step
+
+    def make():
+        s = AcceleratedPGM(f=loss.SquaredL2Loss(y=y, A=A), L0=1.0, x0=0.5 * y,
+                           g=2e-2 * functional.IsotropicTVNorm(), maxiter=8)
+        assert s._fused is not None
+        s.step()
+        s.t = t
+        return s
+
+    se, sc = make(), make()
+    c = se._momentum()  # of t
+    se.t = t
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        if what == "step":
+            sc.step()
+        else:
+            sc._fused.enqueue(c)
+    sc.t = t
+    kept = [(se.x, se.x.clone())]
+    for k in range(4):
+        graph.replay()
+        torch.cuda.synchronize()
+        junk = [torch.rand(shape, device="cuda") for _ in range(6)]
+        del junk
+        se.step()
+        se.t = t
+        kept.append((se.x, se.x.clone()))
+        torch.cuda.synchronize()
+        assert torch.equal(sc.x, se.x) and torch.equal(sc.v, se.v), k
+    sc.step()
+    se.step()
+    assert torch.equal(sc.x, se.x) and torch.equal(sc.v, se.v)
+    assert all(torch.equal(a, b) for a, b in kept)
+
+
+@pytest.mark.parametrize("shape", [(60, 64), (1024, 1024)])
+def test_fused_apgm_captured_from_assigned_state(gpu, shape):
+    """A step captured right after x and v were assigned starts, at every
+    replay, from what the assigned tensors then hold."""
+    A = CircularConvolve(gaussian_psf(3, 1.0), shape)
+    rng = np.random.default_rng(41)
+    y = dev(rng.random(shape).astype(np.float32))
+
+    def make():
+        s = AcceleratedPGM(f=loss.SquaredL2Loss(y=y, A=A), L0=1.0, x0=y,
+                           g=2e-2 * functional.IsotropicTVNorm(), maxiter=8)
+        s.step()
+        return s
+
+    sc = make()
+    x, v = 0.5 * y, 0.25 * y
+    sc.x, sc.v, sc.t = x, v, 3.0
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        sc.step()
+    for k in range(3):
+        a, b = (dev(rng.random(shape).astype(np.float32)) for _ in range(2))
+        x.copy_(a)
+        v.copy_(b)
+        graph.replay()
+        torch.cuda.synchronize()
+        se = make()
+        se.x, se.v, se.t = a, b, 3.0
+        se.step()
+        assert torch.equal(sc.x, se.x) and torch.equal(sc.v, se.v), k
