@@ -279,11 +279,14 @@ class _FusedDeconv:
 
     def adopt_state(self, same: bool = False):
         """Own contiguous x and v, and the first gradient step from them
-        (``same``: v is known to equal x, as in a new solver)."""
+        (``same``: v is known to equal x, as in a new solver).  The kernels take
+        pointers, so both are brought to the device and to float32, and one of
+        another shape is refused."""
         p = self.pgm
         self._stepped = False
-        self.x = p.x.contiguous().clone()
-        self.v = p.v.contiguous().clone() if hasattr(p, "v") else self.x.clone()
+        x = dev.input_array(p.x, (self.M, self.N), "x")
+        v = dev.input_array(p.v, (self.M, self.N), "v") if hasattr(p, "v") else x
+        self.x, self.v = x.clone(), v.clone()
         self._publish()
         self._L = float(p.L)
         self._prime(same)

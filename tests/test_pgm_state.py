@@ -1,0 +1,58 @@
+"""Host side of the fused AcceleratedPGM deconvolution: what it takes over
+from the solver, without a GPU (the device conversions and the kernels are
+replaced)."""
+
+import types
+
+import numpy as np
+import pytest
+import torch
+
+from scico_amd import _device as dev
+from scico_amd.optimize import _pgm
+
+
+@pytest.fixture
+def fused(monkeypatch):
+    """A fused iteration of a 4 x 5 problem with its kernels left out; calls
+    that would launch are counted in ``primed``."""
+
+    def as_device(x, dtype=np.float32):
+        return torch.as_tensor(x).to(dev.torch_dtype(dtype)).contiguous()
+
+    monkeypatch.setattr(dev, "as_device", as_device)
+    f = object.__new__(_pgm._FusedDeconv)
+    f.M, f.N = 4, 5
+    y = torch.zeros(4, 5)
+    f.pgm = types.SimpleNamespace(x=torch.zeros(4, 5), v=torch.zeros(4, 5), L=1.0,
+                                  f=types.SimpleNamespace(A=object(), y=y, scale=0.5),
+                                  g=types.SimpleNamespace(scale=1.0))
+    f.primed = 0
+
+    def prime(same):
+        f.primed += 1
+
+    f._prime = prime
+    f._made_from = f._inputs(f.pgm)
+    f.adopt_state()
+    return f
+
+
+@pytest.mark.parametrize("name", ["x", "v"])
+@pytest.mark.parametrize("shape", [(4, 4), (5, 4), (20,), (1, 4, 5), ()])
+def test_assigned_state_of_another_shape_is_refused(fused, name, shape):
+    setattr(fused.pgm, name, torch.zeros(shape))
+    with pytest.raises(ValueError, match="Shapes do not conform"):
+        fused.current()
+    assert fused.primed == 1
+    assert fused.x.shape == fused.v.shape == (4, 5)
+
+
+@pytest.mark.parametrize("given", [torch.ones(4, 5, dtype=torch.float64), np.ones((4, 5)),
+                                   torch.ones(5, 4).T, torch.ones(4, 5, dtype=torch.int32)])
+def test_assigned_state_is_converted(fused, given):
+    fused.pgm.v = given
+    assert fused.current() is fused and fused.primed == 2
+    v = fused.pgm.v
+    assert v is fused.v and v is not given
+    assert v.dtype == torch.float32 and v.is_contiguous() and torch.equal(v, torch.ones(4, 5))
