@@ -190,8 +190,9 @@ class _FusedDeconv:
         """What the set-up is made from: the objects, and with their identities
         the values that change in place (torch counts a tensor's changes)."""
         f, g = pgm.f, pgm.g
-        A, y, base = f.A, f.y, getattr(g, "functional", g)
-        return (f, A, y, g, base), (id(f), id(A), id(y), id(g), id(base), f.scale, y._version,
+        A, y, base = getattr(f, "A", None), getattr(f, "y", None), getattr(g, "functional", g)
+        return (f, A, y, g, base), (id(f), id(A), id(y), id(g), id(base),
+                                    getattr(f, "scale", None), getattr(y, "_version", None),
                                     getattr(g, "scale", 1.0), getattr(base, "isotropic", None),
                                     getattr(base, "circular", None))
 

@@ -56,3 +56,21 @@ def test_assigned_state_is_converted(fused, given):
     v = fused.pgm.v
     assert v is fused.v and v is not given
     assert v.dtype == torch.float32 and v.is_contiguous() and torch.equal(v, torch.ones(4, 5))
+
+
+def test_replaced_problem_asks_for_another_path(fused, monkeypatch):
+    """Functionals without the attributes of the fused structure, and changes
+    of those it was made from, go back to the choice of a path."""
+    built = []
+    monkeypatch.setattr(_pgm._FusedDeconv, "build", staticmethod(lambda p: built.append(p)))
+    assert fused.current() is fused and not built
+    keep = fused.pgm.f, fused.pgm.g
+    for f, g in ((object(), keep[1]), (keep[0], object()),
+                 (types.SimpleNamespace(A=keep[0].A, y=np.zeros((4, 5)), scale=0.5), keep[1])):
+        fused.pgm.f, fused.pgm.g = f, g
+        assert fused.current() is None and len(built) == 1
+        built.clear()
+        fused.pgm.f, fused.pgm.g = keep
+        assert fused.current() is fused and not built
+    fused.pgm.f.y.add_(1.0)
+    assert fused.current() is None and len(built) == 1
