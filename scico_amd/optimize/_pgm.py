@@ -152,6 +152,14 @@ class AcceleratedPGM(PGM):
         return ["x", "v", "t", "L"]
 
 
+def _version(t):
+    """torch's count of a tensor's in-place changes; None where there is none
+    (inference tensors, host arrays)."""
+    if not isinstance(t, torch.Tensor) or t.is_inference():
+        return None
+    return t._version
+
+
 class _FusedDeconv:
     """Fused device implementation of AcceleratedPGM-TV deconvolution."""
 
@@ -188,11 +196,12 @@ class _FusedDeconv:
     @staticmethod
     def _inputs(pgm):
         """What the set-up is made from: the objects, and with their identities
-        the values that change in place (torch counts a tensor's changes)."""
+        the values that change in place (torch counts a tensor's changes,
+        except those of a y made in inference mode, which are not followed)."""
         f, g = pgm.f, pgm.g
         A, y, base = getattr(f, "A", None), getattr(f, "y", None), getattr(g, "functional", g)
         return (f, A, y, g, base), (id(f), id(A), id(y), id(g), id(base),
-                                    getattr(f, "scale", None), getattr(y, "_version", None),
+                                    getattr(f, "scale", None), _version(y),
                                     getattr(g, "scale", 1.0), getattr(base, "isotropic", None),
                                     getattr(base, "circular", None))
 
@@ -287,7 +296,8 @@ class _FusedDeconv:
         self._stepped = False
         x = dev.input_array(p.x, (self.M, self.N), "x")
         v = dev.input_array(p.v, (self.M, self.N), "v") if hasattr(p, "v") else x
-        self.x, self.v = x.clone(), v.clone()
+        with torch.inference_mode(False):  # (tensors with a count of their changes)
+            self.x, self.v = x.clone(), v.clone()
         self._publish()
         self._L = float(p.L)
         self._prime(same)
@@ -320,6 +330,9 @@ class _FusedDeconv:
         # goes on from the last one's results.
         if torch.cuda.is_current_stream_capturing():
             self.enqueue(c)
+        elif torch.is_inference_mode_enabled():
+            with torch.inference_mode(False):  # (tensors with a count of their changes)
+                self.enqueue(c, torch.empty_like(self.x), torch.empty_like(self.v))
         else:
             self.enqueue(c, torch.empty_like(self.x), torch.empty_like(self.v))
         self.n_steps += 1

@@ -665,3 +665,29 @@ def test_fused_apgm_captured_from_assigned_state(gpu, shape):
         se.x, se.v, se.t = a, b, 3.0
         se.step()
         assert torch.equal(sc.x, se.x) and torch.equal(sc.v, se.v), k
+
+
+@pytest.mark.parametrize("shape", [(45, 50), (1024, 1024)])
+def test_fused_apgm_inference_mode(gpu, shape):
+    """A solver made and run in torch.inference_mode(), with data made inside
+    or outside it, gives what it gives elsewhere, bit for bit, also after an
+    in-place change of x."""
+    h, yh = gaussian_psf(5, 1.0), np.random.default_rng(43).random(shape).astype(np.float32)
+    outside = CircularConvolve(h, shape), dev(yh)
+
+    def run(A, y):
+        s = AcceleratedPGM(f=loss.SquaredL2Loss(y=y, A=A), L0=1.0,
+                           g=2e-2 * functional.IsotropicTVNorm(),
+                           x0=torch.zeros(shape, device="cuda"), maxiter=4)
+        assert s._fused is not None
+        s.solve()
+        s.x.mul_(0.5)
+        s.step()
+        return s.x.clone(), s.v.clone(), float(s.objective())
+
+    ref = run(*outside)
+    with torch.inference_mode():
+        for A, y in (outside, (CircularConvolve(h, shape), dev(yh))):
+            got = run(A, y)
+            assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
+            assert got[2] == ref[2]

@@ -74,3 +74,19 @@ def test_replaced_problem_asks_for_another_path(fused, monkeypatch):
         assert fused.current() is fused and not built
     fused.pgm.f.y.add_(1.0)
     assert fused.current() is None and len(built) == 1
+
+
+def test_inference_mode(fused):
+    """In inference mode, and with data made there, the state is taken over
+    and followed as elsewhere: torch keeps no count of changes for tensors of
+    that mode, so the solver's own are made outside it."""
+    with torch.inference_mode():
+        fused.pgm.x = torch.ones(4, 5)
+        fused.pgm.f.y = torch.ones(4, 5)
+        fused._made_from = fused._inputs(fused.pgm)
+        assert fused.current() is fused and fused.primed == 2
+        assert fused.current() is fused and fused.primed == 2
+        assert torch.equal(fused.x, torch.ones(4, 5))
+        fused.pgm.v.mul_(2.0)
+        assert fused.current() is fused and fused.primed == 3
+    assert fused.current() is fused and fused.primed == 3
