@@ -19,13 +19,14 @@ c_float_p = POINTER(c_float)
 c_double_p = POINTER(c_double)
 
 SCXR_OK = 0
+SCXR_ERR_UNSUPPORTED = -6
 _STATUS = {
     -1: "invalid argument",
     -2: "shape mismatch",
     -3: "unsupported geometry",
     -4: "HIP runtime error",
     -5: "device allocation failed",
-    -6: "unsupported",
+    SCXR_ERR_UNSUPPORTED: "unsupported",
 }
 
 

@@ -28,7 +28,7 @@ import torch
 
 from .. import _device as dev
 from .. import _vec as vec
-from .._lib import ScxrError, call, load
+from .._lib import SCXR_ERR_UNSUPPORTED, ScxrError, call, load
 from ._common import Optimizer
 
 
@@ -189,8 +189,10 @@ class _FusedDeconv:
         try:
             if int(load().scxr_cconv_apgm_parts(A.plan)) <= 0:
                 return None
-        except ScxrError:  # no plan for this size: the generic path reports it when used
-            return None
+        except ScxrError as e:
+            if e.code != SCXR_ERR_UNSUPPORTED:
+                raise
+            return None  # no plan for this size: the generic path reports it when used
         return _FusedDeconv(pgm, float(scale), base)
 
     @staticmethod

@@ -90,3 +90,31 @@ def test_inference_mode(fused):
         fused.pgm.v.mul_(2.0)
         assert fused.current() is fused and fused.primed == 3
     assert fused.current() is fused and fused.primed == 3
+
+
+@pytest.mark.parametrize("code", [-6, -5, -4])
+def test_plan_failures(monkeypatch, code):
+    """Only a size without a plan declines the fused iteration; a plan that
+    could not be made is reported."""
+    from scico_amd._lib import ScxrError
+    from scico_amd.functional import IsotropicTVNorm
+    from scico_amd.linop import CircularConvolve
+    from scico_amd.loss import SquaredL2Loss
+
+    def plan(self):
+        raise ScxrError("scxr_cconv_plan_create", code, "")
+
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(_pgm, "load", lambda: types.SimpleNamespace(scxr_cconv_apgm_parts=int))
+    monkeypatch.setattr(CircularConvolve, "plan", property(plan))
+    A = object.__new__(CircularConvolve)
+    A.ndims, A.input_shape, A.fft_shape = 2, (4, 5), (4, 5)
+    f = object.__new__(SquaredL2Loss)
+    f.A, f.y, f.scale = A, torch.zeros(4, 5), 0.5
+    pgm = types.SimpleNamespace(f=f, g=IsotropicTVNorm(), x=torch.zeros(4, 5))
+    if code == -6:
+        assert _pgm._FusedDeconv.build(pgm) is None
+    else:
+        with pytest.raises(ScxrError) as e:
+            _pgm._FusedDeconv.build(pgm)
+        assert e.value.code == code
