@@ -412,11 +412,17 @@ __global__ __launch_bounds__(256) void fwd_slice16_kernel(
       }
       // the second pixel of its bin group? (lane before, within the row)
       const int prev = __builtin_amdgcn_update_dpp(-BIG, gi, 0x111, 0xf, 0xf, false);
+      // Lanes clear, file and read one another's entries: LDS executes a
+      // wave's accesses in order, the fences keep the compiler to it.
       ent[lane] = make_int4(0, 0, 0, 0);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_wave_barrier();
       if (gi >= -1 && gi < FBL)
         ent[lr * 16 + 2 * (gi + 1) + (gi == prev)] =
             make_int4(off, __float_as_int(wl), __float_as_int(wr), 1);
     }
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll 1
     for (int rr = 0; rr < min(4, nslow - r0); ++rr) {
       const int4 e = ent[rr * 16 + kk];
@@ -447,6 +453,8 @@ __global__ __launch_bounds__(256) void fwd_slice16_kernel(
       use(SCXR_X3_SLOT(12)); use(SCXR_X3_SLOT(13)); use(SCXR_X3_SLOT(14)); use(SCXR_X3_SLOT(15));
 #undef SCXR_X3_SLOT
     }
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_wave_barrier();
   }
   if (!qok) return;
 #pragma unroll
