@@ -109,7 +109,8 @@ int scxr_xr2d_weights(const scxr_xr2d_plan* plan, int32_t* inds, float* weights,
 
 /* FBP row filter (scico/linop/xray/_xray2d.py:158-221): out (A, Dout) =
  * rows of y (A, D) linearly convolved with taps (device, D), keeping
- * outputs [shift, shift + Dout) of the full convolution. D <= 4096. */
+ * outputs [shift, shift + Dout) of the full convolution. D <= 4096.  With
+ * Dout = D, out may be y. */
 int scxr_ramp_filter(int32_t A, int32_t D, int32_t Dout, int32_t shift, const float* taps,
                      const float* y, float* out, const int32_t* pred, void* stream);
 

@@ -1288,6 +1288,24 @@ __global__ __launch_bounds__(256 * ADJ_VS) __attribute__((amdgpu_waves_per_eu(4)
 // against one row per workgroup with two LDS reads per multiply-add.
 // The matrix products include the zeros beyond the taps, so a tile with an
 // input that is not finite takes the plain sums, which leave them out.
+//
+// An output that overlaps the input (a row may be filtered in place) takes a
+// workgroup per row, which reads all of it before it writes.
+__global__ __launch_bounds__(256) void ramp_row_kernel(const float* y, float* out,
+                                                       const float* __restrict__ taps, int D,
+                                                       int Dout, int s, const int32_t* pred) {
+  if (pred_off(pred)) return;
+  __shared__ float row[4096];
+  for (int k = threadIdx.x; k < D; k += 256) row[k] = y[static_cast<size_t>(blockIdx.x) * D + k];
+  __syncthreads();
+  for (int t = threadIdx.x; t < Dout; t += 256) {
+    const int c = t + s;
+    float v = 0.0f;
+    for (int m = max(0, c - D + 1); m <= min(D - 1, c); ++m) v = fmaf(taps[m], row[c - m], v);
+    out[static_cast<size_t>(blockIdx.x) * Dout + t] = v;
+  }
+}
+
 constexpr int RAMP_K = 256, RAMP_T = 64, RAMP_A = 16;
 
 __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
@@ -1837,6 +1855,12 @@ int scxr_ramp_filter(int32_t A, int32_t D, int32_t Dout, int32_t shift, const fl
                      const float* y, float* out, const int32_t* pred, void* stream) {
   SCXR_REQUIRE(A > 0 && D > 0 && D <= 4096 && Dout > 0 && taps && y && out, SCXR_ERR_ARG,
                "bad ramp_filter arguments (D must be in [1, 4096])");
+  if (y < out + static_cast<size_t>(A) * Dout && out < y + static_cast<size_t>(A) * D) {
+    hipLaunchKernelGGL(ramp_row_kernel, dim3(A), dim3(256), 0, as_stream(stream), y, out, taps, D,
+                       Dout, shift, pred);
+    SCXR_LAUNCHED("ramp filter in place");
+    return SCXR_OK;
+  }
   hipLaunchKernelGGL(ramp_kernel, dim3(ceil_div(Dout, RAMP_T), ceil_div(A, RAMP_A)), dim3(256), 0,
                      as_stream(stream), y, out, taps, A, D, Dout, shift, pred);
   SCXR_LAUNCHED("ramp filter");

@@ -396,3 +396,26 @@ def test_adjoint_mul_epilogue(gpu, shape, views, det):
          torch.cuda.current_stream().cuda_stream)
     ref = vec.scale_mul(0.37, w, H.back_project(y))
     assert torch.equal(out.view(torch.int32), ref.view(torch.int32))
+
+
+@pytest.mark.parametrize("A,D", [(1, 1), (17, 63), (300, 1001), (3, 4096)])
+def test_ramp_filter_in_place(gpu, A, D):
+    """Rows filtered in place: float64 convolution, bar as above."""
+    from scico_amd._lib import call
+
+    rng = np.random.default_rng(A * 10000 + D)
+    s = (D - 1) // 2
+    h, y = rng.standard_normal(D).astype(np.float32), rng.standard_normal((A, D)).astype(np.float32)
+    hd, yd = torch.as_tensor(h, device="cuda"), torch.as_tensor(y, device="cuda")
+    call("scxr_ramp_filter", A, D, D, s, hd.data_ptr(), yd.data_ptr(), yd.data_ptr(), None,
+         torch.cuda.current_stream().cuda_stream)
+    h64, y64 = h.astype(np.float64), y.astype(np.float64)
+
+    def full(rows, taps):
+        return np.stack([np.convolve(r, taps)[s : s + D] for r in rows])
+
+    ref = np.zeros((A, D))
+    ref[:, : min(D, 2 * D - 1 - s)] = full(y64, h64)
+    bar = np.zeros((A, D))
+    bar[:, : min(D, 2 * D - 1 - s)] = D * 2.0**-24 * full(np.abs(y64), np.abs(h64))
+    assert np.all(np.abs(yd.cpu().numpy() - ref) <= bar + 1e-30)
