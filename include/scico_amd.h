@@ -529,8 +529,9 @@ int scxr_batch_admm_itstat(const scxr_xr2d_batch* plan, const double* res, const
  * keeps the slice adjoint that reads the detector rows from global memory
  * instead of staging them in LDS (the two give bitwise-equal results; the
  * staged one is faster); bit 2 set keeps the general-mode gathers from
- * global memory instead of the kernels with windows in LDS (equal up to
- * float32 rounding; the latter are faster).  Pass 1 for the default.
+ * global memory instead of the kernels with windows in LDS, bit 3 the latter
+ * also where the volume and the views are few (equal up to float32 rounding;
+ * with neither the faster one is taken).  Pass 1 for the default.
  */
 typedef struct scxr_xr3d_plan scxr_xr3d_plan;
 

@@ -1416,6 +1416,28 @@ static int dev_alloc(void** ptr, size_t bytes) {
   return SCXR_OK;
 }
 
+// Where the windows in LDS are the faster path (all figures of graph replays;
+// a flag forces either).  The forward takes three launches and a workspace:
+// its time meets the gather's at about 280000 voxels times views (16^3 with
+// 60 views 20.9 against 21.1 us, 32^3 with 8 19.8 against 20.2, 64^3 with one
+// 23.7 against 23.5; 16^3 with 10 17.1 against 10.7, 32^3 with 20 27 against
+// 20.6 us).
+static bool splat_pays(const Plan& p) {
+  return static_cast<double>(p.X) * p.Y * p.Z * p.V >= 280e3;
+}
+
+// The adjoint's waves walk their views one after the other, and with fewer
+// than 32 views a block has two of them: below some work that chain is longer
+// than the gather's (16^3 with 30 views 16.0 against 10.4 us, 32^3 with 31 17.0
+// against 10.3; 40^3 with 31 17.1 against 16.5, 48^3 with 31 17.1 against 17.6,
+// 64^3 with 5 7.2 against 8.1 us; from 32 views on 8^3 takes 9.6 against 10.7
+// us).  With a single view half the waves have none, at any size (256^3 87.6
+// against 68.1 us).
+static bool adj_tiles_pay(const Plan& p) {
+  const double work = static_cast<double>(p.X) * p.Y * p.Z * p.V;
+  return p.V >= 32 || (p.V > 1 && work >= 1.2e6 + 3e4 * p.V);
+}
+
 // Detector coordinates of every voxel centre stay below this (float32
 // rounding of P far below the window margins, window offsets within int32).
 constexpr double GEN_PMAX = 8192.0;
@@ -1729,8 +1751,9 @@ int create(Plan& p, int X, int Y, int Z, int V, const float* mats, int D0, int D
     std::vector<SplatItem> items;
     std::vector<float> zt;
     if (!(allow_slice & 4) && gen_in_range(p, m)) {
-      p.splat = build_splat(p, m, gv, views, items);
-      p.adj_tiled = build_adj_tiles(p, m, zt);
+      const bool always = allow_slice & 8;
+      p.splat = (always || splat_pays(p)) && build_splat(p, m, gv, views, items);
+      p.adj_tiled = (always || adj_tiles_pay(p)) && build_adj_tiles(p, m, zt);
     }
     return upload_tables(p, m, gv, views, items, zt);
   }

@@ -79,7 +79,8 @@ class XRayTransform3D(LinearOperator):
                 self.matrices.ctypes.data_as(ctypes.POINTER(ctypes.c_float)),
                 self.det_shape[0], self.det_shape[1],
                 int(self._allow_slice) | (0 if self._stage_adjoint else 2) |
-                (0 if self._windows else 4), ctypes.byref(h),
+                (4 if not self._windows else 8 if self._windows == "always" else 0),
+                ctypes.byref(h),
             )
             self._plan = h
             self._ws_floats = int(lib.scxr_xr3d_forward_ws(h))

@@ -294,3 +294,33 @@ def test_slice_strips(gpu, shape, views, scale, shift):
     eps = 2.0**-24
     assert np.all(np.abs(fwd - ref[0, :, 1:-1]) <= eps * (ref[2] * ref[1])[:, 1:-1] + 1e-30)
     assert np.all(np.abs(adj - back[0]) <= eps * 2 * views * back[1] + 1e-30)
+
+
+@pytest.mark.parametrize("case", list(WINDOW_CASES))
+def test_general_windows_small(gpu, case):
+    """The kernels with windows in LDS on volumes so small that the gathers
+    are the default: against the gathers (bar as in test_general_windows)."""
+    shape, det, mk = WINDOW_CASES[case]
+    M = mk(shape, det)
+    H, G = XRayTransform3D(shape, M, det), XRayTransform3D(shape, M, det)
+    H._windows, G._windows = "always", False
+    rng = np.random.default_rng(12)
+    x = torch.as_tensor(rng.random(shape).astype(np.float32), device="cuda")
+    y = torch.as_tensor(rng.standard_normal(H.output_shape).astype(np.float32), device="cuda")
+    e = rel_l2(H(x).cpu(), G(x).cpu()), rel_l2(H.adj(y).cpu(), G.adj(y).cpu())
+    assert max(e) <= 1e-5 and H._ws_floats > 0 and G._ws_floats == 0
+
+
+@pytest.mark.parametrize("n,views,splat", [(16, 1, False), (23, 23, False), (23, 24, True),
+                                           (64, 1, False), (66, 1, True), (66, 40, True)])
+def test_general_windows_rule(gpu, n, views, splat):
+    """The default takes the forward's windows from 280000 voxels times views
+    on, and is the path that it takes, bit for bit."""
+    shape, det = (n, n, n), (n + 8, n)
+    M = _tilted(shape, det, "XY", views)
+    H = XRayTransform3D(shape, M, det)
+    W = XRayTransform3D(shape, M, det)
+    H._allow_slice = W._allow_slice = False
+    W._windows = "always" if splat else False
+    x = torch.as_tensor(np.random.default_rng(5).random(shape).astype(np.float32), device="cuda")
+    assert torch.equal(H(x), W(x)) and (H._ws_floats > 0) == splat
