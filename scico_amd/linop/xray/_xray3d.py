@@ -17,6 +17,7 @@ import ctypes
 import weakref
 
 import numpy as np
+import torch
 
 from ... import _device as dev
 from ... import _pred
@@ -102,8 +103,14 @@ class XRayTransform3D(LinearOperator):
         out = dev.output_buffer(out, self.output_shape)
         plan = self.plan
         # general mode: detector windows, from the caching allocator so that
-        # calls on several streams (and captured ones) have their own
-        ws = dev.empty((self._ws_floats,)) if self._ws_floats else None
+        # calls on several streams (and captured ones) have their own; without
+        # memory for them the gather, which needs none
+        try:
+            ws = dev.empty((self._ws_floats,)) if self._ws_floats else None
+        except torch.OutOfMemoryError:
+            call("scxr_xr3d_forward", plan, im.data_ptr(), out.data_ptr(),
+                 dev.ptr(_pred.resolve(pred)), dev.stream())
+            return out
         call("scxr_xr3d_forward_with", plan, im.data_ptr(), out.data_ptr(), dev.ptr(ws),
              dev.ptr(_pred.resolve(pred)), dev.stream())
         return out

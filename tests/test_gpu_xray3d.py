@@ -324,3 +324,21 @@ def test_general_windows_rule(gpu, n, views, splat):
     W._windows = "always" if splat else False
     x = torch.as_tensor(np.random.default_rng(5).random(shape).astype(np.float32), device="cuda")
     assert torch.equal(H(x), W(x)) and (H._ws_floats > 0) == splat
+
+
+def test_general_forward_without_memory(gpu, monkeypatch):
+    """No memory for the windows: the forward is the gather's, bit for bit."""
+    from scico_amd.linop.xray import _xray3d
+
+    shape, det, mk = WINDOW_CASES["any"]
+    H, G = (XRayTransform3D(shape, mk(shape, det), det) for _ in range(2))
+    G._windows = False
+    x = torch.as_tensor(np.random.default_rng(6).random(shape).astype(np.float32), device="cuda")
+    ref, out = G(x), torch.empty(H.output_shape, device="cuda")
+    assert H.plan and H._ws_floats > 0
+
+    def empty(shape, dtype=np.float32):
+        raise torch.OutOfMemoryError("no memory")
+
+    monkeypatch.setattr(_xray3d.dev, "empty", empty)
+    assert torch.equal(H.project(x, out=out), ref)
