@@ -442,8 +442,11 @@ __device__ __forceinline__ const float2* pass_twiddles(float2* X, int tot, int n
   return X + tot;
 }
 
+// At least four waves per SIMD: with 131 registers, above the 128 that allow
+// them, 1000 and 4000 lines of 2048 took 34.5 and 107 us against 26.5 and 92.
 template <bool MIXED, int MAXV>
-__global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __restrict__ in,
+__global__ __launch_bounds__(SH_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void
+stockham_kernel(const void* __restrict__ in,
                                                               void* __restrict__ out, Pass P,
                                                               Stages S, float scale,
                                                               const int32_t* pred) {
@@ -539,7 +542,8 @@ __global__ __launch_bounds__(SH_THREADS) void stockham_kernel(const void* __rest
         if (threadIdx.x + q * SH_THREADS < tot)
           times(threadIdx.x + q * SH_THREADS, hv[q]);
     } else {
-      for (int e = threadIdx.x; e < tot; e += SH_THREADS) times(e, spectrum(e));
+      for (int e = threadIdx.x; e < tot; e += SH_THREADS)
+        if (e / n < nl) times(e, spectrum(e));
     }
     __syncthreads();
     transform<MIXED, MAXV>(X, n, P.log2n, S, lpb, twl, true);
