@@ -219,7 +219,9 @@ class _UnrolledAPGMTV(torch.autograd.Function):
         ybar = torch.zeros_like(y)
         wbar = torch.zeros_like(w)
         gw = torch.empty_like(w)
-        us = ctx.us
+        # the kept inputs go as they are used (a second backward computes them
+        # again), so that no other segment's are held beside them
+        us, ctx.us = ctx.us, None
         for s in reversed(sorted(ctx.ckpts)):
             end = min(s + every, K)
             if us is None:
@@ -231,7 +233,7 @@ class _UnrolledAPGMTV(torch.autograd.Function):
                     if k + 1 < end:
                         x, v = _prox_step(us[-1], x, w, L, lam, cs[k], iso)
             for k in reversed(range(s, end)):
-                u = us[k - s]
+                u = us.pop()
                 # v_{k+1} = x_{k+1} + c_k (x_{k+1} - x_k)
                 xk1 = vec.axpby(1.0, xbar, 1.0 + cs[k], vbar)
                 xk_part = vec.scale(-cs[k], vbar)

@@ -238,3 +238,32 @@ def test_unrolled_gradient_central_fd_512(gpu):
     print(f"  512^2 unrolled grad vs central FD: median rel err {np.median(errs):.2e}, "
           f"90th pct {np.percentile(errs, 90):.2e}", flush=True)
     assert np.median(errs) <= 1e-2 and np.percentile(errs, 90) <= 5e-2
+
+
+def test_unrolled_backward_memory(gpu):
+    """The backward holds the prox inputs of one segment at a time: those of
+    the last are held before it and go as it uses them, so its peak over what
+    is held is a segment's inputs (one of them may still be in use) below that
+    of a second backward, which computes them all again to the same
+    gradients."""
+    n, K, every = 256, 20, 5
+    H = XRayTransform2D((n, n), np.linspace(0, np.pi, 30, endpoint=False))
+    rng = np.random.default_rng(7)
+    y = dev(rng.standard_normal(H.output_shape).astype(np.float32)).requires_grad_()
+    w = dev(rng.random((n, n)).astype(np.float32)).requires_grad_()
+    img = n * n * 4
+    x = AG.unrolled_apgm_tv(H, y, w, 4000.0, 2.0, K=K, checkpoint_every=every)
+    g = torch.ones_like(x)
+
+    def grads():
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        held = torch.cuda.memory_allocated()
+        out = torch.autograd.grad(x, (y, w), g, retain_graph=True)
+        return out, (torch.cuda.max_memory_allocated() - held) / img
+
+    first, peak1 = grads()
+    second, peak2 = grads()  # nothing kept any more: every segment computed again
+    print(f"  unrolled backward: {peak1:.1f} images over those held, {peak2:.1f} again", flush=True)
+    assert all(torch.equal(a, b) for a, b in zip(first, second))
+    assert peak1 <= peak2 - (every - 1)
