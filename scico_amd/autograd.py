@@ -183,22 +183,22 @@ def _prox_step(u, x_old, w, L, lam, c, iso):
 
 class _UnrolledAPGMTV(torch.autograd.Function):
     # The backward runs over segments of `every` steps.  The forward keeps
-    # (x, v) at the start of each, and the prox inputs of the last one, which
-    # the backward needs first (the others' it computes again: as many images,
-    # one segment at a time).
+    # (x, v) at the start of each, and with keep_last the prox inputs of the
+    # last one, which the backward needs first (the others' it computes again:
+    # as many images, one segment at a time).
     @staticmethod
-    def forward(ctx, y, w, x0, H, L, lam, K, every, iso):
+    def forward(ctx, y, w, x0, H, L, lam, K, every, iso, keep_last):
         y, w = y.detach().contiguous(), w.detach().contiguous()
         cs = _momentum(K)
         x = v = x0.detach().contiguous().clone()
-        ckpts, us = {}, []
+        ckpts, us = {}, None
         keep = any(ctx.needs_input_grad)
         for k in range(K):
             if k % every == 0 and keep:
                 ckpts[k] = (x, v)
-                us = []
+                us = [] if keep_last else None
             u = _prox_input(H, y, v, L)
-            if keep:
+            if us is not None:
                 us.append(u)
             if k + 1 < K:
                 x, v = _prox_step(u, x, w, L, lam, cs[k], iso)
@@ -246,16 +246,22 @@ class _UnrolledAPGMTV(torch.autograd.Function):
                 vbar = vec.axpby(1.0, ubar, -gam, H.back_project(Au))
                 xbar = xk_part
             us = None
-        return ybar, wbar, None, None, None, None, None, None, None
+        return ybar, wbar, None, None, None, None, None, None, None, None
 
 
 def unrolled_apgm_tv(H, y, w, L: float, lam: float, K: int = 20, checkpoint_every: int = 5,
-                     x0=None, isotropic: bool = True):
+                     x0=None, isotropic: bool = True, keep_last: bool = True):
     """``x_K`` of ``K`` AcceleratedPGM steps on
     ``0.5 ||H x - y||^2 + lam * sum_p w[p] |grad x|_p`` (Haar TV prox),
     step ``1/L``, from ``x0`` (zeros by default).  Differentiable with
-    respect to ``y`` and ``w`` (torch autograd)."""
+    respect to ``y`` and ``w`` (torch autograd).
+
+    Between forward and backward two images are held for every
+    ``checkpoint_every`` steps, and up to ``checkpoint_every`` more so that the
+    backward need not compute the last of those segments again.  With many
+    reconstructions before one backward pass, ``keep_last=False`` leaves the
+    latter out; the gradients are the same."""
     if x0 is None:
         x0 = torch.zeros(H.input_shape, dtype=torch.float32, device=dev.DEVICE)
     return _UnrolledAPGMTV.apply(y, w, x0, H, float(L), float(lam), int(K),
-                                 int(checkpoint_every), bool(isotropic))
+                                 int(checkpoint_every), bool(isotropic), bool(keep_last))

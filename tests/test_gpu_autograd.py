@@ -267,3 +267,26 @@ def test_unrolled_backward_memory(gpu):
     print(f"  unrolled backward: {peak1:.1f} images over those held, {peak2:.1f} again", flush=True)
     assert all(torch.equal(a, b) for a, b in zip(first, second))
     assert peak1 <= peak2 - (every - 1)
+
+
+@pytest.mark.parametrize("K,every", [(3, 5), (5, 5), (7, 3), (8, 1)])
+def test_unrolled_keep_last(gpu, K, every):
+    """keep_last=False holds nothing between the passes but the result and two
+    images for every segment; the same result and gradients, bit for bit."""
+    n = 256
+    H = XRayTransform2D((n, n), np.linspace(0, np.pi, 30, endpoint=False))
+    rng = np.random.default_rng(8)
+    y = dev(rng.standard_normal(H.output_shape).astype(np.float32)).requires_grad_()
+    w = dev(rng.random((n, n)).astype(np.float32)).requires_grad_()
+    H(w.detach())
+    got = []
+    for keep in (True, False):
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        x = AG.unrolled_apgm_tv(H, y, w, 4000.0, 2.0, K=K, checkpoint_every=every, keep_last=keep)
+        held = (torch.cuda.memory_allocated() - before) / (n * n * 4)
+        got.append((x.detach().clone(), *torch.autograd.grad(x.square().sum(), (y, w))))
+        if not keep:
+            assert held <= 1 + 2 * -(-K // every)
+        del x
+    assert all(torch.equal(a, b) for a, b in zip(*got))
