@@ -799,7 +799,9 @@ __device__ __forceinline__ void fwd_body_staged(float* acc, const float* share, 
 #pragma unroll
   for (int r = 0; r < S; ++r) flr[r] = static_cast<float>(loff + r);
   const float* col = share + wave * pitch;
-  for (int base = K * static_cast<int>(blockIdx.y); base < N;
+  // (a wave without a column in the last set has nothing to add there: 88 x 97
+  // with 300 views, whose seventh set holds one column, 12.0 -> 11.2 us)
+  for (int base = K * static_cast<int>(blockIdx.y); base + wave < N;
        base += K * static_cast<int>(gridDim.y), col += K * pitch) {
     float t[CH][1];
 #pragma unroll
