@@ -1639,14 +1639,20 @@ int forward(const Plan& p, const float* im, float* sino, const int32_t* pred, hi
   // Column-fast views stream the transposed image (the caller's, or the
   // plan's workspace filled here) or stage their columns of the image itself:
   // where rows and share take at most 64 KiB (128^2 unsplit takes 78: 12.5 us
-  // staged, 11.5 transposed; 100 x 80 takes 50: 8.8 against 9.4) and every
-  // workgroup of the launch finds room on a CU at once (256^2 in 8 parts with
-  // 45 views 10.2 -> 9.7 us, but with 180 views, three turns, 16 -> 21 us).
+  // staged, 11.5 transposed; 100 x 80 takes 50: 8.8 against 9.4) and the CUs'
+  // LDS has room for every workgroup of the launch at once (256^2 in 8 parts
+  // with 45 views 10.2 -> 9.7 us, but with 180 views, three turns, 16 -> 21 us;
+  // 88 x 97 with 700 views, two of 54 KiB on a CU, 16.5 -> 17.2).  Small shares
+  // have room for more than the four workgroups that a CU's 32 waves allow: the
+  // launch then takes turns, and staging is the faster path all the same (64^2
+  // with 200 views in 8 parts 8.0 against 10.3 us, 100^2 in 6 10.2 against 12.0).
   const size_t rows_lds = fwd_lds_bytes(p.vpg, p.D, p.fwd_ch);
   const size_t share = fwd_share_bytes(p.fwd_ch, p.N, p.fwd_sp, p.fwd_pitch);
+  const size_t room = (rows_lds + share + FWD_LDS_STATIC + LDS_GRANULE - 1) / LDS_GRANULE *
+                      LDS_GRANULE;
   const bool stage = !imT && p.fwd_pitch > 0 && rows_lds + share <= FWD_LDS_MAX &&
                      static_cast<size_t>(p.n_groups) * p.fwd_sp <=
-                         p.cus * (LDS_PER_CU / (rows_lds + share));
+                         p.cus * (LDS_PER_CU / room);
   const float* srcT = imT ? imT : p.work;
   if (p.any_colfast && !imT && !stage) {
     dim3 g(ceil_div(p.N, 32), ceil_div(p.M, 32));

@@ -25,6 +25,8 @@ constexpr int FWD_WAVES = 8;
 constexpr int FWD_SP_MAX = 8;  // most workgroups one forward group's lines are split over
 constexpr size_t FWD_LDS_MAX = 64 * 1024;
 constexpr size_t LDS_PER_CU = 160 * 1024;
+constexpr size_t LDS_GRANULE = 1280;     // LDS is given out in units of this
+constexpr size_t FWD_LDS_STATIC = 256;   // at most, beside the rows and the staged share
 constexpr int FWD_SMAX = 64;  // largest lane stride of the forward projector
 inline size_t fwd_lds_bytes(int vpg, int D, int ch) {
   return sizeof(float) * static_cast<size_t>(vpg) * FWD_WAVES * ch *
