@@ -103,10 +103,10 @@ __device__ __forceinline__ double fma_(double a, double b, double c) { return fm
 // and runs the inverse stages on the same buffer.
 constexpr int SH_THREADS = 256;
 // Values per thread and stage: 4 for workgroups of at most 1024 values, else 32
-// (lpb n <= 8192).  The kernels unroll over them for every radix, and at 32
-// the mixed-radix column pass is 160 KB of code, which does not stay in the
-// instruction cache (convolution of 3 x 360 x 480: 39 -> 25 us, 512 x 512: 27 ->
-// 22 us).
+// (lpb n <= 8192; powers of two).  The kernels unroll over them for every
+// radix, and at 32 the mixed-radix column pass was 160 KB of code, which does
+// not stay in the instruction cache (convolution of 3 x 360 x 480: 39 -> 25 us,
+// 512 x 512: 27 -> 22 us).
 constexpr int SH_MAXV = 32, SH_FEW = 4;
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) {
@@ -1201,8 +1201,9 @@ struct Plan {
   AxisTables ax[3];
   float2* h = nullptr;     // spectrum (fsize)
   float2* work = nullptr;  // complex workspace (batch * fsize)
-  // real 2D path (two axes of 3 or more): Hermitian part of the spectrum on the half grid (F0, F1/2 + 1) and lines per workgroup of the
-  // row and column passes
+  // real 2D path (two axes of 3 or more): Hermitian part of the spectrum on
+  // the half grid (F0, F1/2 + 1) and lines per workgroup of the row and column
+  // passes
   bool r2c = false;
   float2* hs = nullptr;
   int lpb_rows = 1, lpb_cols = 1;
@@ -1259,19 +1260,26 @@ size_t pass_lds(const AxisTables& t, int lpb) {
 
 // Lines that a workgroup may take: 1024 values, the instances of four values
 // a thread (8 x 512 x 512 convolution, 4 lines against 2: 53.7 against 48.2
-// us, 8 x 450 x 480 64.3 against 41.3 us); lines longer than that 8192 (7168
-// beside the twiddles of p-term sums).
+// us, 8 x 450 x 480 64.3 against 41.3 us); lines longer than that (powers of
+// two) 8192.
 int line_cap(const AxisTables& t) {
-  const int values = t.n <= SH_FEW * SH_THREADS ? SH_FEW * SH_THREADS
-                                                : (t.log2n >= 0 ? 8192 : 7168);
+  const int values = t.n <= SH_FEW * SH_THREADS ? SH_FEW * SH_THREADS : 8192;
   return std::max(1, values / t.n);
 }
 
-// The instance of a pass's kernel for lpb lines of t (see SH_MAXV).
-#define SCXR_FFT_KERNEL(K, t, lpb, ...)                                          \
-  (static_cast<long long>(lpb) * (t).n <= SH_FEW * SH_THREADS                    \
-       ? ((t).log2n < 0 ? &K<true, SH_FEW, ##__VA_ARGS__> : &K<false, SH_FEW, ##__VA_ARGS__>) \
-       : ((t).log2n < 0 ? &K<true, SH_MAXV, ##__VA_ARGS__> : &K<false, SH_MAXV, ##__VA_ARGS__>))
+// Whether a pass of l lines of t has an instance that holds them.
+bool lines_fit(const AxisTables& t, int l) {
+  const int most = t.log2n < 0 ? SH_FEW * SH_THREADS : SH_MAXV * SH_THREADS;
+  return l >= 1 && l <= 64 && static_cast<long long>(l) * t.n <= most;
+}
+
+// The instance of a pass's kernel for lpb lines of t (see SH_MAXV); mixed
+// lengths never take more than 1024 values.
+#define SCXR_FFT_KERNEL(K, t, lpb, ...)                            \
+  ((t).log2n < 0 ? &K<true, SH_FEW, ##__VA_ARGS__>                 \
+   : static_cast<long long>(lpb) * (t).n <= SH_FEW * SH_THREADS    \
+       ? &K<false, SH_FEW, ##__VA_ARGS__>                          \
+       : &K<false, SH_MAXV, ##__VA_ARGS__>)
 
 int make_tables(AxisTables& t, int n) {
   t.n = n;
@@ -1480,8 +1488,8 @@ int scxr_cconv_plan_create(int32_t ndim, const int32_t* fshape, int64_t batch,
     p.lpb_cols = pick(p.batch * H1, p.ax[0]);
     if (const char* env = std::getenv("SCXR_FFT_LPB")) {
       int a = 0, b = 0;
-      if (std::sscanf(env, "%d,%d", &a, &b) == 2 && a >= 1 && b >= 1 && a <= 64 && b <= 64 &&
-          pass_lds(p.ax[1], a) <= 65536 && pass_lds(p.ax[0], b) <= 65536) {
+      if (std::sscanf(env, "%d,%d", &a, &b) == 2 && lines_fit(p.ax[1], a) &&
+          lines_fit(p.ax[0], b)) {
         p.lpb_rows = a;
         p.lpb_cols = b;
       }

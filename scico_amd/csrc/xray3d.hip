@@ -207,7 +207,8 @@ __device__ __forceinline__ void slice_block(int& bg, int& vg) {
 // centres are at least |f| apart along the fast axis), so the whole row is
 // straight-line code apart from wave-uniform branches: every occupied
 // slot's row of slices is loaded independently and accumulated into
-// static registers.
+// static registers.  For spacings below 0.67 (32 or 64 candidates a row); the
+// others take fwd_slice16_kernel.
 template <int CPR, int SPG>
 __global__ __launch_bounds__(256) void fwd_slice_kernel(const float4* __restrict__ vol,
                                                         float4* __restrict__ proj,
@@ -274,14 +275,8 @@ __global__ __launch_bounds__(256) void fwd_slice_kernel(const float4* __restrict
 #pragma unroll
       for (int gg = -1; gg <= FB; ++gg) {
         const unsigned long long bal = __ballot(gi < gg);
-        int cnt;
-        if (CPR == 64) {
-          cnt = __popcll(bal);
-        } else {
-          const unsigned part = static_cast<unsigned>(bal >> (rr * CPR)) &
-                                (CPR == 32 ? 0xffffffffu : ((1u << CPR) - 1u));
-          cnt = __popc(part);
-        }
+        const int cnt =
+            CPR == 64 ? __popcll(bal) : __popc(static_cast<unsigned>(bal >> (rr * CPR)));
         first[gg + 1] = base + cnt;
       }
       // Groups in chunks of GC: the loads of a chunk's occupied slots are
@@ -1361,7 +1356,7 @@ static bool try_slice(Plan& p, const std::vector<float>& m, int sax, int dax) {
   if (!(fmin > 0.0f)) return false;
   const double need = std::ceil((FB + 1) / static_cast<double>(fmin)) + 6.0;
   if (need > 64.0) return false;
-  p.cpr = need <= 16.0 ? 16 : (need <= 32.0 ? 32 : 64);
+  p.cpr = need <= 32.0 ? 32 : 64;
   // pixels of one bin group (left in [g, g + 1)) along the fast axis
   const double spg = std::ceil(1.0 / static_cast<double>(fmin) + 0.01);
   if (spg > 3.0) return false;
@@ -1369,6 +1364,7 @@ static bool try_slice(Plan& p, const std::vector<float>& m, int sax, int dax) {
   // 16 candidates hold a strip of FBL + 1 bins, rounded outwards and widened
   // by a pixel each side
   p.slot16 = (FBL + 1) / static_cast<double>(fmin) < 11.99;
+  if (p.slot16) p.cpr = 16;
   p.mode = MODE_SLICE;
   p.sax = sax;
   p.dax = dax;
@@ -1939,21 +1935,13 @@ int forward(const Plan& p, const float* vol, float* proj, float* ws, const int32
 #define SCXR_FWD3(C, G)                                                                       \
   hipLaunchKernelGGL((fwd_slice_kernel<C, G>), grid, dim3(256), 0, s, v4, y4, p.geom, p.P, p.Q, \
                      p.SQ, p.U, p.V, pred)
-  if (p.spg == 2) {
-    if (p.cpr == 16)
-      SCXR_FWD3(16, 2);
-    else if (p.cpr == 32)
-      SCXR_FWD3(32, 2);
-    else
-      SCXR_FWD3(64, 2);
-  } else {
-    if (p.cpr == 16)
-      SCXR_FWD3(16, 3);
-    else if (p.cpr == 32)
-      SCXR_FWD3(32, 3);
-    else
-      SCXR_FWD3(64, 3);
-  }
+  // (two slots: spacings of 0.5 to 0.67, at most 24 candidates)
+  if (p.spg == 2)
+    SCXR_FWD3(32, 2);
+  else if (p.cpr == 32)
+    SCXR_FWD3(32, 3);
+  else
+    SCXR_FWD3(64, 3);
 #undef SCXR_FWD3
   SCXR_LAUNCHED("xr3d slice forward");
   if (!p.proj_direct) return canon_to_proj(p, yc, proj, pred, s);
