@@ -372,19 +372,30 @@ __device__ __forceinline__ void prime_stage(V* X, int n, int lpb, int R, int Ns,
       int l, s, g, k;
       where(e, l, s, g, k);
       const V* x = X + l * n + g * Ns + k;
-      int step = k * tstep + s * nb, idx = 0;
-      if (step >= n) step -= n;
-      Real<V> re = 0, im = 0;
-      for (int r = 0; r < R; ++r) {
-        V w = tw[idx];
-        if (inv) w = conjf2(w);
-        const V p = cmul(x[r * nb], w);
-        re = re + p.x;
-        im = im + p.y;
-        idx += step;
-        if (idx >= n) idx -= n;
+      int step = k * tstep + s * nb, idx = step;
+      if (step >= n) idx = step -= n;
+      // Term 0 has weight 1.  The R - 1 others (an even number) are added in two
+      // halves, and each half's four kinds of product apart, with one rounding
+      // per product and sum.  One chain of rounded products left the convolution
+      // on half spectra, whose rows come in pairs, further off than sums over
+      // the full spectrum: 509 x 503 8.2e-7 against 7.4e-7 of the result, 5.8e-7
+      // with these.
+      Real<V> xx[2] = {x[0].x, 0}, yy[2] = {0, 0}, xy[2] = {0, 0}, yx[2] = {x[0].y, 0};
+      for (int r = 1; r < R; r += 2) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          V w = tw[idx];
+          if (inv) w = conjf2(w);
+          const V a = x[(r + h) * nb];
+          xx[h] = fma_(a.x, w.x, xx[h]);
+          yy[h] = fma_(a.y, w.y, yy[h]);
+          xy[h] = fma_(a.x, w.y, xy[h]);
+          yx[h] = fma_(a.y, w.x, yx[h]);
+          idx += step;
+          if (idx >= n) idx -= n;
+        }
       }
-      o[q] = cmake<V>(re, im);
+      o[q] = cmake<V>((xx[0] + xx[1]) - (yy[0] + yy[1]), (xy[0] + xy[1]) + (yx[0] + yx[1]));
     }
   }
   __syncthreads();

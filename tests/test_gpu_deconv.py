@@ -691,3 +691,21 @@ def test_fused_apgm_inference_mode(gpu, shape):
             got = run(A, y)
             assert torch.equal(got[0], ref[0]) and torch.equal(got[1], ref[1])
             assert got[2] == ref[2]
+
+
+@pytest.mark.parametrize("shape,bar", [((127, 131), 3.9e-7), ((257, 251), 5.3e-7),
+                                       ((512, 509), 5.6e-7), ((509, 503), 7.4e-7)])
+def test_circconv_prime_sizes_error(gpu, shape, bar):
+    """Lengths with large prime factors: the convolution on half spectra is no
+    further from float64 (rel-L2) than the measured error of sums over all n
+    inputs on the full spectrum, the bar."""
+    rng = np.random.default_rng(0)
+    h = rng.standard_normal((3, 3)).astype(np.float32)
+    x = rng.standard_normal(shape).astype(np.float32)
+    A = CircularConvolve(h, shape)
+    H = np.fft.fft2(h.astype(np.float64), s=shape)
+    X = np.fft.fft2(x.astype(np.float64))
+    for got, hd in ((A(dev(x)), H), (A.adj(dev(x)), H.conj())):
+        e = rel_l2(got.cpu(), np.fft.ifft2(hd * X).real)
+        print(f"  circconv {shape}: rel-L2 vs float64 {e:.2e}", flush=True)
+        assert e <= bar
