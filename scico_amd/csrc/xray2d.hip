@@ -1282,12 +1282,17 @@ __global__ __launch_bounds__(256 * ADJ_VS) __attribute__((amdgpu_waves_per_eu(4)
 // with the ramp taps h[0..D) by zero-padded FFT of length 2D - 1 and keeps
 // [s, 2D - 1 - s), s = (D - 1) / 2; here the same linear convolution is
 // summed directly: out[a, t] = sum_k y[a, k] h[t + s - k], a product of the
-// rows with the Toeplitz matrix of the taps, on the float32 matrix cores.
+// rows with the Toeplitz matrix of the taps, on the float64 matrix cores.
 // A workgroup takes 16 rows x 64 outputs (16 x 16 per wave) and walks the
 // inputs that reach them in chunks of 256 through LDS, four per MFMA; two
-// accumulators take alternate steps.  Bound by the latency of one or two
-// waves per SIMD (a sinogram has few rows); 301 rows of 595: 54 -> 9.9 us
-// against one row per workgroup with two LDS reads per multiply-add.
+// accumulators take alternate steps.  Bound by the matrix cores and the
+// latency of one or two waves per SIMD (a sinogram has few rows); 301 rows of
+// 595: 53.0 -> 12.8 us, 720 of 724 68.5 -> 23.5 us against one row per workgroup
+// with two LDS reads per multiply-add.  In float32 the products take 9.2 and
+// 14.7 us, but the ramp's centre tap cancels against all others on a smooth
+// row, and their order, unlike the plain one, carries the large partial sums
+// through the chain: 1.6e-5 off float64 for smooth rows of 595, the plain sums
+// 2.1e-6, these 2.5e-8 (the rounding of the result).
 // The matrix products include the zeros beyond the taps, so a tile with an
 // input that is not finite takes the plain sums, which leave them out.
 //
@@ -1315,7 +1320,7 @@ __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
                                                    const float* __restrict__ taps, int A, int D,
                                                    int Dout, int s, const int32_t* pred) {
   if (pred_off(pred)) return;
-  typedef float f4 __attribute__((ext_vector_type(4)));
+  typedef double d4 __attribute__((ext_vector_type(4)));
   __shared__ float rows[RAMP_A][RAMP_K + 4];
   __shared__ float h[RAMP_K + RAMP_T];
   __shared__ int bad;
@@ -1324,7 +1329,7 @@ __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
   if (threadIdx.x == 0) bad = 0;
   // inputs k with 0 <= t + s - k < D for some output t of the tile
   const int kb = max(0, t0 + s - (D - 1)), ke = min(D, t0 + RAMP_T + s);
-  f4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  d4 acc[2] = {{0., 0., 0., 0.}, {0., 0., 0., 0.}};
   const int i = lane & 15, kk = lane >> 4;
   bool fin = true;
   for (int k0 = kb; k0 < ke; k0 += RAMP_K) {
@@ -1354,8 +1359,8 @@ __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
     for (int q0 = 0; q0 < steps; q0 += 8) {
 #pragma unroll
       for (int q = q0; q < q0 + 8; ++q)
-        acc[q & 1] =
-            __builtin_amdgcn_mfma_f32_16x16x4f32(rp[4 * q], hp[-4 * q], acc[q & 1], 0, 0, 0);
+        acc[q & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+            static_cast<double>(rp[4 * q]), static_cast<double>(hp[-4 * q]), acc[q & 1], 0, 0, 0);
     }
   }
   if (!fin) bad = 1;
@@ -1364,9 +1369,9 @@ __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
   if (t >= Dout) return;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const int a = a0 + 4 * kk + r;
+    const int a = a0 + kk + 4 * r;  // (the float64 products' layout)
     if (a >= A) break;
-    float v = acc[0][r] + acc[1][r];
+    float v = static_cast<float>(acc[0][r] + acc[1][r]);
     if (bad) {
       const int c = t + s;
       v = 0.0f;

@@ -419,3 +419,26 @@ def test_ramp_filter_in_place(gpu, A, D):
     bar = np.zeros((A, D))
     bar[:, : min(D, 2 * D - 1 - s)] = D * 2.0**-24 * full(np.abs(y64), np.abs(h64))
     assert np.all(np.abs(yd.cpu().numpy() - ref) <= bar + 1e-30)
+
+
+@pytest.mark.parametrize("A,D", [(1, 2), (16, 33), (17, 129), (40, 363), (5, 1001), (3, 4096)])
+def test_ramp_filter_smooth_rows(gpu, A, D):
+    """Rows whose ramp-filtered values are small against their terms: the
+    float64 sum rounded once (half a unit of the result and D float64
+    roundings of the absolute sum)."""
+    from scico_amd._lib import call
+    from scico_amd.linop.xray._fbp import filter_window, ramp_filter
+
+    s, Dout = filter_window(D)
+    h = ramp_filter(np.arange(D) - s, 1.0).astype(np.float32)
+    t = (np.arange(D) - D / 2 - 5 * np.sin(np.arange(A))[:, None]) / (D / 3)
+    y = (50.0 * np.maximum(0.0, 1.0 - t * t)).astype(np.float32)
+    hd, yd = torch.as_tensor(h, device="cuda"), torch.as_tensor(y, device="cuda")
+    out = torch.empty((A, Dout), device="cuda")
+    call("scxr_ramp_filter", A, D, Dout, s, hd.data_ptr(), yd.data_ptr(), out.data_ptr(), None,
+         torch.cuda.current_stream().cuda_stream)
+    h64, y64 = h.astype(np.float64), y.astype(np.float64)
+    ref = np.stack([np.convolve(r, h64)[s : s + Dout] for r in y64])
+    mag = np.stack([np.convolve(r, np.abs(h64))[s : s + Dout] for r in y64])
+    bar = 2.0**-24 * np.abs(ref) + 2 * D * 2.0**-53 * mag + 1e-30
+    assert np.all(np.abs(out.cpu().numpy() - ref) <= bar)
