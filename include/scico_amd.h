@@ -406,6 +406,10 @@ int32_t scxr_cconv_apgm_parts(const scxr_cconv_plan* plan);
 int64_t scxr_cconv_apgm_setup_ws(const scxr_cconv_plan* plan);
 int scxr_cconv_apgm_setup(const scxr_cconv_plan* plan, const float* y, float* gs, float* Yh,
                           double* ws, void* stream);
+/* The same, and aty = A^T y (F0 F1 floats) evaluated in float64 and rounded
+ * once; gs and Yh, or aty, may be null. */
+int scxr_cconv_apgm_setup_aty(const scxr_cconv_plan* plan, const float* y, float* gs, float* Yh,
+                              float* aty, double* ws, void* stream);
 /* Gradient step of the fused iteration; G = A^T A is the convolution by gs:
  *   gx <- G x;  u <- v + b ((1 + c) gx - c gx_prev - aty)
  * with gx_prev the gx on entry (G v for v = x + c (x - x_prev), by

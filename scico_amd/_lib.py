@@ -171,6 +171,8 @@ SIGNATURES = [
     ("scxr_cconv_apgm_setup_ws", c_int64, [c_void_p]),
     ("scxr_cconv_apgm_setup", c_int32,
      [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    ("scxr_cconv_apgm_setup_aty", c_int32,
+     [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     ("scxr_apgm_itstat", c_int32,
      [c_void_p, c_int32, c_double, c_void_p, c_int32, c_double, c_void_p, c_int32, c_void_p,
       c_void_p, c_int32, c_void_p]),

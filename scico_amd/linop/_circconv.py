@@ -124,6 +124,17 @@ class CircularConvolve(LinearOperator):
     def _adj(self, y, out=None, pred=None):
         return self._apply(y, True, out, pred)
 
+    def adj_once_rounded(self, y):
+        """``adj(y)``, for one image evaluated in float64 and rounded once."""
+        n = int(load().scxr_cconv_apgm_setup_ws(self.plan))
+        if n <= 0:
+            return self.adj(y)
+        y = dev.input_array(y, self.input_shape, "y")
+        ws, out = dev.empty((n,), np.float64), dev.empty(self.input_shape)
+        call("scxr_cconv_apgm_setup_aty", self.plan, y.data_ptr(), None, None, out.data_ptr(),
+             ws.data_ptr(), dev.stream())
+        return out
+
     def fftn(self, x, inverse=False):
         """Complex fftn (ifftn) of ``x`` over the convolution axes."""
         x = x if isinstance(x, torch.Tensor) else torch.as_tensor(np.asarray(x))

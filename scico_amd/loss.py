@@ -81,7 +81,7 @@ class SquaredL2Loss(Loss):
             g = hs.real**2 + hs.imag**2
             G = CircularConvolve(g.astype(np.complex64), A.input_shape, ndims=A.ndims,
                                  h_is_dft=True)
-            cache = (A, key, G, A.adj(self.y))
+            cache = (A, key, G, A.adj_once_rounded(self.y))
             self._gram_cache = cache
         return cache[2], cache[3]
 

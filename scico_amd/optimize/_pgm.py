@@ -242,16 +242,16 @@ class _FusedDeconv:
         f64 = dict(dtype=torch.float64, device=dev.DEVICE)
         y = dev.as_device(pgm.f.y)
         self._made_from = self._inputs(pgm)
-        # the half-grid spectra of G = A^T A and of y, formed in float64 on the
-        # device and rounded once (host FFTs took 15 ms of a new 1024 x 1024
-        # problem)
+        # the half-grid spectra of G = A^T A and of y, and A^T y, formed in
+        # float64 on the device and rounded once (host FFTs took 15 ms of a new
+        # 1024 x 1024 problem; the rounding of A^T y stays in every gradient)
         H1 = self.N // 2 + 1
         self.gs = torch.empty(self.M * H1, **f32)
         self.Yh = torch.empty(2 * self.M * H1, **f32)
         ws = torch.empty(int(lib.scxr_cconv_apgm_setup_ws(self.A.plan)), **f64)
-        call("scxr_cconv_apgm_setup", self.A.plan, y.data_ptr(), self.gs.data_ptr(),
-             self.Yh.data_ptr(), ws.data_ptr(), dev.stream())
-        self.aty = self.A.adj(y)
+        self.aty = torch.empty((self.M, self.N), **f32)
+        call("scxr_cconv_apgm_setup_aty", self.A.plan, y.data_ptr(), self.gs.data_ptr(),
+             self.Yh.data_ptr(), self.aty.data_ptr(), ws.data_ptr(), dev.stream())
         self.n_obj = int(lib.scxr_cconv_apgm_parts(self.A.plan))
         self.n_res = int(lib.scxr_tv_prox_apgm_parts(self.M, self.N))
         self.n_tv = self.n_res  # the prox kernel's TV partials, one per workgroup
