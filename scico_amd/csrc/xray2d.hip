@@ -1281,22 +1281,9 @@ __global__ __launch_bounds__(256 * ADJ_VS) __attribute__((amdgpu_waves_per_eu(4)
 // FBP row filter (_xray2d.py:187-194): the reference convolves each row
 // with the ramp taps h[0..D) by zero-padded FFT of length 2D - 1 and keeps
 // [s, 2D - 1 - s), s = (D - 1) / 2; here the same linear convolution is
-// summed directly: out[a, t] = sum_k y[a, k] h[t + s - k], a product of the
-// rows with the Toeplitz matrix of the taps, on the float64 matrix cores.
-// A workgroup takes 16 rows x 64 outputs (16 x 16 per wave) and walks the
-// inputs that reach them in chunks of 256 through LDS, four per MFMA; two
-// accumulators take alternate steps.  Bound by the matrix cores and the
-// latency of one or two waves per SIMD (a sinogram has few rows); 301 rows of
-// 595: 53.0 -> 12.8 us, 720 of 724 68.5 -> 23.5 us against one row per workgroup
-// with two LDS reads per multiply-add.  In float32 the products take 9.2 and
-// 14.7 us, but the ramp's centre tap cancels against all others on a smooth
-// row, and their order, unlike the plain one, carries the large partial sums
-// through the chain: 1.6e-5 off float64 for smooth rows of 595, the plain sums
-// 2.1e-6, these 2.5e-8 (the rounding of the result).
-// The matrix products include the zeros beyond the taps, so a tile with an
-// input that is not finite takes the plain sums, which leave them out.
-//
-// An output that overlaps the input (a row may be filtered in place) takes a
+// summed directly: out[a, t] = sum_k y[a, k] h[t + s - k].
+
+// An output that overlaps the input (a row may be filtered in place): a
 // workgroup per row, which reads all of it before it writes.
 __global__ __launch_bounds__(256) void ramp_row_kernel(const float* y, float* out,
                                                        const float* __restrict__ taps, int D,
@@ -1313,18 +1300,33 @@ __global__ __launch_bounds__(256) void ramp_row_kernel(const float* y, float* ou
   }
 }
 
+// Otherwise a product of the rows with the Toeplitz matrix of the taps, on the
+// float64 matrix cores.  A workgroup takes 16 rows x 64 outputs (16 x 16 per
+// wave, of two halves of the workgroup that share the inputs) and walks the
+// inputs that reach them in chunks of 256 through LDS, four per MFMA; two
+// accumulators take alternate steps.  Bound by the latency of a few waves per
+// SIMD (a sinogram has few rows) and, from a thousand rows on, the matrix
+// cores; 301 rows of 595: 53.0 -> 9.9 us (12.8 without the halves), 720 of 724
+// 68.5 -> 20.5 us against one row per workgroup with two LDS reads per
+// multiply-add.  In float32 the products took 9.2 and 14.7 us, but the ramp's
+// centre tap cancels against all others on a smooth row, and their order,
+// unlike the plain one, carries the large partial sums through the chain:
+// 1.6e-5 off float64 for smooth rows of 595, the plain sums 2.1e-6, these
+// 2.5e-8 (the rounding of the result).
+// The matrix products include the zeros beyond the taps, so a tile with an
+// input that is not finite takes the plain sums, which leave them out.
 constexpr int RAMP_K = 256, RAMP_T = 64, RAMP_A = 16;
 
-__global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
+__global__ __launch_bounds__(512) void ramp_kernel(const float* __restrict__ y,
                                                    float* __restrict__ out,
                                                    const float* __restrict__ taps, int A, int D,
                                                    int Dout, int s, const int32_t* pred) {
   if (pred_off(pred)) return;
   typedef double d4 __attribute__((ext_vector_type(4)));
-  __shared__ float rows[RAMP_A][RAMP_K + 4];
+  __shared__ __align__(16) float rows[RAMP_A][RAMP_K + 4];
   __shared__ float h[RAMP_K + RAMP_T];
   __shared__ int bad;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = (threadIdx.x >> 6) & 3, half = threadIdx.x >> 8, lane = threadIdx.x & 63;
   const int a0 = blockIdx.y * RAMP_A, t0 = blockIdx.x * RAMP_T;
   if (threadIdx.x == 0) bad = 0;
   // inputs k with 0 <= t + s - k < D for some output t of the tile
@@ -1334,19 +1336,21 @@ __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
   bool fin = true;
   for (int k0 = kb; k0 < ke; k0 += RAMP_K) {
     __syncthreads();
-    float v[RAMP_A];  // all loads in flight at once
+    constexpr int NR = RAMP_A / 2;  // rows of each half of the workgroup
+    const int e = threadIdx.x & 255, r0 = half * NR;
+    float v[NR];  // all loads in flight at once
 #pragma unroll
-    for (int r = 0; r < RAMP_A; ++r) {
-      const int a = a0 + r, k = k0 + threadIdx.x;
+    for (int r = 0; r < NR; ++r) {
+      const int a = a0 + r0 + r, k = k0 + e;
       v[r] = (a < A && k < ke) ? y[static_cast<size_t>(a) * D + k] : 0.0f;
     }
 #pragma unroll
-    for (int r = 0; r < RAMP_A; ++r) {
+    for (int r = 0; r < NR; ++r) {
       fin = fin && fabsf(v[r]) <= 3.402823466e38f;
-      rows[r][threadIdx.x] = v[r];
+      rows[r0 + r][e] = v[r];
     }
     // h[e] = tap of distance t - k = e - (RAMP_K - 1) from the chunk's origin
-    for (int e = threadIdx.x; e < RAMP_K + RAMP_T; e += 256) {
+    for (int e = threadIdx.x; e < RAMP_K + RAMP_T; e += 512) {
       const int m = t0 - k0 + s + e - (RAMP_K - 1);
       const float g = m >= 0 && m < D ? taps[m] : 0.0f;
       fin = fin && fabsf(g) <= 3.402823466e38f;
@@ -1355,8 +1359,9 @@ __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
     __syncthreads();
     const float* hp = h + 16 * wave + i + (RAMP_K - 1) - kk;
     const float* rp = &rows[i][kk];
-    const int steps = (min(RAMP_K, ke - k0) + 3) / 4;  // rounded up to 8 below: rows are 0 there
-    for (int q0 = 0; q0 < steps; q0 += 8) {
+    // each half takes half of the steps, rounded up to 8: rows are 0 beyond
+    const int steps = (min(RAMP_K, ke - k0) + 63) / 64 * 8;
+    for (int q0 = half * steps; q0 < (half + 1) * steps; q0 += 8) {
 #pragma unroll
       for (int q = q0; q < q0 + 8; ++q)
         acc[q & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(
@@ -1365,13 +1370,18 @@ __global__ __launch_bounds__(256) void ramp_kernel(const float* __restrict__ y,
   }
   if (!fin) bad = 1;
   __syncthreads();
+  double(*other)[4] = reinterpret_cast<double(*)[4]>(&rows[0][0]) + 64 * wave + lane;
+  if (half == 1)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) (*other)[r] = acc[0][r] + acc[1][r];
+  __syncthreads();
   const int t = t0 + 16 * wave + i;
-  if (t >= Dout) return;
+  if (half == 1 || t >= Dout) return;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int a = a0 + kk + 4 * r;  // (the float64 products' layout)
     if (a >= A) break;
-    float v = static_cast<float>(acc[0][r] + acc[1][r]);
+    float v = static_cast<float>(acc[0][r] + acc[1][r] + (*other)[r]);
     if (bad) {
       const int c = t + s;
       v = 0.0f;
@@ -1874,7 +1884,7 @@ int scxr_ramp_filter(int32_t A, int32_t D, int32_t Dout, int32_t shift, const fl
     SCXR_LAUNCHED("ramp filter in place");
     return SCXR_OK;
   }
-  hipLaunchKernelGGL(ramp_kernel, dim3(ceil_div(Dout, RAMP_T), ceil_div(A, RAMP_A)), dim3(256), 0,
+  hipLaunchKernelGGL(ramp_kernel, dim3(ceil_div(Dout, RAMP_T), ceil_div(A, RAMP_A)), dim3(512), 0,
                      as_stream(stream), y, out, taps, A, D, Dout, shift, pred);
   SCXR_LAUNCHED("ramp filter");
   return SCXR_OK;
