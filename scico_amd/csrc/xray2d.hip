@@ -950,7 +950,12 @@ __device__ __forceinline__ void fwd_group(const float* __restrict__ im,
 // 256^2 with 180 views, 4 parts).  The parts cross between workgroups, so
 // they are stored and loaded at agent scope, past the XCD's cache, and every
 // wave's stores are complete before the workgroup is counted.  (A release
-// fence instead writes the whole L2 back in every workgroup: 130 us.)
+// fence instead writes the whole L2 back in every workgroup: 130 us.)  This
+// leans on the AMDGPU memory model for gfx942 and gfx950, where a monotonic
+// agent-scope store or load carries sc1 and is performed past the XCD's L2
+// and vmcnt counts a store until then: the release that C++ asks for before
+// the count is the waitcnt alone, as long as every part store is such a store
+// (fwd_group's `part` branch) and every part load such a load.
 template <int V, int CH, bool FR, bool STG>
 __global__ __launch_bounds__(64 * FWD_WAVES) void fwd_kernel(const float* __restrict__ im,
                                                   const float* __restrict__ imT,

@@ -1764,8 +1764,9 @@ int create(Plan& p, int X, int Y, int Z, int V, const float* mats, int D0, int D
     // Staged adjoint: a 4 x 8 tile's rows per view, at most
     // ceil(3 |a| + 7 |b| + rounding) + 2 (the corner bins' spread plus the
     // right-hand tap), must fit ADJ_NW.  The rounding margin covers the
-    // float32 evaluation of the corner centres (a few ulps of |P|).  The
-    // kernel packs two detector-row indices into 16-bit fields: U < 65536.
+    // float32 evaluation of the corner centres (a few ulps of |P|); beyond
+    // 65536 detector rows, where those reach a tap, rows are read from global
+    // memory.
     p.adj_staged = !(allow_slice & 2) && p.U < 65536;
     for (int v = 0; v < V && p.adj_staged; ++v) {
       const double a = std::fabs(static_cast<double>(g[v].x)),
