@@ -31,6 +31,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <cstring>
@@ -1412,26 +1413,54 @@ static int dev_alloc(void** ptr, size_t bytes) {
   return SCXR_OK;
 }
 
-// Where the windows in LDS are the faster path (all figures of graph replays;
-// a flag forces either).  The forward takes three launches and a workspace:
-// its time meets the gather's at about 280000 voxels times views (16^3 with
-// 60 views 20.9 against 21.1 us, 32^3 with 8 19.8 against 20.2, 64^3 with one
-// 23.7 against 23.5; 16^3 with 10 17.1 against 10.7, 32^3 with 20 27 against
-// 20.6 us).
-static bool splat_pays(const Plan& p) {
-  return static_cast<double>(p.X) * p.Y * p.Z * p.V >= 280e3;
+// Where the windows in LDS are the faster path: both sides' times in us,
+// fitted to graph replays over volumes of 8^3 to 256^3 and thin ones, few and
+// many views, detectors smaller and larger than the volume (most within a
+// fifth).  A flag forces either.
+//
+// The gather of the forward pays for every detector pixel, for the candidate
+// voxels of the pixels that the volume covers, and for the march of a pixel
+// along its planes; the windows take two or three launches and a workspace,
+// and at these sizes little else.  (Windows against gather: 16^3 with 10 views
+// 18 against 12, with 60 views 22 against 22, 64^3 with one view 25 against 25,
+// 40^3 with 6 23 against 28; on a detector of 500^2 pixels 32^3 with 3 views 19
+// against 81; 512 x 512 x 1 with one view 36 against 531.)
+static bool splat_pays(const Plan& p, const std::vector<float>& m, const std::vector<GenView>& gv) {
+  const int dims[3] = {p.X, p.Y, p.Z};
+  double pixels = 0.0, candidates = 0.0;
+  int planes = 0;
+  bool copy = false;
+  for (int v = 0; v < p.V; ++v) {
+    const int na = dims[gv[v].a];
+    double e[2];
+    for (int r = 0; r < 2; ++r)
+      e[r] = std::fabs(mat(m, v, r, 0)) * p.X + std::fabs(mat(m, v, r, 1)) * p.Y +
+             std::fabs(mat(m, v, r, 2)) * p.Z + 2.0;
+    pixels += 1e-6 * p.D0 * p.D1 * (45.0 + na);
+    candidates += 1e-6 * std::min<double>(p.D0, e[0]) * std::min<double>(p.D1, e[1]) * na *
+                  gv[v].nb * gv[v].nc;
+    planes = std::max(planes, na);
+    copy = copy || gv[v].a == 2;
+  }
+  const double gather = 6.0 + pixels + std::max(0.2 * planes, candidates + 0.1 * planes);
+  return gather >= 16.0 + 0.07 * planes + (copy ? 3.5 : 0.0);
 }
 
-// The adjoint's waves walk their views one after the other, and with fewer
-// than 32 views a block has two of them: below some work that chain is longer
-// than the gather's (16^3 with 30 views 16.0 against 10.4 us, 32^3 with 31 17.0
-// against 10.3; 40^3 with 31 17.1 against 16.5, 48^3 with 31 17.1 against 17.6,
-// 64^3 with 5 7.2 against 8.1 us; from 32 views on 8^3 takes 9.6 against 10.7
-// us).  With a single view half the waves have none, at any size (256^3 87.6
-// against 68.1 us).
+// The adjoint's waves walk their share of the views one after the other (half
+// of them below 32 views, a quarter from there on), and a block that the
+// volume fills in part costs as much as a whole one; the gather's threads walk
+// all views, at a rate that depends on how many of a wave's voxels lie along
+// the fast axis.  (Tiles against gather: 16^3 with 30 views 16.0 against 10.4,
+// with 32 9.9 against 10.9; 64^3 with 2 views 5.6 against 4.5, with 5 7.2 against
+// 8.1; 256^3 with one view 88 against 68, with two 91 against 149; 512 x 512 x 1
+// with 40 views 52 against 24, 512 x 512 x 4 51 against 74.)
 static bool adj_tiles_pay(const Plan& p) {
-  const double work = static_cast<double>(p.X) * p.Y * p.Z * p.V;
-  return p.V >= 32 || (p.V > 1 && work >= 1.2e6 + 3e4 * p.V);
+  const double n = static_cast<double>(p.X) * p.Y * p.Z, V = p.V;
+  const double blocks = std::ceil(p.X / 8.0) * std::ceil(p.Y / 8.0) * std::ceil(p.Z / 8.0);
+  const double rate = p.Z < 8 ? 1.85 : p.Z < 32 ? 2.5 : std::min(p.X, p.Y) < 8 ? 5.5 : 4.3;
+  const double tiles = std::max(2.6 + (V >= 32 ? 0.217 : 0.445) * V,
+                                3.5 + 1e-3 * blocks * (2.0 + 0.26 * V));
+  return tiles <= std::max(1.9 + 0.28 * V, 2.0 + 1e-6 * rate * n * V);
 }
 
 // Detector coordinates of every voxel centre stay below this (float32
@@ -1748,7 +1777,7 @@ int create(Plan& p, int X, int Y, int Z, int V, const float* mats, int D0, int D
     std::vector<float> zt;
     if (!(allow_slice & 4) && gen_in_range(p, m)) {
       const bool always = allow_slice & 8;
-      p.splat = (always || splat_pays(p)) && build_splat(p, m, gv, views, items);
+      p.splat = (always || splat_pays(p, m, gv)) && build_splat(p, m, gv, views, items);
       p.adj_tiled = (always || adj_tiles_pay(p)) && build_adj_tiles(p, m, zt);
     }
     return upload_tables(p, m, gv, views, items, zt);

@@ -311,12 +311,13 @@ def test_general_windows_small(gpu, case):
     assert max(e) <= 1e-5 and H._ws_floats > 0 and G._ws_floats == 0
 
 
-@pytest.mark.parametrize("n,views,splat", [(16, 1, False), (23, 23, False), (23, 24, True),
-                                           (64, 1, False), (66, 1, True), (66, 40, True)])
-def test_general_windows_rule(gpu, n, views, splat):
-    """The default takes the forward's windows from 280000 voxels times views
-    on, and is the path that it takes, bit for bit."""
-    shape, det = (n, n, n), (n + 8, n)
+@pytest.mark.parametrize("shape,det,views,splat", [
+    ((16, 16, 16), (24, 16), 1, False), ((23, 24, 25), (40, 42), 4, False),
+    ((66, 66, 66), (74, 66), 40, True), ((96, 96, 96), (120, 120), 3, True),
+    ((32, 32, 32), (500, 500), 3, True), ((256, 256, 1), (300, 300), 4, True)])
+def test_general_windows_rule(gpu, shape, det, views, splat):
+    """The default takes the forward's windows where the gather has more to
+    do, and is the path that it takes, bit for bit."""
     M = _tilted(shape, det, "XY", views)
     H = XRayTransform3D(shape, M, det)
     W = XRayTransform3D(shape, M, det)
