@@ -178,6 +178,7 @@ __device__ __forceinline__ float rlf(float v, int lane) {
 // ------------------------------------------------------ slice kernels --
 
 // Bin group and view group of a workgroup of the slice forward.
+template <bool UP>
 __device__ __forceinline__ void slice_block(int& bg, int& vg) {
   // Workgroup order: consecutive workgroups go to the 8 XCDs in turn; each
   // XCD is given a contiguous run of an order that takes the view groups
@@ -186,12 +187,16 @@ __device__ __forceinline__ void slice_block(int& bg, int& vg) {
   // (neighbouring views' strips share most of their pixel rows, so they
   // share its L2) across all bin groups (whose strips differ in length,
   // so every XCD gets a similar share of work).  A bijection of the grid.
-  // (An eighth rounded up: rounded down, a run ends in the long strips of one
-  // block more; 256^3 with 360 and 180 views 1256, 741 -> 1196, 698 us.)
+  // (UP: an eighth rounded up: rounded down, a run ends in the long strips of
+  // one block more; fwd_slice16_kernel at 256^3 with 360 and 180 views 1256, 741
+  // -> 1196, 698 us, two slots at a spacing of 0.57 with 180 and 45 views 812,
+  // 447 -> 750, 418.  Three slots a bin group are 3 to 8 % slower with it at a
+  // spacing of 0.35, 0 to 7 % faster or slower at 0.4 to 0.5, and keep the
+  // eighth rounded down.)
   const int GX = gridDim.x, GY = gridDim.y, G = GX * GY, G8 = (G / 8) * 8;
   int L = blockIdx.y * GX + blockIdx.x;
   if (L < G8) L = (L % 8) * (G8 / 8) + L / 8;
-  const int VB = (GY + 7) / 8;  // view groups per block
+  const int VB = UP ? (GY + 7) / 8 : max(GY / 8, 1);  // view groups per block
   const int blk = L / (GX * VB);
   const int nb = min(VB, GY - blk * VB);  // the last block may be short
   const int within = L - blk * GX * VB;
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(256) void fwd_slice_kernel(const float4* __restrict
   constexpr int BIG = INT_MAX / 2;
   const int lane = threadIdx.x & 63;
   int bg, vg;
-  slice_block(bg, vg);
+  slice_block<(SPG < 3)>(bg, vg);
   const int v = vg * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (v >= V) return;
   const int u0 = bg * FB;
@@ -363,7 +368,7 @@ __global__ __launch_bounds__(256) void fwd_slice16_kernel(
   __shared__ int4 table[4][64];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int bg, vg;
-  slice_block(bg, vg);
+  slice_block<true>(bg, vg);
   const int v = vg * 4 + w;
   if (v >= V) return;
   const int u0 = bg * FBL;
